@@ -1573,8 +1573,8 @@ RTC_API void rtcgOccluded1MAsync(RTCScene scene, const RTCIntersectContext* cont
 }
 
 // No reference counterpart: rtcgIntersect1MAsync / rtcgOccluded1MAsync for
-// callers that cannot allocate. The kernels' ray counter and error bits are
-// words 0 and 1 of the GPU's fixed scratch array; nothing here allocates
+// callers that cannot allocate. The kernels' ray counters and error bits are
+// in the GPU's fixed scratch array; nothing here allocates
 // device memory or creates a stream.
 RTC_API void rtcgQuery1MNoAlloc(RTCScene scene, const RTCIntersectContext* context, void* d_rays, unsigned int M,
                                 size_t byteStride, int occluded, void* hipStream) {
@@ -2131,7 +2131,7 @@ RTC_API void rtcgSplitModelCollectInstanced(RTCGSplitModel model, RTCScene scene
   copy.reserve((size_t)M * byteStride);
   RTG_HIP(hipMemcpyAsync(copy.ptr, d_rays, (size_t)M * byteStride, hipMemcpyDeviceToDevice, t.stream));
   m->m.visits.reserve((size_t)nn * 4);
-  m->m.counts.reserve(256);
+  m->m.counts.reserve(rtg::COUNTER_BYTES);
   RTG_HIP(hipMemsetAsync(m->m.visits.ptr, 0, (size_t)nn * 4, t.stream));
   uint32_t* vis = m->m.visits.as<uint32_t>();
   rtg::launch_trace_inst_counted(v, copy.ptr, M, byteStride, t.errword.as<uint32_t>(), m->m.counts.as<uint32_t>(),
@@ -2362,7 +2362,7 @@ RTC_API void rtcgTraceBatch(const RTCGBatchItem* items, unsigned int numItems, i
   d->activate();
   ThreadDev& t = d->td();
   t.batch.reserve(pb.items.size() * sizeof(rtg::BatchItem));
-  t.batch_counter.reserve(256);
+  t.batch_counter.reserve(rtg::COUNTER_BYTES);
   RTG_HIP(hipMemcpyAsync(t.batch.ptr, pb.items.data(), pb.items.size() * sizeof(rtg::BatchItem), hipMemcpyHostToDevice,
                          t.stream));
   rtg::launch_trace_batch(pb.sc, t.batch.as<rtg::BatchItem>(), (uint32_t)pb.items.size(), pb.total, occluded != 0,
@@ -2406,7 +2406,7 @@ RTC_API float rtcgAutotuneBatch(const RTCGBatchItem* items, unsigned int numItem
   }
   table.reserve(wi.size() * sizeof(rtg::BatchItem));
   RTG_HIP(hipMemcpyAsync(table.ptr, wi.data(), wi.size() * sizeof(rtg::BatchItem), hipMemcpyHostToDevice, t.stream));
-  t.batch_counter.reserve(256);
+  t.batch_counter.reserve(rtg::COUNTER_BYTES);
   auto time_launch = [&](const rtg::TraceParams& c) {
     float total = 0.0f;
     const int reps = 2;
@@ -2477,7 +2477,7 @@ RTC_API RTCGBatchGraph rtcgNewBatchGraph(const RTCGBatchItem* items, unsigned in
       g->slots.push_back(s->slot);
     }
     g->table.reserve(pb.items.size() * sizeof(rtg::BatchItem) + 16);
-    g->counter.reserve(256);
+    g->counter.reserve(rtg::COUNTER_BYTES);
     g->err.reserve(256);
     if (!pb.items.empty())
       RTG_HIP(hipMemcpyAsync(g->table.ptr, pb.items.data(), pb.items.size() * sizeof(rtg::BatchItem),

@@ -17,7 +17,7 @@ struct TraceParams {
   uint32_t sort_min = 65536;  // smallest stream that is reordered
   int persistent = 1;       // persistent waves pulling rays from a counter
   // Idle lanes of a wave that trigger a refill. A refill stalls the wave
-  // for one ray-record load (and, once per 256 rays, the global counter
+  // for one ray-record load (and, once per RAY_RUN rays, a global counter's
   // atomic); on the 2^20-triangle soup with 2^24 incoherent rays 10 gave
   // 1936 Mrays/s closest hit (8-14 within 1 %, 24: 1854, 32: 1818) and 24
   // gave 3795 Mrays/s occlusion (48: 3339).
@@ -32,8 +32,13 @@ struct TraceParams {
   // closest hit (speculative node visits before a pending leaf's hits).
   int dual = 2;
   int cus = 256;            // compute units (set from the device)
-  int blocks_per_cu = 8;    // resident 256-thread blocks per compute unit for the persistent grid
+  int blocks_per_cu = 8;    // 256-thread blocks per compute unit for the persistent grid (at most those resident)
 };
+
+// Ray counters of a persistent launch, one for each XCD, 256 B apart.
+constexpr uint32_t COUNTERS_LOG2 = 3, COUNTERS = 1u << COUNTERS_LOG2;
+constexpr uint32_t COUNTER_STRIDE = 64;  // in words
+constexpr size_t COUNTER_BYTES = COUNTERS * COUNTER_STRIDE * 4;
 
 // One ray stream of a batched traversal (device memory).
 struct BatchItem {
@@ -57,7 +62,7 @@ struct RaySorter {
 // triangle tests. err receives bit 0 on a traversal stack overflow.
 // node_visits (optional, with the counters): one atomic increment per node
 // visit, indexed like the QNode8 array.
-// counter (optional): the persistent kernel's ray counter (one device word);
+// counter (optional): the persistent kernel's ray counters (COUNTER_BYTES);
 // without it the sorter's is used, and with neither the grid covers every ray.
 void launch_trace(const DevScene& sc, void* rays, uint32_t M, uint64_t stride, bool occluded, uint32_t inst_id,
                   uint32_t* cnt_nodes, uint32_t* cnt_tris, uint32_t* err, hipStream_t s,
@@ -66,15 +71,15 @@ void launch_trace(const DevScene& sc, void* rays, uint32_t M, uint64_t stride, b
 
 // One persistent launch over several ray streams of scenes that share sc's
 // node and triangle arrays (a batched build). items (device memory) sorted
-// by first; M = total rays. Records traced in place. counter: one device
-// word, cleared by a kernel (the sequence can be captured in a hipGraph).
+// by first; M = total rays. Records traced in place. counter:
+// COUNTER_BYTES of device memory, cleared by a kernel (the sequence can be captured in a hipGraph).
 void launch_trace_batch(const DevScene& sc, const BatchItem* items, uint32_t nitems, uint32_t M, bool occluded,
                         bool aligned, uint32_t* err, uint32_t* counter, hipStream_t s, const TraceParams& tp);
 
 // Two-level traversal of a scene with instances (top tree over InstRec
 // leaves, object trees in top.objects); otherwise as launch_trace. ctx_inst
-// is the query context's instID[0]; counter (one device word) or, if null,
-// the sorter's supplies the ray counter.
+// is the query context's instID[0]; counter (COUNTER_BYTES) or, if null,
+// the sorter's supplies the ray counters.
 void launch_trace_inst(const DevTop& top, void* rays, uint32_t M, uint64_t stride, bool occluded, uint32_t ctx_inst,
                        uint32_t* err, hipStream_t s, const TraceParams& tp, RaySorter* sorter,
                        uint32_t* counter = nullptr);
@@ -87,10 +92,10 @@ void launch_trace_inst_counted(const DevTop& top, void* rays, uint32_t M, uint64
                                uint32_t* counter, uint32_t* top_visits, uint32_t* obj_visits, uint32_t target_obj,
                                hipStream_t s, const TraceParams& tp);
 
-// Scratch of the no-allocation queries: word 0 is the persistent kernel's
-// ray counter, word 1 the traversal error bits; one fixed array per GPU
-// (NOALLOC_SCRATCH_WORDS words), held until the process ends.
-constexpr uint32_t NOALLOC_SCRATCH_WORDS = 64;
+// Scratch of the no-allocation queries: the persistent kernel's ray counters
+// (the words at multiples of COUNTER_STRIDE), with the traversal error bits
+// in word 1; one fixed array per GPU, held until the process ends.
+constexpr uint32_t NOALLOC_SCRATCH_WORDS = COUNTERS * COUNTER_STRIDE;
 constexpr uint32_t NOALLOC_MAX_RAYS = 1u << 31;  // the counter word's range, with room for every wave's overshoot
 // Looks up the device address of this GPU's copy of the scratch array; the
 // GPU `ordinal` must be current. Once per GPU (later calls return at once);

@@ -23,10 +23,12 @@
 // 2^-12 relative).
 #include "trace.h"
 
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
 
-// Scratch of the no-allocation queries (word 0: ray counter, word 1: error
-// bits), one copy per GPU. In host code this name is a host-side stand-in,
+// Scratch of the no-allocation queries (ray counters, with the error bits
+// in word 1), one copy per GPU. In host code this name is a host-side stand-in,
 // not a device address: kernels get the address noalloc_setup() looked up.
 static __device__ __align__(256) uint32_t scratch[rtg::NOALLOC_SCRATCH_WORDS];
 
@@ -137,29 +139,53 @@ struct RingStack<0> {
   __device__ inline void clear() { sp = 0; }
 };
 
-// Rays of a persistent wave come from a private run of consecutive slots
-// that the wave takes from the global counter CHUNK at a time, so a refill
-// costs a global atomic only once every CHUNK rays (the atomic's latency
-// stalls the whole wave). Every lane computes the same values (all inputs
-// are wave-uniform), so the state needs no broadcast after the one atomic.
+// How a persistent launch shares out its M rays: in `count` runs of RAY_RUN
+// consecutive slots, dealt in groups of 1 << qs to as many queues (one for each
+// XCD: blocks are dealt to the XCDs in turn). Run j of queue q is run
+// (j << qs) + ((q + j) & ((1 << qs) - 1)): the turn keeps a queue from getting
+// one column of an image.
+struct RayRuns {
+  uint32_t count, qs;
+};
+
+// Slots of a run: one refill of a whole wave. Longer runs need fewer atomics
+// but leave more to the last waves: with one counter for all, 256 gave 573 us
+// and 64 gave 616 us for 2 M camera rays on a 2.1 M triangle terrain (the
+// atomics on one address pass one at a time), with a counter for each XCD 64
+// gives 430 us (128: 473, 32: 451, 16: 517). 2^24 incoherent rays in the
+// 2^20-triangle soup take 7.22 ms at 64 and 7.43 at 256, two million rays
+// through 10,000 instances and their shadow rays 3.56 ms against 4.07.
+constexpr uint32_t RAY_RUN = 64;
+
+// A persistent wave's rays. Its first run is its own (the wave's place in its
+// queue), the next ones come from its queue's counter, so a refill costs a
+// global atomic only once every RAY_RUN rays (its latency stalls the whole
+// wave), and a stream that the first runs cover needs no counter. Every lane
+// computes the same values (all inputs are wave-uniform), so the state needs
+// no broadcast.
 struct WavePool {
-  static constexpr uint32_t CHUNK = 256;
-  uint32_t lb = 0, le = 0;  // unassigned slots [lb, le) of the current run
-  bool gdone = false;       // the global counter has passed M
+  uint32_t lb, le;  // unassigned slots [lb, le) of the current run
+  bool gdone;       // the wave's queue has no more runs
+  __device__ inline void run(const RayRuns& rr, uint32_t M, uint32_t j, uint32_t& nb, uint32_t& ne) {
+    const uint32_t k = (j << rr.qs) + ((blockIdx.x + j) & ((1u << rr.qs) - 1u));
+    gdone = ((j + 1u) << rr.qs) >= rr.count;
+    nb = k < rr.count ? k * RAY_RUN : M;
+    ne = M - nb < RAY_RUN ? M : nb + RAY_RUN;
+  }
+  __device__ inline void init(const RayRuns& rr, uint32_t M) {
+    run(rr, M, (blockIdx.x >> rr.qs) * (TB / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lb, le);
+    gdone = gdone || ((gridDim.x * (TB / 64)) >= rr.count);
+  }
   // Hands out nidle slots (idle lane `rank` gets the rank-th); returns this
   // lane's slot or 0xffffffff when the rays have run out.
-  __device__ inline uint32_t take(uint32_t* next, uint32_t M, int nidle, uint32_t rank, int lane) {
+  __device__ inline uint32_t take(const RayRuns& rr, uint32_t* next, uint32_t M, int nidle, uint32_t rank, int lane) {
     const uint32_t have = le - lb;
     uint32_t nb = 0, ne = 0;
     if (have < (uint32_t)nidle && !gdone) {
       uint32_t g = 0;
-      if (lane == 0) g = atomicAdd(next, CHUNK);
-      g = __shfl(g, 0, 64);
-      if ((uint64_t)g + CHUNK >= M) gdone = true;
-      if (g < M) {
-        nb = g;
-        ne = (uint64_t)g + CHUNK < M ? g + CHUNK : M;
-      }
+      if (lane == 0) g = atomicAdd(next + (blockIdx.x & ((1u << rr.qs) - 1u)) * COUNTER_STRIDE, 1u);
+      g = (uint32_t)__builtin_amdgcn_readfirstlane((int)g);
+      run(rr, M, (gridDim.x >> rr.qs) * (TB / 64) + g, nb, ne);
     }
     uint32_t slot = 0xffffffffu;
     if (rank < have) slot = lb + rank;
@@ -635,7 +661,7 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
                                                 uint32_t inst_id, uint32_t* __restrict__ cnt_nodes,
                                                 uint32_t* __restrict__ cnt_tris, uint32_t* __restrict__ err,
                                                 const uint32_t* __restrict__ perm, uint32_t* __restrict__ next,
-                                                int refill_min, uint32_t* node_visits,
+                                                int refill_min, RayRuns rr, uint32_t* node_visits,
                                                 const BatchItem* __restrict__ items, uint32_t nitems) {
   const int lane = threadIdx.x & 63;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -653,6 +679,7 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
   uint32_t lroot = 0;       // BATCH: its scene's root
   bool active = false, occluded = false, pool_empty = false;
   WavePool pool;
+  pool.init(rr, M);
   // a ray touches each node and triangle record at most once
   // (node and triangle counts are below 2^31 each, so the bound fits 32 bits)
   const uint32_t max_iter = sc.num_nodes + sc.num_tris + 16u;
@@ -664,7 +691,7 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
       const uint64_t idle = __ballot(!active);
       const int nidle = __popcll(idle);
       if (nidle >= refill_min) {
-        const uint32_t slot = pool.take(next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
+        const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
         pool_empty = pool.empty();
         if (!active) {
           if (slot != 0xffffffffu) {
@@ -830,7 +857,7 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
                                                                     uint32_t* __restrict__ err,
                                                                     const uint32_t* __restrict__ perm,
                                                                     uint32_t* __restrict__ next, int refill_min,
-                                                                    uint32_t* node_visits) {
+                                                                    RayRuns rr, uint32_t* node_visits) {
   constexpr uint32_t NONE_REF = 0xffffffffu;
   const int lane = threadIdx.x & 63;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -846,6 +873,7 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
   uint32_t cur = NONE_REF, tri = NONE_REF, ray = 0, nvis = 0, ntri = 0;
   bool active = false, occluded = false, pool_empty = false;
   WavePool pool;
+  pool.init(rr, M);
   // (node and triangle counts are below 2^31 each, so the bound fits 32 bits)
   const uint32_t max_iter = sc.num_nodes + sc.num_tris + 16u;
   uint32_t iter = 0;
@@ -855,7 +883,7 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
       const uint64_t idle = __ballot(!active);
       const int nidle = __popcll(idle);
       if (nidle >= refill_min) {
-        const uint32_t slot = pool.take(next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
+        const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
         pool_empty = pool.empty();
         if (!active && slot != 0xffffffffu) {
           ray = perm ? perm[slot] : slot;
@@ -1005,7 +1033,7 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
 template <bool OCCLUDED, bool ALIGNED, bool CNT = false>
 __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restrict__ rays, uint32_t M,
                                                       uint64_t stride, uint32_t ctx_inst, uint32_t* __restrict__ err,
-                                                      uint32_t* __restrict__ next, int refill_min,
+                                                      uint32_t* __restrict__ next, int refill_min, RayRuns rr,
                                                       uint32_t* __restrict__ top_visits = nullptr,
                                                       uint32_t* __restrict__ obj_visits = nullptr,
                                                       uint32_t target_obj = 0xffffffffu) {
@@ -1034,6 +1062,7 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
   bool orobust = false;
   bool active = false, occluded = false, pool_empty = false;
   WavePool pool;
+  pool.init(rr, M);
   uint64_t iter = 0;
 
   while (true) {
@@ -1042,7 +1071,7 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
       const uint64_t idle = __ballot(!active);
       const int nidle = __popcll(idle);
       if (nidle >= refill_min) {
-        const uint32_t slot = pool.take(next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
+        const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
         pool_empty = pool.empty();
         if (!active) {
           if (slot != 0xffffffffu) {
@@ -1243,7 +1272,7 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
   }
 }
 
-__global__ void k_zero_u32(uint32_t* p) { *p = 0u; }
+__global__ void k_zero_counters(uint32_t* p) { p[threadIdx.x * COUNTER_STRIDE] = 0u; }
 
 // Sort key of a ray: 30-bit Morton code of its origin in the scene box
 // (origins outside are clamped to the box faces); inactive rays sort last.
@@ -1265,6 +1294,35 @@ __global__ __launch_bounds__(TB) void k_ray_keys(const char* __restrict__ rays, 
   vals[i] = i;
 }
 
+// Grid and runs of a persistent launch over M rays, and whether it needs the
+// counters (runs beyond every wave's first).
+struct RayPlan {
+  dim3 grid;
+  RayRuns runs;
+  bool counter;
+};
+
+RayPlan ray_plan(uint32_t M, int resident, const TraceParams& tp) {
+  // no more blocks than are resident at once: a wave's own first run must not
+  // wait for another wave to end
+  const uint32_t per_cu = (uint32_t)std::max(1, std::min(tp.blocks_per_cu, resident));
+  const uint32_t runs = div_up(M, RAY_RUN);
+  uint32_t blocks = std::min((uint32_t)tp.cus * per_cu, div_up(runs, TB / 64));
+  const uint32_t qs = blocks >= COUNTERS ? COUNTERS_LOG2 : 0u;  // (a grid is a multiple of its queues)
+  blocks = (((blocks - 1u) >> qs) + 1u) << qs;
+  return {dim3(blocks), {runs, qs}, (uint64_t)blocks * (TB / 64) < runs};
+}
+
+// Resident blocks per compute unit of a kernel (asked once per kernel).
+template <auto KERNEL>
+int resident_blocks() {
+  static const int n = [] {
+    int b = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, KERNEL, TB, 0) == hipSuccess && b > 0 ? b : TRACE_MIN_BLOCKS;
+  }();
+  return n;
+}
+
 struct LaunchArgs {
   DevScene sc;
   char* rays;
@@ -1277,31 +1335,37 @@ struct LaunchArgs {
   int refill;
   uint32_t* node_visits;
   bool persistent;
-  dim3 grid, pgrid;
-  int lds_slots;
+  const TraceParams* tp;
   hipStream_t s;
   bool dual;
 };
 
 template <bool OCC, bool AL, bool CNT, int SL, bool PL>
 void launch_one(const LaunchArgs& a) {
-  if (a.persistent && a.dual)  // (its ring has 8 slots whatever SL is)
-    hipLaunchKernelGGL((k_trace_d<OCC, AL, CNT, PL>), a.pgrid, dim3(TB), 0, a.s, a.sc, a.rays, a.M, a.stride,
-                       a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.counter, a.refill, a.node_visits);
-  else if (a.persistent)
-    hipLaunchKernelGGL((k_trace_p<OCC, AL, CNT, SL, PL>), a.pgrid, dim3(TB), 0, a.s, a.sc, a.rays, a.M, a.stride,
-                       a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.counter, a.refill, a.node_visits,
-                       nullptr, 0u);
+  if (!a.persistent) {
+    hipLaunchKernelGGL((k_trace<OCC, AL, CNT, SL, PL>), dim3(div_up(a.M, TB)), dim3(TB), 0, a.s, a.sc, a.rays, a.M,
+                       a.stride, a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.node_visits);
+    return;
+  }
+  // (the dual-cursor kernel's ring has 8 slots whatever SL is)
+  const RayPlan p = ray_plan(
+      a.M, a.dual ? resident_blocks<k_trace_d<OCC, AL, CNT, PL>>() : resident_blocks<k_trace_p<OCC, AL, CNT, SL, PL>>(), *a.tp);
+  if (p.counter) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(COUNTERS), 0, a.s, a.counter);
+  if (a.dual)
+    hipLaunchKernelGGL((k_trace_d<OCC, AL, CNT, PL>), p.grid, dim3(TB), 0, a.s, a.sc, a.rays, a.M, a.stride,
+                       a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.counter, a.refill, p.runs,
+                       a.node_visits);
   else
-    hipLaunchKernelGGL((k_trace<OCC, AL, CNT, SL, PL>), a.grid, dim3(TB), 0, a.s, a.sc, a.rays, a.M, a.stride,
-                       a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.node_visits);
+    hipLaunchKernelGGL((k_trace_p<OCC, AL, CNT, SL, PL>), p.grid, dim3(TB), 0, a.s, a.sc, a.rays, a.M, a.stride,
+                       a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.counter, a.refill, p.runs,
+                       a.node_visits, nullptr, 0u);
 }
 
 template <bool OCC, bool AL, bool CNT, bool PL>
 void launch_slots(const LaunchArgs& a) {
-  if (a.lds_slots <= 0) launch_one<OCC, AL, CNT, 0, PL>(a);
-  else if (a.lds_slots <= 8) launch_one<OCC, AL, CNT, 8, PL>(a);
-  else if (a.lds_slots <= 12) launch_one<OCC, AL, CNT, 12, PL>(a);
+  if (a.tp->lds_slots <= 0) launch_one<OCC, AL, CNT, 0, PL>(a);
+  else if (a.tp->lds_slots <= 8) launch_one<OCC, AL, CNT, 8, PL>(a);
+  else if (a.tp->lds_slots <= 12) launch_one<OCC, AL, CNT, 12, PL>(a);
   else launch_one<OCC, AL, CNT, 16, PL>(a);
 }
 
@@ -1339,88 +1403,93 @@ void launch_trace(const DevScene& sc, void* rays, uint32_t M, uint64_t stride, b
   const bool persistent = tp.persistent && (sorter || counter);
   const int rmin = occluded ? tp.refill_min_occ : tp.refill_min;
   const int refill = rmin < 1 ? 1 : (rmin > 64 ? 64 : rmin);  // 64 idle lanes always refill
-  dim3 pgrid(1);
-  if (persistent) {
-    if (!counter) {
-      sorter->counter.reserve(256);
-      counter = sorter->counter.as<uint32_t>();
-    }
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, counter);
-    const uint32_t want = (uint32_t)tp.cus * (uint32_t)tp.blocks_per_cu;
-    pgrid = dim3(want < grid.x ? want : grid.x);
+  if (persistent && !counter) {
+    sorter->counter.reserve(COUNTER_BYTES);
+    counter = sorter->counter.as<uint32_t>();
   }
-  LaunchArgs la{sc, rp, M, stride, inst_id, cnt_nodes, cnt_tris, err, perm,
-                persistent ? counter : nullptr, refill, count ? node_visits : nullptr,
-                persistent, grid, pgrid, tp.lds_slots, s, tp.dual == 1 || (tp.dual == 2 && occluded)};
+  LaunchArgs la{sc, rp, M, stride, inst_id, cnt_nodes, cnt_tris, err, perm, persistent ? counter : nullptr, refill,
+                count ? node_visits : nullptr, persistent, &tp, s, tp.dual == 1 || (tp.dual == 2 && occluded)};
   if (sc.robust) launch_pl<true>(la, count, occluded, aligned);
   else launch_pl<false>(la, count, occluded, aligned);
   RTG_HIP(hipGetLastError());
 }
 
+template <bool OCC, bool AL, bool PL, int SL>
+void launch_batch_slots(const DevScene& sc, const BatchItem* items, uint32_t nitems, uint32_t M, uint32_t* err,
+                        uint32_t* counter, hipStream_t s, const TraceParams& tp) {
+  const int rmin = OCC ? tp.refill_min_occ : tp.refill_min;
+  const int refill = rmin < 1 ? 1 : (rmin > 64 ? 64 : rmin);
+  const RayPlan p = ray_plan(M, resident_blocks<k_trace_p<OCC, AL, false, SL, PL, true>>(), tp);
+  if (p.counter) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(COUNTERS), 0, s, counter);
+  hipLaunchKernelGGL((k_trace_p<OCC, AL, false, SL, PL, true>), p.grid, dim3(TB), 0, s, sc, (char*)nullptr, M,
+                     (uint64_t)0, 0xffffffffu, (uint32_t*)nullptr, (uint32_t*)nullptr, err, (const uint32_t*)nullptr,
+                     counter, refill, p.runs, (uint32_t*)nullptr, items, nitems);
+}
+
 // (LDS stack rings of 8 or of 12 entries per lane: lds_slots up to 8, or more)
 template <bool OCC, bool AL, bool PL>
 void launch_batch_one(const DevScene& sc, const BatchItem* items, uint32_t nitems, uint32_t M, uint32_t* err,
-                      uint32_t* counter, int refill, dim3 pgrid, hipStream_t s, int lds_slots) {
-  if (lds_slots <= 8)
-    hipLaunchKernelGGL((k_trace_p<OCC, AL, false, 8, PL, true>), pgrid, dim3(TB), 0, s, sc, (char*)nullptr, M,
-                       (uint64_t)0, 0xffffffffu, (uint32_t*)nullptr, (uint32_t*)nullptr, err,
-                       (const uint32_t*)nullptr, counter, refill, (uint32_t*)nullptr, items, nitems);
-  else
-    hipLaunchKernelGGL((k_trace_p<OCC, AL, false, 12, PL, true>), pgrid, dim3(TB), 0, s, sc, (char*)nullptr, M,
-                       (uint64_t)0, 0xffffffffu, (uint32_t*)nullptr, (uint32_t*)nullptr, err,
-                       (const uint32_t*)nullptr, counter, refill, (uint32_t*)nullptr, items, nitems);
+                      uint32_t* counter, hipStream_t s, const TraceParams& tp) {
+  if (tp.lds_slots <= 8) launch_batch_slots<OCC, AL, PL, 8>(sc, items, nitems, M, err, counter, s, tp);
+  else launch_batch_slots<OCC, AL, PL, 12>(sc, items, nitems, M, err, counter, s, tp);
 }
 
 void launch_trace_batch(const DevScene& sc, const BatchItem* items, uint32_t nitems, uint32_t M, bool occluded,
                         bool aligned, uint32_t* err, uint32_t* counter, hipStream_t s, const TraceParams& tp) {
   if (M == 0 || nitems == 0 || sc.num_nodes == 0) return;
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, counter);
-  const int rmin = occluded ? tp.refill_min_occ : tp.refill_min;
-  const int refill = rmin < 1 ? 1 : (rmin > 64 ? 64 : rmin);
-  const uint32_t want = (uint32_t)tp.cus * (uint32_t)tp.blocks_per_cu;
-  const uint32_t blocks = div_up(M, TB);
-  const dim3 pgrid(want < blocks ? want : blocks);
   if (sc.robust) {
     if (occluded) {
-      if (aligned) launch_batch_one<true, true, true>(sc, items, nitems, M, err, counter, refill, pgrid, s, tp.lds_slots);
-      else launch_batch_one<true, false, true>(sc, items, nitems, M, err, counter, refill, pgrid, s, tp.lds_slots);
+      if (aligned) launch_batch_one<true, true, true>(sc, items, nitems, M, err, counter, s, tp);
+      else launch_batch_one<true, false, true>(sc, items, nitems, M, err, counter, s, tp);
     } else {
-      if (aligned) launch_batch_one<false, true, true>(sc, items, nitems, M, err, counter, refill, pgrid, s, tp.lds_slots);
-      else launch_batch_one<false, false, true>(sc, items, nitems, M, err, counter, refill, pgrid, s, tp.lds_slots);
+      if (aligned) launch_batch_one<false, true, true>(sc, items, nitems, M, err, counter, s, tp);
+      else launch_batch_one<false, false, true>(sc, items, nitems, M, err, counter, s, tp);
     }
   } else {
     if (occluded) {
-      if (aligned) launch_batch_one<true, true, false>(sc, items, nitems, M, err, counter, refill, pgrid, s, tp.lds_slots);
-      else launch_batch_one<true, false, false>(sc, items, nitems, M, err, counter, refill, pgrid, s, tp.lds_slots);
+      if (aligned) launch_batch_one<true, true, false>(sc, items, nitems, M, err, counter, s, tp);
+      else launch_batch_one<true, false, false>(sc, items, nitems, M, err, counter, s, tp);
     } else {
-      if (aligned) launch_batch_one<false, true, false>(sc, items, nitems, M, err, counter, refill, pgrid, s, tp.lds_slots);
-      else launch_batch_one<false, false, false>(sc, items, nitems, M, err, counter, refill, pgrid, s, tp.lds_slots);
+      if (aligned) launch_batch_one<false, true, false>(sc, items, nitems, M, err, counter, s, tp);
+      else launch_batch_one<false, false, false>(sc, items, nitems, M, err, counter, s, tp);
     }
   }
   RTG_HIP(hipGetLastError());
+}
+
+template <bool OCC, bool AL, bool CNT>
+void launch_inst_one(const DevTop& top, char* rays, uint32_t M, uint64_t stride, uint32_t ctx_inst, uint32_t* err,
+                     uint32_t* counter, int refill, hipStream_t s, const TraceParams& tp, uint32_t* top_visits,
+                     uint32_t* obj_visits, uint32_t target_obj) {
+  const RayPlan p = ray_plan(M, resident_blocks<k_trace_inst<OCC, AL, CNT>>(), tp);
+  if (p.counter) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(COUNTERS), 0, s, counter);
+  hipLaunchKernelGGL((k_trace_inst<OCC, AL, CNT>), p.grid, dim3(TB), 0, s, top, rays, M, stride, ctx_inst, err,
+                     counter, refill, p.runs, top_visits, obj_visits, target_obj);
 }
 
 void launch_trace_inst(const DevTop& top, void* rays, uint32_t M, uint64_t stride, bool occluded, uint32_t ctx_inst,
                        uint32_t* err, hipStream_t s, const TraceParams& tp, RaySorter* sorter, uint32_t* counter) {
   if (M == 0 || top.num_nodes == 0) return;
   const bool aligned = ((uintptr_t)rays % 16 == 0) && (stride % 16 == 0);
-  const uint32_t blocks = div_up(M, TB);
-  const uint32_t want = (uint32_t)tp.cus * (uint32_t)tp.blocks_per_cu;
-  const dim3 grid(want < blocks ? want : blocks), block(TB);
   const int rmin = occluded ? tp.refill_min_occ_inst : tp.refill_min;
   const int refill = rmin < 1 ? 1 : (rmin > 64 ? 64 : rmin);
   if (!counter) {
-    sorter->counter.reserve(256);
+    sorter->counter.reserve(COUNTER_BYTES);
     counter = sorter->counter.as<uint32_t>();
   }
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, counter);
   char* rp = (char*)rays;
+  auto go = [&](auto occ, auto al) {
+    launch_inst_one<occ(), al(), false>(top, rp, M, stride, ctx_inst, err, counter, refill, s, tp, nullptr, nullptr,
+                                        0xffffffffu);
+  };
+  using T = std::true_type;
+  using F = std::false_type;
   if (occluded) {
-    if (aligned) hipLaunchKernelGGL((k_trace_inst<true, true>), grid, block, 0, s, top, rp, M, stride, ctx_inst, err, counter, refill);
-    else hipLaunchKernelGGL((k_trace_inst<true, false>), grid, block, 0, s, top, rp, M, stride, ctx_inst, err, counter, refill);
+    if (aligned) go(T(), T());
+    else go(T(), F());
   } else {
-    if (aligned) hipLaunchKernelGGL((k_trace_inst<false, true>), grid, block, 0, s, top, rp, M, stride, ctx_inst, err, counter, refill);
-    else hipLaunchKernelGGL((k_trace_inst<false, false>), grid, block, 0, s, top, rp, M, stride, ctx_inst, err, counter, refill);
+    if (aligned) go(F(), T());
+    else go(F(), F());
   }
   RTG_HIP(hipGetLastError());
 }
@@ -1430,18 +1499,14 @@ void launch_trace_inst_counted(const DevTop& top, void* rays, uint32_t M, uint64
                                hipStream_t s, const TraceParams& tp) {
   if (M == 0 || top.num_nodes == 0) return;
   const bool aligned = ((uintptr_t)rays % 16 == 0) && (stride % 16 == 0);
-  const uint32_t blocks = div_up(M, TB);
-  const uint32_t want = (uint32_t)tp.cus * (uint32_t)tp.blocks_per_cu;
-  const dim3 grid(want < blocks ? want : blocks), block(TB);
   const int refill = tp.refill_min < 1 ? 1 : (tp.refill_min > 64 ? 64 : tp.refill_min);
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, counter);
   char* rp = (char*)rays;
   if (aligned)
-    hipLaunchKernelGGL((k_trace_inst<false, true, true>), grid, block, 0, s, top, rp, M, stride, 0xffffffffu, err,
-                       counter, refill, top_visits, obj_visits, target_obj);
+    launch_inst_one<false, true, true>(top, rp, M, stride, 0xffffffffu, err, counter, refill, s, tp, top_visits,
+                                       obj_visits, target_obj);
   else
-    hipLaunchKernelGGL((k_trace_inst<false, false, true>), grid, block, 0, s, top, rp, M, stride, 0xffffffffu, err,
-                       counter, refill, top_visits, obj_visits, target_obj);
+    launch_inst_one<false, false, true>(top, rp, M, stride, 0xffffffffu, err, counter, refill, s, tp, top_visits,
+                                        obj_visits, target_obj);
   RTG_HIP(hipGetLastError());
 }
 

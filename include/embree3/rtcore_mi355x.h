@@ -31,8 +31,8 @@ RTC_API void rtcgOccluded1MAsync(RTCScene scene, const struct RTCIntersectContex
  * forbid hipMalloc): the query of rtcgIntersect1MAsync (occluded = 0,
  * RTCRayHit records) or rtcgOccluded1MAsync (occluded = 1, RTCRay records)
  * over records in this device's memory, with the same results, allocating
- * nothing. Its kernels keep their ray counter and error bits in a fixed
- * 256-byte array per GPU that the library holds until the process ends.
+ * nothing. Its kernels keep their ray counters and error bits in a fixed
+ * 2 KB array per GPU that the library holds until the process ends.
  * At most 2^31 rays per call (more is RTC_ERROR_INVALID_ARGUMENT); host
  * records are RTC_ERROR_INVALID_ARGUMENT; the device's ray-reordering setting
  * is not applied. Every call on one GPU shares that GPU's array, so calls that
