@@ -2424,7 +2424,8 @@ RTC_API float rtcgAutotuneBatch(const RTCGBatchItem* items, unsigned int numItem
     check_trace_error(t);
     return total / (float)reps;
   };
-  const rtg::TraceParams tp = d->trace_params();
+  rtg::TraceParams tp = d->trace_params();
+  tp.groups = 0;  // the settings are those of the one-lane kernel, also where the batch is small
   rtg::TraceParams bestt = tp;
   float best = INFINITY;
   for (int slots : {8, 12})
@@ -2605,8 +2606,12 @@ RTC_API float rtcgAutotune(RTCScene scene, const void* d_rays, unsigned int M, s
   const int reps = 2;
   // The sweep works on local copies; the device's settings change once, at
   // the end, under its settings lock, so that commits and queries on other
-  // threads never see a trial value.
-  const rtg::TraceParams tp = d->trace_params();
+  // threads never see a trial value. Every trial runs the one-lane kernels
+  // that the settings are for, also on a sample small enough for eight lanes
+  // a ray.
+  rtg::TraceParams tp = d->trace_params();
+  const int groups = tp.groups;
+  tp.groups = 0;
   const rtg::BuildParams start = d->build_settings();
   rtg::BuildParams bestb = start;
   float best = time_config(s, t, tp, d_rays, work.ptr, M, byteStride, occluded != 0, reps);
@@ -2655,6 +2660,7 @@ RTC_API float rtcgAutotune(RTCScene scene, const void* d_rays, unsigned int M, s
     d->build.width = bestb.width;
     d->build.max_leaf = bestb.max_leaf;
     d->build.cost_tri = bestb.cost_tri;
+    bestt.groups = groups;
     d->trace = bestt;
   }
   if (out && outSize) {

@@ -68,6 +68,7 @@ struct DeviceBVH {
     s.num_nodes = stats.num_nodes;
     s.num_tris = stats.num_prims;
     s.robust = robust;
+    s.max_stack = stats.max_stack;
     const SceneSlot& sl = slot < slots.size() ? slots[slot] : SceneSlot();
     s.root = sl.root;
     for (int k = 0; k < 3; k++) {

@@ -131,6 +131,7 @@ struct DevScene {
   float scale[3];  // 1023.99 / extent per axis (0 for a flat axis)
   uint32_t robust; // triangle records hold (v0, v1, v2) for the Pluecker test
   uint32_t root;   // root node of this scene (scenes of a batch share the arrays)
+  uint32_t max_stack;  // traversal stack entries the deepest path can need
 };
 
 // What the two-level traversal needs: the top tree over instance records

@@ -31,6 +31,7 @@ struct TraceParams {
   // incoherent rays it gave 3934 vs 3789 Mrays/s occlusion but 1724 vs 1939
   // closest hit (speculative node visits before a pending leaf's hits).
   int dual = 2;
+  int groups = 1;           // small streams with eight lanes a ray (0: one lane, as large ones)
   int cus = 256;            // compute units (set from the device)
   int blocks_per_cu = 8;    // 256-thread blocks per compute unit for the persistent grid (at most those resident)
 };

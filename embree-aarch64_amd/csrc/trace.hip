@@ -653,6 +653,16 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
 // same code as 6. A 16-entry LDS stack (32 KB per block) leaves room for 5.
 constexpr int TRACE_MIN_BLOCKS = 6;
 
+// The stream of a batch that ray slot `slot` belongs to.
+__device__ inline const BatchItem& stream_of(const BatchItem* __restrict__ items, uint32_t nitems, uint32_t slot) {
+  uint32_t lo = 0, hi = nitems - 1;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    if (items[mid].first <= slot) lo = mid; else hi = mid - 1;
+  }
+  return items[lo];
+}
+
 // BATCH: the ray slots 0..M-1 are the concatenation of the streams in
 // `items` (sorted by `first`); a lane finds its stream by binary search and
 // starts at that stream's scene root.
@@ -697,12 +707,7 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
           if (slot != 0xffffffffu) {
             char* src;
             if (BATCH) {
-              uint32_t lo = 0, hi = nitems - 1;
-              while (lo < hi) {
-                const uint32_t mid = (lo + hi + 1) >> 1;
-                if (items[mid].first <= slot) lo = mid; else hi = mid - 1;
-              }
-              const BatchItem& it = items[lo];
+              const BatchItem& it = stream_of(items, nitems, slot);
               ray = slot - it.first;
               lrp = it.rays + (uint64_t)ray * it.stride;
               lroot = it.root;
@@ -1013,6 +1018,209 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
       }
       active = false;
     }
+  }
+}
+
+// ------------------------------------------------------- small streams --
+
+// A stream too small to fill the GPU with one ray per lane: eight lanes share
+// a ray. In a node step lane c tests child c, in a leaf step triangle c of the
+// leaf, and a pop looks at eight entries, so a step is a fraction of the
+// one-lane kernels' instructions, and a wave waits for the longest of 8 rays
+// instead of 64. What bounds it is the chain of dependent steps of the longest
+// ray (about 0.8 us each, most of it the node's load): 1073 camera rays on a
+// 131 k triangle terrain take 38 us a call, 85 with a lane a ray. Ray state is the same in a group's eight lanes; every branch depends on
+// it (or on a ballot of the group), so the group stays together.
+constexpr int GL = 8;            // lanes of a ray
+constexpr int GR = 64 / GL;      // rays of a block (one wave)
+
+template <int CTRL>
+__device__ inline uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xf, 0xf, false);
+}
+// The value of lane (c ^ X) of the group.
+__device__ inline uint32_t gx1(uint32_t v) { return dpp<0xB1>(v); }   // quad_perm [1,0,3,2]
+__device__ inline uint32_t gx2(uint32_t v) { return dpp<0x4E>(v); }   // quad_perm [2,3,0,1]
+__device__ inline uint32_t gx3(uint32_t v) { return dpp<0x1B>(v); }   // quad_perm [3,2,1,0]
+__device__ inline uint32_t gx7(uint32_t v) { return dpp<0x141>(v); }  // row_half_mirror
+__device__ inline float gmin(float v) {
+  v = fminf(v, __uint_as_float(gx1(__float_as_uint(v))));
+  v = fminf(v, __uint_as_float(gx2(__float_as_uint(v))));
+  return fminf(v, __uint_as_float(gx7(__float_as_uint(v))));
+}
+
+template <bool OCCLUDED, bool ALIGNED, bool PL, bool BATCH = false>
+__global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ rays, uint32_t M, uint64_t stride,
+                                                uint32_t inst_id, uint32_t* __restrict__ err, uint32_t cap,
+                                                const BatchItem* __restrict__ items, uint32_t nitems) {
+  extern __shared__ uint64_t group_stack[];  // cap entries for each ray, entry e of ray g at [e * GR + g]
+  const uint32_t c = threadIdx.x & (GL - 1), g = threadIdx.x / GL;
+  const uint32_t i = blockIdx.x * GR + g;
+  if (i >= M) return;
+  char* rp = rays + (uint64_t)i * stride;
+  uint32_t root = sc.root;
+  if (BATCH) {
+    const BatchItem& it = stream_of(items, nitems, i);
+    rp = it.rays + (uint64_t)(i - it.first) * it.stride;
+    root = it.root;
+  }
+  float4 a, b;
+  float tfar;
+  load_ray<ALIGNED>(rp, a, b, tfar);
+  if (!(a.w <= tfar)) return;
+  TRay r;
+  setup_ray(r, a, b, tfar);
+  Hit best;  // the best of the triangles that this lane tested
+  best.found = false;
+  best.t = INFINITY;
+  best.prim = best.geom = 0xffffffffu;
+  best.u = best.v = best.ngx = best.ngy = best.ngz = 0.0f;
+  float lim = widen_up(tfar);
+  bool occluded = false;
+  lds_u64* stack = (lds_u64*)group_stack + g;
+  uint32_t sp = 0, cur = root;
+  const uint32_t gshift = g * GL;
+  auto group = [&](bool x) { return (uint32_t)(__ballot(x) >> gshift) & 0xffu; };
+  // this lane's plane bytes: near and far of each axis
+  const uint32_t onx = 32u + (r.negx ? 8u : 0u) + c, ony = 48u + (r.negy ? 8u : 0u) + c, onz = 64u + (r.negz ? 8u : 0u) + c;
+  const uint32_t ofx = 72u + 2 * c - onx, ofy = 104u + 2 * c - ony, ofz = 136u + 2 * c - onz;  // (the other of the two)
+  const uint32_t max_iter = sc.num_nodes + sc.num_tris + 16u;
+  uint32_t iter = 0;
+  while (true) {
+    if (++iter > max_iter) {
+      atomicOr(err, 2u);
+      break;
+    }
+    if (!(cur & REF_LEAF)) {
+      if (cur >= sc.num_nodes) {
+        atomicOr(err, 4u);
+        break;
+      }
+      const char* np = reinterpret_cast<const char*>(sc.nodes + cur);
+      const uint4 w0 = *reinterpret_cast<const uint4*>(np), w1 = *reinterpret_cast<const uint4*>(np + 16);
+      const uint8_t* nb = reinterpret_cast<const uint8_t*>(np);
+      const float qnx = (float)nb[onx], qfx = (float)nb[ofx], qny = (float)nb[ony], qfy = (float)nb[ofy],
+                  qnz = (float)nb[onz], qfz = (float)nb[ofz];
+      const uint64_t meta = (uint64_t)w1.z | ((uint64_t)w1.w << 32);
+      const uint32_t mb = (uint32_t)(meta >> (8 * c)) & 0xffu;
+      // (the same operations as intersect_node())
+      const float sx = __uint_as_float((w0.w & 0xffu) << 23), sy = __uint_as_float(((w0.w >> 8) & 0xffu) << 23),
+                  sz = __uint_as_float(((w0.w >> 16) & 0xffu) << 23);
+      const float dx = __uint_as_float(w0.x) - r.ox, dy = __uint_as_float(w0.y) - r.oy, dz = __uint_as_float(w0.z) - r.oz;
+      const float tnx = __builtin_fmaf(qnx, sx * r.rnx, dx * r.rnx), tfx = __builtin_fmaf(qfx, sx * r.rfx, dx * r.rfx);
+      const float tny = __builtin_fmaf(qny, sy * r.rny, dy * r.rny), tfy = __builtin_fmaf(qfy, sy * r.rfy, dy * r.rfy);
+      const float tnz = __builtin_fmaf(qnz, sz * r.rnz, dz * r.rnz), tfz = __builtin_fmaf(qfz, sz * r.rfz, dz * r.rfz);
+      const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, r.tlo));
+      const float tf = fminf(fminf(tfx, tfy), fminf(tfz, lim));
+      const bool hit = (tn <= tf) && (mb != 0u);
+      const uint32_t mask = group(hit);
+      if (mask) {
+        const uint32_t cb = w1.x - 0x80u, tb = (w1.y | REF_LEAF) - 1u;
+        const uint32_t n = (uint32_t)__popc(mask);
+        uint32_t rank, first;
+        if (OCCLUDED) {
+          rank = (uint32_t)__popc(mask & ((1u << c) - 1u));
+          first = (uint32_t)__builtin_ctz(mask);
+        } else {
+          // rank by entry distance; the low bits make the keys distinct
+          const uint32_t key = hit ? (__float_as_uint(tn) & ~7u) | c : 0xffffffffu;
+          const uint32_t m = gx7(key);
+          rank = (gx1(key) < key) + (gx2(key) < key) + (gx3(key) < key) + (m < key) + (gx1(m) < key) + (gx2(m) < key) +
+                 (gx3(m) < key);
+          first = (uint32_t)__builtin_ctz(group(hit && rank == 0u));
+        }
+        if (sp + n > cap) {
+          atomicOr(err, 1u);
+          break;
+        }
+        // the nearest is next, the others are pushed farthest first
+        if (hit && rank > 0u)
+          stack[(sp + n - 1u - rank) * GR] = pack_entry(make_uint2(meta_ref(mb, cb, tb), __float_as_uint(tn)));
+        sp += n - 1u;
+        cur = meta_ref((uint32_t)(meta >> (8 * first)) & 0xffu, cb, tb);
+        continue;
+      }
+    } else {
+      const uint32_t ti = cur & ~REF_LEAF;
+      if (ti >= sc.num_tris) {
+        atomicOr(err, 4u);
+        break;
+      }
+      TriTest h;
+      bool valid = false;
+      h.flags = 0u;
+      if (c < sc.num_tris - ti) valid = tri_test<PL>(r, sc.tris + ti + c, h);
+      // records up to the leaf's last one
+      const uint32_t last = group((h.flags & TRI_LAST) != 0u);
+      valid = valid && (last == 0u || c <= (uint32_t)__builtin_ctz(last));
+      if (OCCLUDED) {
+        if (group(valid)) {
+          occluded = true;
+          break;
+        }
+      } else {
+        if (valid && (!best.found || h.t < best.t ||
+                      (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim))))) {
+          best.found = true;
+          best.t = h.t;
+          best.u = h.un / h.dn;
+          best.v = h.vn / h.dn;
+          best.ngx = h.ngx; best.ngy = h.ngy; best.ngz = h.ngz;
+          best.prim = h.prim; best.geom = h.geom;
+        }
+        if (group(valid)) lim = widen_up(fminf(gmin(best.t), tfar));
+      }
+      if (last == 0u) {
+        cur += GL;
+        continue;
+      }
+    }
+    // pop the next entry that can still hold a closer hit, eight at a time
+    bool got = false;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    while (sp > 0u) {
+      const uint2 e = c < sp ? unpack_entry(stack[(sp - 1u - c) * GR]) : make_uint2(0u, 0x7f800000u);
+      const uint32_t ok = group(c < sp && (OCCLUDED || __uint_as_float(e.y) <= lim));
+      if (ok) {
+        const uint32_t k = (uint32_t)__builtin_ctz(ok);
+        sp -= k + 1u;
+        cur = unpack_entry(stack[sp * GR]).x;
+        got = true;
+        break;
+      }
+      sp = sp > GL ? sp - GL : 0u;
+    }
+    if (!got) break;
+  }
+  if (OCCLUDED) {
+    if (occluded && c == 0u) *reinterpret_cast<float*>(rp + 32) = -INFINITY;
+    return;
+  }
+  // the least (t, geomID, primID) of the group; a lane that holds it writes it
+  // (two may hold the same triangle, reached through two leaves)
+  float t = best.t;
+  uint32_t geom = best.geom, prim = best.prim;
+  auto least = [&](float t2, uint32_t g2, uint32_t p2) {
+    const bool less = t2 < t || (t2 == t && (g2 < geom || (g2 == geom && p2 < prim)));
+    t = less ? t2 : t;
+    geom = less ? g2 : geom;
+    prim = less ? p2 : prim;
+  };
+  least(__uint_as_float(gx1(__float_as_uint(t))), gx1(geom), gx1(prim));
+  least(__uint_as_float(gx2(__float_as_uint(t))), gx2(geom), gx2(prim));
+  least(__uint_as_float(gx7(__float_as_uint(t))), gx7(geom), gx7(prim));
+  if (best.found && best.t == t && best.geom == geom && best.prim == prim) {
+    float* f = reinterpret_cast<float*>(rp);
+    uint32_t* u = reinterpret_cast<uint32_t*>(rp);
+    f[8] = best.t;
+    f[12] = best.ngx;
+    f[13] = best.ngy;
+    f[14] = best.ngz;
+    f[15] = best.u;
+    f[16] = best.v;
+    u[17] = best.prim;
+    u[18] = best.geom;
+    u[19] = inst_id;
   }
 }
 
@@ -1369,8 +1577,42 @@ void launch_slots(const LaunchArgs& a) {
   else launch_one<OCC, AL, CNT, 16, PL>(a);
 }
 
+// The largest streams that eight lanes a ray serve better (us a call, with 14
+// of launching and of making the records; eight lanes against one):
+//                                     1024       16384      65536      131072
+//   camera, 131 k terrain          42 :  82   48 : 103   63 :  96   97 : 120
+//   random, 262 k soup            102 : 223  174 : 286  279 : 304  448 : 315
+//   random occlusion, 262 k soup   31 :  54   40 :  58   83 :  70  129 :  75
+//   camera, 16 k sphere            41 :  70   44 :  78   69 :  86   90 :  93
+// From there on the GPU is full, and one lane a ray needs fewer instructions.
+constexpr uint32_t GROUP_MAX_RAYS = 65536, GROUP_MAX_RAYS_OCC = 32768;
+// A ray's stack is all in LDS: 256 entries are 16 KB a wave. (Trees of a few
+// million triangles need fewer than 80.)
+constexpr uint32_t GROUP_MAX_STACK = 256;
+
+bool use_groups(const DevScene& sc, uint32_t M, bool occluded, const TraceParams& tp) {
+  return tp.persistent && tp.groups && M <= (occluded ? GROUP_MAX_RAYS_OCC : GROUP_MAX_RAYS) && sc.max_stack < GROUP_MAX_STACK;
+}
+
+template <bool OCC, bool AL, bool PL>
+void launch_group(const LaunchArgs& a) {
+  const uint32_t cap = a.sc.max_stack + 1u;
+  hipLaunchKernelGGL((k_trace_g<OCC, AL, PL>), dim3(div_up(a.M, GR)), dim3(64), cap * GR * 8, a.s, a.sc, a.rays, a.M,
+                     a.stride, a.inst_id, a.err, cap, nullptr, 0u);
+}
+
 template <bool PL>
 void launch_pl(const LaunchArgs& a, bool count, bool occluded, bool aligned) {
+  if (!count && !a.perm && use_groups(a.sc, a.M, occluded, *a.tp)) {
+    if (occluded) {
+      if (aligned) launch_group<true, true, PL>(a);
+      else launch_group<true, false, PL>(a);
+    } else {
+      if (aligned) launch_group<false, true, PL>(a);
+      else launch_group<false, false, PL>(a);
+    }
+    return;
+  }
   if (count) {
     if (occluded) launch_slots<true, false, true, PL>(a);
     else launch_slots<false, false, true, PL>(a);
@@ -1419,6 +1661,12 @@ void launch_batch_slots(const DevScene& sc, const BatchItem* items, uint32_t nit
                         uint32_t* counter, hipStream_t s, const TraceParams& tp) {
   const int rmin = OCC ? tp.refill_min_occ : tp.refill_min;
   const int refill = rmin < 1 ? 1 : (rmin > 64 ? 64 : rmin);
+  if (use_groups(sc, M, OCC, tp)) {
+    const uint32_t cap = sc.max_stack + 1u;
+    hipLaunchKernelGGL((k_trace_g<OCC, AL, PL, true>), dim3(div_up(M, GR)), dim3(64), cap * GR * 8, s, sc,
+                       (char*)nullptr, M, (uint64_t)0, 0xffffffffu, err, cap, items, nitems);
+    return;
+  }
   const RayPlan p = ray_plan(M, resident_blocks<k_trace_p<OCC, AL, false, SL, PL, true>>(), tp);
   if (p.counter) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(COUNTERS), 0, s, counter);
   hipLaunchKernelGGL((k_trace_p<OCC, AL, false, SL, PL, true>), p.grid, dim3(TB), 0, s, sc, (char*)nullptr, M,

@@ -1,7 +1,10 @@
-"""The rays of a launch are shared out in runs of 64 to waves and queues:
-every record of every stream length around the edges of a run, a block, the
-eight queues and the waves' first runs is traced once, byte-identical to the
-oracle."""
+"""Small streams are traced with eight lanes a ray, larger ones with one, whose
+rays are shared out in runs of 64 to waves and queues: every record of every
+stream length around the edges of a block, of the change between the two, of
+the eight queues and the waves' first runs is traced once, byte-identical to
+the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -9,10 +12,10 @@ from conftest import mismatches
 
 pytestmark = pytest.mark.gpu
 
-# one lane, a run, a block of four, eight blocks (the queues start), all
-# resident waves' first runs at 5, 6 and 7 blocks on 256 compute units, and
-# past them (the counters start)
-SIZES = [1, 63, 64, 65, 255, 257, 1792, 1793, 2049, 327679, 327681, 393215, 393217, 458753, 600001]
+# one ray, a block of eight, the last sizes with eight lanes a ray (occlusion,
+# closest hit) and the first with one, all resident waves' first runs at 5, 6
+# and 7 blocks on 256 compute units, and past them (the counters start)
+SIZES = [1, 7, 8, 9, 1021, 32767, 32769, 65535, 65537, 327679, 327681, 393215, 393217, 458753, 600001]
 
 
 @pytest.fixture(scope="module")
@@ -63,7 +66,43 @@ def test_every_record_through_an_instance(rtc, device, oracle, scene, n):
     top.release()
 
 
-@pytest.mark.parametrize("n", [65, 2049, 393217, 600001])
+@pytest.mark.parametrize("config,robust", [("", False), ("", True), ("bvh_leaf=15,cost_tri=0.02", False),
+                                           ("bvh_leaf=15,cost_tri=0.02", True), ("bvh_width=2", False)])
+@pytest.mark.parametrize("n,stride", [(999, 80), (999, 84), (70001, 80), (70001, 84)])
+def test_both_kernels_on_other_trees(rtc, oracle, config, robust, n, stride):
+    # leaves of more than eight triangles, binary trees, robust scenes, records
+    # that are not 16-byte aligned, intervals that start behind the origin
+    dev = rtc.Device(config)
+    soup = rtc.gen_soup(3000, seed=5, h=0.06)
+    sc = rtc.Scene(dev, [soup, rtc.gen_sphere(9, center=(0.5, 0.5, 0.5), radius=0.3)],
+                   flags=rtc.RTC_SCENE_FLAG_ROBUST if robust else 0).commit()
+    bvh = oracle.BVH([soup, rtc.gen_sphere(9, center=(0.5, 0.5, 0.5), radius=0.3)])
+    rays = rtc.gen_random_rays(n, seed=6)
+    rays["tnear"][::3] = -0.5
+    rays["tfar"][1::5] = 0.2
+    ref = rays.copy()
+    bvh.intersect(ref, robust=robust)
+    wide = np.zeros((n, stride), np.uint8)
+    wide[:, :80] = rays.view(np.uint8).reshape(n, 80)
+    d = dev.malloc(wide.nbytes)
+    dev.memcpy(d, wide.ctypes.data, wide.nbytes)
+    rtc.lib().rtcIntersect1M(sc.h, ctypes.byref(rtc.init_context()), d, n, stride)
+    dev.check("rtcIntersect1M")
+    dev.memcpy(wide.ctypes.data, d, wide.nbytes)
+    dev.free(d)
+    assert len(mismatches(np.ascontiguousarray(wide[:, :80]).reshape(-1).view(rtc.RTCRayHit), ref)) == 0
+    occ = np.zeros(n, rtc.RTCRay)
+    for k in rtc.RTCRay.names:
+        occ[k] = rays[k]
+    dark = occ.copy()
+    sc.occluded1M(occ)
+    bvh.occluded(dark, robust=robust)
+    assert len(mismatches(occ, dark)) == 0
+    sc.release()
+    dev.release()
+
+
+@pytest.mark.parametrize("n", [65, 32771, 65539, 393217, 600001])
 def test_every_record_of_a_batch(rtc, device, scene, n):
     _, rays, hits, _, _ = scene
     mesh = rtc.gen_sphere(8)
