@@ -53,36 +53,53 @@ typedef __attribute__((address_space(3))) uint64_t lds_u64;
 __device__ inline uint64_t pack_entry(uint2 e) { return (uint64_t)e.x | ((uint64_t)e.y << 32); }
 __device__ inline uint2 unpack_entry(uint64_t v) { return make_uint2((uint32_t)v, (uint32_t)(v >> 32)); }
 
-// Second word of a closest-hit stack entry: the entry distance rounded down
-// to a bfloat16 pattern (high half; -inf for a negative distance) and the
-// least distance of the entries below it (low half), so that a pop can tell
-// when every entry left is farther than the closest hit.
-__device__ inline uint32_t pack_dist(uint32_t d16, float& smin) {
-  const uint32_t y = (d16 << 16) | (__float_as_uint(smin) >> 16);
-  smin = fminf(smin, __uint_as_float(d16 << 16));
+// Second word of a closest-hit stack entry: in the high half the entry
+// distance's bits, rounded down, and in the low half the least such of the
+// entries below it, so that a pop can tell when every entry left is farther
+// than the closest hit. Distances compare as signed integers: positive ones
+// order like the floats, and a negative one (tnear < 0) is below all of them.
+__device__ inline uint32_t pack_dist(int key, int& smin) {
+  const uint32_t y = __builtin_amdgcn_perm((uint32_t)key, (uint32_t)smin, 0x07060302u);
+  smin = min(smin, key);
   return y;
 }
-__device__ inline float entry_dist(uint32_t y) { return __uint_as_float(y & 0xffff0000u); }
-__device__ inline float below_dist(uint32_t y) { return __uint_as_float(y << 16); }
+__device__ inline int below_dist(uint32_t y) { return (int)(y << 16); }
+// A word above this belongs to an entry beyond `lim` (which no key of a
+// negative distance is, whatever lim).
+__device__ inline int dist_limit(float lim) { return max((int)__float_as_uint(lim), 0) | 0xffff; }
+constexpr int DIST_NONE = 0x7f800000;         // of an empty stack
+constexpr int DIST_ALWAYS = (int)0xff800000;  // of an entry that is never skipped
 
 template <int LDS_SLOTS>
 struct RingStack {
   // A power-of-two ring finds entry i's slot as i & (LDS_SLOTS - 1); any
-  // other size keeps the slot of entry sp in `top`. When the ring is full,
-  // the oldest ring entry (lo = sp - LDS_SLOTS) sits in entry sp's slot.
+  // other size keeps the byte offset of entry sp's slot in `top`. When the
+  // ring is full, the oldest ring entry (lo = sp - LDS_SLOTS) sits in entry
+  // sp's slot.
   static constexpr bool POW2 = (LDS_SLOTS & (LDS_SLOTS - 1)) == 0;
-  lds_u64* lds;    // this lane's slot 0; slot k is lds + k * TB
-  uint64_t* spill; // STACK_CAP entries, private
-  int sp, lo;      // [0, lo) spilled, [lo, sp) in the ring
-  int top;         // sp mod LDS_SLOTS (other sizes than powers of two)
-  __device__ inline int slot() const {
-    if constexpr (POW2) return sp & (LDS_SLOTS - 1);
-    else return top;
+  static constexpr uint32_t STEP = TB * 8, RING = LDS_SLOTS * STEP;  // bytes between a lane's slots, and of the ring
+  typedef __attribute__((address_space(3))) char lds_char;
+  lds_char* lds;
+  uint64_t* spill;  // STACK_CAP entries, private
+  int sp, lo;       // [0, lo) spilled, [lo, sp) in the ring
+  uint32_t top;     // (other sizes than powers of two)
+  __device__ inline lds_u64& slot() const {
+    if constexpr (POW2) return *(lds_u64*)(lds + (uint32_t)(sp & (LDS_SLOTS - 1)) * STEP);
+    else return *(lds_u64*)(lds + top);
   }
-  __device__ inline void init(uint64_t* base, uint64_t* spill_mem) {
-    lds = (lds_u64*)base;
+  // (the one of x and x -/+ RING that is in the ring is the smaller as unsigned)
+  __device__ inline void up() {
+    sp++;
+    if constexpr (!POW2) top = min(top + STEP, top + STEP - RING);
+  }
+  __device__ inline void down() {
+    sp--;
+    if constexpr (!POW2) top = min(top - STEP, top - STEP + RING);
+  }
+  __device__ inline void init(uint64_t* ring, uint64_t* spill_mem) {
+    lds = (lds_char*)(POW2 ? ring + threadIdx.x : ring);
     spill = spill_mem;
-    sp = lo = top = 0;
+    clear();
   }
   // Whether a node's entries (at most 7) may be put(): true while the stack
   // holds at most STACK entries, which a tree the builder accepted never
@@ -91,12 +108,11 @@ struct RingStack {
   __device__ inline bool fits() const { return sp <= STACK; }
   __device__ inline void put(uint2 e) {
     if (sp - lo == LDS_SLOTS) {
-      spill[lo] = lds[slot() * TB];
+      spill[lo] = slot();
       lo++;
     }
-    lds[slot() * TB] = pack_entry(e);
-    sp++;
-    if constexpr (!POW2) top = top == LDS_SLOTS - 1 ? 0 : top + 1;
+    slot() = pack_entry(e);
+    up();
   }
   __device__ inline bool push(uint2 e) {
     if (sp >= STACK) return false;
@@ -104,18 +120,20 @@ struct RingStack {
     return true;
   }
   __device__ inline uint2 pop() {
-    sp--;
-    if constexpr (!POW2) top = top == 0 ? LDS_SLOTS - 1 : top - 1;
+    down();
     // an entry below the ring comes back through its ring slot, so that the
     // read below is always an LDS read
     if (sp < lo) {
       lo = sp;
-      lds[slot() * TB] = spill[sp];
+      slot() = spill[sp];
     }
-    return unpack_entry(lds[slot() * TB]);
+    return unpack_entry(slot());
   }
   __device__ inline bool empty() const { return sp == 0; }
-  __device__ inline void clear() { sp = lo = top = 0; }
+  __device__ inline void clear() {
+    sp = lo = 0;
+    top = threadIdx.x * 8;
+  }
 };
 
 // LDS_SLOTS == 0: the whole stack is a private array.
@@ -252,6 +270,7 @@ struct NodeHit {
 // (the expression the builder verified against every widened child box),
 // with rdir rounded down for near and up for far planes as the reference's
 // robust TravRay does (kernels/bvh/node_intersector1.h:122-190).
+template <bool OCCLUDED>
 __device__ inline void intersect_node(const QNode8* __restrict__ nodes, uint32_t i, const TRay& r, float thi,
                                       NodeHit& h) {
   const uint4* np = reinterpret_cast<const uint4*>(nodes + i);
@@ -302,7 +321,8 @@ __device__ inline void intersect_node(const QNode8* __restrict__ nodes, uint32_t
     const float tny = __builtin_fmaf(qny, any, bny), tfy = __builtin_fmaf(qfy, afy, bfy);
     const float tnz = __builtin_fmaf(qnz, anz, bnz), tfz = __builtin_fmaf(qfz, afz, bfz);
     const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, r.tlo));
-    const float tf = fminf(fminf(tfx, tfy), fminf(tfz, thi));
+    // (closest hit: push_near_to_far compares the entry distances with the limit)
+    const float tf = OCCLUDED ? fminf(fminf(tfx, tfy), fminf(tfz, thi)) : fminf(fminf(tfx, tfy), tfz);
     h.tn[c] = tn;
     h.hit[c] = (tn <= tf) && (mb != 0u);
     mask |= h.hit[c] ? (1u << c) : 0u;
@@ -344,33 +364,35 @@ __device__ inline bool push_any_order(const NodeHit& h, Stack& stack, uint32_t* 
 
 // Closest hit: pushes the hit children except the nearest, farthest first,
 // each with its entry distance, sets `next` to the nearest child and returns
-// whether any child was hit.
+// whether any child was hit within the limit.
 // A key is the entry distance's bit pattern with the child's meta byte in the
-// low 8 bits (distinct among a node's children), or 0xffffffff for a child
-// that is not hit. Entry distances are never below the ray's widened tnear,
-// so for tnear >= 0 the bit patterns order like the distances (a negative
-// distance, possible only with tnear < 0, orders as farther than every
-// positive one: a different visiting order, the same result). The
-// perturbation of the low 8 bits changes only the order among nearly equal
-// children. A 19-comparator network (Batcher's odd-even merge sort) orders
-// the keys decreasingly without branches: children not hit first, the
-// nearest hit child last. The stored distance is the key's high half
-// (rounded down; -inf for a negative distance), never above the true entry
-// distance, so the pop test stays conservative.
+// low 8 bits (distinct among a node's children), or NO_HIT for a child that is
+// not hit; keys compare as signed integers (see pack_dist). The perturbation of
+// the low 8 bits changes only the order among nearly equal children. A
+// 19-comparator network (Batcher's odd-even merge sort) orders the keys
+// decreasingly without branches: children not hit and those beyond the limit
+// first, the nearest hit child last. The stored distance is the key's high half
+// (rounded down), never above a positive entry distance, so the pop test stays
+// conservative. The limit is compared with the sorted keys (which a push tests
+// anyway) instead of taking part in every child's slab test. (With integer
+// distances and this, 274 VALU instructions a ray instead of 290 on the
+// 2^20-triangle soup, 7.00 ms instead of 7.14 for 2^24 rays: the kernel is
+// bound as much by the return path of the vector memory, busy 95 % of the
+// time, where every lane's 16 bytes of a node are an access of their own.)
 template <class Stack>
-__device__ inline bool push_near_to_far(const NodeHit& h, Stack& stack, float& smin, uint32_t* err,
+__device__ inline bool push_near_to_far(const NodeHit& h, Stack& stack, int& smin, float lim, uint32_t* err,
                                         uint32_t& next) {
-  constexpr uint32_t NO_HIT = 0xffffffffu;
-  uint32_t k[8];
+  constexpr int NO_HIT = 0x7fffffff;
+  int k[8];
   // v_perm_b32 selector: byte 0 from the meta word (byte c & 3), bytes 1-3
   // from the distance
 #pragma unroll
   for (int c = 0; c < 8; c++)
-    k[c] = h.hit[c] ? __builtin_amdgcn_perm(__float_as_uint(h.tn[c]), c < 4 ? h.meta_lo : h.meta_hi,
-                                            0x07060500u | (uint32_t)(c & 3))
+    k[c] = h.hit[c] ? (int)__builtin_amdgcn_perm(__float_as_uint(h.tn[c]), c < 4 ? h.meta_lo : h.meta_hi,
+                                                 0x07060500u | (uint32_t)(c & 3))
                     : NO_HIT;
   auto ce = [&](int i, int j) {
-    const uint32_t hi = max(k[i], k[j]), lo = min(k[i], k[j]);
+    const int hi = max(k[i], k[j]), lo = min(k[i], k[j]);
     k[i] = hi;
     k[j] = lo;
   };
@@ -380,23 +402,22 @@ __device__ inline bool push_near_to_far(const NodeHit& h, Stack& stack, float& s
   ce(0, 4); ce(1, 5); ce(2, 6); ce(3, 7);
   ce(2, 4); ce(3, 5);
   ce(1, 2); ce(3, 4); ce(5, 6);
-  if (k[7] == NO_HIT) return false;
+  // at most the pattern of +inf with a full low byte, below NO_HIT
+  const int klim = max((int)__float_as_uint(lim), 0) | 0xff;
+  if (k[7] > klim) return false;
   const uint32_t cb = h.cb, tb = h.tb;
   if (stack.fits()) {
 #pragma unroll
     for (int j = 0; j < 7; j++) {
-      if (k[j] != NO_HIT) {
-        const uint32_t dk = ((int32_t)k[j] < 0) ? 0xff800000u : k[j];
-        // (dk's high half, smin's high half)
-        stack.put(make_uint2(meta_ref(k[j] & 0xffu, cb, tb), __builtin_amdgcn_perm(dk, __float_as_uint(smin), 0x07060302u)));
-        const float d = __uint_as_float(dk & 0xffff0000u);
-        smin = d < smin ? d : smin;
+      if (k[j] <= klim) {
+        const uint32_t y = pack_dist(k[j], smin);
+        stack.put(make_uint2(meta_ref((uint32_t)k[j] & 0xffu, cb, tb), y));
       }
     }
   } else {
     atomicOr(err, 1u);
   }
-  next = meta_ref(k[7] & 0xffu, cb, tb);
+  next = meta_ref((uint32_t)k[7] & 0xffu, cb, tb);
   return true;
 }
 
@@ -539,8 +560,8 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
   __shared__ uint64_t lds_stack[LDS_SLOTS > 0 ? LDS_SLOTS * TB : 1];
   uint64_t spill_mem[STACK_CAP];
   RingStack<LDS_SLOTS> stack;
-  stack.init(lds_stack + threadIdx.x, spill_mem);
-  float smin = INFINITY;  // least entry distance on the stack (closest hit)
+  stack.init(lds_stack, spill_mem);
+  int smin = DIST_NONE;  // least entry distance on the stack (closest hit)
   uint32_t cur = sc.root;
   bool occluded = false;
   // every node and triangle record is reached at most once per ray, so the
@@ -560,12 +581,12 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
         break;
       }
       NodeHit h;
-      intersect_node(sc.nodes, cur, r, lim, h);
+      intersect_node<OCCLUDED>(sc.nodes, cur, r, lim, h);
       if (COUNT) {
         nvis++;
         if (node_visits) atomicAdd(&node_visits[cur], 1u);
       }
-      if (OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, err, cur)) {
+      if (OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)) {
         continue;
       }
     } else {
@@ -602,18 +623,19 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
     }
     // pop the next entry that can still hold a closer hit
     bool got = false;
+    const int dlim = dist_limit(lim);
     while (!stack.empty()) {
       const uint2 e = stack.pop();
       if (!OCCLUDED) smin = below_dist(e.y);
-      if (OCCLUDED || entry_dist(e.y) <= lim) {
+      if (OCCLUDED || (int)e.y <= dlim) {
         cur = e.x;
         got = true;
         break;
       }
-      if (smin > lim) {
+      if (smin > dlim) {
         // every entry left is farther than the closest hit so far
         stack.clear();
-        smin = INFINITY;
+        smin = DIST_NONE;
         break;
       }
     }
@@ -678,8 +700,8 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
   __shared__ uint64_t lds_stack[LDS_SLOTS > 0 ? LDS_SLOTS * TB : 1];
   uint64_t spill_mem[STACK_CAP];
   RingStack<LDS_SLOTS> stack;
-  stack.init(lds_stack + threadIdx.x, spill_mem);
-  float smin = INFINITY;  // least entry distance on the stack (closest hit)
+  stack.init(lds_stack, spill_mem);
+  int smin = DIST_NONE;  // least entry distance on the stack (closest hit)
 
   TRay r;
   Hit best;
@@ -727,8 +749,8 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
               best.u = best.v = best.ngx = best.ngy = best.ngz = 0.0f;
               lim = widen_up(tfar);
               cur = BATCH ? lroot : sc.root;
-              stack.init(lds_stack + threadIdx.x, spill_mem);
-              smin = INFINITY;
+              stack.init(lds_stack, spill_mem);
+              smin = DIST_NONE;
               occluded = false;
               nvis = ntri = 0;
               iter = 0;
@@ -758,12 +780,12 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
         done = true;
       } else {
         NodeHit h;
-        intersect_node(sc.nodes, cur, r, lim, h);
+        intersect_node<OCCLUDED>(sc.nodes, cur, r, lim, h);
         if (COUNT) {
           nvis++;
           if (node_visits) atomicAdd(&node_visits[cur], 1u);
         }
-        if (OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, err, cur)) {
+        if (OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)) {
           continue;  // next step descends into cur
         }
       }
@@ -806,18 +828,19 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
     if (!done) {
       // pop the next entry that can still hold a closer hit
       bool got = false;
+      const int dlim = dist_limit(lim);
       while (!stack.empty()) {
         const uint2 e = stack.pop();
         if (!OCCLUDED) smin = below_dist(e.y);
-        if (OCCLUDED || entry_dist(e.y) <= lim) {
+        if (OCCLUDED || (int)e.y <= dlim) {
           cur = e.x;
           got = true;
           break;
         }
-        if (smin > lim) {
+        if (smin > dlim) {
           // every entry left is farther than the closest hit so far
           stack.clear();
-          smin = INFINITY;
+          smin = DIST_NONE;
           break;
         }
       }
@@ -869,8 +892,8 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
   __shared__ uint64_t lds_stack[8 * TB];
   uint64_t spill_mem[STACK_CAP];
   RingStack<8> stack;
-  stack.init(lds_stack + threadIdx.x, spill_mem);
-  float smin = INFINITY;  // least entry distance on the stack (closest hit)
+  stack.init(lds_stack, spill_mem);
+  int smin = DIST_NONE;  // least entry distance on the stack (closest hit)
 
   TRay r;
   Hit best;
@@ -904,8 +927,8 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
             lim = widen_up(tfar);
             cur = sc.root;
             tri = NONE_REF;
-            stack.init(lds_stack + threadIdx.x, spill_mem);
-            smin = INFINITY;
+            stack.init(lds_stack, spill_mem);
+            smin = DIST_NONE;
             occluded = false;
             nvis = ntri = 0;
             iter = 0;
@@ -940,12 +963,12 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
         done = true;
       } else {
         NodeHit h;
-        intersect_node(sc.nodes, cur, r, lim, h);
+        intersect_node<OCCLUDED>(sc.nodes, cur, r, lim, h);
         if (COUNT) {
           nvis++;
           if (node_visits) atomicAdd(&node_visits[cur], 1u);
         }
-        if (!(OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, err, cur))) {
+        if (!(OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur))) {
           cur = NONE_REF;
         }
       }
@@ -982,17 +1005,18 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
     }
     // the node cursor takes the next entry that can still hold a closer hit
     if (!done && cur == NONE_REF) {
+      const int dlim = dist_limit(lim);
       while (!stack.empty()) {
         const uint2 e = stack.pop();
         if (!OCCLUDED) smin = below_dist(e.y);
-        if (OCCLUDED || entry_dist(e.y) <= lim) {
+        if (OCCLUDED || (int)e.y <= dlim) {
           cur = e.x;
           break;
         }
-        if (smin > lim) {
+        if (smin > dlim) {
           // every entry left is farther than the closest hit so far
           stack.clear();
-          smin = INFINITY;
+          smin = DIST_NONE;
           break;
         }
       }
@@ -1253,8 +1277,8 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
   __shared__ float4 lds_world[3 * TB];
   uint64_t spill_mem[STACK_CAP];
   RingStack<8> stack;
-  stack.init(lds_stack + threadIdx.x, spill_mem);
-  float smin = INFINITY;  // least entry distance on the stack (closest hit)
+  stack.init(lds_stack, spill_mem);
+  int smin = DIST_NONE;  // least entry distance on the stack (closest hit)
 
   TRay r;
   Hit best;
@@ -1298,8 +1322,8 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
               cur = top.root;
               in_obj = false;
               moved = false;
-              stack.init(lds_stack + threadIdx.x, spill_mem);
-              smin = INFINITY;
+              stack.init(lds_stack, spill_mem);
+              smin = DIST_NONE;
               occluded = false;
               iter = 0;
               active = true;
@@ -1334,8 +1358,8 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
           }
         }
         NodeHit h;
-        intersect_node(nodes, cur, r, lim, h);
-        if (OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, err, cur)) {
+        intersect_node<OCCLUDED>(nodes, cur, r, lim, h);
+        if (OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)) {
           continue;
         }
       }
@@ -1400,12 +1424,12 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
         const uint4 w = reinterpret_cast<const uint4*>(top.insts + ii)[3];
         const bool identity = (w.z & INST_IDENTITY) != 0u;
         // the rest of a multi-record leaf resumes after this instance
-        if (!(w.z & TRI_LAST) && !stack.push(make_uint2((ii + 1u) | REF_LEAF, pack_dist(0xff80u, smin))))
+        if (!(w.z & TRI_LAST) && !stack.push(make_uint2((ii + 1u) | REF_LEAF, pack_dist(DIST_ALWAYS, smin))))
           atomicOr(err, 1u);
         if ((identity || ctx_inst == 0xffffffffu) && w.y < top.num_objects) {
           const DevScene o = top.objects[w.y];
           if (o.num_nodes > 0) {
-            if (!stack.push(make_uint2(REF_INST_EXIT, pack_dist(0xff80u, smin)))) atomicOr(err, 1u);
+            if (!stack.push(make_uint2(REF_INST_EXIT, pack_dist(DIST_ALWAYS, smin)))) atomicOr(err, 1u);
             if (!identity) {
               lds_world[threadIdx.x] = make_float4(r.ox, r.oy, r.oz, r.dx);
               lds_world[TB + threadIdx.x] = make_float4(r.dy, r.dz, r.rnx, r.rny);
@@ -1438,6 +1462,7 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
       // pop the next entry that can still hold a closer hit; an exit entry
       // returns the ray to world space
       bool got = false;
+      const int dlim = dist_limit(lim);
       while (!stack.empty()) {
         const uint2 e = stack.pop();
         if (!OCCLUDED) smin = below_dist(e.y);
@@ -1456,15 +1481,15 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
           }
           continue;
         }
-        if (OCCLUDED || entry_dist(e.y) <= lim) {
+        if (OCCLUDED || (int)e.y <= dlim) {
           cur = e.x;
           got = true;
           break;
         }
-        if (smin > lim) {
+        if (smin > dlim) {
           // every entry left is farther than the closest hit so far
           stack.clear();
-          smin = INFINITY;
+          smin = DIST_NONE;
           break;
         }
       }
