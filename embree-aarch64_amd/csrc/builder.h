@@ -99,12 +99,12 @@ struct DeviceBVH {
 // Scratch reused across builds on one device.
 struct BuildScratch {
   DevBuf geoms, lo4, hi4, keys, vals, slo, shi, child, parent_int, parent_leaf, range, nlo, nhi, cost,
-      isleaf, split8, visit, queue, counters, sacc, depth, lvl_hist, lvl_order, leaf_src;
+      isleaf, split8, visit, queue, counters, sacc, leaf_src;
+  DevBuf refit_list[2], refit_count;  // nodes that span chunks
   RadixSorter sorter;
   SahScratch sah;
   SpatialScratch spatial;
   LevelReadback rb;  // collapse level counters
-  PinnedBuf lvl_host;  // refit level histogram and offsets
 };
 
 // A binary tree over caller boxes with the SAH-optimal collapse decisions

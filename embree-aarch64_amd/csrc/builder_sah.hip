@@ -87,8 +87,7 @@ struct Counters {
                         // and clears (L + 2) % 3 for the level after)
   uint32_t ntiny;       // tiny segments so far (all levels)
   uint32_t error;    // bit 0: a segment list overflowed, bit 1: bin counts disagree, bit 2: destination out of range,
-                     // bit 3: median subtree stack overflow, bit 4: a tiny segment out of range,
-                     // bit 5: a depth beyond 254
+                     // bit 3: median subtree stack overflow, bit 4: a tiny segment out of range
 };
 
 struct Lists {
@@ -109,13 +108,7 @@ struct Tree {
   uint32_t* vals;
   Counters* cnt;
   uint32_t* roots;  // per tree
-  uint8_t* depth;   // binary depth of each inner node (0xff: unused id)
 };
-
-__device__ inline void set_depth(const Tree& t, uint32_t m, uint32_t d) {
-  if (d > 254u) atomicOr(&t.cnt->error, 32u);
-  t.depth[m] = (uint8_t)(d > 254u ? 254u : d);
-}
 
 struct Mapping {
   float ofs[3], scale[3];
@@ -251,7 +244,6 @@ __device__ inline void link_inner(const Tree& t, const Seg& sg, uint32_t m) {
     t.parent_int[m] = sg.parent;
   }
   t.range[m] = make_uint2(sg.first, sg.first + sg.count - 1);
-  set_depth(t, m, sg.meta >> 1);
 }
 
 // The whole subtree of a small segment [first, first+count) (child `side`
@@ -272,7 +264,6 @@ __device__ inline void finish_median(const Tree& t, uint32_t m, uint32_t side, u
     t.child[2 * p + (meta & 1u)] = mid;
     t.parent_int[mid] = p;
     t.range[mid] = make_uint2(f, f + c - 1);
-    set_depth(t, mid, d);
     const uint32_t cf[2] = {f, f + nl}, cc[2] = {nl, c - nl};
 #pragma unroll
     for (int s = 0; s < 2; s++) {
@@ -1393,7 +1384,6 @@ __device__ inline void tiny_groups(const TinyItem* q, int nq, const Bufs& B, con
       t.child[2 * np + (nm & 1u)] = mid;
       t.parent_int[mid] = np;
       t.range[mid] = make_uint2(first + nf, first + nf + nc - 1u);
-      set_depth(t, mid, nm >> 1);
     }
     group_sync<true>();
     if (busy) {
@@ -1451,7 +1441,7 @@ __global__ void k_fill_seg_ids(uint32_t* sid, const Seg* segs) {
 
 void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4* shi,
                     const std::vector<SahRoot>& trees, uint32_t* child, uint32_t* parent_int,
-                    uint32_t* parent_leaf, uint2* range, uint8_t* depth, const LearnedCost* learned,
+                    uint32_t* parent_leaf, uint2* range, const LearnedCost* learned,
                     uint32_t fin_max, SahScratch& S, SahTreeOut& out, hipStream_t s) {
   if (fin_max > MEDIAN_MAX) fin_max = MEDIAN_MAX;
   LearnedCost lcost{};
@@ -1489,7 +1479,6 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
   hipLaunchKernelGGL(k_fill_u32, dim3(div_up(n - 1, TBS)), dim3(TBS), 0, s, parent_int, (size_t)(n - 1), REF_EMPTY);
   hipLaunchKernelGGL(k_fill_u32, dim3(div_up(trees.size(), TBS)), dim3(TBS), 0, s, S.roots.as<uint32_t>(),
                      trees.size(), NIL);
-  RTG_HIP(hipMemsetAsync(depth, 0xff, (size_t)(n - 1), s));
 
   // trees start as big, mid or small segments of the level loop (a tree's
   // root is split by bins even when tiny)
@@ -1527,7 +1516,7 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
   RTG_HIP(hipMemcpyAsync(cnt, &hc, sizeof(hc), hipMemcpyHostToDevice, s));
   RTG_HIP(hipStreamSynchronize(s));  // the host staging above must outlive its copies
 
-  Tree t{child, parent_int, parent_leaf, range, vals, cnt, S.roots.as<uint32_t>(), depth};
+  Tree t{child, parent_int, parent_leaf, range, vals, cnt, S.roots.as<uint32_t>()};
   // Level l reads the segment lists of parity l & 1 and fills those of the
   // other parity; its kernels take their segment counts from the device, so
   // the host queues level l + 1 before it knows whether level l left any
