@@ -99,12 +99,13 @@ struct DeviceBVH {
 // Scratch reused across builds on one device.
 struct BuildScratch {
   DevBuf geoms, lo4, hi4, keys, vals, slo, shi, child, parent_int, parent_leaf, range, nlo, nhi, cost,
-      isleaf, split8, visit, queue, counters, sacc, leaf_src;
+      isleaf, split8, visit, counters, sacc, leaf_src, roots;
+  DevBuf walk_top, walk_sub, walk_rest, walk_count, walk_stats;  // wide nodes, numbered and then written
   DevBuf refit_list[2], refit_count;  // nodes that span chunks
   RadixSorter sorter;
+  Scanner scanner;
   SahScratch sah;
   SpatialScratch spatial;
-  LevelReadback rb;  // collapse level counters
 };
 
 // A binary tree over caller boxes with the SAH-optimal collapse decisions

@@ -23,7 +23,8 @@ struct BuildCounters {
   uint32_t valid;
   uint32_t node_count;
   uint32_t tri_count;
-  uint32_t qcount[3];  // collapse level k reads slot (k + 2) % 3, fills k % 3, clears (k + 1) % 3
+  uint32_t top_nodes;  // nodes that k_walk_top numbered
+  uint32_t subtrees;   // subtrees that it left to k_walk_rest
   uint32_t max_depth;
   uint32_t error;  // bit 0: refit walk too long, bit 1: collapse index out of range, bit 2: bad tree
   uint32_t max_stack;  // most traversal stack entries any root-to-node path can need
@@ -34,11 +35,12 @@ struct BuildCounters {
 constexpr uint32_t NONE = 0xffffffffu;
 constexpr int BT = 256;
 
-struct QItem {
-  uint32_t bref;  // binary ref: REF_LEAF | sorted prim index, or inner node index
-  uint32_t node;  // QNode8 slot
-  uint32_t depth;
-  uint32_t need;  // stack entries the traversal may hold on reaching this node
+// A node of the 8-wide tree to come.
+struct WideNode {
+  uint32_t bref;   // binary ref: REF_LEAF | sorted prim index, or inner node index
+  uint32_t tri;    // first of its subtree's leaf records (as many as it has primitives)
+  uint32_t level;  // depth << 16 | stack entries the traversal may hold on reaching it
+  uint32_t link;   // while it waits: its own number; when walked: the number of its first inner child
 };
 
 // ------------------------------------------------------------ reductions --
@@ -108,9 +110,8 @@ __global__ void k_init_counters(BuildCounters* c, uint32_t nscenes) {
   c->node_count = nscenes;
   c->roots_seen = 0;
   c->tri_count = 0;
-  c->qcount[0] = 0;
-  c->qcount[1] = 0;
-  c->qcount[2] = nscenes;  // the collapse's first level reads slot 2: one root item per scene
+  c->top_nodes = 0;
+  c->subtrees = 0;
   c->max_depth = 0;
   c->max_stack = 0;
   c->error = 0;
@@ -652,12 +653,8 @@ __global__ __launch_bounds__(BT) void k_check_tree(const uint32_t* __restrict__ 
 
 // ---------------------------------------------------------------- collapse --
 
+// The binary tree and its collapse table as the walk and the emission read them.
 struct CollapseArgs {
-  const QItem* qin;
-  QItem* qout;
-  const uint32_t* nin;  // items in qin (a device counter)
-  uint32_t qout_slot;
-  uint32_t* qclear;     // the count the next level fills, cleared here (no kernel of this level uses it)
   const uint32_t* child;
   const uint2* range;
   const float4* nlo;
@@ -666,13 +663,21 @@ struct CollapseArgs {
   const uint8_t* split8;
   const float4* slo;
   const float4* shi;
+  BuildCounters* cnt;
+  uint32_t nscenes;
+  uint32_t n;         // primitives
+  uint32_t width;     // children per node (2..8)
+  uint32_t max_sub;   // subtrees that the arrays below hold
+  WideNode* top;      // top node i
+  WideNode* sub;      // roots of the subtrees, waiting
+  WideNode* rest;     // node i of subtree f at sub[f].tri + i
+  uint32_t* count;    // nodes of each subtree without its root, and (prefix) their exclusive sums
+  const uint32_t* prefix;
   QNode8* nodes;
   uint32_t* leaf_src; // position of each leaf record's primitive, bit 31: last of its leaf
   NodeInfo* info;
-  BuildCounters* cnt;
-  uint32_t n;         // capacity of nodes and of each queue
-  uint32_t tri_cap;   // capacity of tris
-  uint32_t width;     // children per node (2..8)
+  uint32_t cap;       // capacity of nodes
+  struct CollapseStats* stats;  // of each workgroup of the emission
 };
 
 constexpr uint32_t LEAF_SRC_LAST = 0x80000000u;  // positions are below 2^31 (REF_LEAF marks them likewise)
@@ -712,280 +717,257 @@ __device__ inline uint32_t quant_hi(float v, float p, float s) {
 // Byte k of a node's eight split bytes loaded as one uint2.
 __device__ inline uint32_t split_byte(uint2 s8, uint32_t k) { return ((k < 4 ? s8.x : s8.y) >> (8 * (k & 3))) & 0xffu; }
 
-// Statistics of the nodes a thread wrote, reduced over the wave before
-// the global atomics (one per item would serialise on their addresses).
+// The children of a wide node: the optimal distribution of `width` slots below
+// inner node b, handed to `found` in order. Returns their number, 0 on a table
+// that asks for more than 8.
+template <class Found>
+__device__ inline int wide_children(const CollapseArgs& a, uint32_t b, Found found) {
+  uint32_t st_ref[8], st_s[8];
+  int n = 0, sp = 2;
+  const uint32_t j8 = (a.split8[8 * (size_t)b + a.width - 1]) & 7u;
+  st_ref[0] = a.child[2 * b + 1]; st_s[0] = a.width - j8;
+  st_ref[1] = a.child[2 * b];     st_s[1] = j8;
+  while (sp > 0 && n < 8) {
+    sp--;
+    uint32_t c = st_ref[sp], slots = st_s[sp];
+    uint2 s8 = make_uint2(0u, 0u), cp = make_uint2(0u, 0u);
+    if (!(c & REF_LEAF)) {
+      // the node's eight split bytes and its child pair: two 8 B loads
+      // issued together, not a byte load per slot count and then the pair
+      s8 = *reinterpret_cast<const uint2*>(a.split8 + 8 * (size_t)c);
+      cp = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)c);
+      while (slots > 1 && (split_byte(s8, slots - 1) & 0x80u)) slots--;
+    } else {
+      slots = 1;
+    }
+    if (slots <= 1) {
+      found(n, c);
+      n++;
+    } else {
+      const uint32_t jj = split_byte(s8, slots - 1) & 7u;
+      if (sp + 2 > 8) {
+        atomicOr(&a.cnt->error, 128u);
+        return 0;
+      }
+      st_ref[sp] = cp.y; st_s[sp] = slots - jj; sp++;
+      st_ref[sp] = cp.x; st_s[sp] = jj;         sp++;
+    }
+  }
+  return n;
+}
+
+// The collapse numbers the wide nodes first (the walk: only links, counts and
+// leaf flags are read) and then writes them all at once (the emission: boxes
+// and quantisation). A wide node owns as many leaf records as it has
+// primitives: its leaves take the first, its inner children the rest in turn.
+// Node numbers need a counter, which lives in LDS: one workgroup walks the top
+// of the tree, then each subtree has a workgroup, and the subtrees' node counts
+// are summed before the emission. (A launch for each level with its slots from
+// counters in HBM took 28 us a level on small trees, and on large ones the
+// atomics of all workgroups on those counters passed one at a time, about
+// 40 ns each: 2^20 triangles 1.20 -> 0.95 ms for a Morton build, 3.20 -> 2.96
+// for binned SAH; 131,000 triangles 0.68 -> 0.50 and 1.46 -> 1.33 ms.)
+// The top is every node with more than 1/256 of the primitives, so fewer than
+// 256 on a level (a thread each), and the subtrees take about the same time.
+constexpr uint32_t TOP_SHARE = 256, TOP_LEVELS = 256;
+constexpr uint32_t TOP_MIN = 512;   // primitives that are always one subtree (a level of the top takes 12 us, of a subtree 8)
+constexpr uint32_t SUB_MAX = 2047;  // subtrees beside the scenes (their sums are one scan launch)
+// Top nodes: fewer than TOP_SHARE on each level, the subtrees' roots, the scenes.
+__host__ __device__ inline uint32_t top_cap(uint32_t max_sub) { return max_sub + TOP_SHARE * TOP_LEVELS; }
+
+// Walks one wide node: `take` gives the first of ni numbers for its inner
+// children, `put` gets each of them with its primitive count, and `record` the
+// first number, for the node's own record.
+template <class Take, class Put, class Record>
+__device__ inline void walk_node(const CollapseArgs& a, const WideNode& w, Take take, Put put, Record record) {
+  uint32_t ref[8], cnt[8];
+  int n = 0;
+  if (w.bref != REF_EMPTY && is_inner(w.bref, a.isleaf))
+    n = wide_children(a, w.bref, [&](int i, uint32_t c) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) ref[j] = i == j ? c : ref[j];
+    });
+  uint32_t ni = 0, nt = 0, inner = 0;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    if (j >= n) continue;
+    cnt[j] = 1u;
+    bool in = false;
+    if (!(ref[j] & REF_LEAF)) {
+      const uint2 r = a.range[ref[j]];
+      cnt[j] = r.y - r.x + 1u;
+      in = !a.isleaf[ref[j]];
+    }
+    if (in) {
+      inner |= 1u << j;
+      ni++;
+    } else {
+      nt += cnt[j];
+    }
+  }
+  const uint32_t first = ni ? take(ni) : 0u;
+  const uint32_t level = w.level + (1u << 16) + (n ? (uint32_t)n - 1u : 0u);  // a node pushes at most n-1 of its n children
+  uint32_t k = 0, tri = w.tri + nt;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    if (!((inner >> j) & 1u)) continue;
+    put(cnt[j], WideNode{ref[j], tri, level, first + k});
+    tri += cnt[j];
+    k++;
+  }
+  record(first);
+}
+
+__global__ __launch_bounds__(BT) void k_walk_top(CollapseArgs a, const uint32_t* __restrict__ roots,
+                                                 const uint32_t* __restrict__ first,
+                                                 const uint32_t* __restrict__ prims) {
+  __shared__ WideNode level[2][TOP_SHARE];
+  __shared__ uint32_t nlevel[2], nodes, nsub, run;
+  if (threadIdx.x == 0) {
+    run = a.cnt->error ? 0u : 1u;  // a tree that failed its check is not followed
+    nodes = a.nscenes;
+    nsub = nlevel[0] = nlevel[1] = 0u;
+  }
+  __syncthreads();
+  if (!run) return;
+  uint32_t in = 0;
+  const uint32_t share = max(a.n / TOP_SHARE, TOP_MIN);
+  // a wide node joins the next level's list or the subtrees
+  auto place = [&](uint32_t to, uint32_t cnt, const WideNode& w) {
+    if (cnt > share) {
+      const uint32_t at = atomicAdd(&nlevel[to], 1u);
+      if (at < TOP_SHARE) level[to][at] = w;
+      else atomicOr(&a.cnt->error, 2u);
+    } else {
+      const uint32_t at = atomicAdd(&nsub, 1u);
+      if (at < a.max_sub) a.sub[at] = w;
+      else atomicOr(&a.cnt->error, 2u);
+    }
+  };
+  for (uint32_t i = threadIdx.x; i < a.nscenes; i += BT) place(0, prims[i], WideNode{roots[i], first[i], 1u << 16, i});
+  __syncthreads();
+  while (true) {
+    const uint32_t count = min(nlevel[in], TOP_SHARE);
+    // (each walked node may add 8 subtrees)
+    if (count == 0u || nsub + 8u * count > a.max_sub) break;
+    if (threadIdx.x < count) {
+      const WideNode w = level[in][threadIdx.x];
+      walk_node(
+          a, w, [&](uint32_t ni) { return atomicAdd(&nodes, ni); },
+          [&](uint32_t cnt, const WideNode& c) { place(in ^ 1u, cnt, c); },
+          [&](uint32_t f) {
+            if (w.link < top_cap(a.max_sub)) a.top[w.link] = WideNode{w.bref, w.tri, w.level, f};
+            else atomicOr(&a.cnt->error, 2u);
+          });
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) nlevel[in] = 0u;
+    in ^= 1u;
+    __syncthreads();
+  }
+  // (of unusually narrow trees) the level that was not walked
+  const uint32_t count = min(nlevel[in], TOP_SHARE);
+  if (threadIdx.x < count && nsub + threadIdx.x < a.max_sub) a.sub[nsub + threadIdx.x] = level[in][threadIdx.x];
+  if (threadIdx.x == 0) {
+    a.cnt->top_nodes = nodes;
+    a.cnt->subtrees = min(nsub + count, a.max_sub);
+  }
+}
+
+// The subtrees, a workgroup each: up to 256 waiting nodes are walked at a time,
+// last first, from a stack in LDS. Where the stack could fill up, fewer are
+// taken, down to one, which needs 7 entries a level.
+constexpr uint32_t REST_STACK = 3072, REST_SPARE = 7 * 128;
+
+__global__ __launch_bounds__(BT) void k_walk_rest(CollapseArgs a) {
+  __shared__ WideNode stack[REST_STACK];
+  __shared__ uint32_t count, nodes, run;
+  if (threadIdx.x == 0) run = a.cnt->error ? 0u : 1u;
+  __syncthreads();
+  const uint32_t nsub = run ? a.cnt->subtrees : 0u;
+  for (uint32_t f = blockIdx.x; f <= a.max_sub; f += gridDim.x) {
+    if (f >= nsub) {  // (the sums run over all of the array)
+      if (threadIdx.x == 0) a.count[f] = 0u;
+      continue;
+    }
+    const WideNode root = a.sub[f];
+    if (threadIdx.x == 0) {
+      stack[0] = root;
+      count = 1u;
+      nodes = 0u;
+    }
+    __syncthreads();
+    for (bool top = true;; top = false) {
+      const uint32_t c = count;
+      if (c == 0u) break;
+      const uint32_t room = REST_STACK - REST_SPARE > c ? (REST_STACK - REST_SPARE - c) / 7u : 0u;
+      const uint32_t m = min(min(c, (uint32_t)BT), max(room, 1u));
+      WideNode w{};
+      if (threadIdx.x < m) w = stack[c - 1u - threadIdx.x];
+      __syncthreads();
+      if (threadIdx.x == 0) count = c - m;
+      __syncthreads();
+      if (threadIdx.x < m) {
+        uint32_t at = 0;
+        walk_node(
+            a, w,
+            [&](uint32_t ni) {
+              at = atomicAdd(&count, ni);
+              return atomicAdd(&nodes, ni);
+            },
+            [&](uint32_t, const WideNode& ch) {
+              if (at < REST_STACK) stack[at++] = ch;
+              else atomicOr(&a.cnt->error, 2u);
+            },
+            [&](uint32_t i) {
+              if (top && root.link < top_cap(a.max_sub)) a.top[root.link] = WideNode{w.bref, w.tri, w.level, REF_LEAF | f};
+              else if (!top && root.tri + w.link < a.n) a.rest[root.tri + w.link] = WideNode{w.bref, w.tri, w.level, i};
+              else atomicOr(&a.cnt->error, 2u);
+            });
+      }
+      __syncthreads();
+      if (threadIdx.x == 0 && count > REST_STACK) count = 0u;  // (reported above)
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) a.count[f] = nodes;
+    __syncthreads();
+  }
+}
+
+// Statistics of the nodes that a thread, then a workgroup, wrote.
 struct CollapseStats {
-  uint32_t max_depth = 0, max_stack = 0;
+  uint32_t max_depth = 0, max_stack = 0, records = 0;
   double sah_nodes = 0.0, sah_leaves = 0.0, sah_leaves_tri = 0.0;
+  __device__ void add(const CollapseStats& o) {
+    max_depth = max(max_depth, o.max_depth);
+    max_stack = max(max_stack, o.max_stack);
+    records += o.records;
+    sah_nodes += o.sah_nodes;
+    sah_leaves += o.sah_leaves;
+    sah_leaves_tri += o.sah_leaves_tri;
+  }
 };
 
-// Node, record and queue slots for the workgroup's items in one atomic per
-// counter (atomics on one address from every wave would serialise): the
-// bit-sliced ballot sums give each lane its offset within the wave, LDS
-// the waves' offsets within the workgroup. Called by every thread of the
-// workgroup; ni (children that are inner nodes) is below 16 and nt (leaf
-// records) below 512.
-__device__ inline void block_alloc(BuildCounters* cnt, uint32_t qslot, uint32_t ni, uint32_t nt, uint32_t& child_base,
-                                   uint32_t& tri_base, uint32_t& qbase) {
-  __shared__ uint32_t wtot[BT / 64][2], bbase[3];
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint64_t below = lane == 0u ? 0ull : (~0ull >> (64u - lane));
-  uint32_t pi = 0u, ti = 0u, pt = 0u, tt = 0u;
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    const uint64_t m = __ballot((ni >> b) & 1u);
-    pi += (uint32_t)__popcll(m & below) << b;
-    ti += (uint32_t)__popcll(m) << b;
-  }
-#pragma unroll
-  for (int b = 0; b < 9; b++) {
-    const uint64_t m = __ballot((nt >> b) & 1u);
-    pt += (uint32_t)__popcll(m & below) << b;
-    tt += (uint32_t)__popcll(m) << b;
-  }
-  if (lane == 0u) {
-    wtot[wave][0] = ti;
-    wtot[wave][1] = tt;
-  }
+// The workgroup's statistics, in thread 0.
+__device__ inline void block_stats(CollapseStats& st) {
+  __shared__ __align__(8) char mem[BT / 64 * sizeof(CollapseStats)];
+  CollapseStats* w = reinterpret_cast<CollapseStats*>(mem);
+  st.max_depth = wave_umax(st.max_depth);
+  st.max_stack = wave_umax(st.max_stack);
+  st.records = wave_sum(st.records);
+  st.sah_nodes = wave_sum(st.sah_nodes);
+  st.sah_leaves = wave_sum(st.sah_leaves);
+  st.sah_leaves_tri = wave_sum(st.sah_leaves_tri);
+  if ((threadIdx.x & 63u) == 0u) w[threadIdx.x >> 6] = st;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t si = 0u, st = 0u;
-    for (int w = 0; w < BT / 64; w++) {
-      si += wtot[w][0];
-      st += wtot[w][1];
-    }
-    bbase[0] = si ? atomicAdd(&cnt->node_count, si) : 0u;
-    bbase[1] = st ? atomicAdd(&cnt->tri_count, st) : 0u;
-    bbase[2] = si ? atomicAdd(&cnt->qcount[qslot], si) : 0u;
-  }
-  __syncthreads();
-  uint32_t oi = 0u, ot = 0u;
-  for (uint32_t w = 0; w < wave; w++) {
-    oi += wtot[w][0];
-    ot += wtot[w][1];
-  }
-  child_base = bbase[0] + oi + pi;
-  tri_base = bbase[1] + ot + pt;
-  qbase = bbase[2] + oi + pi;
-  __syncthreads();  // wtot and bbase are reused by the next item
+  if (threadIdx.x == 0)
+    for (int i = 1; i < BT / 64; i++) st.add(w[i]);
 }
 
-// One item (an 8-wide node to write) per thread, for the levels with many
-// items (throughput); every thread of the workgroup calls it (active: the
-// thread has an item), for block_alloc.
-__device__ inline void collapse_item1(const CollapseArgs& a, uint32_t t, bool active, CollapseStats& st) {
-  bool go = active;
-  QItem item{};
-  if (go) item = a.qin[t];
-  const float eps = o2f(a.cnt->maxabs) * BOX_EPS_REL;
-  if (go && item.bref == REF_EMPTY) {  // root of a scene without primitives: a node with no children
-    go = false;
-    if (item.node >= a.n) {
-      atomicOr(&a.cnt->error, 2u);
-    } else {
-    QNode8 q;
-    q.px = q.py = q.pz = 0.0f;
-    q.ex = q.ey = q.ez = 127;
-    q.imask = 0;
-    q.child_base = q.tri_base = 0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      q.meta[k] = 0;
-      q.qlox[k] = q.qloy[k] = q.qloz[k] = 255;
-      q.qhix[k] = q.qhiy[k] = q.qhiz[k] = 0;
-    }
-    a.nodes[item.node] = q;
-    NodeInfo inf;
-    inf.lo[0] = inf.lo[1] = inf.lo[2] = 0.0f;
-    inf.hi[0] = inf.hi[1] = inf.hi[2] = 0.0f;
-    inf.count = 0;
-    inf.depth = item.depth;
-    a.info[item.node] = inf;
-    }
-  }
-
-  // children: the optimal distribution of 8 slots below item.bref
-  uint32_t ch[8];
-  int n = 0;
-  if (!go) {
-  } else if (!is_inner(item.bref, a.isleaf)) {
-    ch[0] = item.bref;  // whole (small) scene as one leaf
-    n = 1;
-  } else {
-    uint32_t st_ref[8], st_s[8];
-    int sp = 0;
-    {
-      const uint32_t j8 = (a.split8[8 * (size_t)item.bref + a.width - 1]) & 7u;
-      st_ref[0] = a.child[2 * item.bref + 1]; st_s[0] = a.width - j8;
-      st_ref[1] = a.child[2 * item.bref];     st_s[1] = j8;
-      sp = 2;
-    }
-    while (sp > 0 && n < 8) {
-      sp--;
-      uint32_t c = st_ref[sp], slots = st_s[sp];
-      uint2 s8 = make_uint2(0u, 0u), cp = make_uint2(0u, 0u);
-      if (!(c & REF_LEAF)) {
-        // the node's eight split bytes and its child pair: two 8 B loads
-        // issued together, not a byte load per slot count and then the pair
-        s8 = *reinterpret_cast<const uint2*>(a.split8 + 8 * (size_t)c);
-        cp = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)c);
-        while (slots > 1 && (split_byte(s8, slots - 1) & 0x80u)) slots--;
-      } else {
-        slots = 1;
-      }
-      if (slots <= 1) {
-        ch[n++] = c;
-      } else {
-        const uint32_t jj = split_byte(s8, slots - 1) & 7u;
-        if (sp + 2 > 8) {
-          atomicOr(&a.cnt->error, 128u);
-          go = false;
-          n = 0;
-          break;
-        }
-        st_ref[sp] = cp.y; st_s[sp] = slots - jj; sp++;
-        st_ref[sp] = cp.x; st_s[sp] = jj;         sp++;
-      }
-    }
-  }
-
-  // per-child primitive ranges live in LDS (one row per thread)
-  __shared__ uint32_t s_first[BT][8];
-  __shared__ uint32_t s_count[BT][8];
-  const uint32_t* rng32 = reinterpret_cast<const uint32_t*>(a.range);
-  float bl[8][3], bh[8][3];
-  uint32_t ni = 0, nt = 0, ninner_prims = 0;
-  uint32_t innerm = 0;  // bit k: child k is an inner node (kept for the writes below)
-  float ul[3] = {INFINITY, INFINITY, INFINITY}, uh[3] = {-INFINITY, -INFINITY, -INFINITY};
-  double sah_leaf = 0.0, sah_leaf_tri = 0.0;
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    if (k < n) {
-      const uint32_t c = ch[k];
-      float4 l, h;
-      uint32_t f, cnt;
-      if (c & REF_LEAF) {
-        l = a.slo[c & ~REF_LEAF];
-        h = a.shi[c & ~REF_LEAF];
-        f = c & ~REF_LEAF;
-        cnt = 1u;
-      } else {
-        l = a.nlo[c];
-        h = a.nhi[c];
-        f = rng32[2 * c];
-        cnt = rng32[2 * c + 1] - f + 1u;
-      }
-      s_first[threadIdx.x][k] = f;
-      s_count[threadIdx.x][k] = cnt;
-      bl[k][0] = l.x; bl[k][1] = l.y; bl[k][2] = l.z;
-      bh[k][0] = h.x; bh[k][1] = h.y; bh[k][2] = h.z;
-#pragma unroll
-      for (int d = 0; d < 3; d++) {
-        ul[d] = fminf(ul[d], bl[k][d]);
-        uh[d] = fmaxf(uh[d], bh[k][d]);
-      }
-      if (is_inner(c, a.isleaf)) {
-        innerm |= 1u << k;
-        ni++;
-        ninner_prims += cnt;
-      } else {
-        nt += cnt;
-        const float A = box_half_area(l, h);
-        sah_leaf += (double)A * (double)((cnt + 3) / 4);
-        sah_leaf_tri += (double)A * (double)cnt;
-      }
-    }
-  }
-  // the children partition the parent's range: a second count of the leaf primitives
-  if (go) {
-    const uint32_t b = item.bref;
-    const uint32_t total_prims = (b & REF_LEAF) ? 1u : (rng32[2 * b + 1] - rng32[2 * b] + 1u);
-    if (total_prims - ninner_prims != nt) atomicOr(&a.cnt->error, 64u);
-  }
-  // node, record and queue slots: one atomic per workgroup and counter
-  uint32_t child_base, tri_base, qbase;
-  block_alloc(a.cnt, a.qout_slot, go ? ni : 0u, go ? nt : 0u, child_base, tri_base, qbase);
-  if (!go) return;
-  if ((uint64_t)child_base + ni > a.n || (uint64_t)tri_base + nt > a.tri_cap || (uint64_t)qbase + ni > a.n ||
-      item.node >= a.n) {
-    atomicOr(&a.cnt->error, 2u);
-    return;
-  }
-  st.max_depth = max(st.max_depth, item.depth);
-  // a node pushes at most n-1 of its n children
-  const uint32_t need = item.need + (uint32_t)n - 1u;
-  st.max_stack = max(st.max_stack, need);
-  st.sah_nodes += (double)half_area(uh[0] - ul[0], uh[1] - ul[1], uh[2] - ul[2]);
-  if (nt) {
-    st.sah_leaves += sah_leaf;
-    st.sah_leaves_tri += sah_leaf_tri;
-  }
-
-  // quantisation grid over the widened union box
-  QNode8 q;
-  float p[3], s[3];
-  uint32_t e[3];
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    p[d] = ul[d] - eps;
-    e[d] = grid_exponent(p[d], uh[d] + eps);
-    s[d] = __uint_as_float(e[d] << 23);
-  }
-  q.px = p[0]; q.py = p[1]; q.pz = p[2];
-  q.ex = (uint8_t)e[0]; q.ey = (uint8_t)e[1]; q.ez = (uint8_t)e[2];
-  q.child_base = child_base;
-  q.tri_base = tri_base;
-  uint32_t imask = 0, rank_i = 0, off_t = 0;
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    if (k < n) {
-      const uint32_t c = ch[k];
-      const uint32_t qlx = quant_lo(bl[k][0] - eps, p[0], s[0]), qhx = quant_hi(bh[k][0] + eps, p[0], s[0]);
-      const uint32_t qly = quant_lo(bl[k][1] - eps, p[1], s[1]), qhy = quant_hi(bh[k][1] + eps, p[1], s[1]);
-      const uint32_t qlz = quant_lo(bl[k][2] - eps, p[2], s[2]), qhz = quant_hi(bh[k][2] + eps, p[2], s[2]);
-      q.qlox[k] = (uint8_t)qlx; q.qhix[k] = (uint8_t)qhx;
-      q.qloy[k] = (uint8_t)qly; q.qhiy[k] = (uint8_t)qhy;
-      q.qloz[k] = (uint8_t)qlz; q.qhiz[k] = (uint8_t)qhz;
-      if ((innerm >> k) & 1u) {
-        imask |= 1u << k;
-        q.meta[k] = (uint8_t)(0x80u | rank_i);
-        a.qout[qbase + rank_i] = QItem{c, child_base + rank_i, item.depth + 1, need};
-        rank_i++;
-      } else {
-        q.meta[k] = (uint8_t)(1u + off_t);
-        // leaf records are written afterwards, one thread each (k_write_leaves)
-        const uint32_t cntk = s_count[threadIdx.x][k];
-        const uint32_t firstk = s_first[threadIdx.x][k];
-        for (uint32_t j = 0; j < cntk; j++)
-          a.leaf_src[tri_base + off_t + j] = (firstk + j) | ((j + 1 == cntk) ? LEAF_SRC_LAST : 0u);
-        off_t += cntk;
-      }
-    } else {
-      q.meta[k] = 0;
-      q.qlox[k] = q.qloy[k] = q.qloz[k] = 255;
-      q.qhix[k] = q.qhiy[k] = q.qhiz[k] = 0;
-    }
-  }
-  q.imask = (uint8_t)imask;
-  a.nodes[item.node] = q;
-  NodeInfo inf;
-  inf.lo[0] = ul[0]; inf.lo[1] = ul[1]; inf.lo[2] = ul[2];
-  inf.hi[0] = uh[0]; inf.hi[1] = uh[1]; inf.hi[2] = uh[2];
-  inf.count = ninner_prims + nt;
-  inf.depth = item.depth;
-  a.info[item.node] = inf;
-}
-
-// One item (an 8-wide node to write) per group of CG = 8 lanes, for the
-// levels with few items (latency), lane k of the group taking slot k of the
-// node: the group descends the binary tree
-// together (every lane the same way) to the node's children, lane k keeps
-// child k, and the lanes then load, count, quantise and write their own
-// child's slot, with the node's union box, counts and slot ranks formed by
-// reductions and scans over the group. Every thread of the workgroup calls
-// it (active: the group has an item), for block_alloc.
+// Writing a node takes a group of CG lanes: every lane finds the children, lane
+// k then loads, quantises and writes child k, with shuffles for the node's box,
+// reductions and scans over the group.
 constexpr uint32_t CG = 8;
-constexpr uint32_t COLLAPSE_GROUPED_MAX = 8192;  // items of a level up to which groups take them
 
 template <class T>
 __device__ inline T group_sum(T v) {
@@ -1014,88 +996,49 @@ __device__ inline uint32_t group_prefix(uint32_t v, uint32_t k) {
   return x - v;
 }
 
-__device__ inline void collapse_item(const CollapseArgs& a, uint32_t t, bool active, uint32_t k, CollapseStats& st) {
-  bool go = active;
-  QItem item{};
-  if (go) item = a.qin[t];
+// Writes node number `number` (w.link: the number of its first inner child).
+__device__ inline void emit_node(const CollapseArgs& a, const WideNode& w, uint32_t number, uint32_t k, CollapseStats& st) {
   const float eps = o2f(a.cnt->maxabs) * BOX_EPS_REL;
-  if (go && item.bref == REF_EMPTY) {  // root of a scene without primitives: a node with no children
-    go = false;
+  const uint32_t depth = w.level >> 16;
+  if (number >= a.cap) {
+    if (k == 0) atomicOr(&a.cnt->error, 2u);
+    return;
+  }
+  if (w.bref == REF_EMPTY) {  // root of a scene without primitives: a node with no children
     if (k == 0) {
-      if (item.node >= a.n) {
-        atomicOr(&a.cnt->error, 2u);
-      } else {
-        QNode8 q;
-        q.px = q.py = q.pz = 0.0f;
-        q.ex = q.ey = q.ez = 127;
-        q.imask = 0;
-        q.child_base = q.tri_base = 0;
+      QNode8 q;
+      q.px = q.py = q.pz = 0.0f;
+      q.ex = q.ey = q.ez = 127;
+      q.imask = 0;
+      q.child_base = q.tri_base = 0;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-          q.meta[j] = 0;
-          q.qlox[j] = q.qloy[j] = q.qloz[j] = 255;
-          q.qhix[j] = q.qhiy[j] = q.qhiz[j] = 0;
-        }
-        a.nodes[item.node] = q;
-        NodeInfo inf;
-        inf.lo[0] = inf.lo[1] = inf.lo[2] = 0.0f;
-        inf.hi[0] = inf.hi[1] = inf.hi[2] = 0.0f;
-        inf.count = 0;
-        inf.depth = item.depth;
-        a.info[item.node] = inf;
+      for (int j = 0; j < 8; j++) {
+        q.meta[j] = 0;
+        q.qlox[j] = q.qloy[j] = q.qloz[j] = 255;
+        q.qhix[j] = q.qhiy[j] = q.qhiz[j] = 0;
       }
+      a.nodes[number] = q;
+      NodeInfo inf;
+      inf.lo[0] = inf.lo[1] = inf.lo[2] = 0.0f;
+      inf.hi[0] = inf.hi[1] = inf.hi[2] = 0.0f;
+      inf.count = 0;
+      inf.depth = depth;
+      a.info[number] = inf;
     }
+    return;
   }
 
-  // children: the optimal distribution of 8 slots below item.bref (the
-  // group's lanes take the same path); lane k keeps child k
+  // children (the group's lanes take the same path); lane k keeps child k
   uint32_t mine = 0u;
-  int n = 0;
-  if (!go) {
-  } else if (!is_inner(item.bref, a.isleaf)) {
-    mine = item.bref;  // whole (small) scene as one leaf
-    n = 1;
+  int n = 1;
+  if (!is_inner(w.bref, a.isleaf)) {
+    mine = w.bref;  // whole (small) scene as one leaf
   } else {
-    uint32_t st_ref[8], st_s[8];
-    int sp = 0;
-    {
-      const uint32_t j8 = (a.split8[8 * (size_t)item.bref + a.width - 1]) & 7u;
-      st_ref[0] = a.child[2 * item.bref + 1]; st_s[0] = a.width - j8;
-      st_ref[1] = a.child[2 * item.bref];     st_s[1] = j8;
-      sp = 2;
-    }
-    while (sp > 0 && n < 8) {
-      sp--;
-      uint32_t c = st_ref[sp], slots = st_s[sp];
-      uint2 s8 = make_uint2(0u, 0u), cp = make_uint2(0u, 0u);
-      if (!(c & REF_LEAF)) {
-        // the node's eight split bytes and its child pair: two 8 B loads
-        // issued together, not a byte load per slot count and then the pair
-        s8 = *reinterpret_cast<const uint2*>(a.split8 + 8 * (size_t)c);
-        cp = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)c);
-        while (slots > 1 && (split_byte(s8, slots - 1) & 0x80u)) slots--;
-      } else {
-        slots = 1;
-      }
-      if (slots <= 1) {
-        if ((uint32_t)n == k) mine = c;
-        n++;
-      } else {
-        const uint32_t jj = split_byte(s8, slots - 1) & 7u;
-        if (sp + 2 > 8) {
-          if (k == 0) atomicOr(&a.cnt->error, 128u);
-          go = false;
-          n = 0;
-          break;
-        }
-        st_ref[sp] = cp.y; st_s[sp] = slots - jj; sp++;
-        st_ref[sp] = cp.x; st_s[sp] = jj;         sp++;
-      }
-    }
+    n = wide_children(a, w.bref, [&](int i, uint32_t c) { mine = (uint32_t)i == k ? c : mine; });
   }
 
   // this lane's child: box, primitive range and kind
-  const bool has = go && k < (uint32_t)n;
+  const bool has = k < (uint32_t)n;
   const uint32_t* rng32 = reinterpret_cast<const uint32_t*>(a.range);
   float4 l = make_float4(INFINITY, INFINITY, INFINITY, 0.0f), h = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
   uint32_t f = 0u, cnt = 0u;
@@ -1129,30 +1072,20 @@ __device__ inline void collapse_item(const CollapseArgs& a, uint32_t t, bool act
   sah_leaf = group_sum(sah_leaf);
   sah_leaf_tri = group_sum(sah_leaf_tri);
   // the children partition the parent's range: a second count of the leaf primitives
-  if (go && k == 0) {
-    const uint32_t b = item.bref;
+  if (k == 0) {
+    const uint32_t b = w.bref;
     const uint32_t total_prims = (b & REF_LEAF) ? 1u : (rng32[2 * b + 1] - rng32[2 * b] + 1u);
     if (total_prims - ninner_prims != nt) atomicOr(&a.cnt->error, 64u);
   }
-  // node, record and queue slots: one atomic per workgroup and counter (the
-  // group's first lane asks for the group)
-  uint32_t child_base, tri_base, qbase;
-  block_alloc(a.cnt, a.qout_slot, (go && k == 0) ? ni : 0u, (go && k == 0) ? nt : 0u, child_base, tri_base, qbase);
-  const int first_lane = (int)((threadIdx.x & 63u) & ~(CG - 1u));
-  child_base = (uint32_t)__shfl((int)child_base, first_lane, 64);
-  tri_base = (uint32_t)__shfl((int)tri_base, first_lane, 64);
-  qbase = (uint32_t)__shfl((int)qbase, first_lane, 64);
-  if (!go) return;
-  if ((uint64_t)child_base + ni > a.n || (uint64_t)tri_base + nt > a.tri_cap || (uint64_t)qbase + ni > a.n ||
-      item.node >= a.n) {
+  const uint32_t child_base = w.link, tri_base = w.tri;
+  if ((uint64_t)child_base + ni > a.cap || (uint64_t)tri_base + nt + ninner_prims > a.n) {
     if (k == 0) atomicOr(&a.cnt->error, 2u);
     return;
   }
-  // a node pushes at most n-1 of its n children
-  const uint32_t need = item.need + (uint32_t)n - 1u;
   if (k == 0) {
-    st.max_depth = max(st.max_depth, item.depth);
-    st.max_stack = max(st.max_stack, need);
+    st.records += nt;
+    st.max_depth = max(st.max_depth, depth);
+    st.max_stack = max(st.max_stack, (w.level & 0xffffu) + (uint32_t)n - 1u);  // a node pushes at most n-1 of its n children
     st.sah_nodes += (double)half_area(uh[0] - ul[0], uh[1] - ul[1], uh[2] - ul[2]);
     if (nt) {
       st.sah_leaves += sah_leaf;
@@ -1169,7 +1102,7 @@ __device__ inline void collapse_item(const CollapseArgs& a, uint32_t t, bool act
     e[d] = grid_exponent(p[d], uh[d] + eps);
     sc[d] = __uint_as_float(e[d] << 23);
   }
-  uint8_t* node = reinterpret_cast<uint8_t*>(a.nodes + item.node);
+  uint8_t* node = reinterpret_cast<uint8_t*>(a.nodes + number);
   uint32_t meta = 0u, qlx = 255u, qhx = 0u, qly = 255u, qhy = 0u, qlz = 255u, qhz = 0u;
   if (has) {
     qlx = quant_lo(l.x - eps, p[0], sc[0]);
@@ -1180,7 +1113,6 @@ __device__ inline void collapse_item(const CollapseArgs& a, uint32_t t, bool act
     qhz = quant_hi(h.z + eps, p[2], sc[2]);
     if (inner) {
       meta = 0x80u | rank_i;
-      a.qout[qbase + rank_i] = QItem{mine, child_base + rank_i, item.depth + 1, need};
     } else {
       meta = 1u + off_t;
       // leaf records are written afterwards, one thread each (k_write_leaves)
@@ -1208,8 +1140,8 @@ __device__ inline void collapse_item(const CollapseArgs& a, uint32_t t, bool act
     inf.lo[0] = ul[0]; inf.lo[1] = ul[1]; inf.lo[2] = ul[2];
     inf.hi[0] = uh[0]; inf.hi[1] = uh[1]; inf.hi[2] = uh[2];
     inf.count = ninner_prims + nt;
-    inf.depth = item.depth;
-    a.info[item.node] = inf;
+    inf.depth = depth;
+    a.info[number] = inf;
   }
 }
 
@@ -1221,9 +1153,9 @@ __global__ __launch_bounds__(BT) void k_write_leaves(const uint32_t* __restrict_
                                                      const uint32_t* __restrict__ vals, const float4* __restrict__ lo4,
                                                      const float4* __restrict__ hi4, const GeomDesc* __restrict__ geoms,
                                                      const BuildCounters* cnt, TriRec* __restrict__ tris,
-                                                     InstRec* __restrict__ insts, uint32_t robust) {
+                                                     InstRec* __restrict__ insts, uint32_t robust, uint32_t n) {
   const uint32_t r = blockIdx.x * BT + threadIdx.x;
-  if (cnt->error || r >= cnt->tri_count) return;
+  if (cnt->error || cnt->tri_count != n || r >= n) return;
   const uint32_t e = leaf_src[r];
   const uint32_t o = vals[e & ~LEAF_SRC_LAST];
   const uint32_t last = (e & LEAF_SRC_LAST) ? TRI_LAST : 0u;
@@ -1255,45 +1187,55 @@ __global__ __launch_bounds__(BT) void k_write_leaves(const uint32_t* __restrict_
   tris[r] = tr;
 }
 
-// One level of the collapse: the grid strides over the level's queue, whose
-// length it reads on the device. A tree that failed its check (error bits
-// set) is not followed.
-__global__ __launch_bounds__(BT, 3) void k_collapse(CollapseArgs a) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *a.qclear = 0u;
-  // the workgroup decides together (block_alloc synchronises it)
+// Every node, in the order of their numbers: the top nodes, then the subtrees'
+// nodes. A tree that failed its check (error bits set) is not written.
+__global__ __launch_bounds__(BT) void k_emit_nodes(CollapseArgs a) {
   __shared__ uint32_t s_run;
   if (threadIdx.x == 0) s_run = a.cnt->error ? 0u : 1u;
   __syncthreads();
-  const uint32_t nin = *a.nin;
-  // few items: a group of CG lanes per item, which shortens each item's
-  // chain of work; many: a thread per item, fewer workgroup steps (each
-  // step's block_alloc atomics serialise on their addresses)
-  const bool grouped = nin <= COLLAPSE_GROUPED_MAX;
-  if (s_run && blockIdx.x * (grouped ? BT / CG : BT) < nin) {
-    CollapseStats st;
-    // block-uniform loops: every thread takes part in each item's block_alloc
-    if (grouped) {
-      constexpr uint32_t PER_BLOCK = BT / CG;
-      for (uint32_t base = blockIdx.x * PER_BLOCK; base < nin; base += gridDim.x * PER_BLOCK) {
-        const uint32_t t = base + threadIdx.x / CG;
-        collapse_item(a, t, t < nin, threadIdx.x % CG, st);
-      }
+  if (!s_run) return;
+  const uint32_t top = a.cnt->top_nodes, nsub = a.cnt->subtrees;
+  const uint32_t total = top + a.prefix[a.max_sub];
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.cnt->node_count = total;
+  CollapseStats st;
+  for (uint32_t i = (blockIdx.x * BT + threadIdx.x) / CG; i < total; i += gridDim.x * (BT / CG)) {
+    WideNode w;
+    if (i < top) {
+      w = a.top[i];
+      if (w.link & REF_LEAF) w.link = top + a.prefix[w.link & ~REF_LEAF];
     } else {
-      for (uint32_t base = blockIdx.x * BT; base < nin; base += gridDim.x * BT)
-        collapse_item1(a, base + threadIdx.x, base + threadIdx.x < nin, st);
+      const uint32_t j = i - top;
+      uint32_t lo = 0, hi = nsub - 1u;  // the subtree: the last whose first node is at most j
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1u) >> 1;
+        if (a.prefix[mid] <= j) lo = mid; else hi = mid - 1u;
+      }
+      const uint32_t p = a.prefix[lo];
+      w = a.rest[a.sub[lo].tri + (j - p)];
+      w.link += top + p;
     }
-    const uint32_t md = wave_umax(st.max_depth), ms = wave_umax(st.max_stack);
-    const double sn = wave_sum(st.sah_nodes), sl = wave_sum(st.sah_leaves), slt = wave_sum(st.sah_leaves_tri);
-    if ((threadIdx.x & 63u) == 0u) {
-      if (md) atomicMax(&a.cnt->max_depth, md);
-      if (ms) atomicMax(&a.cnt->max_stack, ms);
-      if (sn != 0.0) atomicAdd(&a.cnt->sah_nodes, sn);
-      if (sl != 0.0) atomicAdd(&a.cnt->sah_leaves, sl);
-      if (slt != 0.0) atomicAdd(&a.cnt->sah_leaves_tri, slt);
-    }
+    emit_node(a, w, i, threadIdx.x % CG, st);
   }
+  block_stats(st);
+  if (threadIdx.x == 0) a.stats[blockIdx.x] = st;
 }
 
+// The sum of the emission's statistics (atomics of every workgroup on a few
+// counters took longer than the emission; this order of summation is fixed).
+__global__ __launch_bounds__(BT) void k_sum_stats(const CollapseStats* __restrict__ part, uint32_t n, BuildCounters* cnt) {
+  if (cnt->error) return;  // (nothing was emitted)
+  CollapseStats st;
+  for (uint32_t i = threadIdx.x; i < n; i += BT) st.add(part[i]);
+  block_stats(st);
+  if (threadIdx.x == 0) {
+    cnt->max_depth = st.max_depth;
+    cnt->max_stack = st.max_stack;
+    cnt->tri_count = st.records;
+    cnt->sah_nodes = st.sah_nodes;
+    cnt->sah_leaves = st.sah_leaves;
+    cnt->sah_leaves_tri = st.sah_leaves_tri;
+  }
+}
 
 // ------------------------------------------------------------------ host --
 
@@ -1539,12 +1481,16 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   if (inst_build) out.insts.reserve((size_t)n * sizeof(InstRec));
   else out.tris.reserve((size_t)n * sizeof(TriRec));
   out.info.reserve((size_t)cap * sizeof(NodeInfo));
-  S.queue.reserve((size_t)2 * cap * sizeof(QItem));
-  QItem* q0 = S.queue.as<QItem>();
-  QItem* q1 = q0 + cap;
-  std::vector<QItem> roots(nscenes);
-  for (uint32_t sI = 0; sI < nscenes; sI++) roots[sI] = QItem{root_ref[sI], sI, 1u, 0u};
-  RTG_HIP(hipMemcpyAsync(q0, roots.data(), nscenes * sizeof(QItem), hipMemcpyHostToDevice, s));
+  // the scenes' roots, first positions and primitive counts, then the walk's arrays
+  const uint32_t max_sub = nscenes > 1 ? nscenes + SUB_MAX : SUB_MAX;
+  S.roots.reserve((size_t)nscenes * 12);
+  root_ref.insert(root_ref.end(), first.begin(), first.end());
+  root_ref.insert(root_ref.end(), count.begin(), count.end());
+  RTG_HIP(hipMemcpyAsync(S.roots.ptr, root_ref.data(), (size_t)nscenes * 12, hipMemcpyHostToDevice, s));
+  S.walk_top.reserve((size_t)top_cap(max_sub) * sizeof(WideNode));
+  S.walk_sub.reserve((size_t)max_sub * sizeof(WideNode));
+  S.walk_rest.reserve((size_t)n * sizeof(WideNode));
+  S.walk_count.reserve(((size_t)max_sub + 1) * 8);
 
   CollapseArgs ca;
   ca.child = S.child.as<uint32_t>();
@@ -1555,54 +1501,34 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   ca.split8 = S.split8.as<uint8_t>();
   ca.slo = S.slo.as<float4>();
   ca.shi = S.shi.as<float4>();
+  ca.cnt = cnt;
+  ca.nscenes = nscenes;
+  ca.n = n;
+  ca.width = width;
+  ca.max_sub = max_sub;
+  ca.top = S.walk_top.as<WideNode>();
+  ca.sub = S.walk_sub.as<WideNode>();
+  ca.rest = S.walk_rest.as<WideNode>();
+  ca.count = S.walk_count.as<uint32_t>();
+  ca.prefix = ca.count + max_sub + 1;
   ca.nodes = out.nodes.as<QNode8>();
   S.leaf_src.reserve((size_t)n * 4);
   ca.leaf_src = S.leaf_src.as<uint32_t>();
   ca.info = out.info.as<NodeInfo>();
-  ca.cnt = cnt;
-  ca.n = cap;
-  ca.tri_cap = n;
-  ca.width = width;
-  // one launch per level of the 8-wide tree; the kernels read their queue
-  // lengths on the device, so the host queues level k + 1 before it learns
-  // (through a pinned slot) whether level k produced any items
-  // 2048 workgroups: a thread per item covers the large levels in one step
-  const uint32_t cgrid = std::min<uint32_t>(div_up(cap, BT), 2048u);
-  auto enqueue_level = [&](uint32_t k) {
-    const uint32_t o = k & 1u;
-    ca.qin = o ? q1 : q0;
-    ca.qout = o ? q0 : q1;
-    ca.nin = &cnt->qcount[(k + 2u) % 3u];
-    ca.qout_slot = k % 3u;
-    ca.qclear = &cnt->qcount[(k + 1u) % 3u];
-    hipLaunchKernelGGL(k_collapse, dim3(cgrid), dim3(BT), 0, s, ca);
-    RTG_HIP(hipGetLastError());
-    RTG_HIP(hipMemcpyAsync(S.rb.slot((int)k), cnt, sizeof(BuildCounters), hipMemcpyDeviceToHost, s));
-    RTG_HIP(hipEventRecord(S.rb.ev[k % LevelReadback::K], s));
-  };
-  S.rb.ensure(sizeof(BuildCounters));
-  std::string level_sizes;
-  enqueue_level(0);
-  for (uint32_t k = 1;; k++) {
-    if (k > 4096) {
-      (void)hipStreamSynchronize(s);
-      throw hip_error(hipErrorUnknown, "BVH collapse did not terminate");
-    }
-    enqueue_level(k);  // speculative: without input it does nothing
-    RTG_HIP(hipEventSynchronize(S.rb.ev[(k - 1) % LevelReadback::K]));
-    memcpy(&hc, S.rb.slot((int)(k - 1)), sizeof(hc));
-    const uint32_t next = hc.qcount[(k - 1) % 3u];
-    level_sizes += " " + std::to_string(next);
-    if (next == 0 || hc.error) break;
-    if (next > cap) {
-      (void)hipStreamSynchronize(s);
-      throw hip_error(hipErrorUnknown, "BVH collapse queue overflow");
-    }
-  }
+  ca.cap = cap;
+  hipLaunchKernelGGL(k_walk_top, dim3(1), dim3(BT), 0, s, ca, S.roots.as<uint32_t>(), S.roots.as<uint32_t>() + nscenes,
+                     S.roots.as<uint32_t>() + 2 * (size_t)nscenes);
+  hipLaunchKernelGGL(k_walk_rest, dim3(std::min(max_sub + 1u, 2048u)), dim3(BT), 0, s, ca);
+  S.scanner.exclusive(ca.count, S.walk_count.as<uint32_t>() + max_sub + 1, (size_t)max_sub + 1, s);
+  const uint32_t egrid = std::min(div_up(cap, BT / CG), 4096u);
+  S.walk_stats.reserve((size_t)egrid * sizeof(CollapseStats));
+  ca.stats = S.walk_stats.as<CollapseStats>();
+  hipLaunchKernelGGL(k_emit_nodes, dim3(egrid), dim3(BT), 0, s, ca);
+  hipLaunchKernelGGL(k_sum_stats, dim3(1), dim3(BT), 0, s, ca.stats, egrid, cnt);
   hipLaunchKernelGGL(k_write_leaves, dim3(div_up(n, BT)), dim3(BT), 0, s, S.leaf_src.as<uint32_t>(),
                      S.vals.as<uint32_t>(), S.lo4.as<float4>(), S.hi4.as<float4>(), S.geoms.as<GeomDesc>(), cnt,
                      inst_build ? nullptr : out.tris.as<TriRec>(), inst_build ? out.insts.as<InstRec>() : nullptr,
-                     prm.robust ? 1u : 0u);
+                     prm.robust ? 1u : 0u, n);
   RTG_HIP(hipGetLastError());
   RTG_HIP(hipMemcpyAsync(&hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, s));
   RTG_HIP(hipStreamSynchronize(s));
@@ -1612,8 +1538,7 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   if (hc.error || hc.tri_count != n)
     throw hip_error(hipErrorUnknown, "BVH build consistency check failed: error bits " + std::to_string(hc.error) +
                                          ", primitives " + std::to_string(n) + ", triangle records " +
-                                         std::to_string(hc.tri_count) + ", nodes " + std::to_string(hc.node_count) +
-                                         ", queue sizes per level" + level_sizes);
+                                         std::to_string(hc.tri_count) + ", nodes " + std::to_string(hc.node_count));
   if (hc.max_stack + 1 > TRACE_STACK)
     throw hip_error(hipErrorUnknown, "BVH too deep for the traversal stack: " + std::to_string(hc.max_stack + 1) +
                                          " entries needed, " + std::to_string(TRACE_STACK) + " available");

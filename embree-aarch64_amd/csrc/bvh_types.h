@@ -4,9 +4,9 @@
 // Layout in HBM (one scene):
 //   nodes : QNode8[num_nodes], 80 B of node in each 128 B slot (one slot
 //           per 128 B cache line, so a node visit never touches two lines),
-//           breadth-first; the root is node 0 (node s for scene s of a
-//           batched build); the internal children of a node are contiguous
-//           from child_base.
+//           the top of the tree first, then subtree by subtree; the root is
+//           node 0 (node s for scene s of a batched build); the internal
+//           children of a node are contiguous from child_base.
 //   tris  : TriRec[num_tris], 48 B each; the leaf children of a node are
 //           contiguous from tri_base; a leaf ends at the record whose
 //           TRI_LAST flag is set.

@@ -43,3 +43,28 @@ def test_skewed_and_equal_primitives(rtc, oracle, device, quality):
     v *= (0.9995 ** np.arange(len(v), dtype=np.float64)).astype(np.float32)[:, None, None]
     v[5000:8000] = v[5000]
     check(rtc, oracle, device, (v.reshape(-1, 3), ix), quality)
+
+
+@pytest.mark.parametrize("width", [2, 3, 8])
+@pytest.mark.parametrize("n", [1, 9, 511, 513, 4097, 70001])
+def test_widths_and_subtrees(rtc, oracle, n, width):
+    # the wide nodes are numbered by subtrees of at most 512 primitives or 1/256 of them
+    dev = rtc.Device(f"bvh_width={width}")
+    check(rtc, oracle, dev, rtc.gen_soup(n, seed=n + 1, h=0.03), 1)
+    dev.release()
+
+
+def test_more_scenes_than_top_nodes(rtc, oracle, device):
+    # 2300 scenes of one build: empty ones, single triangles, small meshes and a large one
+    meshes = [rtc.gen_soup(k % 7, seed=k + 1, h=0.2) if k % 500 else rtc.gen_soup(20000, seed=k + 1, h=0.02)
+              for k in range(2300)]
+    scs = [rtc.Scene(device, [m]) for m in meshes]
+    rtc.commit_scenes(scs)
+    for k in (0, 1, 2, 6, 7, 500, 501, 1999, 2000, 2299):
+        rays = rtc.gen_random_rays(200, seed=k)
+        ref = rays.copy()
+        scs[k].intersect1M(rays)
+        oracle.BVH([meshes[k]]).intersect(ref)
+        assert len(mismatches(rays, ref)) == 0, k
+    for s in scs:
+        s.release()
