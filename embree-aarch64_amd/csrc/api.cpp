@@ -16,9 +16,13 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <condition_variable>
+#include <exception>
+#include <functional>
 #include <memory>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -49,14 +53,108 @@ inline void ref_dec(RefObj* o) {
 
 struct Device;
 
+// One host thread's share of a transfer of host memory: a stream of its own
+// (transfers and traces of several chunks overlap) and two chunks, one packed
+// or unpacked by the host while the GPU works on the other.
+struct HostLane {
+  struct Slot {
+    rtg::PinnedBuf in, out;
+    rtg::DevBuf dev;
+    hipEvent_t ev = nullptr;
+    size_t first = 0, n = 0;  // records in flight (n = 0: none)
+  };
+  hipStream_t stream = nullptr;
+  Slot slot[2];
+  rtg::RaySorter sorter;
+  HostLane() {
+    RTG_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+    for (Slot& s : slot) RTG_HIP(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming));
+  }
+  void drain() {
+    (void)hipStreamSynchronize(stream);
+    for (Slot& s : slot) s.n = 0;
+  }
+  ~HostLane() {
+    if (stream) (void)hipStreamSynchronize(stream);
+    for (Slot& s : slot)
+      if (s.ev) (void)hipEventDestroy(s.ev);
+    if (stream) (void)hipStreamDestroy(stream);
+  }
+};
+
+// A device's helper threads for transfers of host memory, each with a lane.
+// They are started when first wanted (at most MAX) and end with the device;
+// between jobs they sleep. A caller does the work itself and does not wait for
+// a helper that has not begun: on a busy host a helper may get a CPU only after
+// the work is done.
+struct HostPool {
+  static constexpr size_t MAX = 7;
+  struct Job {
+    std::function<void(HostLane&)> work;
+    size_t open = 0, active = 0;  // helpers that may still join, and those at work
+    std::exception_ptr failed;
+  };
+  std::mutex mtx;
+  std::condition_variable wake, done;
+  std::vector<Job*> jobs;  // with open places
+  std::vector<std::thread> threads;
+  bool stop = false;
+  void submit(Job& job, size_t helpers, int ordinal) {
+    std::lock_guard<std::mutex> g(mtx);
+    job.open = std::min(helpers, MAX);
+    jobs.push_back(&job);
+    try {
+      while (threads.size() < job.open) threads.emplace_back([this, ordinal] { serve(ordinal); });
+    } catch (const std::system_error&) {  // no more threads: the caller does what they would have done
+    }
+    wake.notify_all();
+  }
+  void finish(Job& job) {
+    std::unique_lock<std::mutex> g(mtx);
+    jobs.erase(std::remove(jobs.begin(), jobs.end(), &job), jobs.end());
+    done.wait(g, [&] { return job.active == 0; });
+  }
+  void serve(int ordinal) {
+    std::unique_ptr<HostLane> lane;
+    std::unique_lock<std::mutex> g(mtx);
+    while (true) {
+      wake.wait(g, [&] { return stop || !jobs.empty(); });
+      if (stop) return;
+      Job& job = *jobs.front();
+      job.active++;
+      if (--job.open == 0) jobs.erase(jobs.begin());
+      g.unlock();
+      std::exception_ptr failed;
+      try {
+        if (!lane) {
+          RTG_HIP(hipSetDevice(ordinal));
+          lane.reset(new HostLane());
+        }
+        job.work(*lane);
+      } catch (...) {
+        failed = std::current_exception();
+      }
+      g.lock();
+      if (failed && !job.failed) job.failed = failed;
+      if (--job.active == 0) done.notify_all();
+    }
+  }
+  ~HostPool() {
+    {
+      std::lock_guard<std::mutex> g(mtx);
+      stop = true;
+    }
+    wake.notify_all();
+    for (auto& t : threads) t.join();
+  }
+};
+
 struct ThreadDev {
   hipStream_t stream = nullptr;
-  rtg::DevBuf staging;
-  rtg::DevBuf errword;
+  rtg::PinnedBuf errword;  // traversal error bits: the host reads them after a synchronisation, without a copy
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  // host records: two pinned chunks the queries of host memory move through
-  rtg::PinnedBuf stage[2];
-  hipEvent_t ev_stage[2] = {nullptr, nullptr};
+  rtg::PinnedBuf small;    // records of small queries in host memory, which the kernel reads and writes in place
+  std::unique_ptr<HostLane> lane;  // of large ones
   rtg::RaySorter sorter;
   rtg::DevBuf batch, batch_counter;  // batched traversal: stream table, work counter
 };
@@ -81,6 +179,7 @@ struct Device : RefObj {
   float spatial_budget = 0.3f;
   std::mutex tls_mtx;
   std::unordered_map<std::thread::id, ThreadDev*> threads;
+  HostPool pool;
   ~Device() override {
     (void)hipSetDevice(ordinal);
     for (auto& kv : threads) {
@@ -88,8 +187,6 @@ struct Device : RefObj {
       if (t->stream) (void)hipStreamDestroy(t->stream);
       if (t->ev0) (void)hipEventDestroy(t->ev0);
       if (t->ev1) (void)hipEventDestroy(t->ev1);
-      for (hipEvent_t e : t->ev_stage)
-        if (e) (void)hipEventDestroy(e);
       delete t;
     }
   }
@@ -102,9 +199,8 @@ struct Device : RefObj {
     RTG_HIP(hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking));
     RTG_HIP(hipEventCreate(&t->ev0));
     RTG_HIP(hipEventCreate(&t->ev1));
-    for (hipEvent_t& e : t->ev_stage) RTG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     t->errword.reserve(256);
-    RTG_HIP(hipMemsetAsync(t->errword.ptr, 0, 4, t->stream));
+    *t->errword.as<uint32_t>() = 0;
     threads[std::this_thread::get_id()] = t;
     return *t;
   }
@@ -472,14 +568,91 @@ void build_scene_tree(Scene* sc, Device* d, const std::vector<rtg::GeomDesc>& de
   if (plain.stats.sah <= sc->bvh->stats.sah) sc->bvh->swap_tree(plain);
 }
 
+// Host threads that help a transfer of `bytes`: one for each 2 MB beyond the
+// first, at most 7 and half of the host's.
+size_t host_helpers(size_t bytes) {
+  const unsigned hw = std::thread::hardware_concurrency();
+  return std::min<size_t>({HostPool::MAX, hw > 1 ? hw / 2 - 1 : 0, bytes / (2u << 20)});
+}
+
+// Runs work(lane) on this thread and on up to `helpers` of the device's helper
+// threads; work takes its pieces from a common counter until there are none.
+template <class Work>
+void on_lanes(Device* d, ThreadDev& t, size_t helpers, Work work) {
+  if (!t.lane) t.lane.reset(new HostLane());
+  HostPool::Job job;
+  job.work = [&](HostLane& lane) {
+    try {
+      work(lane);
+    } catch (...) {
+      lane.drain();
+      throw;
+    }
+  };
+  if (helpers) d->pool.submit(job, helpers, d->ordinal);
+  std::exception_ptr mine;
+  try {
+    job.work(*t.lane);
+  } catch (...) {
+    mine = std::current_exception();
+  }
+  if (helpers) d->pool.finish(job);
+  if (mine) std::rethrow_exception(mine);
+  if (job.failed) std::rethrow_exception(job.failed);
+}
+
+// Copies host memory to the device. Large copies go through the lanes' pinned
+// chunks, filled by several host threads while earlier chunks are on their way
+// (the runtime's own copy of pageable memory reaches half the rate of PCIe);
+// they are complete on return, small ones are queued on t.stream.
+constexpr size_t UPLOAD_CHUNK = size_t(1) << 20, UPLOAD_MIN = size_t(4) << 20;
+
+void upload_host(Device* d, ThreadDev& t, void* dst, const void* src, size_t bytes) {
+  if (bytes < UPLOAD_MIN) {
+    RTG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, t.stream));
+    return;
+  }
+  RTG_HIP(hipStreamSynchronize(t.stream));  // (nothing queued before reads or writes dst any more)
+  std::atomic<size_t> next{0};
+  on_lanes(d, t, host_helpers(bytes), [&](HostLane& lane) {
+    for (auto& s : lane.slot) s.in.reserve(UPLOAD_CHUNK);
+    for (unsigned k = 0;; k ^= 1u) {
+      HostLane::Slot& s = lane.slot[k];
+      if (s.n) RTG_HIP(hipEventSynchronize(s.ev));
+      s.n = 0;
+      const size_t at = next.fetch_add(1) * UPLOAD_CHUNK;
+      if (at >= bytes) break;
+      const size_t n = std::min(UPLOAD_CHUNK, bytes - at);
+      memcpy(s.in.ptr, (const char*)src + at, n);
+      RTG_HIP(hipMemcpyAsync((char*)dst + at, s.in.ptr, n, hipMemcpyHostToDevice, lane.stream));
+      RTG_HIP(hipEventRecord(s.ev, lane.stream));
+      s.n = n;
+    }
+    lane.drain();
+  });
+}
+
 // Uploads the enabled triangle geometries of sc (scene index `scene` of a
 // build) into device buffers owned by sc, appending their descriptors;
 // prim_offset advances over their triangles.
 void upload_geometry(Scene* sc, Device* d, ThreadDev& t, uint32_t scene, uint32_t& prim_offset,
                      std::vector<rtg::GeomDesc>& out) {
-  for (auto* b : sc->gdata) delete b;
-  sc->gdata.clear();
+  // buffers of the last commit are used again where they fit (an allocation of
+  // this size, and the synchronisation of freeing the old one, cost more than
+  // the copy on small scenes)
+  std::vector<rtg::DevBuf*> old;
+  old.swap(sc->gdata);
   sc->descs.clear();
+  size_t used = 0;
+  auto buffer = [&](size_t bytes) {
+    auto* b = used < old.size() ? old[used] : new rtg::DevBuf();
+    if (used < old.size()) old[used] = nullptr;
+    used++;
+    sc->gdata.push_back(b);
+    if (b->bytes > 2 * bytes + (size_t(1) << 20)) b->release();
+    b->reserve(bytes);
+    return b;
+  };
   for (size_t id = 0; id < sc->geoms.size(); id++) {
     Geometry* g = sc->geoms[id];
     if (!g || !g->enabled || g->type != RTC_GEOMETRY_TYPE_TRIANGLE) continue;
@@ -488,14 +661,10 @@ void upload_geometry(Scene* sc, Device* d, ThreadDev& t, uint32_t scene, uint32_
     const size_t ibytes = (g->index.count - 1) * g->index.stride + 12;
     if ((uint64_t)prim_offset + g->index.count > 0xffffffffull) RTC_THROW(RTC_ERROR_INVALID_OPERATION, "too many primitives");
     d->monitor((ssize_t)(vbytes + ibytes));
-    auto* vb = new rtg::DevBuf();
-    sc->gdata.push_back(vb);
-    auto* ib = new rtg::DevBuf();
-    sc->gdata.push_back(ib);
-    vb->reserve(vbytes ? vbytes : 16);
-    ib->reserve(ibytes);
-    if (vbytes) RTG_HIP(hipMemcpyAsync(vb->ptr, g->vertex.ptr, vbytes, hipMemcpyHostToDevice, t.stream));
-    RTG_HIP(hipMemcpyAsync(ib->ptr, g->index.ptr, ibytes, hipMemcpyHostToDevice, t.stream));
+    rtg::DevBuf* vb = buffer(vbytes ? vbytes : 16);
+    rtg::DevBuf* ib = buffer(ibytes);
+    if (vbytes) upload_host(d, t, vb->ptr, g->vertex.ptr, vbytes);
+    upload_host(d, t, ib->ptr, g->index.ptr, ibytes);
     rtg::GeomDesc gd;
     gd.vertices = (const char*)vb->ptr;
     gd.indices = (const char*)ib->ptr;
@@ -511,6 +680,7 @@ void upload_geometry(Scene* sc, Device* d, ThreadDev& t, uint32_t scene, uint32_
     sc->descs.push_back(gd);
     out.push_back(gd);
   }
+  for (auto* b : old) delete b;
 }
 
 // ------------------------------------------------------------ instances --
@@ -727,17 +897,20 @@ void check_top(Scene* sc) {
 
 bool scene_empty(Scene* sc) { return sc->two_level ? false : sc->bvh->empty(sc->slot); }
 
-// Traverses the scene over device records on `stream`.
-void launch_scene(Scene* sc, ThreadDev& t, void* rays, unsigned M, size_t stride, bool occluded, uint32_t inst,
-                  hipStream_t stream, const rtg::TraceParams& tp) {
+// Traverses the scene over device (or pinned) records on `stream`.
+void launch_scene(Scene* sc, uint32_t* err, rtg::RaySorter& sorter, void* rays, unsigned M, size_t stride, bool occluded,
+                  uint32_t inst, hipStream_t stream, const rtg::TraceParams& tp) {
   if (sc->two_level) {
     check_top(sc);
-    rtg::launch_trace_inst(sc->top_view, rays, M, stride, occluded, inst, t.errword.as<uint32_t>(), stream, tp,
-                           &t.sorter);
+    rtg::launch_trace_inst(sc->top_view, rays, M, stride, occluded, inst, err, stream, tp, &sorter);
   } else if (!sc->bvh->empty(sc->slot)) {
-    rtg::launch_trace(sc->bvh->view(sc->slot), rays, M, stride, occluded, inst, nullptr, nullptr,
-                      t.errword.as<uint32_t>(), stream, tp, &t.sorter);
+    rtg::launch_trace(sc->bvh->view(sc->slot), rays, M, stride, occluded, inst, nullptr, nullptr, err, stream, tp,
+                      &sorter);
   }
+}
+void launch_scene(Scene* sc, ThreadDev& t, void* rays, unsigned M, size_t stride, bool occluded, uint32_t inst,
+                  hipStream_t stream, const rtg::TraceParams& tp) {
+  launch_scene(sc, t.errword.as<uint32_t>(), t.sorter, rays, M, stride, occluded, inst, stream, tp);
 }
 
 void single_level_only(Scene* sc, const char* what) {
@@ -782,51 +955,18 @@ bool is_device_ptr(Device* d, const void* p) {
 }
 
 void check_trace_error(ThreadDev& t) {
-  uint32_t err = 0;
-  RTG_HIP(hipMemcpyAsync(&err, t.errword.ptr, 4, hipMemcpyDeviceToHost, t.stream));
   RTG_HIP(hipStreamSynchronize(t.stream));
-  if (err) {
-    RTG_HIP(hipMemsetAsync(t.errword.ptr, 0, 4, t.stream));
-    RTG_HIP(hipStreamSynchronize(t.stream));
-    RTC_THROW(RTC_ERROR_UNKNOWN, (err & 1u) ? "traversal stack overflow" : "corrupt acceleration structure");
-  }
+  const uint32_t err = __atomic_exchange_n(t.errword.as<uint32_t>(), 0u, __ATOMIC_RELAXED);
+  if (err) RTC_THROW(RTC_ERROR_UNKNOWN, (err & 1u) ? "traversal stack overflow" : "corrupt acceleration structure");
 }
+
+// Rays up to which a query in host memory is traced in place in pinned memory
+// (one ray 17 us, 43 with copies; 4000 rays 100 us in place, 106 in chunks), and
+// records of a chunk of a larger one: each costs about 60 us of launches beside
+// its transfers, and there are a few for every thread.
+constexpr size_t SMALL_RAYS = 8192, HOST_CHUNK_MIN = 16384, HOST_CHUNK_MAX = 65536;
 
 // Stream query over host or device records (reference rtcore.cpp:595-623, 848-874).
-// Host records per chunk of a query in host memory (80 MB of RTCRayHit).
-constexpr size_t HOST_CHUNK_RAYS = size_t(1) << 20;
-
-// Copies n records of rec bytes from src (stride sstride) to dst (stride
-// dstride), on several host threads when there are many.
-void copy_records(void* dst, size_t dstride, const void* src, size_t sstride, size_t n, size_t rec) {
-  auto part = [&](size_t a, size_t b) {
-    if (dstride == rec && sstride == rec) {
-      memcpy((char*)dst + a * rec, (const char*)src + a * rec, (b - a) * rec);
-    } else {
-      for (size_t i = a; i < b; i++) memcpy((char*)dst + i * dstride, (const char*)src + i * sstride, rec);
-    }
-  };
-  const unsigned hw = std::thread::hardware_concurrency();
-  const size_t nt = std::min<size_t>({8, hw > 1 ? hw / 2 : 1, std::max<size_t>(1, n * rec / (4u << 20))});
-  if (nt <= 1) {
-    part(0, n);
-    return;
-  }
-  std::vector<std::thread> th;
-  const size_t per = (n + nt - 1) / nt;
-  size_t j = 1;
-  try {
-    for (; j < nt; j++) {
-      const size_t a = std::min(n, j * per), b = std::min(n, (j + 1) * per);
-      if (a < b) th.emplace_back(part, a, b);
-    }
-  } catch (...) {  // no more threads: this one copies the parts not started
-  }
-  part(0, std::min(n, per));
-  for (; j < nt; j++) part(std::min(n, j * per), std::min(n, (j + 1) * per));
-  for (auto& x : th) x.join();
-}
-
 void trace_stream(Scene* sc, const RTCIntersectContext* ctx, void* rays, unsigned M, size_t stride, bool occluded) {
   if (!sc->committed) RTC_THROW(RTC_ERROR_INVALID_OPERATION, "scene not committed");
   if (ctx && ctx->filter) RTC_THROW(RTC_ERROR_INVALID_OPERATION, "filter functions are not supported");
@@ -844,32 +984,69 @@ void trace_stream(Scene* sc, const RTCIntersectContext* ctx, void* rays, unsigne
     check_trace_error(t);
     return;
   }
-  // Host records move in chunks through two pinned buffers: host threads
-  // pack chunk k into one while the GPU uploads, traces and downloads chunk
-  // k - 1 through the other, and unpack a chunk once its download is done.
-  // (Pageable memory cannot be registered for DMA here, so every byte goes
-  // through a host copy; several threads copy faster than one.)
-  const size_t chunk = std::min<size_t>(M, HOST_CHUNK_RAYS);
-  const size_t nchunks = (M + chunk - 1) / chunk;
-  t.staging.reserve((size_t)M * rec);
-  for (auto& b : t.stage) b.reserve(chunk * rec);
   const rtg::TraceParams tp = d->trace_params();
-  auto unpack = [&](size_t k) {
-    const size_t first = k * chunk, n = std::min<size_t>(chunk, M - first);
-    RTG_HIP(hipEventSynchronize(t.ev_stage[k & 1]));
-    copy_records((char*)rays + first * stride, stride, t.stage[k & 1].ptr, rec, n, rec);
-  };
-  for (size_t k = 0; k < nchunks; k++) {
-    if (k >= 2) unpack(k - 2);  // frees this chunk's pinned buffer
-    const size_t first = k * chunk, n = std::min<size_t>(chunk, M - first);
-    char* dev = t.staging.as<char>() + first * rec;
-    copy_records(t.stage[k & 1].ptr, rec, (const char*)rays + first * stride, stride, n, rec);
-    RTG_HIP(hipMemcpyAsync(dev, t.stage[k & 1].ptr, n * rec, hipMemcpyHostToDevice, t.stream));
-    launch_scene(sc, t, dev, (unsigned)n, rec, occluded, inst, t.stream, tp);
-    RTG_HIP(hipMemcpyAsync(t.stage[k & 1].ptr, dev, n * rec, hipMemcpyDeviceToHost, t.stream));
-    RTG_HIP(hipEventRecord(t.ev_stage[k & 1], t.stream));
+  if (M <= SMALL_RAYS) {
+    // the kernel works on the pinned records themselves: no copies to queue
+    t.small.reserve(SMALL_RAYS * sizeof(RTCRayHit));
+    char* rec0 = t.small.as<char>();
+    for (unsigned i = 0; i < M; i++) memcpy(rec0 + i * rec, (const char*)rays + i * stride, rec);
+    launch_scene(sc, t, rec0, M, rec, occluded, inst, t.stream, tp);
+    check_trace_error(t);
+    for (unsigned i = 0; i < M; i++) memcpy((char*)rays + i * stride, rec0 + i * rec, rec);
+    return;
   }
-  for (size_t k = nchunks >= 2 ? nchunks - 2 : 0; k < nchunks; k++) unpack(k);
+  // Chunks of records, each packed to what the query reads, traced, and what
+  // the query wrote unpacked (pageable memory cannot be registered for DMA
+  // here, so every byte goes through a host copy). A thread packs or unpacks
+  // one chunk while the GPU works on its other one, and several threads'
+  // chunks keep both directions of PCIe and the GPU busy at once.
+  const size_t helpers = host_helpers((size_t)M * rec);
+  const size_t chunk = std::max<size_t>(HOST_CHUNK_MIN, std::min<size_t>(HOST_CHUNK_MAX, M / ((helpers + 1) * 2)));
+  const size_t nchunks = ((size_t)M + chunk - 1) / chunk;
+  std::atomic<size_t> next{0};
+  uint32_t* err = t.errword.as<uint32_t>();
+  on_lanes(d, t, std::min(helpers, nchunks - 1), [&](HostLane& lane) {
+    const size_t out_words = occluded ? 1 : rtg::HIT_WORDS;
+    for (auto& s : lane.slot) {
+      s.in.reserve(chunk * rtg::RAY_WORDS * 4);
+      s.out.reserve(chunk * rtg::HIT_WORDS * 4);
+      s.dev.reserve(chunk * sizeof(RTCRayHit));
+    }
+    auto unpack = [&](HostLane::Slot& s) {
+      if (!s.n) return;
+      RTG_HIP(hipEventSynchronize(s.ev));
+      const uint32_t* o = s.out.as<uint32_t>();
+      for (size_t i = 0; i < s.n; i++, o += out_words) {
+        char* r = (char*)rays + (s.first + i) * stride;
+        if (occluded) {
+          memcpy(r + 32, o, 4);
+        } else if (o[1] != rtg::NO_NORMAL) {
+          memcpy(r + 32, o, 4);
+          memcpy(r + 48, o + 1, 32);
+        }
+      }
+      s.n = 0;
+    };
+    for (unsigned k = 0;; k ^= 1u) {
+      HostLane::Slot& s = lane.slot[k];
+      unpack(s);
+      const size_t c = next.fetch_add(1);
+      if (c >= nchunks) {
+        unpack(lane.slot[k ^ 1u]);
+        break;
+      }
+      s.first = c * chunk;
+      const size_t n = std::min<size_t>(chunk, M - s.first);
+      char* p = s.in.as<char>();
+      for (size_t i = 0; i < n; i++) memcpy(p + i * rtg::RAY_WORDS * 4, (const char*)rays + (s.first + i) * stride, rtg::RAY_WORDS * 4);
+      rtg::unpack_rays(s.in.as<uint32_t>(), s.dev.ptr, (uint32_t)n, occluded, lane.stream);
+      launch_scene(sc, err, lane.sorter, s.dev.ptr, (unsigned)n, rec, occluded, inst, lane.stream, tp);
+      rtg::pack_hits(s.dev.ptr, s.out.as<uint32_t>(), (uint32_t)n, occluded, lane.stream);
+      RTG_HIP(hipGetLastError());
+      RTG_HIP(hipEventRecord(s.ev, lane.stream));
+      s.n = n;
+    }
+  });
   check_trace_error(t);
 }
 

@@ -60,7 +60,8 @@ struct RaySorter {
 // Traces M ray records (RTCRayHit for closest hit, RTCRay for occlusion)
 // spaced `stride` bytes apart in device memory, in place. cnt_nodes /
 // cnt_tris (optional, M entries each) receive per-ray node visits and
-// triangle tests. err receives bit 0 on a traversal stack overflow.
+// triangle tests. err (device or pinned host memory) receives
+// bit 0 on a traversal stack overflow.
 // node_visits (optional, with the counters): one atomic increment per node
 // visit, indexed like the QNode8 array.
 // counter (optional): the persistent kernel's ray counters (COUNTER_BYTES);
@@ -92,6 +93,16 @@ void launch_trace_inst(const DevTop& top, void* rays, uint32_t M, uint64_t strid
 void launch_trace_inst_counted(const DevTop& top, void* rays, uint32_t M, uint64_t stride, uint32_t* err,
                                uint32_t* counter, uint32_t* top_visits, uint32_t* obj_visits, uint32_t target_obj,
                                hipStream_t s, const TraceParams& tp);
+
+// Words of a record that a query reads, and of RTCRayHit that a hit writes (the
+// distance, then words 12 to 19).
+constexpr uint32_t RAY_WORDS = 9, HIT_WORDS = 9;
+constexpr uint32_t NO_NORMAL = 0x7fffffffu;  // first word of the normal of a record without a hit
+// n device records (80 B RTCRayHit or 48 B RTCRay) from their RAY_WORDS words,
+// and what the query wrote of them (HIT_WORDS, or for occlusion the distance).
+// in and out: pinned host memory. n is below 2^24.
+void unpack_rays(const uint32_t* in, void* recs, uint32_t n, bool occluded, hipStream_t s);
+void pack_hits(const void* recs, uint32_t* out, uint32_t n, bool occluded, hipStream_t s);
 
 // Scratch of the no-allocation queries: the persistent kernel's ray counters
 // (the words at multiples of COUNTER_STRIDE), with the traversal error bits

@@ -40,6 +40,13 @@ constexpr int STACK = (int)TRACE_STACK;  // entries per ray (the builder checks 
 // holds at most STACK (fits()), so the arrays have room for 7 more.
 constexpr int STACK_CAP = STACK + 8;
 
+// Sets error bits. The word may be in host memory, which has no atomic OR over
+// PCIe: of bits that two lanes set at once, one may be lost, never both.
+__device__ inline void raise_error(uint32_t* err, uint32_t bits) {
+  const uint32_t old = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(err, old | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Per-lane traversal stack: the top LDS_SLOTS entries live in LDS (slot-major,
 // so lanes touching the same slot hit distinct banks), older entries spill
 // to a private array only when the ring is full. Entry = (ref, entry distance).
@@ -356,7 +363,7 @@ __device__ inline bool push_any_order(const NodeHit& h, Stack& stack, uint32_t* 
       stack.put(make_uint2(meta_ref((uint32_t)(meta >> (8 * c)) & 0xffu, cb, tb), 0u));
     }
   } else {
-    atomicOr(err, 1u);
+    raise_error(err, 1u);
   }
   next = meta_ref((uint32_t)(meta >> (8 * c0)) & 0xffu, cb, tb);
   return true;
@@ -415,7 +422,7 @@ __device__ inline bool push_near_to_far(const NodeHit& h, Stack& stack, int& smi
       }
     }
   } else {
-    atomicOr(err, 1u);
+    raise_error(err, 1u);
   }
   next = meta_ref((uint32_t)k[7] & 0xffu, cb, tb);
   return true;
@@ -572,12 +579,12 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
   uint32_t iter = 0;
   while (true) {
     if (++iter > max_iter) {
-      atomicOr(err, 2u);
+      raise_error(err, 2u);
       break;
     }
     if (!(cur & REF_LEAF)) {
       if (cur >= sc.num_nodes) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         break;
       }
       NodeHit h;
@@ -593,7 +600,7 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
       uint32_t ti = cur & ~REF_LEAF;
       while (true) {
         if (ti >= sc.num_tris) {
-          atomicOr(err, 4u);
+          raise_error(err, 4u);
           break;
         }
         TriTest h;
@@ -772,11 +779,11 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
     // ---- one traversal step
     bool done = false;
     if (++iter > max_iter) {
-      atomicOr(err, 2u);
+      raise_error(err, 2u);
       done = true;
     } else if (!(cur & REF_LEAF)) {
       if (cur >= sc.num_nodes) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         done = true;
       } else {
         NodeHit h;
@@ -794,7 +801,7 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
       // wave's other lanes in a triangle loop
       const uint32_t ti = cur & ~REF_LEAF;
       if (ti >= sc.num_tris) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         done = true;
       } else {
         TriTest h;
@@ -948,7 +955,7 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
 
     bool done = false;
     if (++iter > max_iter) {
-      atomicOr(err, 2u);
+      raise_error(err, 2u);
       done = true;
     }
     // a waiting leaf starts once the triangle cursor is free
@@ -959,7 +966,7 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
     // node step
     if (!done && cur != NONE_REF && !(cur & REF_LEAF)) {
       if (cur >= sc.num_nodes) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         done = true;
       } else {
         NodeHit h;
@@ -976,7 +983,7 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
     // triangle step
     if (!done && tri != NONE_REF) {
       if (tri >= sc.num_tris) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         done = true;
       } else {
         TriTest h;
@@ -1112,12 +1119,12 @@ __global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ 
   uint32_t iter = 0;
   while (true) {
     if (++iter > max_iter) {
-      atomicOr(err, 2u);
+      raise_error(err, 2u);
       break;
     }
     if (!(cur & REF_LEAF)) {
       if (cur >= sc.num_nodes) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         break;
       }
       const char* np = reinterpret_cast<const char*>(sc.nodes + cur);
@@ -1154,7 +1161,7 @@ __global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ 
           first = (uint32_t)__builtin_ctz(group(hit && rank == 0u));
         }
         if (sp + n > cap) {
-          atomicOr(err, 1u);
+          raise_error(err, 1u);
           break;
         }
         // the nearest is next, the others are pushed farthest first
@@ -1167,7 +1174,7 @@ __global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ 
     } else {
       const uint32_t ti = cur & ~REF_LEAF;
       if (ti >= sc.num_tris) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         break;
       }
       TriTest h;
@@ -1341,13 +1348,13 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
     // ---- one traversal step
     bool done = false;
     if (++iter > top.max_iter) {
-      atomicOr(err, 2u);
+      raise_error(err, 2u);
       done = true;
     } else if (!(cur & REF_LEAF)) {
       const QNode8* nodes = in_obj ? onodes : top.nodes;
       const uint32_t nn = in_obj ? onn : top.num_nodes;
       if (cur >= nn) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         done = true;
       } else {
         if (CNT) {
@@ -1367,7 +1374,7 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
       // one triangle of the current object
       const uint32_t ti = cur & ~REF_LEAF;
       if (ti >= otn) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         done = true;
       } else {
         TriTest h;
@@ -1416,7 +1423,7 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
       // an instance record of the top tree
       const uint32_t ii = cur & ~REF_LEAF;
       if (ii >= top.num_insts) {
-        atomicOr(err, 4u);
+        raise_error(err, 4u);
         done = true;
       } else {
         const float4* q = reinterpret_cast<const float4*>(top.insts + ii);
@@ -1425,11 +1432,11 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
         const bool identity = (w.z & INST_IDENTITY) != 0u;
         // the rest of a multi-record leaf resumes after this instance
         if (!(w.z & TRI_LAST) && !stack.push(make_uint2((ii + 1u) | REF_LEAF, pack_dist(DIST_ALWAYS, smin))))
-          atomicOr(err, 1u);
+          raise_error(err, 1u);
         if ((identity || ctx_inst == 0xffffffffu) && w.y < top.num_objects) {
           const DevScene o = top.objects[w.y];
           if (o.num_nodes > 0) {
-            if (!stack.push(make_uint2(REF_INST_EXIT, pack_dist(DIST_ALWAYS, smin)))) atomicOr(err, 1u);
+            if (!stack.push(make_uint2(REF_INST_EXIT, pack_dist(DIST_ALWAYS, smin)))) raise_error(err, 1u);
             if (!identity) {
               lds_world[threadIdx.x] = make_float4(r.ox, r.oy, r.oz, r.dx);
               lds_world[TB + threadIdx.x] = make_float4(r.dy, r.dz, r.rnx, r.rny);
@@ -1506,6 +1513,28 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
 }
 
 __global__ void k_zero_counters(uint32_t* p) { p[threadIdx.x * COUNTER_STRIDE] = 0u; }
+
+// Records of queries in host memory. What a query reads of a record is its
+// first RAY_WORDS words, what it may write the distance and the hit: PCIe carries
+// those 36 of 80 bytes each way, straight between pinned host memory and the
+// device records (a word a thread, so that both sides' accesses are whole lines).
+// A hit always writes its normal, and no hit's normal is NO_NORMAL (a NaN fails
+// the hit tests).
+__global__ __launch_bounds__(TB) void k_unpack_rays(const uint32_t* __restrict__ in, uint32_t* __restrict__ recs,
+                                                    uint32_t words, uint32_t rec_words) {
+  const uint32_t t = blockIdx.x * TB + threadIdx.x;
+  if (t >= words) return;
+  const uint32_t i = t / RAY_WORDS, w = t - i * RAY_WORDS;
+  recs[(size_t)i * rec_words + w] = in[t];
+  if (w == 0 && rec_words > 12) recs[(size_t)i * rec_words + 12] = NO_NORMAL;
+}
+__global__ __launch_bounds__(TB) void k_pack_hits(const uint32_t* __restrict__ recs, uint32_t* __restrict__ out,
+                                                  uint32_t words, uint32_t rec_words) {
+  const uint32_t t = blockIdx.x * TB + threadIdx.x;
+  if (t >= words) return;
+  const uint32_t per = rec_words > 12 ? HIT_WORDS : 1u, i = t / per, w = t - i * per;
+  out[t] = recs[(size_t)i * rec_words + (w == 0 ? 8u : 11u + w)];
+}
 
 // Sort key of a ray: 30-bit Morton code of its origin in the scene box
 // (origins outside are clamped to the box faces); inactive rays sort last.
@@ -1781,6 +1810,17 @@ void launch_trace_inst_counted(const DevTop& top, void* rays, uint32_t M, uint64
     launch_inst_one<false, false, true>(top, rp, M, stride, 0xffffffffu, err, counter, refill, s, tp, top_visits,
                                         obj_visits, target_obj);
   RTG_HIP(hipGetLastError());
+}
+
+void unpack_rays(const uint32_t* in, void* recs, uint32_t n, bool occluded, hipStream_t s) {
+  hipLaunchKernelGGL(k_unpack_rays, dim3(div_up((size_t)n * RAY_WORDS, TB)), dim3(TB), 0, s, in, (uint32_t*)recs,
+                     n * RAY_WORDS, occluded ? 12u : 20u);
+}
+
+void pack_hits(const void* recs, uint32_t* out, uint32_t n, bool occluded, hipStream_t s) {
+  const uint32_t words = n * (occluded ? 1u : HIT_WORDS);
+  hipLaunchKernelGGL(k_pack_hits, dim3(div_up(words, TB)), dim3(TB), 0, s, (const uint32_t*)recs, out, words,
+                     occluded ? 12u : 20u);
 }
 
 namespace {

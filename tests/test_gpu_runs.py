@@ -4,6 +4,7 @@ stream length around the edges of a block, of the change between the two, of
 the eight queues and the waves' first runs is traced once, byte-identical to
 the oracle."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -37,15 +38,83 @@ def scene(rtc, device, oracle):
     sc.release()
 
 
+def on_device(rtc, device, sc, recs, call):
+    d = device.malloc(recs.nbytes)
+    device.memcpy(d, recs.ctypes.data, recs.nbytes)
+    call(sc.h, ctypes.byref(rtc.init_context()), d, len(recs), recs.itemsize)
+    device.check("query")
+    device.memcpy(recs.ctypes.data, d, recs.nbytes)
+    device.free(d)
+    return recs
+
+
 @pytest.mark.parametrize("n", SIZES)
 def test_every_record_of_a_stream(rtc, device, scene, n):
     sc, rays, hits, shadow, dark = scene
-    out = rays[:n].copy()
-    sc.intersect1M(out)
-    assert len(mismatches(out, hits[:n])) == 0
-    occ = shadow[:n].copy()
-    sc.occluded1M(occ)
-    assert len(mismatches(occ, dark[:n])) == 0
+    L = rtc.lib()
+    assert len(mismatches(on_device(rtc, device, sc, rays[:n].copy(), L.rtcIntersect1M), hits[:n])) == 0
+    assert len(mismatches(on_device(rtc, device, sc, shadow[:n].copy(), L.rtcOccluded1M), dark[:n])) == 0
+
+
+# in place in pinned memory up to 8192 records, then chunks of 16384 to 65536 on up to eight threads
+@pytest.mark.parametrize("stride", [0, 12])
+@pytest.mark.parametrize("n", [1, 2, 8191, 8192, 8193, 16384, 16385, 50001, 300001, 600001])
+def test_every_record_in_host_memory(rtc, device, scene, n, stride):
+    sc, rays, hits, shadow, dark = scene
+    L = rtc.lib()
+    for src, ref, call in ((rays, hits, L.rtcIntersect1M), (shadow, dark, L.rtcOccluded1M)):
+        step = src.itemsize + stride
+        buf = np.full((n, step), 0xA5, np.uint8)
+        buf[:, :src.itemsize] = src[:n].view(np.uint8).reshape(n, -1)
+        call(sc.h, ctypes.byref(rtc.init_context()), buf.ctypes.data, n, step)
+        device.check("query")
+        got = np.ascontiguousarray(buf[:, :src.itemsize]).reshape(-1).view(src.dtype)
+        assert len(mismatches(got, ref[:n])) == 0
+        assert (buf[:, src.itemsize:] == 0xA5).all()
+
+
+def test_host_queries_of_several_threads(rtc, device, scene):
+    sc, rays, hits, _, _ = scene
+    bad = []
+
+    def one(n, first):
+        out = rays[first:first + n].copy()
+        sc.intersect1M(out)
+        bad.append(len(mismatches(out, hits[first:first + n])))
+
+    th = [threading.Thread(target=one, args=(100000 + 7 * k, 20000 * k)) for k in range(6)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert bad == [0] * 6
+
+
+def test_geometry_uploads_in_pieces_and_again(rtc, oracle):
+    # buffers above and below the size that several threads copy, with a vertex
+    # stride, in one geometry that changes size from commit to commit
+    dev = rtc.Device("")
+    L = rtc.lib()
+    sc = rtc.Scene(dev)
+    g = L.rtcNewGeometry(dev.h, rtc.RTC_GEOMETRY_TYPE_TRIANGLE)
+    L.rtcAttachGeometry(sc.h, g)
+    rays = rtc.gen_random_rays(2000, seed=8)
+    for n in (500, 400000, 399000, 900000, 40, 400000):
+        v, ix = rtc.gen_soup(n, seed=n, h=0.02)
+        wide = np.full((len(v) + 1, 5), np.nan, np.float32)
+        wide[:-1, :3] = v
+        ix = np.ascontiguousarray(ix)
+        L.rtcSetSharedGeometryBuffer(g, rtc.RTC_BUFFER_TYPE_VERTEX, 0, rtc.RTC_FORMAT_FLOAT3, wide.ctypes.data, 0, 20, len(v))
+        L.rtcSetSharedGeometryBuffer(g, rtc.RTC_BUFFER_TYPE_INDEX, 0, rtc.RTC_FORMAT_UINT3, ix.ctypes.data, 0, 12, n)
+        L.rtcCommitGeometry(g)
+        sc.commit()
+        out, ref = rays.copy(), rays.copy()
+        sc.intersect1M(out)
+        oracle.BVH([(v, ix)]).intersect(ref)
+        assert len(mismatches(out, ref)) == 0, n
+    L.rtcReleaseGeometry(g)
+    sc.release()
+    dev.release()
 
 
 @pytest.mark.parametrize("n", [1, 65, 2049, 327681, 600001])
@@ -56,8 +125,7 @@ def test_every_record_through_an_instance(rtc, device, oracle, scene, n):
     top = rtc.Scene(device)
     top.add_instance(sc, l2w)
     top.commit()
-    out = rays[:n].copy()
-    top.intersect1M(out)
+    out = on_device(rtc, device, top, rays[:n].copy(), rtc.lib().rtcIntersect1M)
     ref = rays[:n].copy()
     o = oracle.Instances()
     o.add_instance(o.add_object([rtc.gen_sphere(8)]), l2w, 0)
