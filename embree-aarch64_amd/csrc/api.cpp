@@ -170,6 +170,7 @@ struct Device : RefObj {
   void* memptr = nullptr;
   std::mutex build_mtx;
   rtg::BuildScratch scratch;
+  rtg::DeviceBVH other;  // scratch of HIGH commits: the tree that was not kept (under build_mtx)
   // tri_builder / builder setting: "default" lets the build quality choose
   // (reference bvh8_factory.cpp:865-870); an unknown name fails the commit.
   enum { TB_DEFAULT, TB_SAH, TB_MORTON, TB_UNKNOWN } tri_builder = TB_DEFAULT;
@@ -562,10 +563,9 @@ void build_scene_tree(Scene* sc, Device* d, const std::vector<rtg::GeomDesc>& de
   if (sc->bvh->stats.num_split == 0) return;
   rtg::BuildParams q = p;
   q.split_budget = 0.0f;
-  rtg::DeviceBVH plain;
-  rtg::build_bvh(descs, q, d->scratch, plain, st);
+  rtg::build_bvh(descs, q, d->scratch, d->other, st);
   RTG_HIP(hipStreamSynchronize(st));
-  if (plain.stats.sah <= sc->bvh->stats.sah) sc->bvh->swap_tree(plain);
+  if (d->other.stats.sah <= sc->bvh->stats.sah) sc->bvh->swap_tree(d->other);
 }
 
 // Host threads that help a transfer of `bytes`: one for each 2 MB beyond the
