@@ -9,7 +9,6 @@
 #include "bvh_types.h"
 #include "gpu_util.h"
 #include "mlp.h"
-#include "sort.h"
 
 namespace rtg {
 
@@ -42,8 +41,7 @@ struct LevelReadback {
 };
 
 struct SahScratch {
-  DevBuf idx[2], blo[2], bhi[2], sid[2], segs[3][3], tiny, bins, splits, flags, scan, counters, roots;
-  Scanner scanner;
+  DevBuf idx[2], blo[2], bhi[2], sid[2], segs[3][3], tiny, bins[2], splits, below, before, counters, roots;
   LevelReadback rb;
 };
 

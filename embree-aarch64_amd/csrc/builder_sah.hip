@@ -18,9 +18,11 @@
 // Segments (contiguous position ranges still to split) are split by size
 // class; the class fixes how a segment is split, whatever kernel does it:
 //   big   (> 4096): positions in chunks of 1024 bin into LDS, the chunk bins
-//                   merge into per-segment bins in HBM with atomics, one
-//                   workgroup per segment picks the split, and a global scan
-//                   of left flags gives every position its stable destination;
+//                   merge into per-segment bins in HBM with atomics and the
+//                   chunk keeps its counts below each bin; one workgroup per
+//                   segment picks the split and sums the chunks' left counts
+//                   it implies, from which every position finds its stable
+//                   destination;
 //   mid   (513..4096): a 256-lane workgroup bins, picks and partitions in LDS;
 //   small (17..512): one wave, same code;
 //   tiny  (2..16): exact SAH splits over the references sorted by centroid
@@ -687,22 +689,33 @@ __global__ void k_fill_u32(uint32_t* p, size_t n, uint32_t v) {
   if (i < n) p[i] = v;
 }
 
-// Bins of the level's big segments; the grid covers the list's capacity
-// and the count is read on the device.
-__global__ void k_init_gbins(uint32_t* g, const uint32_t* nseg) {
+__device__ inline uint32_t empty_bin_word(int w) { return w >= 3 * NB && w < 3 * NB + 9 * NB ? NIL : 0u; }
+
+// Empty bins for the first level's big segments; k_big_split empties those
+// of each level after.
+__global__ void k_init_gbins(uint32_t* g, uint32_t nseg) {
   const size_t i = (size_t)blockIdx.x * TBS + threadIdx.x;
-  if (i >= (size_t)*nseg * BIN_WORDS) return;
-  const int w = (int)(i % BIN_WORDS);
-  g[i] = w < 3 * NB ? 0u : (w < 3 * NB + 9 * NB ? NIL : 0u);
+  if (i >= (size_t)nseg * BIN_WORDS) return;
+  g[i] = empty_bin_word((int)(i % BIN_WORDS));
 }
 
+// A chunk of CHUNK positions meets at most two big segments, because each is
+// longer than the chunk: one that holds the chunk's first position, and one
+// that begins after it. The chunk's counts below each bin and its left
+// references before it are kept per chunk under that side.
+static_assert(CHUNK <= MID_MAX, "a big segment must be longer than a chunk");
+constexpr int AXIS_BINS = 3 * NB;
+__device__ inline size_t chunk_row(uint32_t chunk, bool begins_inside) {
+  return ((size_t)chunk * 2 + (begins_inside ? 1 : 0)) * AXIS_BINS;
+}
 
-// A chunk of CHUNK positions meets at most two big segments (each is longer
-// than the chunk): they are binned in LDS and merged into HBM; any other
-// segment id (not expected) bins straight into HBM.
+// Bins the chunk's references into LDS, merges the bins into HBM and writes
+// the chunk's counts below each bin: below[chunk_row + axis * NB + k] is how
+// many of them a split "bin < k" sends left.
 __global__ __launch_bounds__(TBS) void k_big_bins(const uint32_t* __restrict__ sid, const float4* __restrict__ blo,
                                                   const float4* __restrict__ bhi, uint32_t n,
-                                                  const Seg* __restrict__ segs, uint32_t* gbins) {
+                                                  const Seg* __restrict__ segs, uint32_t* gbins,
+                                                  uint32_t* __restrict__ below, Counters* cnt) {
   // one set of bins per wave and segment slot (fewer lanes per LDS atomic),
   // merged before the merge into HBM
   constexpr int NW = TBS / 64;
@@ -777,7 +790,7 @@ __global__ __launch_bounds__(TBS) void k_big_bins(const uint32_t* __restrict__ s
     const float4 l = rl[j], h = rh[j];
     const int slot = s == slo_id ? 0 : (s == shi_id ? 1 : 2);
     if (slot == 2) {
-      bin_prim(gbins + (size_t)s * BIN_WORDS, make_mapping(segs[s]), l, h);
+      atomicOr(&cnt->error, 4u);
       continue;
     }
     if (slot != cslot) {
@@ -815,6 +828,19 @@ __global__ __launch_bounds__(TBS) void k_big_bins(const uint32_t* __restrict__ s
     for (int a = 0; a < 3; a++) flush(a);
   }
   __syncthreads();
+  if (tid < 2 * AXIS_BINS && (tid < AXIS_BINS || shi_id != slo_id)) {
+    // half-waves of NB lanes: exclusive prefix of an axis's counts
+    const int slot = tid / AXIS_BINS, e = tid % AXIS_BINS, b = e & (NB - 1);
+    uint32_t c = 0u;
+    for (int w = 0; w < NW; w++) c += sb[slot][w][e];
+    uint32_t x = c;
+#pragma unroll
+    for (int d = 1; d < NB; d <<= 1) {
+      const uint32_t y = __shfl_up(x, d, NB);
+      if (b >= d) x += y;
+    }
+    below[chunk_row(blockIdx.x, segs[slot ? shi_id : slo_id].first > c0) + e] = x - c;
+  }
   for (int slot = 0; slot < 2; slot++) {
     if (slot == 1 && shi_id == slo_id) break;
     uint32_t* g = gbins + (size_t)(slot ? shi_id : slo_id) * BIN_WORDS;
@@ -837,10 +863,18 @@ __global__ __launch_bounds__(TBS) void k_big_bins(const uint32_t* __restrict__ s
   }
 }
 
+// One workgroup per big segment: picks the split from its bins, empties the
+// bins of the up to two big children (their ids are below twice the count of
+// this level's segments) and turns the chunks' counts below the split into
+// the number of the segment's left references before each chunk. With these
+// k_big_scatter finds every destination by itself: no pass writes flags and
+// no scan runs over the positions (a build of 2^20 references takes 2.71 ms,
+// 2.95 with them; 300 k 1.52 and 1.61).
 template <bool LEARNED>
 __global__ __launch_bounds__(TBS, 4) void k_big_split(const Seg* __restrict__ segs, const uint32_t* __restrict__ nseg,
-                                                   const uint32_t* __restrict__ gbins, Split* __restrict__ splits,
-                                                   Lists nx, Tree t, LearnedCost lc) {
+                                                   const uint32_t* __restrict__ gbins, uint32_t* __restrict__ next_bins,
+                                                   const uint32_t* __restrict__ below, uint32_t* __restrict__ before,
+                                                   Split* __restrict__ splits, Lists nx, Tree t, LearnedCost lc) {
   __shared__ ChooseLds L;
   __shared__ uint32_t w[BIN_WORDS];  // the segment's bins, read once from HBM
   const uint32_t i = blockIdx.x;
@@ -848,10 +882,40 @@ __global__ __launch_bounds__(TBS, 4) void k_big_split(const Seg* __restrict__ se
   const Seg sg = segs[i];
   const uint32_t depth = sg.meta >> 1;
   const Mapping m = make_mapping(sg);
-  for (int k = threadIdx.x; k < BIN_WORDS; k += TBS) w[k] = gbins[(size_t)i * BIN_WORDS + k];
+  const int tid = threadIdx.x, lane = tid & 63;
+  for (int k = tid; k < BIN_WORDS; k += TBS) {
+    w[k] = gbins[(size_t)i * BIN_WORDS + k];
+    const uint32_t e = empty_bin_word(k);
+    if (2 * i < nx.cap[0]) next_bins[(size_t)(2 * i) * BIN_WORDS + k] = e;
+    if (2 * i + 1 < nx.cap[0]) next_bins[(size_t)(2 * i + 1) * BIN_WORDS + k] = e;
+  }
   __syncthreads();
-  Split sp = choose_split<TBS, false, LEARNED>(w, m, sg, lc, L, &t.cnt->error, threadIdx.x);
-  if (threadIdx.x != 0) return;
+  Split sp = choose_split<TBS, false, LEARNED>(w, m, sg, lc, L, &t.cnt->error, tid);
+  if (tid >= TBS - 64) {
+    // the last wave: chunks whose first position is the segment's, 64 at a
+    // time (an object median sends the first positions left)
+    const uint32_t ca = (sg.first + CHUNK - 1) / CHUNK, cz = (sg.first + sg.count - 1) / CHUNK;
+    const uint32_t col = (uint32_t)(sp.axis * NB + sp.k);
+    uint32_t sum = 0u;
+    if (sp.axis < 3 && ca * CHUNK != sg.first) sum = below[chunk_row(ca - 1, true) + col];
+    for (uint32_t c0 = ca; c0 <= cz; c0 += 64) {
+      const uint32_t c = c0 + (uint32_t)lane;
+      if (sp.axis == 3) {
+        if (c <= cz) before[c] = min(c * CHUNK - sg.first, sp.nleft);
+        continue;
+      }
+      const uint32_t v = c <= cz ? below[chunk_row(c, false) + col] : 0u;
+      uint32_t x = v;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(x, d);
+        if (lane >= d) x += y;
+      }
+      if (c <= cz) before[c] = sum + x - v;
+      sum += __shfl(x, 63);
+    }
+  }
+  if (tid != 0) return;
   // child centroid bounds: lo+hi of a primitive lies in [2 lo, 2 hi] of its
   // side's box, and in the parent's bounds
   float lcl[3], lch[3], rcl[3], rch[3];
@@ -883,49 +947,78 @@ __global__ __launch_bounds__(TBS, 4) void k_big_split(const Seg* __restrict__ se
   splits[i] = sp;
 }
 
-__global__ __launch_bounds__(TBS) void k_big_flags(const uint32_t* __restrict__ sid, const float4* __restrict__ blo,
-                                                   const float4* __restrict__ bhi, uint32_t n,
-                                                   const Seg* __restrict__ segs, const Split* __restrict__ splits,
-                                                   uint32_t* __restrict__ flags) {
-  const uint32_t i = blockIdx.x * TBS + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t s = sid[i];
-  uint32_t f = 0u;
-  if (s != NIL) f = goes_left(splits[s], blo[i], bhi[i], i - segs[s].first) ? 1u : 0u;
-  flags[i] = f;
-}
-
+// Moves a chunk's references to their side of their segment, in order: the
+// left ones of a position's segment before it are those before the chunk
+// (of a segment that began earlier) plus those of the chunk's positions
+// before it, counted by ballots over its 16 rows of 64.
 __global__ __launch_bounds__(TBS) void k_big_scatter(const uint32_t* __restrict__ sid, const uint32_t* __restrict__ idx,
                                                      const float4* __restrict__ blo, const float4* __restrict__ bhi,
                                                      uint32_t n, const Seg* __restrict__ segs,
                                                      const Split* __restrict__ splits,
-                                                     const uint32_t* __restrict__ flags,
-                                                     const uint32_t* __restrict__ scan, uint32_t* __restrict__ sid_o,
+                                                     const uint32_t* __restrict__ before, uint32_t* __restrict__ sid_o,
                                                      uint32_t* __restrict__ idx_o, float4* __restrict__ blo_o,
                                                      float4* __restrict__ bhi_o, uint32_t* __restrict__ vals,
                                                      Counters* cnt) {
-  const uint32_t i = blockIdx.x * TBS + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t s = sid[i];
-  if (s == NIL) {  // not in a big segment: the position keeps its place
-    sid_o[i] = NIL;
-    return;
+  constexpr int ROUNDS = (int)(CHUNK / TBS), NW = TBS / 64;
+  __shared__ uint32_t rows[ROUNDS * NW];  // left references of each row of 64 positions
+  __shared__ uint32_t s_skip;             // left references before the segment that begins in the chunk
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t c0 = blockIdx.x * CHUNK;
+  uint32_t sd[ROUNDS], id[ROUNDS], rank[ROUNDS];
+  float4 l[ROUNDS], h[ROUNDS];
+  bool left[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; r++) {
+    const uint32_t i = c0 + (uint32_t)(r * TBS + tid);
+    sd[r] = i < n ? sid[i] : NIL;
+    if (sd[r] != NIL) {
+      l[r] = blo[i];
+      h[r] = bhi[i];
+      id[r] = idx[i];
+    } else if (i < n) {
+      sid_o[i] = NIL;  // not in a big segment: the position keeps its place
+    }
   }
-  const uint32_t first = segs[s].first;
-  const Split& sp = splits[s];
-  const uint32_t lr = scan[i] - scan[first];
-  const bool left = flags[i] != 0u;
-  const uint32_t dst = left ? first + lr : first + sp.nleft + (i - first - lr);
-  if (dst >= first + segs[s].count) {
-    atomicOr(&cnt->error, 4u);
-    return;
+  const uint64_t below_lane = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+#pragma unroll
+  for (int r = 0; r < ROUNDS; r++) {
+    const uint32_t i = c0 + (uint32_t)(r * TBS + tid);
+    left[r] = sd[r] != NIL && goes_left(splits[sd[r]], l[r], h[r], i - segs[sd[r]].first);
+    const uint64_t m = __ballot(left[r]);
+    rank[r] = (uint32_t)__popcll(m & below_lane);
+    if (lane == 0) rows[r * NW + wave] = (uint32_t)__popcll(m);
   }
-  const uint32_t v = idx[i];
-  idx_o[dst] = v;
-  blo_o[dst] = blo[i];
-  bhi_o[dst] = bhi[i];
-  vals[dst] = v;
-  sid_o[dst] = left ? sp.lsid : sp.rsid;
+  __syncthreads();
+  uint32_t sum = 0u;
+#pragma unroll
+  for (int k = 0; k < ROUNDS * NW; k++) {
+    if (wave == k % NW) rank[k / NW] += sum;
+    sum += rows[k];
+  }
+#pragma unroll
+  for (int r = 0; r < ROUNDS; r++) {
+    const uint32_t i = c0 + (uint32_t)(r * TBS + tid);
+    if (sd[r] != NIL && i > c0 && segs[sd[r]].first == i) s_skip = rank[r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < ROUNDS; r++) {
+    if (sd[r] == NIL) continue;
+    const uint32_t i = c0 + (uint32_t)(r * TBS + tid);
+    const uint32_t first = segs[sd[r]].first;
+    const Split& sp = splits[sd[r]];
+    const uint32_t lr = first > c0 ? rank[r] - s_skip : before[blockIdx.x] + rank[r];
+    const uint32_t dst = left[r] ? first + lr : first + sp.nleft + (i - first - lr);
+    if (dst >= first + segs[sd[r]].count) {
+      atomicOr(&cnt->error, 4u);
+      continue;
+    }
+    idx_o[dst] = id[r];
+    blo_o[dst] = l[r];
+    bhi_o[dst] = h[r];
+    vals[dst] = id[r];
+    sid_o[dst] = left[r] ? sp.lsid : sp.rsid;
+  }
 }
 
 // ------------------------------------------------- mid and small segments --
@@ -1464,10 +1557,11 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
   for (int c = 0; c < 3; c++)
     for (int l = 0; l < 3; l++) S.segs[c][l].reserve((size_t)cap[c] * sizeof(Seg));
   S.tiny.reserve((size_t)tiny_cap * sizeof(TinyItem));
-  S.bins.reserve((size_t)cap[0] * BIN_WORDS * 4);
+  const uint32_t nchunks = div_up(n, CHUNK);
+  for (int p = 0; p < 2; p++) S.bins[p].reserve((size_t)cap[0] * BIN_WORDS * 4);
   S.splits.reserve((size_t)cap[0] * sizeof(Split));
-  S.flags.reserve((size_t)n * 4);
-  S.scan.reserve((size_t)n * 4);
+  S.below.reserve((size_t)nchunks * 2 * AXIS_BINS * 4);
+  S.before.reserve((size_t)nchunks * 4);
   S.counters.reserve(sizeof(Counters));
   S.roots.reserve(trees.size() * 4);
   Counters* cnt = S.counters.as<Counters>();
@@ -1508,6 +1602,8 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
     for (const Seg& sg : init[0]) longest = std::max(longest, sg.count);
     hipLaunchKernelGGL(k_fill_seg_ids, dim3(div_up(longest, TBS), cur[0]), dim3(TBS), 0, s, S.sid[0].as<uint32_t>(),
                        S.segs[0][0].as<Seg>());
+    hipLaunchKernelGGL(k_init_gbins, dim3(div_up((size_t)cur[0] * BIN_WORDS, TBS)), dim3(TBS), 0, s,
+                       S.bins[0].as<uint32_t>(), cur[0]);
   }
   Counters hc{};
   for (int c = 0; c < 3; c++) hc.nseg[0][c] = cur[c];
@@ -1563,23 +1659,15 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
     uint32_t gb[3];
     grid_bound(L, gb);
     if (big_live && gb[0]) {
-      hipLaunchKernelGGL(k_init_gbins, dim3(div_up((size_t)gb[0] * BIN_WORDS, TBS)), dim3(TBS), 0, s,
-                         S.bins.as<uint32_t>(), &cnt->nseg[li][0]);
-      hipLaunchKernelGGL(k_big_bins, dim3(div_up(n, CHUNK)), dim3(TBS), 0, s, S.sid[in].as<uint32_t>(),
-                         S.blo[in].as<float4>(), S.bhi[in].as<float4>(), n, bs, S.bins.as<uint32_t>());
-      if (lcost.P)
-        hipLaunchKernelGGL(k_big_split<true>, dim3(gb[0]), dim3(TBS), 0, s, bs, &cnt->nseg[li][0],
-                           S.bins.as<uint32_t>(), S.splits.as<Split>(), nx, t, lcost);
-      else
-        hipLaunchKernelGGL(k_big_split<false>, dim3(gb[0]), dim3(TBS), 0, s, bs, &cnt->nseg[li][0],
-                           S.bins.as<uint32_t>(), S.splits.as<Split>(), nx, t, lcost);
-      hipLaunchKernelGGL(k_big_flags, dim3(div_up(n, TBS)), dim3(TBS), 0, s, S.sid[in].as<uint32_t>(),
-                         S.blo[in].as<float4>(), S.bhi[in].as<float4>(), n, bs, S.splits.as<Split>(),
-                         S.flags.as<uint32_t>());
-      S.scanner.exclusive(S.flags.as<uint32_t>(), S.scan.as<uint32_t>(), n, s);
-      hipLaunchKernelGGL(k_big_scatter, dim3(div_up(n, TBS)), dim3(TBS), 0, s, S.sid[in].as<uint32_t>(),
+      hipLaunchKernelGGL(k_big_bins, dim3(nchunks), dim3(TBS), 0, s, S.sid[in].as<uint32_t>(),
+                         S.blo[in].as<float4>(), S.bhi[in].as<float4>(), n, bs, S.bins[in].as<uint32_t>(),
+                         S.below.as<uint32_t>(), cnt);
+      hipLaunchKernelGGL(lcost.P ? k_big_split<true> : k_big_split<false>, dim3(gb[0]), dim3(TBS), 0, s, bs,
+                         &cnt->nseg[li][0], S.bins[in].as<uint32_t>(), S.bins[o].as<uint32_t>(),
+                         S.below.as<uint32_t>(), S.before.as<uint32_t>(), S.splits.as<Split>(), nx, t, lcost);
+      hipLaunchKernelGGL(k_big_scatter, dim3(nchunks), dim3(TBS), 0, s, S.sid[in].as<uint32_t>(),
                          S.idx[in].as<uint32_t>(), S.blo[in].as<float4>(), S.bhi[in].as<float4>(), n, bs,
-                         S.splits.as<Split>(), S.flags.as<uint32_t>(), S.scan.as<uint32_t>(), S.sid[o].as<uint32_t>(),
+                         S.splits.as<Split>(), S.before.as<uint32_t>(), S.sid[o].as<uint32_t>(),
                          S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(), S.bhi[o].as<float4>(), vals, cnt);
     }
     // (k_seg clears the next level's counts: it runs even with no mid segment)
