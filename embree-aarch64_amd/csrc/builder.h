@@ -100,6 +100,8 @@ struct DeviceBVH {
 struct BuildScratch {
   DevBuf geoms, lo4, hi4, keys, vals, slo, shi, child, parent_int, parent_leaf, range, nlo, nhi, cost,
       isleaf, split8, visit, counters, sacc, leaf_src, roots;
+  PinnedBuf stage;  // geometries and scene ranges, read by kernels
+  HostPost post;    // the counters, as the host needs them
   DevBuf walk_top, walk_sub, walk_rest, walk_count, walk_stats;  // wide nodes, numbered and then written
   DevBuf refit_list[2], refit_count;  // nodes that span chunks
   RadixSorter sorter;

@@ -8,6 +8,7 @@
 //   leaf/inner decision by SAH cost and the 8-wide collapse that repeatedly
 //     opens the child with the largest half area: kernels/builders/bvh_builder_sah.h:222-330;
 //   leaf fill e1 = v0-v1, e2 = v2-v0: kernels/geometry/triangle.h:40-41,98-120.
+#include <algorithm>
 #include <chrono>
 #include <cstring>
 #include <string>
@@ -26,11 +27,15 @@ struct BuildCounters {
   uint32_t top_nodes;  // nodes that k_walk_top numbered
   uint32_t subtrees;   // subtrees that it left to k_walk_rest
   uint32_t max_depth;
-  uint32_t error;  // bit 0: refit walk too long, bit 1: collapse index out of range, bit 2: bad tree
+  uint32_t error;  // bit 0: refit walk too long, bit 1: collapse index out of range, bit 2: bad tree,
+                   // bit 8: the binary tree's build failed
   uint32_t max_stack;  // most traversal stack entries any root-to-node path can need
   uint32_t roots_seen; // tree roots met by the tree check
   double sah_nodes, sah_leaves, sah_leaves_tri;
 };
+
+constexpr uint32_t COUNTER_WORDS = sizeof(BuildCounters) / 4;
+static_assert(COUNTER_WORDS <= 63, "the counters are posted by one wave");
 
 constexpr uint32_t NONE = 0xffffffffu;
 constexpr int BT = 256;
@@ -98,7 +103,13 @@ __global__ void k_iota(uint32_t* v, uint32_t n) {
   if (i < n) v[i] = i;
 }
 
-__global__ void k_init_counters(BuildCounters* c, uint32_t nscenes) {
+// The counters of a new build, and its geometries from pinned memory.
+__global__ __launch_bounds__(BT) void k_init_build(BuildCounters* c, uint32_t nscenes,
+                                                   const uint32_t* __restrict__ stage, uint32_t* __restrict__ geoms,
+                                                   uint32_t words) {
+  const uint32_t i = blockIdx.x * BT + threadIdx.x;
+  if (i < words) geoms[i] = stage[i];
+  if (i != 0) return;
   for (int k = 0; k < 3; k++) {
     c->glo[k] = f2o(INFINITY);
     c->ghi[k] = f2o(-INFINITY);
@@ -297,8 +308,10 @@ __device__ inline uint32_t interleave3(uint32_t x) {
 
 __global__ __launch_bounds__(BT) void k_morton(const float4* __restrict__ lo4, const float4* __restrict__ hi4,
                                                uint32_t total, uint32_t* __restrict__ keys,
-                                               uint32_t* __restrict__ vals, const BuildCounters* __restrict__ cnt) {
+                                               uint32_t* __restrict__ vals, const BuildCounters* __restrict__ cnt,
+                                               uint32_t* post, uint32_t seq) {
   const uint32_t i = blockIdx.x * BT + threadIdx.x;
+  if (i < 64) post_words(post, seq, reinterpret_cast<const uint32_t*>(cnt), COUNTER_WORDS);
   if (i >= total) return;
   vals[i] = i;
   if (keys[i] == 0xffffffffu) return;
@@ -317,12 +330,41 @@ __global__ __launch_bounds__(BT) void k_morton(const float4* __restrict__ lo4, c
   keys[i] = interleave3(q[0]) | (interleave3(q[1]) << 1) | (interleave3(q[2]) << 2);
 }
 
+// Where the scenes' roots come from: `stage` (pinned) holds their first
+// positions, their primitive counts and the index of their tree.
+struct RootArgs {
+  uint32_t nscenes;           // 0: the roots are not placed yet
+  const uint32_t* stage;
+  const uint32_t* tree_root;  // null: the radix tree's root, node 0
+  const uint32_t* tree_error;
+  uint32_t* roots;            // binary references, first positions, primitive counts
+  uint32_t* error;
+};
+
+// The boxes in position order; also no node visited yet, and the scenes' roots.
 __global__ __launch_bounds__(BT) void k_gather_sorted(const uint32_t* __restrict__ vals,
                                                       const float4* __restrict__ lo4,
                                                       const float4* __restrict__ hi4, uint32_t n,
-                                                      float4* __restrict__ slo, float4* __restrict__ shi) {
+                                                      float4* __restrict__ slo, float4* __restrict__ shi,
+                                                      uint32_t* __restrict__ visit, RootArgs ra) {
   const uint32_t j = blockIdx.x * BT + threadIdx.x;
+  if (j < ra.nscenes) {
+    const uint32_t f = ra.stage[j], c = ra.stage[ra.nscenes + j];
+    uint32_t ref = c == 0u ? REF_EMPTY : f | REF_LEAF;
+    if (c >= 2u) {
+      ref = ra.tree_root ? ra.tree_root[ra.stage[2 * ra.nscenes + j]] : 0u;
+      if (ref + 1u >= n || ref == REF_EMPTY) {
+        atomicOr(ra.error, 256u);
+        ref = 0u;
+      }
+    }
+    ra.roots[j] = ref;
+    ra.roots[ra.nscenes + j] = f;
+    ra.roots[2 * ra.nscenes + j] = c;
+    if (j == 0u && ra.tree_error && *ra.tree_error) atomicOr(ra.error, 256u);
+  }
   if (j >= n) return;
+  if (j + 1u < n || n == 1u) visit[j] = 0u;
   const uint32_t o = vals[j];
   slo[j] = lo4[o];
   shi[j] = hi4[o];
@@ -1222,9 +1264,11 @@ __global__ __launch_bounds__(BT) void k_emit_nodes(CollapseArgs a) {
 
 // The sum of the emission's statistics (atomics of every workgroup on a few
 // counters took longer than the emission; this order of summation is fixed).
-__global__ __launch_bounds__(BT) void k_sum_stats(const CollapseStats* __restrict__ part, uint32_t n, BuildCounters* cnt) {
-  if (cnt->error) return;  // (nothing was emitted)
+// The counters then go to the host.
+__global__ __launch_bounds__(BT) void k_sum_stats(const CollapseStats* __restrict__ part, uint32_t n, BuildCounters* cnt,
+                                                  uint32_t* post, uint32_t seq) {
   CollapseStats st;
+  if (cnt->error) n = 0;  // (nothing was emitted)
   for (uint32_t i = threadIdx.x; i < n; i += BT) st.add(part[i]);
   block_stats(st);
   if (threadIdx.x == 0) {
@@ -1235,6 +1279,8 @@ __global__ __launch_bounds__(BT) void k_sum_stats(const CollapseStats* __restric
     cnt->sah_leaves = st.sah_leaves;
     cnt->sah_leaves_tri = st.sah_leaves_tri;
   }
+  __syncthreads();
+  if (threadIdx.x < 64) post_words(post, seq, reinterpret_cast<const uint32_t*>(cnt), COUNTER_WORDS);
 }
 
 // ------------------------------------------------------------------ host --
@@ -1266,8 +1312,11 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   const uint32_t min_leaf = prm.min_leaf < 1 ? 1 : (prm.min_leaf > max_leaf ? max_leaf : prm.min_leaf);
   const uint32_t block = prm.block < 1 ? 1 : prm.block;
 
+  if (nscenes == 0 || nscenes > 65535) throw hip_error(hipErrorInvalidValue, "scene count out of range");
   S.geoms.reserve(geoms.size() * sizeof(GeomDesc));
-  RTG_HIP(hipMemcpyAsync(S.geoms.ptr, geoms.data(), geoms.size() * sizeof(GeomDesc), hipMemcpyHostToDevice, s));
+  const uint32_t geom_words = (uint32_t)(geoms.size() * sizeof(GeomDesc) / 4);
+  S.stage.reserve(((size_t)geom_words + 3 * (size_t)nscenes) * 4);
+  memcpy(S.stage.ptr, geoms.data(), (size_t)geom_words * 4);
   S.counters.reserve(sizeof(BuildCounters));
   S.lo4.reserve((size_t)total * 16);
   S.hi4.reserve((size_t)total * 16);
@@ -1275,7 +1324,6 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   S.vals.reserve((size_t)total * 4);
   BuildCounters* cnt = S.counters.as<BuildCounters>();
 
-  if (nscenes == 0 || nscenes > 65535) throw hip_error(hipErrorInvalidValue, "scene count out of range");
   const bool batched = nscenes > 1;
   SceneAcc* sacc = nullptr;
   if (batched) {
@@ -1283,27 +1331,31 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
     sacc = S.sacc.as<SceneAcc>();
     hipLaunchKernelGGL(k_init_sacc, dim3(div_up(nscenes, BT)), dim3(BT), 0, s, sacc, nscenes);
   }
-  hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(1), 0, s, cnt, nscenes);
+  hipLaunchKernelGGL(k_init_build, dim3(div_up(geom_words, BT)), dim3(BT), 0, s, cnt, nscenes,
+                     S.stage.as<uint32_t>(), S.geoms.as<uint32_t>(), geom_words);
   hipLaunchKernelGGL(k_primrefs, dim3(div_up(total, (size_t)BT * PR_PER)), dim3(BT), 0, s, S.geoms.as<GeomDesc>(),
                      (uint32_t)geoms.size(), total, S.lo4.as<float4>(), S.hi4.as<float4>(), S.keys.as<uint32_t>(), cnt,
                      sacc);
+  BuildCounters hc;
+  std::vector<SceneAcc> hs(batched ? nscenes : 0);
   if (batched) {
     // group the references by scene (stable, so each scene keeps primref order); invalid ones sort last
     hipLaunchKernelGGL(k_iota, dim3(div_up(total, BT)), dim3(BT), 0, s, S.vals.as<uint32_t>(), total);
     RTG_HIP(hipGetLastError());
     S.sorter.sort_pairs(S.keys.as<uint32_t>(), S.vals.as<uint32_t>(), total, 0, 16, s);
+    RTG_HIP(hipMemcpyAsync(&hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, s));
+    RTG_HIP(hipMemcpyAsync(hs.data(), sacc, nscenes * sizeof(SceneAcc), hipMemcpyDeviceToHost, s));
+    RTG_HIP(hipStreamSynchronize(s));
   } else {
+    // (the counts and bounds are final here: the host gets them while the sort runs)
+    uint32_t* post = S.post.arm();
     hipLaunchKernelGGL(k_morton, dim3(div_up(total, BT)), dim3(BT), 0, s, S.lo4.as<float4>(), S.hi4.as<float4>(),
-                       total, S.keys.as<uint32_t>(), S.vals.as<uint32_t>(), cnt);
+                       total, S.keys.as<uint32_t>(), S.vals.as<uint32_t>(), cnt, post, S.post.seq);
     RTG_HIP(hipGetLastError());
     S.sorter.sort_pairs(S.keys.as<uint32_t>(), S.vals.as<uint32_t>(), total, 0, 32, s);
+    S.post.wait(s);
+    memcpy(&hc, S.post.words(), sizeof(hc));
   }
-
-  BuildCounters hc;
-  RTG_HIP(hipMemcpyAsync(&hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, s));
-  std::vector<SceneAcc> hs(batched ? nscenes : 0);
-  if (batched) RTG_HIP(hipMemcpyAsync(hs.data(), sacc, nscenes * sizeof(SceneAcc), hipMemcpyDeviceToHost, s));
-  RTG_HIP(hipStreamSynchronize(s));
   uint32_t n = hc.valid;
   out.stats.num_prims = n;
   for (int k = 0; k < 3; k++) {
@@ -1314,7 +1366,7 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   out.slots.assign(nscenes, SceneSlot());
   std::vector<uint32_t> first(nscenes, 0), count(nscenes, 0);
   std::vector<SahRoot> trees;
-  std::vector<uint32_t> tree_scene;
+  std::vector<uint32_t> tree_of(nscenes, 0);
   {
     uint32_t pos = 0;
     for (uint32_t sI = 0; sI < nscenes; sI++) {
@@ -1336,8 +1388,8 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
           r.clo[k] = o2f(batched ? hs[sI].clo[k] : hc.clo[k]);
           r.chi[k] = o2f(batched ? hs[sI].chi[k] : hc.chi[k]);
         }
+        tree_of[sI] = (uint32_t)trees.size();
         trees.push_back(r);
-        tree_scene.push_back(sI);
       }
     }
     if (pos != n) throw hip_error(hipErrorUnknown, "per-scene primitive counts disagree with the total");
@@ -1369,9 +1421,6 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
 
   S.slo.reserve((size_t)n * 16);
   S.shi.reserve((size_t)n * 16);
-  hipLaunchKernelGGL(k_gather_sorted, dim3(div_up(n, BT)), dim3(BT), 0, s, S.vals.as<uint32_t>(), S.lo4.as<float4>(),
-                     S.hi4.as<float4>(), n, S.slo.as<float4>(), S.shi.as<float4>());
-
   const uint32_t ninner = n > 1 ? n - 1 : 1;
   S.child.reserve((size_t)ninner * 8);
   S.parent_int.reserve((size_t)ninner * 4);
@@ -1383,28 +1432,35 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   S.split8.reserve((size_t)ninner * 8);
   S.isleaf.reserve((size_t)ninner);
   S.visit.reserve((size_t)ninner * 4);
-  std::vector<uint32_t> root_ref(nscenes, REF_EMPTY);
-  for (uint32_t sI = 0; sI < nscenes; sI++)
-    if (count[sI] == 1) root_ref[sI] = first[sI] | REF_LEAF;
+  S.roots.reserve((size_t)nscenes * 12);
+  uint32_t* sstage = S.stage.as<uint32_t>() + geom_words;
+  std::copy(first.begin(), first.end(), sstage);
+  std::copy(count.begin(), count.end(), sstage + nscenes);
+  std::copy(tree_of.begin(), tree_of.end(), sstage + 2 * (size_t)nscenes);
+  RootArgs ra_none{}, ra_place{nscenes, sstage, nullptr, nullptr, S.roots.as<uint32_t>(), &cnt->error};
+  auto gather = [&](const RootArgs& r) {
+    hipLaunchKernelGGL(k_gather_sorted, dim3(div_up(std::max(n, r.nscenes), BT)), dim3(BT), 0, s,
+                       S.vals.as<uint32_t>(), S.lo4.as<float4>(), S.hi4.as<float4>(), n, S.slo.as<float4>(),
+                       S.shi.as<float4>(), S.visit.as<uint32_t>(), r);
+  };
   const bool use_sah = batched || prm.builder == BUILDER_SAH || prm.learned;
+  gather(use_sah && !trees.empty() ? ra_none : ra_place);
   if (!trees.empty()) {
-    RTG_HIP(hipMemsetAsync(S.visit.ptr, 0, (size_t)ninner * 4, s));
     if (batched)
       hipLaunchKernelGGL(k_fill_none, dim3(div_up(n, BT)), dim3(BT), 0, s, S.parent_leaf.as<uint32_t>(), n);
     if (use_sah) {
-      SahTreeOut so;
+      SahRoots so;
       build_sah_tree(n, S.vals.as<uint32_t>(), S.slo.as<float4>(), S.shi.as<float4>(), trees, S.child.as<uint32_t>(),
                      S.parent_int.as<uint32_t>(), S.parent_leaf.as<uint32_t>(), S.range.as<uint2>(),
                      prm.learned, prm.median_below, S.sah, so, s);
-      for (size_t k = 0; k < trees.size(); k++) root_ref[tree_scene[k]] = so.roots[k];
       // boxes in the final primitive order
-      hipLaunchKernelGGL(k_gather_sorted, dim3(div_up(n, BT)), dim3(BT), 0, s, S.vals.as<uint32_t>(),
-                         S.lo4.as<float4>(), S.hi4.as<float4>(), n, S.slo.as<float4>(), S.shi.as<float4>());
+      ra_place.tree_root = so.roots;
+      ra_place.tree_error = so.error;
+      gather(ra_place);
     } else {
       hipLaunchKernelGGL(k_radix_tree, dim3(div_up(n - 1, BT)), dim3(BT), 0, s, S.keys.as<uint32_t>(), (int)n,
                          S.child.as<uint32_t>(), S.parent_int.as<uint32_t>(), S.parent_leaf.as<uint32_t>(),
                          S.range.as<uint2>());
-      root_ref[0] = 0;
     }
     RefitArgs ra{n, S.child.as<uint32_t>(), S.range.as<uint2>(), S.slo.as<float4>(), S.shi.as<float4>(),
                  S.nlo.as<float4>(), S.nhi.as<float4>(), S.cost.as<float>(), S.split8.as<uint8_t>(),
@@ -1446,7 +1502,7 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
 
   if (user) {  // the binary tree with its collapse decisions, for the caller's own nodes
     const uint32_t ni = n > 1 ? n - 1 : 0;
-    user->root = root_ref[0];
+    RTG_HIP(hipMemcpyAsync(&user->root, S.roots.ptr, 4, hipMemcpyDeviceToHost, s));
     user->child.resize(2 * (size_t)ni);
     user->range.resize(2 * (size_t)ni);
     user->split8.resize(8 * (size_t)ni);
@@ -1481,12 +1537,7 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   if (inst_build) out.insts.reserve((size_t)n * sizeof(InstRec));
   else out.tris.reserve((size_t)n * sizeof(TriRec));
   out.info.reserve((size_t)cap * sizeof(NodeInfo));
-  // the scenes' roots, first positions and primitive counts, then the walk's arrays
   const uint32_t max_sub = nscenes > 1 ? nscenes + SUB_MAX : SUB_MAX;
-  S.roots.reserve((size_t)nscenes * 12);
-  root_ref.insert(root_ref.end(), first.begin(), first.end());
-  root_ref.insert(root_ref.end(), count.begin(), count.end());
-  RTG_HIP(hipMemcpyAsync(S.roots.ptr, root_ref.data(), (size_t)nscenes * 12, hipMemcpyHostToDevice, s));
   S.walk_top.reserve((size_t)top_cap(max_sub) * sizeof(WideNode));
   S.walk_sub.reserve((size_t)max_sub * sizeof(WideNode));
   S.walk_rest.reserve((size_t)n * sizeof(WideNode));
@@ -1524,14 +1575,16 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   S.walk_stats.reserve((size_t)egrid * sizeof(CollapseStats));
   ca.stats = S.walk_stats.as<CollapseStats>();
   hipLaunchKernelGGL(k_emit_nodes, dim3(egrid), dim3(BT), 0, s, ca);
-  hipLaunchKernelGGL(k_sum_stats, dim3(1), dim3(BT), 0, s, ca.stats, egrid, cnt);
+  uint32_t* post = S.post.arm();
+  hipLaunchKernelGGL(k_sum_stats, dim3(1), dim3(BT), 0, s, ca.stats, egrid, cnt, post, S.post.seq);
   hipLaunchKernelGGL(k_write_leaves, dim3(div_up(n, BT)), dim3(BT), 0, s, S.leaf_src.as<uint32_t>(),
                      S.vals.as<uint32_t>(), S.lo4.as<float4>(), S.hi4.as<float4>(), S.geoms.as<GeomDesc>(), cnt,
                      inst_build ? nullptr : out.tris.as<TriRec>(), inst_build ? out.insts.as<InstRec>() : nullptr,
                      prm.robust ? 1u : 0u, n);
   RTG_HIP(hipGetLastError());
-  RTG_HIP(hipMemcpyAsync(&hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, s));
   RTG_HIP(hipStreamSynchronize(s));
+  S.post.wait(s);
+  memcpy(&hc, S.post.words(), sizeof(hc));
   if (!trees.empty() && (hc.roots_seen != roots_expected || (hc.error & 5u)))
     throw hip_error(hipErrorUnknown, "binary tree check failed: error bits " + std::to_string(hc.error) + ", roots " +
                                          std::to_string(hc.roots_seen) + " of " + std::to_string(roots_expected));

@@ -12,37 +12,10 @@
 
 namespace rtg {
 
-// Pinned host slots and events through which the host reads a level's
-// counters while the next level already runs.
-struct LevelReadback {
-  static constexpr int K = 2;
-  void* host = nullptr;
-  size_t bytes = 0;  // per slot
-  hipEvent_t ev[K] = {};
-  void ensure(size_t b) {
-    if (!ev[0])
-      for (hipEvent_t& e : ev) RTG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    if (b <= bytes) return;
-    if (host) (void)hipHostFree(host);
-    host = nullptr;
-    bytes = 0;
-    RTG_HIP(hipHostMalloc(&host, K * b, hipHostMallocDefault));
-    bytes = b;
-  }
-  void* slot(int k) const { return (char*)host + (size_t)(k % K) * bytes; }
-  ~LevelReadback() {
-    for (hipEvent_t e : ev)
-      if (e) (void)hipEventDestroy(e);
-    if (host) (void)hipHostFree(host);
-  }
-  LevelReadback() = default;
-  LevelReadback(const LevelReadback&) = delete;
-  LevelReadback& operator=(const LevelReadback&) = delete;
-};
-
 struct SahScratch {
   DevBuf idx[2], blo[2], bhi[2], sid[2], segs[3][3], tiny, bins[2], splits, below, before, counters, roots;
-  LevelReadback rb;
+  PinnedBuf stage;  // the trees' segments, read by the first kernel
+  HostPost post;    // a level's counts, read while it runs
 };
 
 // One tree of the forest: positions [first, first+count), count >= 2.
@@ -51,9 +24,11 @@ struct SahRoot {
   float clo[3], chi[3];  // bounds of lo+hi over its references
 };
 
-struct SahTreeOut {
-  std::vector<uint32_t> roots;  // inner node id of each tree's root
-  uint32_t levels = 0;          // top-down levels run
+// Where the device finds the trees' root ids (NIL, 0xffffffff, if missing) and
+// the build's error bits, once the work queued on the stream has run.
+struct SahRoots {
+  const uint32_t* roots = nullptr;
+  const uint32_t* error = nullptr;
 };
 
 // Inputs: n valid references, `vals` holding their primref indices and
@@ -64,11 +39,12 @@ struct SahTreeOut {
 // id is its split position, so ids lie in [0, n-2]; ids no tree uses keep
 // parent_int = REF_EMPTY).
 // `learned` (may be null) replaces the half-area term of the split cost.
+// The build is still queued on the stream when the call returns.
 // Segments of at most median_below (<= 64) references are split at their
 // median position all the way down instead of by binned SAH.
 void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4* shi,
                     const std::vector<SahRoot>& trees, uint32_t* child, uint32_t* parent_int,
                     uint32_t* parent_leaf, uint2* range, const LearnedCost* learned,
-                    uint32_t median_below, SahScratch& S, SahTreeOut& out, hipStream_t s);
+                    uint32_t median_below, SahScratch& S, SahRoots& out, hipStream_t s);
 
 }  // namespace rtg

@@ -37,7 +37,6 @@
 // which is unique, so the output does not depend on the order in which
 // segments are processed.
 #include <algorithm>
-#include <cstring>
 #include <string>
 
 #include "builder_sah.h"
@@ -92,6 +91,16 @@ struct Counters {
                      // bit 3: median subtree stack overflow, bit 4: a tiny segment out of range
 };
 
+// What a level's first kernel does besides its work: it posts the counts of
+// the level's segments to the host and clears the counts that the next level
+// fills. post is null for the first level and for a level's other kernels.
+struct LevelStart {
+  Counters* cnt;
+  uint32_t* post;
+  uint32_t seq;
+  uint32_t in, clear;  // list slots
+};
+
 struct Lists {
   Seg* seg[3];       // next level's big, mid and small segments
   uint32_t* nseg;    // and their counts
@@ -111,6 +120,19 @@ struct Tree {
   Counters* cnt;
   uint32_t* roots;  // per tree
 };
+
+__device__ inline void start_level(const LevelStart& st) {
+  if (!st.post || blockIdx.x != 0 || threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  if (lane < 3) {
+    st.post[1 + lane] = st.cnt->nseg[st.in][lane];
+    st.cnt->nseg[st.clear][lane] = 0u;
+  }
+  if (lane == 3) st.post[4] = __hip_atomic_load(&st.cnt->ntiny, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (lane == 4) st.post[5] = __hip_atomic_load(&st.cnt->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __threadfence_system();
+  if (lane == 0) __hip_atomic_store(st.post, st.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 struct Mapping {
   float ofs[3], scale[3];
@@ -684,20 +706,7 @@ __device__ inline Split choose_split(const uint32_t* w, const Mapping& m, const 
 
 // ------------------------------------------------------------ big segments --
 
-__global__ void k_fill_u32(uint32_t* p, size_t n, uint32_t v) {
-  const size_t i = (size_t)blockIdx.x * TBS + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
 __device__ inline uint32_t empty_bin_word(int w) { return w >= 3 * NB && w < 3 * NB + 9 * NB ? NIL : 0u; }
-
-// Empty bins for the first level's big segments; k_big_split empties those
-// of each level after.
-__global__ void k_init_gbins(uint32_t* g, uint32_t nseg) {
-  const size_t i = (size_t)blockIdx.x * TBS + threadIdx.x;
-  if (i >= (size_t)nseg * BIN_WORDS) return;
-  g[i] = empty_bin_word((int)(i % BIN_WORDS));
-}
 
 // A chunk of CHUNK positions meets at most two big segments, because each is
 // longer than the chunk: one that holds the chunk's first position, and one
@@ -715,13 +724,14 @@ __device__ inline size_t chunk_row(uint32_t chunk, bool begins_inside) {
 __global__ __launch_bounds__(TBS) void k_big_bins(const uint32_t* __restrict__ sid, const float4* __restrict__ blo,
                                                   const float4* __restrict__ bhi, uint32_t n,
                                                   const Seg* __restrict__ segs, uint32_t* gbins,
-                                                  uint32_t* __restrict__ below, Counters* cnt) {
+                                                  uint32_t* __restrict__ below, Counters* cnt, LevelStart st) {
   // one set of bins per wave and segment slot (fewer lanes per LDS atomic),
   // merged before the merge into HBM
   constexpr int NW = TBS / 64;
   __shared__ uint32_t sb[2][NW][BIN_WORDS];
   __shared__ uint32_t s_lo, s_hi;
   __shared__ Mapping sm[2];
+  start_level(st);
   const int tid = threadIdx.x, wave = tid >> 6;
   const uint32_t c0 = blockIdx.x * CHUNK;
   const uint32_t c1 = c0 + CHUNK < n ? c0 + CHUNK : n;
@@ -1207,10 +1217,9 @@ __global__ __launch_bounds__(256, 4) void k_seg(const Seg* __restrict__ segs, co
                                              const uint32_t* __restrict__ idx, const float4* __restrict__ blo,
                                              const float4* __restrict__ bhi, uint32_t* __restrict__ idx_o,
                                              float4* __restrict__ blo_o, float4* __restrict__ bhi_o, Lists nx,
-                                             Tree t, LearnedCost lc, uint32_t* __restrict__ clear) {
+                                             Tree t, LearnedCost lc, LevelStart st) {
   __shared__ SegLds<256> S;
-  // the counts the next level fills (no kernel of this level uses them)
-  if (blockIdx.x == 0 && threadIdx.x < 3) clear[threadIdx.x] = 0u;
+  start_level(st);
   if (blockIdx.x >= *nseg) return;
   const Seg sg = segs[blockIdx.x];
   float lcl[3], lch[3], rcl[3], rch[3];
@@ -1239,9 +1248,10 @@ __global__ __launch_bounds__(SEGW_TB) void k_seg_wave(const Seg* __restrict__ se
                                                       const uint32_t* __restrict__ idx, const float4* __restrict__ blo,
                                                       const float4* __restrict__ bhi, uint32_t* __restrict__ idx_o,
                                                       float4* __restrict__ blo_o, float4* __restrict__ bhi_o, Lists nx,
-                                                      Tree t, LearnedCost lc) {
+                                                      Tree t, LearnedCost lc, LevelStart st) {
   __shared__ SegLds<64> S[SEGW_WAVES];
   __shared__ uint32_t lcount[4], lbase[4];
+  start_level(st);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t i = blockIdx.x * SEGW_WAVES + (uint32_t)wave;
   if (threadIdx.x < 4) lcount[threadIdx.x] = 0u;
@@ -1530,12 +1540,52 @@ __global__ void k_fill_seg_ids(uint32_t* sid, const Seg* segs) {
   if (i < sg.count) sid[sg.first + i] = blockIdx.y;
 }
 
+// Everything that the level loop finds filled: the references' indices, the
+// marks of unused inner node ids, the big-segment id of every position (of the
+// first big segment; k_fill_seg_ids adds the others), empty bins for the big
+// segments, the trees' segments (from pinned memory), their roots and the
+// counters.
+struct Begin {
+  uint32_t n, ntrees;
+  const uint32_t* vals;
+  uint32_t* idx;
+  uint32_t* parent_int;
+  uint32_t* sid;
+  uint32_t* bins;
+  uint32_t* roots;
+  Counters* cnt;
+  uint32_t count[3];         // segments by class
+  uint32_t first0, count0;   // positions of the first big segment
+  const uint32_t* stage;     // the segments, class by class
+  uint32_t* seg[3];
+};
+
+__global__ __launch_bounds__(TBS) void k_begin(Begin b) {
+  const uint32_t i = blockIdx.x * TBS + threadIdx.x;
+  if (i < b.n) {
+    b.idx[i] = b.vals[i];
+    if (i + 1 < b.n) b.parent_int[i] = REF_EMPTY;
+    if (b.count[0]) b.sid[i] = i - b.first0 < b.count0 ? 0u : NIL;
+  }
+  if (i < b.ntrees) b.roots[i] = NIL;
+  if (i < b.count[0] * (uint32_t)BIN_WORDS) b.bins[i] = empty_bin_word((int)(i % BIN_WORDS));
+  constexpr uint32_t SW = sizeof(Seg) / 4;
+  const uint32_t c0 = b.count[0] * SW, c1 = c0 + b.count[1] * SW, c2 = c1 + b.count[2] * SW;
+  for (uint32_t w = i; w < c2; w += gridDim.x * TBS) {
+    const uint32_t v = b.stage[w];
+    if (w < c0) b.seg[0][w] = v;
+    else if (w < c1) b.seg[1][w - c0] = v;
+    else b.seg[2][w - c1] = v;
+  }
+  if (i < sizeof(Counters) / 4) reinterpret_cast<uint32_t*>(b.cnt)[i] = i < 3 ? b.count[i] : 0u;
+}
+
 }  // namespace
 
 void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4* shi,
                     const std::vector<SahRoot>& trees, uint32_t* child, uint32_t* parent_int,
                     uint32_t* parent_leaf, uint2* range, const LearnedCost* learned,
-                    uint32_t fin_max, SahScratch& S, SahTreeOut& out, hipStream_t s) {
+                    uint32_t fin_max, SahScratch& S, SahRoots& out, hipStream_t s) {
   if (fin_max > MEDIAN_MAX) fin_max = MEDIAN_MAX;
   LearnedCost lcost{};
   if (learned) lcost = *learned;
@@ -1566,14 +1616,6 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
   S.roots.reserve(trees.size() * 4);
   Counters* cnt = S.counters.as<Counters>();
 
-  RTG_HIP(hipMemcpyAsync(S.idx[0].ptr, vals, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
-  RTG_HIP(hipMemcpyAsync(S.blo[0].ptr, slo, (size_t)n * 16, hipMemcpyDeviceToDevice, s));
-  RTG_HIP(hipMemcpyAsync(S.bhi[0].ptr, shi, (size_t)n * 16, hipMemcpyDeviceToDevice, s));
-  // inner node ids no tree uses stay marked
-  hipLaunchKernelGGL(k_fill_u32, dim3(div_up(n - 1, TBS)), dim3(TBS), 0, s, parent_int, (size_t)(n - 1), REF_EMPTY);
-  hipLaunchKernelGGL(k_fill_u32, dim3(div_up(trees.size(), TBS)), dim3(TBS), 0, s, S.roots.as<uint32_t>(),
-                     trees.size(), NIL);
-
   // trees start as big, mid or small segments of the level loop (a tree's
   // root is split by bins even when tiny)
   std::vector<Seg> init[3];
@@ -1591,39 +1633,42 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
     init[r.count > MID_MAX ? 0 : (r.count > SMALL_MAX ? 1 : 2)].push_back(sg);
   }
   uint32_t cur[3];
+  Begin bg{n, ntrees, vals, S.idx[0].as<uint32_t>(), parent_int, S.sid[0].as<uint32_t>(), S.bins[0].as<uint32_t>(),
+           S.roots.as<uint32_t>(), cnt, {}, 0, 0, nullptr, {}};
+  S.stage.reserve((size_t)ntrees * sizeof(Seg));
+  Seg* stage = S.stage.as<Seg>();
+  bg.stage = S.stage.as<uint32_t>();
   for (int c = 0; c < 3; c++) {
-    cur[c] = (uint32_t)init[c].size();
-    if (cur[c])
-      RTG_HIP(hipMemcpyAsync(S.segs[c][0].ptr, init[c].data(), init[c].size() * sizeof(Seg), hipMemcpyHostToDevice, s));
+    bg.count[c] = cur[c] = (uint32_t)init[c].size();
+    bg.seg[c] = S.segs[c][0].as<uint32_t>();
+    stage = std::copy(init[c].begin(), init[c].end(), stage);
   }
-  if (cur[0]) {  // the big-segment kernels read every position's big-segment id
-    hipLaunchKernelGGL(k_fill_u32, dim3(div_up(n, TBS)), dim3(TBS), 0, s, S.sid[0].as<uint32_t>(), (size_t)n, NIL);
+  if (cur[0]) {
+    bg.first0 = init[0][0].first;
+    bg.count0 = init[0][0].count;
+  }
+  // (a tree holds two positions or more, a big segment more than BIN_WORDS:
+  // a thread per position covers the roots and the bins)
+  hipLaunchKernelGGL(k_begin, dim3(div_up(n, TBS)), dim3(TBS), 0, s, bg);
+  if (cur[0] > 1) {
     uint32_t longest = 0;
     for (const Seg& sg : init[0]) longest = std::max(longest, sg.count);
     hipLaunchKernelGGL(k_fill_seg_ids, dim3(div_up(longest, TBS), cur[0]), dim3(TBS), 0, s, S.sid[0].as<uint32_t>(),
                        S.segs[0][0].as<Seg>());
-    hipLaunchKernelGGL(k_init_gbins, dim3(div_up((size_t)cur[0] * BIN_WORDS, TBS)), dim3(TBS), 0, s,
-                       S.bins[0].as<uint32_t>(), cur[0]);
   }
-  Counters hc{};
-  for (int c = 0; c < 3; c++) hc.nseg[0][c] = cur[c];
-  hc.ntiny = 0;
-  hc.error = 0;
-  RTG_HIP(hipMemcpyAsync(cnt, &hc, sizeof(hc), hipMemcpyHostToDevice, s));
-  RTG_HIP(hipStreamSynchronize(s));  // the host staging above must outlive its copies
 
   Tree t{child, parent_int, parent_leaf, range, vals, cnt, S.roots.as<uint32_t>()};
   // Level l reads the segment lists of parity l & 1 and fills those of the
   // other parity; its kernels take their segment counts from the device, so
   // the host queues level l + 1 before it knows whether level l left any
-  // work, and reads level l's counters (through a pinned slot) meanwhile.
+  // work, and reads the counts that level l + 1's first kernel posts while
+  // that level runs.
   // big-segment kernels run until a level is known to have left no big
   // segment (children are smaller than their parents, so none comes back)
-  S.rb.ensure(sizeof(Counters));
   bool big_live = cur[0] > 0;
   // Grids: a level's kernels read their counts on the device, so a grid
   // need only cover an upper bound. The host knows the input counts of
-  // level kin_level (read back, or level 0's); a segment has at most two
+  // level kin_level (posted, or level 0's); a segment has at most two
   // children, big ones only from big, mid ones from big or mid.
   uint32_t kin[3] = {cur[0], cur[1], cur[2]};
   uint32_t kin_level = 0;
@@ -1658,79 +1703,73 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
     const Seg* bs = S.segs[0][li].as<Seg>();
     uint32_t gb[3];
     grid_bound(L, gb);
+    // the references' boxes: level 0 reads the caller's
+    const float4* lo_in = L ? S.blo[in].as<float4>() : slo;
+    const float4* hi_in = L ? S.bhi[in].as<float4>() : shi;
+    const LevelStart none{};
+    LevelStart st{cnt, nullptr, 0, (uint32_t)li, (uint32_t)lz};
+    if (L) {
+      st.post = S.post.arm();
+      st.seq = S.post.seq;
+    }
     if (big_live && gb[0]) {
-      hipLaunchKernelGGL(k_big_bins, dim3(nchunks), dim3(TBS), 0, s, S.sid[in].as<uint32_t>(),
-                         S.blo[in].as<float4>(), S.bhi[in].as<float4>(), n, bs, S.bins[in].as<uint32_t>(),
-                         S.below.as<uint32_t>(), cnt);
+      hipLaunchKernelGGL(k_big_bins, dim3(nchunks), dim3(TBS), 0, s, S.sid[in].as<uint32_t>(), lo_in,
+                         hi_in, n, bs, S.bins[in].as<uint32_t>(), S.below.as<uint32_t>(), cnt, st);
+      st = none;
       hipLaunchKernelGGL(lcost.P ? k_big_split<true> : k_big_split<false>, dim3(gb[0]), dim3(TBS), 0, s, bs,
                          &cnt->nseg[li][0], S.bins[in].as<uint32_t>(), S.bins[o].as<uint32_t>(),
                          S.below.as<uint32_t>(), S.before.as<uint32_t>(), S.splits.as<Split>(), nx, t, lcost);
       hipLaunchKernelGGL(k_big_scatter, dim3(nchunks), dim3(TBS), 0, s, S.sid[in].as<uint32_t>(),
-                         S.idx[in].as<uint32_t>(), S.blo[in].as<float4>(), S.bhi[in].as<float4>(), n, bs,
-                         S.splits.as<Split>(), S.before.as<uint32_t>(), S.sid[o].as<uint32_t>(),
-                         S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(), S.bhi[o].as<float4>(), vals, cnt);
+                         S.idx[in].as<uint32_t>(), lo_in, hi_in, n, bs, S.splits.as<Split>(),
+                         S.before.as<uint32_t>(), S.sid[o].as<uint32_t>(), S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(), S.bhi[o].as<float4>(), vals, cnt);
     }
-    // (k_seg clears the next level's counts: it runs even with no mid segment)
-    hipLaunchKernelGGL(lcost.P ? k_seg<true> : k_seg<false>, dim3(std::max(gb[1], 1u)), dim3(256), 0, s, S.segs[1][li].as<Seg>(),
-                       &cnt->nseg[li][1], S.idx[in].as<uint32_t>(), S.blo[in].as<float4>(), S.bhi[in].as<float4>(),
-                       S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(), S.bhi[o].as<float4>(), nx, t, lcost,
-                       cnt->nseg[lz]);
-    if (gb[2])
-      hipLaunchKernelGGL(lcost.P ? k_seg_wave<true> : k_seg_wave<false>, dim3(div_up(gb[2], SEGW_WAVES)), dim3(SEGW_TB), 0, s,
-                       S.segs[2][li].as<Seg>(), &cnt->nseg[li][2], S.idx[in].as<uint32_t>(), S.blo[in].as<float4>(),
-                       S.bhi[in].as<float4>(), S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(), S.bhi[o].as<float4>(),
-                       nx, t, lcost);
+    if (gb[1]) {
+      hipLaunchKernelGGL(lcost.P ? k_seg<true> : k_seg<false>, dim3(gb[1]), dim3(256), 0, s, S.segs[1][li].as<Seg>(),
+                         &cnt->nseg[li][1], S.idx[in].as<uint32_t>(), lo_in, hi_in, S.idx[o].as<uint32_t>(),
+                         S.blo[o].as<float4>(), S.bhi[o].as<float4>(), nx, t, lcost, st);
+      st = none;
+    }
+    // (a level without segments still posts that)
+    if (gb[2] || st.post)
+      hipLaunchKernelGGL(lcost.P ? k_seg_wave<true> : k_seg_wave<false>, dim3(std::max(div_up(gb[2], SEGW_WAVES), 1u)),
+                         dim3(SEGW_TB), 0, s, S.segs[2][li].as<Seg>(), &cnt->nseg[li][2], S.idx[in].as<uint32_t>(),
+                         lo_in, hi_in, S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(), S.bhi[o].as<float4>(), nx, t,
+                         lcost, st);
     RTG_HIP(hipGetLastError());
   };
-  auto readback = [&](uint32_t level) {
-    RTG_HIP(hipMemcpyAsync(S.rb.slot((int)level), cnt, sizeof(Counters), hipMemcpyDeviceToHost, s));
-    RTG_HIP(hipEventRecord(S.rb.ev[level % LevelReadback::K], s));
+  uint32_t ntiny = 0;
+  auto fail = [&](const std::string& what) {
+    (void)hipStreamSynchronize(s);
+    throw hip_error(hipErrorUnknown, what);
   };
-  uint32_t levels = 0;
-  if (cur[0] + cur[1] + cur[2] > 0) {
-    enqueue_level(0);
-    readback(0);
-    for (levels = 1;; levels++) {
-      if (levels > 4096) {
-        (void)hipStreamSynchronize(s);
-        throw hip_error(hipErrorUnknown, "SAH build did not terminate");
-      }
-      enqueue_level(levels);  // speculative: without input it does nothing
-      readback(levels);
-      RTG_HIP(hipEventSynchronize(S.rb.ev[(levels - 1) % LevelReadback::K]));
-      memcpy(&hc, S.rb.slot((int)(levels - 1)), sizeof(hc));
-      if (hc.error) {
-        (void)hipStreamSynchronize(s);
-        throw hip_error(hipErrorUnknown, "SAH build failed: error bits " + std::to_string(hc.error));
-      }
-      const uint32_t* next = hc.nseg[levels % 3u];  // input of the level just queued
-      for (int c = 0; c < 3; c++) kin[c] = next[c];
-      kin_level = levels;
-      if (next[0] + next[1] + next[2] == 0) break;
-      if (next[0] == 0) big_live = false;
-    }
+  enqueue_level(0);
+  for (uint32_t level = 1;; level++) {
+    if (level > 4096) fail("SAH build did not terminate");
+    enqueue_level(level);  // speculative: without input it only posts
+    S.post.wait(s);
+    const uint32_t* w = S.post.words();  // the level's segments by class, the tiny segments so far, the error bits
+    if (w[4]) fail("SAH build failed: error bits " + std::to_string(w[4]));
+    for (int c = 0; c < 3; c++) kin[c] = w[c];
+    kin_level = level;
+    ntiny = w[3];  // (final once a level has no segments)
+    if (kin[0] + kin[1] + kin[2] == 0) break;
+    if (kin[0] == 0) big_live = false;
   }
   // the tiny segments of all levels
-  if (hc.ntiny > tiny_cap) throw hip_error(hipErrorUnknown, "SAH build: tiny segment list overflowed");
-  if (hc.ntiny) {
+  if (ntiny > tiny_cap) fail("SAH build: tiny segment list overflowed");
+  if (ntiny) {
     Bufs B;
     for (int p = 0; p < 2; p++) {
       B.idx[p] = S.idx[p].as<uint32_t>();
       B.blo[p] = S.blo[p].as<float4>();
       B.bhi[p] = S.bhi[p].as<float4>();
     }
-    hipLaunchKernelGGL(k_tiny, dim3(div_up(hc.ntiny, TINY_PER_BLOCK)), dim3(TINY_TB), 0, s, S.tiny.as<TinyItem>(),
-                       hc.ntiny, B, t);
+    hipLaunchKernelGGL(k_tiny, dim3(div_up(ntiny, TINY_PER_BLOCK)), dim3(TINY_TB), 0, s, S.tiny.as<TinyItem>(),
+                       ntiny, B, t);
     RTG_HIP(hipGetLastError());
   }
-  out.roots.assign(trees.size(), NIL);
-  RTG_HIP(hipMemcpyAsync(out.roots.data(), S.roots.ptr, trees.size() * 4, hipMemcpyDeviceToHost, s));
-  RTG_HIP(hipMemcpyAsync(&hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, s));
-  RTG_HIP(hipStreamSynchronize(s));
-  if (hc.error) throw hip_error(hipErrorUnknown, "SAH build failed: error bits " + std::to_string(hc.error));
-  for (uint32_t r : out.roots)
-    if (r == NIL || r + 1 >= n) throw hip_error(hipErrorUnknown, "SAH build produced no root");
-  out.levels = levels;
+  out.roots = S.roots.as<uint32_t>();
+  out.error = &cnt->error;
 }
 
 }  // namespace rtg
