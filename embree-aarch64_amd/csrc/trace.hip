@@ -264,6 +264,17 @@ __device__ inline uint32_t spread3(uint32_t x) {
 
 __device__ inline float byte_f(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xffu); }
 
+// A lane without a ray (REF_EMPTY: one that has to pop its next reference).
+// That state lives in the reference itself, and branches set it instead of
+// leaving the step: a bool that several branches set, or a `continue`, costs a
+// lane mask in scalar registers and scalar instructions at every merge. (The
+// two-level kernel spilled 43 to 55 scalar registers to vector lanes: 3.52 ms
+// for two million rays through 10,000 instances and their shadow rays, 2.82
+// without any; the one-level kernels gained 1.5 to 4.5 %.) REF_DONE: the ray
+// has ended and its hit is still to be written, with those of the wave's other
+// ended rays at the next refill.
+constexpr uint32_t REF_IDLE = 0xffffffffu, REF_DONE = 0xfffffffdu;
+
 struct NodeHit {
   uint32_t mask;
   uint32_t imask;
@@ -428,10 +439,12 @@ __device__ inline bool push_near_to_far(const NodeHit& h, Stack& stack, int& smi
   return true;
 }
 
+// A ray's best hit: none while geom is the invalid ID. u = un / dn and
+// v = vn / dn are divided when the hit is written: nearly every step of a wave
+// improves some lane's hit, and would run the two divisions for it.
 struct Hit {
-  float t, u, v, ngx, ngy, ngz;
+  float t, un, vn, dn, ngx, ngy, ngz;
   uint32_t prim, geom;
-  bool found;
 };
 
 __device__ inline float prod_diff(float a, float b, float c, float d) { return __builtin_fmaf(a, b, -(c * d)); }
@@ -558,10 +571,9 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
   TRay r;
   setup_ray(r, a, b, tfar);
   Hit best;
-  best.found = false;
   best.t = INFINITY;
   best.prim = best.geom = 0xffffffffu;
-  best.u = best.v = best.ngx = best.ngy = best.ngz = 0.0f;
+  best.un = best.vn = best.dn = best.ngx = best.ngy = best.ngz = 0.0f;
   float lim = widen_up(tfar);
 
   __shared__ uint64_t lds_stack[LDS_SLOTS > 0 ? LDS_SLOTS * TB : 1];
@@ -611,13 +623,11 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
             occluded = true;
             break;
           }
-          const bool better = !best.found || h.t < best.t ||
+          const bool better = h.t < best.t ||
                               (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim)));
           if (better) {
-            best.found = true;
             best.t = h.t;
-            best.u = h.un / h.dn;
-            best.v = h.vn / h.dn;
+            best.un = h.un; best.vn = h.vn; best.dn = h.dn;
             best.ngx = h.ngx; best.ngy = h.ngy; best.ngz = h.ngz;
             best.prim = h.prim; best.geom = h.geom;
           }
@@ -626,7 +636,7 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
         ti++;
       }
       if (OCCLUDED && occluded) break;
-      if (!OCCLUDED && best.found) lim = widen_up(fminf(best.t, tfar));
+      if (!OCCLUDED && best.geom != 0xffffffffu) lim = widen_up(fminf(best.t, tfar));
     }
     // pop the next entry that can still hold a closer hit
     bool got = false;
@@ -651,24 +661,42 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
   if (COUNT) { cnt_nodes[i] = nvis; cnt_tris[i] = ntri; }
   if (OCCLUDED) {
     if (occluded) *reinterpret_cast<float*>(rp + 32) = -INFINITY;
-  } else if (best.found) {
+  } else if (best.geom != 0xffffffffu) {
     float* f = reinterpret_cast<float*>(rp);
     uint32_t* u = reinterpret_cast<uint32_t*>(rp);
     f[8] = best.t;
     f[12] = best.ngx;
     f[13] = best.ngy;
     f[14] = best.ngz;
-    f[15] = best.u;
-    f[16] = best.v;
+    f[15] = best.un / best.dn;
+    f[16] = best.vn / best.dn;
     u[17] = best.prim;
     u[18] = best.geom;
     u[19] = inst_id;
   }
 }
 
+__device__ inline void write_hit(const Hit& best, char* rp, uint32_t inst_id) {
+  float* f = reinterpret_cast<float*>(rp);
+  uint32_t* u = reinterpret_cast<uint32_t*>(rp);
+  f[8] = best.t;
+  f[12] = best.ngx;
+  f[13] = best.ngy;
+  f[14] = best.ngz;
+  f[15] = best.un / best.dn;
+  f[16] = best.vn / best.dn;
+  u[17] = best.prim;
+  u[18] = best.geom;
+  u[19] = inst_id;
+}
+
 // Persistent variant: a fixed grid of waves pulls rays from a global counter.
 // A lane whose ray is finished takes a new one as soon as at least
-// `refill_min` lanes of its wave are idle, so incoherent rays of very
+// `refill_min` lanes of its wave are idle (and the hits of the ended rays are
+// written then, all at once: the stores, the two divisions and the branch run
+// for ten lanes or more instead of for one or two in nearly every step; 1920 x
+// 1080 camera rays on a 2.1 M triangle terrain take 379 us, 407 before, the
+// Pluecker test on a soup 995 us, 1092 before), so incoherent rays of very
 // different lengths keep the SIMD lanes busy (Aila and Laine, "Understanding
 // the efficiency of ray traversal on GPUs", HPG 2009). Each loop iteration is
 // one traversal step (one node, or one leaf plus the pop that follows) for
@@ -713,10 +741,10 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
   TRay r;
   Hit best;
   float lim = 0.0f;
-  uint32_t cur = 0, ray = 0, nvis = 0, ntri = 0;
+  uint32_t cur = REF_IDLE, ray = 0, nvis = 0, ntri = 0;
   char* lrp = nullptr;      // BATCH: this lane's record
   uint32_t lroot = 0;       // BATCH: its scene's root
-  bool active = false, occluded = false, pool_empty = false;
+  bool pool_empty = false;
   WavePool pool;
   pool.init(rr, M);
   // a ray touches each node and triangle record at most once
@@ -726,122 +754,109 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
 
   while (true) {
     // ---- refill idle lanes (wave-uniform decision)
-    if (!pool_empty) {
-      const uint64_t idle = __ballot(!active);
-      const int nidle = __popcll(idle);
-      if (nidle >= refill_min) {
-        const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
-        pool_empty = pool.empty();
-        if (!active) {
-          if (slot != 0xffffffffu) {
-            char* src;
-            if (BATCH) {
-              const BatchItem& it = stream_of(items, nitems, slot);
-              ray = slot - it.first;
-              lrp = it.rays + (uint64_t)ray * it.stride;
-              lroot = it.root;
-              src = lrp;
-            } else {
-              ray = perm ? perm[slot] : slot;
-              src = rays + (uint64_t)ray * stride;
-            }
-            float4 a, b;
-            float tfar;
-            load_ray<ALIGNED>(src, a, b, tfar);
-            if (a.w <= tfar) {
-              setup_ray(r, a, b, tfar);
-              best.found = false;
-              best.t = INFINITY;
-              best.prim = best.geom = 0xffffffffu;
-              best.u = best.v = best.ngx = best.ngy = best.ngz = 0.0f;
-              lim = widen_up(tfar);
-              cur = BATCH ? lroot : sc.root;
-              stack.init(lds_stack, spill_mem);
-              smin = DIST_NONE;
-              occluded = false;
-              nvis = ntri = 0;
-              iter = 0;
-              active = true;
-            } else if (COUNT) {
-              cnt_nodes[ray] = 0;
-              cnt_tris[ray] = 0;
-            }
-          }
+    const uint64_t idle = __ballot(cur >= REF_DONE);
+    const int nidle = __popcll(idle);
+    if (nidle >= (pool_empty ? 64 : refill_min)) {
+      if (cur == REF_DONE) {
+        cur = REF_IDLE;
+        if (COUNT) { cnt_nodes[ray] = nvis; cnt_tris[ray] = ntri; }
+        if (!OCCLUDED && best.geom != 0xffffffffu) write_hit(best, BATCH ? lrp : rays + (uint64_t)ray * stride, inst_id);
+      }
+      if (pool_empty) break;
+      const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
+      pool_empty = pool.empty();
+      if (cur == REF_IDLE && slot != 0xffffffffu) {
+        char* src;
+        if (BATCH) {
+          const BatchItem& it = stream_of(items, nitems, slot);
+          ray = slot - it.first;
+          lrp = it.rays + (uint64_t)ray * it.stride;
+          lroot = it.root;
+          src = lrp;
+        } else {
+          ray = perm ? perm[slot] : slot;
+          src = rays + (uint64_t)ray * stride;
+        }
+        float4 a, b;
+        float tfar;
+        load_ray<ALIGNED>(src, a, b, tfar);
+        if (a.w <= tfar) {
+          setup_ray(r, a, b, tfar);
+          best.t = INFINITY;
+          best.prim = best.geom = 0xffffffffu;
+          best.un = best.vn = best.dn = best.ngx = best.ngy = best.ngz = 0.0f;
+          lim = widen_up(tfar);
+          cur = BATCH ? lroot : sc.root;
+          stack.init(lds_stack, spill_mem);
+          smin = DIST_NONE;
+          nvis = ntri = 0;
+          iter = 0;
+        } else if (COUNT) {
+          cnt_nodes[ray] = 0;
+          cnt_tris[ray] = 0;
         }
       }
     }
-    if (__ballot(active) == 0) {
-      if (pool_empty) break;
-      continue;
-    }
-    if (!active) continue;
 
-    // ---- one traversal step
-    bool done = false;
-    if (++iter > max_iter) {
+    // ---- one traversal step; a lane whose ray ends in it becomes REF_DONE
+    if (++iter > max_iter && cur < REF_DONE) {
       raise_error(err, 2u);
-      done = true;
-    } else if (!(cur & REF_LEAF)) {
+      cur = REF_DONE;
+    }
+    if (!(cur & REF_LEAF)) {
       if (cur >= sc.num_nodes) {
         raise_error(err, 4u);
-        done = true;
+        cur = REF_DONE;
       } else {
-        NodeHit h;
-        intersect_node<OCCLUDED>(sc.nodes, cur, r, lim, h);
         if (COUNT) {
           nvis++;
           if (node_visits) atomicAdd(&node_visits[cur], 1u);
         }
-        if (OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)) {
-          continue;  // next step descends into cur
-        }
+        NodeHit h;
+        intersect_node<OCCLUDED>(sc.nodes, cur, r, lim, h);
+        if (!(OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)))
+          cur = REF_EMPTY;
       }
-    } else {
+    } else if (cur < REF_DONE) {
       // one triangle per step: a lane in a long leaf does not hold the
       // wave's other lanes in a triangle loop
       const uint32_t ti = cur & ~REF_LEAF;
       if (ti >= sc.num_tris) {
         raise_error(err, 4u);
-        done = true;
+        cur = REF_DONE;
       } else {
         TriTest h;
         const bool valid = tri_test<PL>(r, sc.tris + ti, h);
         if (COUNT) ntri++;
+        cur = (h.flags & TRI_LAST) ? REF_EMPTY : cur + 1u;  // the leaf's next record
         if (valid) {
           if (OCCLUDED) {
-            occluded = true;
+            *reinterpret_cast<float*>((BATCH ? lrp : rays + (uint64_t)ray * stride) + 32) = -INFINITY;
+            cur = REF_DONE;
           } else {
-            const bool better = !best.found || h.t < best.t ||
+            // (a hit's geometry ID is below the initial one)
+            const bool better = h.t < best.t ||
                                 (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim)));
             if (better) {
-              best.found = true;
               best.t = h.t;
-              best.u = h.un / h.dn;
-              best.v = h.vn / h.dn;
+              best.un = h.un; best.vn = h.vn; best.dn = h.dn;
               best.ngx = h.ngx; best.ngy = h.ngy; best.ngz = h.ngz;
               best.prim = h.prim; best.geom = h.geom;
               lim = widen_up(fminf(best.t, r.tfar));
             }
           }
         }
-        if (OCCLUDED && occluded) {
-          done = true;
-        } else if (!(h.flags & TRI_LAST)) {
-          cur = (ti + 1) | REF_LEAF;  // the leaf's next record
-          continue;
-        }
       }
     }
-    if (!done) {
+    if (cur == REF_EMPTY) {
       // pop the next entry that can still hold a closer hit
-      bool got = false;
+      cur = REF_DONE;
       const int dlim = dist_limit(lim);
       while (!stack.empty()) {
         const uint2 e = stack.pop();
         if (!OCCLUDED) smin = below_dist(e.y);
         if (OCCLUDED || (int)e.y <= dlim) {
           cur = e.x;
-          got = true;
           break;
         }
         if (smin > dlim) {
@@ -851,27 +866,6 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
           break;
         }
       }
-      done = !got;
-    }
-    if (done) {
-      char* rp = BATCH ? lrp : rays + (uint64_t)ray * stride;
-      if (COUNT) { cnt_nodes[ray] = nvis; cnt_tris[ray] = ntri; }
-      if (OCCLUDED) {
-        if (occluded) *reinterpret_cast<float*>(rp + 32) = -INFINITY;
-      } else if (best.found) {
-        float* f = reinterpret_cast<float*>(rp);
-        uint32_t* u = reinterpret_cast<uint32_t*>(rp);
-        f[8] = best.t;
-        f[12] = best.ngx;
-        f[13] = best.ngy;
-        f[14] = best.ngz;
-        f[15] = best.u;
-        f[16] = best.v;
-        u[17] = best.prim;
-        u[18] = best.geom;
-        u[19] = inst_id;
-      }
-      active = false;
     }
   }
 }
@@ -893,7 +887,7 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
                                                                     const uint32_t* __restrict__ perm,
                                                                     uint32_t* __restrict__ next, int refill_min,
                                                                     RayRuns rr, uint32_t* node_visits) {
-  constexpr uint32_t NONE_REF = 0xffffffffu;
+  constexpr uint32_t NONE_REF = 0xffffffffu;  // no leaf in progress (as every lane without a ray)
   const int lane = threadIdx.x & 63;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   __shared__ uint64_t lds_stack[8 * TB];
@@ -905,8 +899,8 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
   TRay r;
   Hit best;
   float lim = 0.0f;
-  uint32_t cur = NONE_REF, tri = NONE_REF, ray = 0, nvis = 0, ntri = 0;
-  bool active = false, occluded = false, pool_empty = false;
+  uint32_t cur = REF_IDLE, tri = NONE_REF, ray = 0, nvis = 0, ntri = 0;
+  bool pool_empty = false;
   WavePool pool;
   pool.init(rr, M);
   // (node and triangle counts are below 2^31 each, so the bound fits 32 bits)
@@ -915,31 +909,27 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
 
   while (true) {
     if (!pool_empty) {
-      const uint64_t idle = __ballot(!active);
+      const uint64_t idle = __ballot(cur == REF_IDLE);
       const int nidle = __popcll(idle);
       if (nidle >= refill_min) {
         const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
         pool_empty = pool.empty();
-        if (!active && slot != 0xffffffffu) {
+        if (cur == REF_IDLE && slot != 0xffffffffu) {
           ray = perm ? perm[slot] : slot;
           float4 a, b;
           float tfar;
           load_ray<ALIGNED>(rays + (uint64_t)ray * stride, a, b, tfar);
           if (a.w <= tfar) {
             setup_ray(r, a, b, tfar);
-            best.found = false;
             best.t = INFINITY;
             best.prim = best.geom = 0xffffffffu;
-            best.u = best.v = best.ngx = best.ngy = best.ngz = 0.0f;
+            best.un = best.vn = best.dn = best.ngx = best.ngy = best.ngz = 0.0f;
             lim = widen_up(tfar);
             cur = sc.root;
-            tri = NONE_REF;
             stack.init(lds_stack, spill_mem);
             smin = DIST_NONE;
-            occluded = false;
             nvis = ntri = 0;
             iter = 0;
-            active = true;
           } else if (COUNT) {
             cnt_nodes[ray] = 0;
             cnt_tris[ray] = 0;
@@ -947,71 +937,67 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
         }
       }
     }
-    if (__ballot(active) == 0) {
+    if (__ballot(cur != REF_IDLE) == 0) {
       if (pool_empty) break;
       continue;
     }
-    if (!active) continue;
 
-    bool done = false;
-    if (++iter > max_iter) {
+    if (++iter > max_iter && cur != REF_IDLE) {
       raise_error(err, 2u);
-      done = true;
+      cur = REF_DONE;
     }
     // a waiting leaf starts once the triangle cursor is free
-    if (!done && tri == NONE_REF && cur != NONE_REF && (cur & REF_LEAF)) {
+    if (tri == NONE_REF && (cur & REF_LEAF) && cur < REF_DONE) {
       tri = cur & ~REF_LEAF;
-      cur = NONE_REF;
+      cur = REF_EMPTY;
     }
     // node step
-    if (!done && cur != NONE_REF && !(cur & REF_LEAF)) {
+    if (!(cur & REF_LEAF)) {
       if (cur >= sc.num_nodes) {
         raise_error(err, 4u);
-        done = true;
+        cur = REF_DONE;
       } else {
-        NodeHit h;
-        intersect_node<OCCLUDED>(sc.nodes, cur, r, lim, h);
         if (COUNT) {
           nvis++;
           if (node_visits) atomicAdd(&node_visits[cur], 1u);
         }
-        if (!(OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur))) {
-          cur = NONE_REF;
-        }
+        NodeHit h;
+        intersect_node<OCCLUDED>(sc.nodes, cur, r, lim, h);
+        if (!(OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)))
+          cur = REF_EMPTY;
       }
     }
     // triangle step
-    if (!done && tri != NONE_REF) {
+    if (tri != NONE_REF) {
       if (tri >= sc.num_tris) {
         raise_error(err, 4u);
-        done = true;
+        cur = REF_DONE;
       } else {
         TriTest h;
         const bool valid = tri_test<PL>(r, sc.tris + tri, h);
         if (COUNT) ntri++;
+        tri = (h.flags & TRI_LAST) ? NONE_REF : tri + 1u;
         if (valid) {
           if (OCCLUDED) {
-            occluded = true;
+            *reinterpret_cast<float*>(rays + (uint64_t)ray * stride + 32) = -INFINITY;
+            cur = REF_DONE;
           } else {
-            const bool better = !best.found || h.t < best.t ||
+            // (a hit's geometry ID is below the initial one)
+            const bool better = h.t < best.t ||
                                 (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim)));
             if (better) {
-              best.found = true;
               best.t = h.t;
-              best.u = h.un / h.dn;
-              best.v = h.vn / h.dn;
+              best.un = h.un; best.vn = h.vn; best.dn = h.dn;
               best.ngx = h.ngx; best.ngy = h.ngy; best.ngz = h.ngz;
               best.prim = h.prim; best.geom = h.geom;
               lim = widen_up(fminf(best.t, r.tfar));
             }
           }
         }
-        if (OCCLUDED && occluded) done = true;
-        else tri = (h.flags & TRI_LAST) ? NONE_REF : tri + 1u;
       }
     }
     // the node cursor takes the next entry that can still hold a closer hit
-    if (!done && cur == NONE_REF) {
+    if (cur == REF_EMPTY) {
       const int dlim = dist_limit(lim);
       while (!stack.empty()) {
         const uint2 e = stack.pop();
@@ -1027,27 +1013,13 @@ __global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, c
           break;
         }
       }
-      if (cur == NONE_REF && tri == NONE_REF) done = true;
+      if (cur == REF_EMPTY && tri == NONE_REF) cur = REF_DONE;
     }
-    if (done) {
-      char* rp = rays + (uint64_t)ray * stride;
+    if (cur == REF_DONE) {
+      cur = REF_IDLE;
+      tri = NONE_REF;
       if (COUNT) { cnt_nodes[ray] = nvis; cnt_tris[ray] = ntri; }
-      if (OCCLUDED) {
-        if (occluded) *reinterpret_cast<float*>(rp + 32) = -INFINITY;
-      } else if (best.found) {
-        float* f = reinterpret_cast<float*>(rp);
-        uint32_t* u = reinterpret_cast<uint32_t*>(rp);
-        f[8] = best.t;
-        f[12] = best.ngx;
-        f[13] = best.ngy;
-        f[14] = best.ngz;
-        f[15] = best.u;
-        f[16] = best.v;
-        u[17] = best.prim;
-        u[18] = best.geom;
-        u[19] = inst_id;
-      }
-      active = false;
+      if (!OCCLUDED && best.geom != 0xffffffffu) write_hit(best, rays + (uint64_t)ray * stride, inst_id);
     }
   }
 }
@@ -1102,10 +1074,9 @@ __global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ 
   TRay r;
   setup_ray(r, a, b, tfar);
   Hit best;  // the best of the triangles that this lane tested
-  best.found = false;
   best.t = INFINITY;
   best.prim = best.geom = 0xffffffffu;
-  best.u = best.v = best.ngx = best.ngy = best.ngz = 0.0f;
+  best.un = best.vn = best.dn = best.ngx = best.ngy = best.ngz = 0.0f;
   float lim = widen_up(tfar);
   bool occluded = false;
   lds_u64* stack = (lds_u64*)group_stack + g;
@@ -1190,12 +1161,10 @@ __global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ 
           break;
         }
       } else {
-        if (valid && (!best.found || h.t < best.t ||
+        if (valid && (h.t < best.t ||
                       (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim))))) {
-          best.found = true;
           best.t = h.t;
-          best.u = h.un / h.dn;
-          best.v = h.vn / h.dn;
+          best.un = h.un; best.vn = h.vn; best.dn = h.dn;
           best.ngx = h.ngx; best.ngy = h.ngy; best.ngz = h.ngz;
           best.prim = h.prim; best.geom = h.geom;
         }
@@ -1240,15 +1209,15 @@ __global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ 
   least(__uint_as_float(gx1(__float_as_uint(t))), gx1(geom), gx1(prim));
   least(__uint_as_float(gx2(__float_as_uint(t))), gx2(geom), gx2(prim));
   least(__uint_as_float(gx7(__float_as_uint(t))), gx7(geom), gx7(prim));
-  if (best.found && best.t == t && best.geom == geom && best.prim == prim) {
+  if (best.geom != 0xffffffffu && best.t == t && best.geom == geom && best.prim == prim) {
     float* f = reinterpret_cast<float*>(rp);
     uint32_t* u = reinterpret_cast<uint32_t*>(rp);
     f[8] = best.t;
     f[12] = best.ngx;
     f[13] = best.ngy;
     f[14] = best.ngz;
-    f[15] = best.u;
-    f[16] = best.v;
+    f[15] = best.un / best.dn;
+    f[16] = best.vn / best.dn;
     u[17] = best.prim;
     u[18] = best.geom;
     u[19] = inst_id;
@@ -1287,78 +1256,79 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
   stack.init(lds_stack, spill_mem);
   int smin = DIST_NONE;  // least entry distance on the stack (closest hit)
 
+  // a ray that ends: closest hit, its hit is still to be finished
+  constexpr uint32_t END = OCCLUDED ? REF_IDLE : REF_DONE;
   TRay r;
   Hit best;
   uint32_t best_inst = 0;
   float lim = 0.0f;
-  uint32_t cur = 0, ray = 0, inst = 0;
-  bool in_obj = false;  // in an object tree (else the top tree)
-  bool moved = false;   // r is in an instance's object space
+  uint32_t cur = REF_IDLE, ray = 0, inst = 0;
+  // in an object tree (else the top tree); r in an instance's object space;
+  // an object of a robust scene (bits of a register: a bool costs a lane mask)
+  constexpr uint32_t IN_OBJ = 1u, MOVED = 2u, ROBUST = 4u;
+  uint32_t where = 0u;
   const QNode8* onodes = nullptr;
   const TriRec* otris = nullptr;
   uint32_t onn = 0, otn = 0;
   uint32_t oidx = 0xffffffffu;  // the object the lane is in (counted variant)
-  bool orobust = false;
-  bool active = false, occluded = false, pool_empty = false;
+  bool pool_empty = false;
   WavePool pool;
   pool.init(rr, M);
-  uint64_t iter = 0;
+  const uint32_t max_iter = (uint32_t)min(top.max_iter, (uint64_t)0xffffffffu);
+  uint32_t iter = 0;
 
   while (true) {
     // ---- refill idle lanes (wave-uniform decision)
-    if (!pool_empty) {
-      const uint64_t idle = __ballot(!active);
-      const int nidle = __popcll(idle);
-      if (nidle >= refill_min) {
-        const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
-        pool_empty = pool.empty();
-        if (!active) {
-          if (slot != 0xffffffffu) {
-            ray = slot;
-            float4 a, b;
-            float tfar;
-            load_ray<ALIGNED>(rays + (uint64_t)ray * stride, a, b, tfar);
-            if (a.w <= tfar) {
-              setup_ray(r, a, b, tfar);
-              best.found = false;
-              best.t = INFINITY;
-              best.prim = best.geom = 0xffffffffu;
-              best.u = best.v = best.ngx = best.ngy = best.ngz = 0.0f;
-              best_inst = 0xffffffffu;
-              lim = widen_up(tfar);
-              cur = top.root;
-              in_obj = false;
-              moved = false;
-              stack.init(lds_stack, spill_mem);
-              smin = DIST_NONE;
-              occluded = false;
-              iter = 0;
-              active = true;
-            }
-          }
+    const uint64_t idle = __ballot(cur >= REF_DONE);
+    const int nidle = __popcll(idle);
+    if (nidle >= (pool_empty ? 64 : refill_min)) {
+      if (!OCCLUDED && cur == REF_DONE) {
+        cur = REF_IDLE;
+        if (best.geom != 0xffffffffu) {
+          float* f = reinterpret_cast<float*>(rays + (uint64_t)ray * stride);
+          const float dn = f[8], un = f[15], vn = f[16];
+          f[8] = best.t;
+          f[15] = un / dn;
+          f[16] = vn / dn;
+        }
+      }
+      if (pool_empty) break;
+      const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
+      pool_empty = pool.empty();
+      if (cur == REF_IDLE && slot != 0xffffffffu) {
+        ray = slot;
+        float4 a, b;
+        float tfar;
+        load_ray<ALIGNED>(rays + (uint64_t)ray * stride, a, b, tfar);
+        if (a.w <= tfar) {
+          setup_ray(r, a, b, tfar);
+          best.t = INFINITY;
+          best.prim = best.geom = 0xffffffffu;
+          best.un = best.vn = best.dn = best.ngx = best.ngy = best.ngz = 0.0f;
+          best_inst = 0xffffffffu;
+          lim = widen_up(tfar);
+          cur = top.root;
+          where = 0u;
+          stack.init(lds_stack, spill_mem);
+          smin = DIST_NONE;
+          iter = 0;
         }
       }
     }
-    if (__ballot(active) == 0) {
-      if (pool_empty) break;
-      continue;
-    }
-    if (!active) continue;
 
     // ---- one traversal step
-    bool done = false;
-    if (++iter > top.max_iter) {
+    if (++iter > max_iter && cur < REF_DONE) {
       raise_error(err, 2u);
-      done = true;
-    } else if (!(cur & REF_LEAF)) {
-      const QNode8* nodes = in_obj ? onodes : top.nodes;
-      const uint32_t nn = in_obj ? onn : top.num_nodes;
-      if (cur >= nn) {
+      cur = END;
+    }
+    if (!(cur & REF_LEAF)) {
+      const QNode8* nodes = where ? onodes : top.nodes;
+      if (cur >= (where ? onn : top.num_nodes)) {
         raise_error(err, 4u);
-        done = true;
+        cur = END;
       } else {
         if (CNT) {
-          if (!in_obj) {
+          if (!where) {
             if (top_visits) atomicAdd(top_visits + cur, 1u);
           } else if (obj_visits && oidx == target_obj) {
             atomicAdd(obj_visits + cur, 1u);
@@ -1366,45 +1336,46 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
         }
         NodeHit h;
         intersect_node<OCCLUDED>(nodes, cur, r, lim, h);
-        if (OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)) {
-          continue;
-        }
+        if (!(OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)))
+          cur = REF_EMPTY;
       }
-    } else if (in_obj) {
-      // one triangle of the current object
-      const uint32_t ti = cur & ~REF_LEAF;
-      if (ti >= otn) {
+    } else if (cur < REF_DONE) {
+      const uint32_t at = cur & ~REF_LEAF;
+      if (at >= (where ? otn : top.num_insts)) {
         raise_error(err, 4u);
-        done = true;
-      } else {
+        cur = END;
+      } else if (where) {
+        // one triangle of the current object
         TriTest h;
-        const bool valid = orobust ? tri_test<true>(r, otris + ti, h) : tri_test<false>(r, otris + ti, h);
+        const bool valid = (where & ROBUST) ? tri_test<true>(r, otris + at, h) : tri_test<false>(r, otris + at, h);
+        cur = (h.flags & TRI_LAST) ? REF_EMPTY : cur + 1u;
         if (valid) {
           if (OCCLUDED) {
-            occluded = true;
+            *reinterpret_cast<float*>(rays + (uint64_t)ray * stride + 32) = -INFINITY;
+            cur = REF_IDLE;
           } else {
             const bool better =
-                !best.found || h.t < best.t ||
+                h.t < best.t ||
                 (h.t == best.t &&
                  (inst < best_inst ||
                   (inst == best_inst &&
                    (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim)))));
             if (better) {
               // the hit goes to the record at once, so that only the fields
-              // the comparison needs stay in registers
-              best.found = true;
+              // the comparison needs stay in registers; u and v wait there as
+              // their numerators, with the denominator where the distance goes
               best.t = h.t;
               best.prim = h.prim;
               best.geom = h.geom;
               best_inst = inst;
               float* f = reinterpret_cast<float*>(rays + (uint64_t)ray * stride);
               uint32_t* u = reinterpret_cast<uint32_t*>(f);
-              f[8] = h.t;
+              f[8] = h.dn;
               f[12] = h.ngx;
               f[13] = h.ngy;
               f[14] = h.ngz;
-              f[15] = h.un / h.dn;
-              f[16] = h.vn / h.dn;
+              f[15] = h.un;
+              f[16] = h.vn;
               u[17] = h.prim;
               u[18] = h.geom;
               u[19] = inst;
@@ -1412,27 +1383,16 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
             }
           }
         }
-        if (OCCLUDED && occluded) {
-          done = true;
-        } else if (!(h.flags & TRI_LAST)) {
-          cur = (ti + 1) | REF_LEAF;
-          continue;
-        }
-      }
-    } else {
-      // an instance record of the top tree
-      const uint32_t ii = cur & ~REF_LEAF;
-      if (ii >= top.num_insts) {
-        raise_error(err, 4u);
-        done = true;
       } else {
-        const float4* q = reinterpret_cast<const float4*>(top.insts + ii);
+        // an instance record of the top tree
+        const float4* q = reinterpret_cast<const float4*>(top.insts + at);
         const float4 m0 = q[0], m1 = q[1], m2 = q[2];
-        const uint4 w = reinterpret_cast<const uint4*>(top.insts + ii)[3];
+        const uint4 w = reinterpret_cast<const uint4*>(top.insts + at)[3];
         const bool identity = (w.z & INST_IDENTITY) != 0u;
         // the rest of a multi-record leaf resumes after this instance
-        if (!(w.z & TRI_LAST) && !stack.push(make_uint2((ii + 1u) | REF_LEAF, pack_dist(DIST_ALWAYS, smin))))
+        if (!(w.z & TRI_LAST) && !stack.push(make_uint2((at + 1u) | REF_LEAF, pack_dist(DIST_ALWAYS, smin))))
           raise_error(err, 1u);
+        cur = REF_EMPTY;
         if ((identity || ctx_inst == 0xffffffffu) && w.y < top.num_objects) {
           const DevScene o = top.objects[w.y];
           if (o.num_nodes > 0) {
@@ -1449,32 +1409,31 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
               const float dy = __builtin_fmaf(r.dx, m0.y, __builtin_fmaf(r.dy, m1.x, r.dz * m1.w));
               const float dz = __builtin_fmaf(r.dx, m0.z, __builtin_fmaf(r.dy, m1.y, r.dz * m2.x));
               setup_ray(r, make_float4(ox, oy, oz, r.tnear), make_float4(dx, dy, dz, 0.0f), r.tfar);
-              moved = true;
+              where = MOVED;
             }
-            in_obj = true;
+            where |= IN_OBJ | (o.robust ? ROBUST : 0u);
             inst = identity ? ctx_inst : w.x;
             if (CNT) oidx = w.y;
             onodes = o.nodes;
             otris = o.tris;
             onn = o.num_nodes;
             otn = o.num_tris;
-            orobust = o.robust != 0u;
             cur = o.root;
-            continue;
           }
         }
       }
     }
-    if (!done) {
+    if (cur == REF_EMPTY) {
       // pop the next entry that can still hold a closer hit; an exit entry
       // returns the ray to world space
-      bool got = false;
+      cur = END;
       const int dlim = dist_limit(lim);
       while (!stack.empty()) {
         const uint2 e = stack.pop();
         if (!OCCLUDED) smin = below_dist(e.y);
         if (e.x == REF_INST_EXIT) {
-          in_obj = false;
+          const bool moved = (where & MOVED) != 0u;
+          where = 0u;
           if (moved) {
             const float4 a = lds_world[threadIdx.x], b = lds_world[TB + threadIdx.x];
             const float4 c = lds_world[2 * TB + threadIdx.x];
@@ -1484,13 +1443,11 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
             r.negx = !(r.rnx >= 0.0f);
             r.negy = !(r.rny >= 0.0f);
             r.negz = !(r.rnz >= 0.0f);
-            moved = false;
           }
           continue;
         }
         if (OCCLUDED || (int)e.y <= dlim) {
           cur = e.x;
-          got = true;
           break;
         }
         if (smin > dlim) {
@@ -1500,14 +1457,6 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
           break;
         }
       }
-      done = !got;
-    }
-    if (done) {
-      char* rp = rays + (uint64_t)ray * stride;
-      if (OCCLUDED) {
-        if (occluded) *reinterpret_cast<float*>(rp + 32) = -INFINITY;
-      }
-      active = false;
     }
   }
 }
