@@ -759,42 +759,93 @@ __device__ inline uint32_t quant_hi(float v, float p, float s) {
 // Byte k of a node's eight split bytes loaded as one uint2.
 __device__ inline uint32_t split_byte(uint2 s8, uint32_t k) { return ((k < 4 ? s8.x : s8.y) >> (8 * (k & 3))) & 0xffu; }
 
-// The children of a wide node: the optimal distribution of `width` slots below
-// inner node b, handed to `found` in order. Returns their number, 0 on a table
-// that asks for more than 8.
-template <class Found>
-__device__ inline int wide_children(const CollapseArgs& a, uint32_t b, Found found) {
-  uint32_t st_ref[8], st_s[8];
-  int n = 0, sp = 2;
-  const uint32_t j8 = (a.split8[8 * (size_t)b + a.width - 1]) & 7u;
-  st_ref[0] = a.child[2 * b + 1]; st_s[0] = a.width - j8;
-  st_ref[1] = a.child[2 * b];     st_s[1] = j8;
-  while (sp > 0 && n < 8) {
-    sp--;
-    uint32_t c = st_ref[sp], slots = st_s[sp];
-    uint2 s8 = make_uint2(0u, 0u), cp = make_uint2(0u, 0u);
-    if (!(c & REF_LEAF)) {
-      // the node's eight split bytes and its child pair: two 8 B loads
-      // issued together, not a byte load per slot count and then the pair
-      s8 = *reinterpret_cast<const uint2*>(a.split8 + 8 * (size_t)c);
-      cp = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)c);
-      while (slots > 1 && (split_byte(s8, slots - 1) & 0x80u)) slots--;
-    } else {
-      slots = 1;
-    }
-    if (slots <= 1) {
-      found(n, c);
-      n++;
-    } else {
-      const uint32_t jj = split_byte(s8, slots - 1) & 7u;
-      if (sp + 2 > 8) {
-        atomicOr(&a.cnt->error, 128u);
-        return 0;
-      }
-      st_ref[sp] = cp.y; st_s[sp] = slots - jj; sp++;
-      st_ref[sp] = cp.x; st_s[sp] = jj;         sp++;
-    }
+// A wide node takes a group of CG lanes: they find its children together, lane k
+// keeps child k.
+constexpr uint32_t CG = 8;
+
+template <class T>
+__device__ inline T group_sum(T v) {
+#pragma unroll
+  for (int d = 1; d < (int)CG; d <<= 1) v += __shfl_xor(v, d, CG);
+  return v;
+}
+__device__ inline float group_min(float v) {
+#pragma unroll
+  for (int d = 1; d < (int)CG; d <<= 1) v = fminf(v, __shfl_xor(v, d, CG));
+  return v;
+}
+__device__ inline float group_max(float v) {
+#pragma unroll
+  for (int d = 1; d < (int)CG; d <<= 1) v = fmaxf(v, __shfl_xor(v, d, CG));
+  return v;
+}
+// exclusive prefix over the group's lanes
+__device__ inline uint32_t group_prefix(uint32_t v, uint32_t k) {
+  uint32_t x = v;
+#pragma unroll
+  for (int d = 1; d < (int)CG; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d, CG);
+    if (k >= (uint32_t)d) x += y;
   }
+  return x - v;
+}
+
+// The children of a wide node: the optimal distribution of `width` slots below
+// inner node b. Lane k of the group gets child k in `mine`; returns their
+// number, 0 on a corrupt table. A lane that holds a reference has the slots from
+// its own place up to the next such lane's; in each round every reference with
+// more than one slot is split, the right part going to the lane at the left
+// part's end. So the chain of loads is as long as the deepest child, not as the
+// number of splits (up to 7, each about 0.8 us): with one lane a node that did
+// them in turn, Morton builds of 20,000 triangles took 0.29 ms, now 0.23, of
+// 2^20 0.88, now 0.81.
+__device__ inline int wide_children(const CollapseArgs& a, uint32_t b, uint32_t k, uint32_t& mine) {
+  const uint32_t shift = (threadIdx.x & 63u) & ~(CG - 1u);
+  auto group = [&](bool x) { return (uint32_t)(__ballot(x) >> shift) & 0xffu; };
+  const uint32_t j8 = a.split8[8 * (size_t)b + a.width - 1] & 7u;
+  const uint2 bc = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)b);
+  uint32_t ref = k ? bc.y : bc.x;
+  uint32_t slots = k == 0u ? j8 : (k == j8 ? a.width - j8 : 0u);
+  bool bad = j8 == 0u || j8 >= a.width;
+  bool open = slots > 1u && !(ref & REF_LEAF);
+  while (group(open)) {
+    uint32_t left = 0u, right = 0u, rref = 0u;  // slots of the parts
+    if (open) {
+      // the node's eight split bytes and its child pair: two 8 B loads
+      const uint2 s8 = *reinterpret_cast<const uint2*>(a.split8 + 8 * (size_t)ref);
+      const uint2 cp = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)ref);
+      while (slots > 1u && (split_byte(s8, slots - 1) & 0x80u)) slots--;
+      if (slots > 1u) {
+        left = split_byte(s8, slots - 1) & 7u;
+        bad = bad || left == 0u || left >= slots;
+        right = slots - left;
+        rref = cp.y;
+        ref = cp.x;
+        slots = left;
+      }
+    }
+    // the lane whose slots include this one: the last at or before it
+    const uint32_t held = group(slots > 0u) & ((2u << k) - 1u);
+    const uint32_t from = held ? 31u - (uint32_t)__builtin_clz(held) : 0u;
+    const uint32_t fl = (uint32_t)__shfl((int)left, (int)from, CG), fr = (uint32_t)__shfl((int)right, (int)from, CG);
+    const uint32_t fref = (uint32_t)__shfl((int)rref, (int)from, CG);
+    if (slots == 0u && fr != 0u && from + fl == k) {
+      ref = fref;
+      slots = fr;
+      open = true;
+    }
+    open = open && slots > 1u && !(ref & REF_LEAF);
+    if (group(bad)) break;
+  }
+  if (group(bad)) {
+    if (k == 0) atomicOr(&a.cnt->error, 128u);
+    return 0;
+  }
+  // child k: the k-th lane that holds a reference
+  uint32_t held = group(slots > 0u);
+  const int n = __builtin_popcount(held);
+  for (uint32_t i = 0; i < k && (held & (held - 1u)); i++) held &= held - 1u;
+  mine = (uint32_t)__shfl((int)ref, __builtin_ctz(held), CG);
   return n;
 }
 
@@ -810,57 +861,48 @@ __device__ inline int wide_children(const CollapseArgs& a, uint32_t b, Found fou
 // 40 ns each: 2^20 triangles 1.20 -> 0.95 ms for a Morton build, 3.20 -> 2.96
 // for binned SAH; 131,000 triangles 0.68 -> 0.50 and 1.46 -> 1.33 ms.)
 // The top is every node with more than 1/256 of the primitives, so fewer than
-// 256 on a level (a thread each), and the subtrees take about the same time.
+// 256 on a level (eight lanes each), and the subtrees take about the same time.
 constexpr uint32_t TOP_SHARE = 256, TOP_LEVELS = 256;
-constexpr uint32_t TOP_MIN = 512;   // primitives that are always one subtree (a level of the top takes 12 us, of a subtree 8)
+// Primitives that are always one subtree (Morton builds of 131,000 terrain
+// triangles 0.347 ms, at 512 0.388, at 4096 0.356; of 20,000 0.225, 0.229, 0.228).
+constexpr uint32_t TOP_MIN = 2048;
 constexpr uint32_t SUB_MAX = 2047;  // subtrees beside the scenes (their sums are one scan launch)
 // Top nodes: fewer than TOP_SHARE on each level, the subtrees' roots, the scenes.
 __host__ __device__ inline uint32_t top_cap(uint32_t max_sub) { return max_sub + TOP_SHARE * TOP_LEVELS; }
 
-// Walks one wide node: `take` gives the first of ni numbers for its inner
-// children, `put` gets each of them with its primitive count, and `record` the
-// first number, for the node's own record.
+// Walks one wide node with a group: `take` gives lane 0 the first of ni numbers
+// for its inner children, `put` gets each of those (in its own lane) with its
+// primitive count, and `record` (in lane 0) the first number, for the node's own
+// record.
 template <class Take, class Put, class Record>
-__device__ inline void walk_node(const CollapseArgs& a, const WideNode& w, Take take, Put put, Record record) {
-  uint32_t ref[8], cnt[8];
+__device__ inline void walk_node(const CollapseArgs& a, const WideNode& w, uint32_t k, Take take, Put put,
+                                 Record record) {
+  uint32_t ref = REF_EMPTY;
   int n = 0;
-  if (w.bref != REF_EMPTY && is_inner(w.bref, a.isleaf))
-    n = wide_children(a, w.bref, [&](int i, uint32_t c) {
-#pragma unroll
-      for (int j = 0; j < 8; j++) ref[j] = i == j ? c : ref[j];
-    });
-  uint32_t ni = 0, nt = 0, inner = 0;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    if (j >= n) continue;
-    cnt[j] = 1u;
-    bool in = false;
-    if (!(ref[j] & REF_LEAF)) {
-      const uint2 r = a.range[ref[j]];
-      cnt[j] = r.y - r.x + 1u;
-      in = !a.isleaf[ref[j]];
-    }
-    if (in) {
-      inner |= 1u << j;
-      ni++;
-    } else {
-      nt += cnt[j];
+  if (w.bref != REF_EMPTY && is_inner(w.bref, a.isleaf)) n = wide_children(a, w.bref, k, ref);
+  uint32_t cnt = 0u;
+  bool in = false;
+  if (k < (uint32_t)n) {
+    cnt = 1u;
+    if (!(ref & REF_LEAF)) {
+      const uint2 r = a.range[ref];
+      cnt = r.y - r.x + 1u;
+      in = !a.isleaf[ref];
     }
   }
-  const uint32_t first = ni ? take(ni) : 0u;
+  const uint32_t nt = group_sum(in ? 0u : cnt), ni = group_sum(in ? 1u : 0u);
+  const uint32_t tri = w.tri + nt + group_prefix(in ? cnt : 0u, k), rank = group_prefix(in ? 1u : 0u, k);
+  uint32_t first = 0u;
+  if (k == 0u && ni) first = take(ni);
+  first = (uint32_t)__shfl((int)first, 0, CG);
   const uint32_t level = w.level + (1u << 16) + (n ? (uint32_t)n - 1u : 0u);  // a node pushes at most n-1 of its n children
-  uint32_t k = 0, tri = w.tri + nt;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    if (!((inner >> j) & 1u)) continue;
-    put(cnt[j], WideNode{ref[j], tri, level, first + k});
-    tri += cnt[j];
-    k++;
-  }
-  record(first);
+  if (in) put(cnt, WideNode{ref, tri, level, first + rank});
+  if (k == 0u) record(first);
 }
 
-__global__ __launch_bounds__(BT) void k_walk_top(CollapseArgs a, const uint32_t* __restrict__ roots,
+constexpr int WT = 1024;  // lanes of a workgroup that walks: 128 nodes at a time
+
+__global__ __launch_bounds__(WT) void k_walk_top(CollapseArgs a, const uint32_t* __restrict__ roots,
                                                  const uint32_t* __restrict__ first,
                                                  const uint32_t* __restrict__ prims) {
   __shared__ WideNode level[2][TOP_SHARE];
@@ -886,16 +928,16 @@ __global__ __launch_bounds__(BT) void k_walk_top(CollapseArgs a, const uint32_t*
       else atomicOr(&a.cnt->error, 2u);
     }
   };
-  for (uint32_t i = threadIdx.x; i < a.nscenes; i += BT) place(0, prims[i], WideNode{roots[i], first[i], 1u << 16, i});
+  for (uint32_t i = threadIdx.x; i < a.nscenes; i += WT) place(0, prims[i], WideNode{roots[i], first[i], 1u << 16, i});
   __syncthreads();
   while (true) {
     const uint32_t count = min(nlevel[in], TOP_SHARE);
     // (each walked node may add 8 subtrees)
     if (count == 0u || nsub + 8u * count > a.max_sub) break;
-    if (threadIdx.x < count) {
-      const WideNode w = level[in][threadIdx.x];
+    for (uint32_t i = threadIdx.x / CG; i < count; i += WT / CG) {
+      const WideNode w = level[in][i];
       walk_node(
-          a, w, [&](uint32_t ni) { return atomicAdd(&nodes, ni); },
+          a, w, threadIdx.x % CG, [&](uint32_t ni) { return atomicAdd(&nodes, ni); },
           [&](uint32_t cnt, const WideNode& c) { place(in ^ 1u, cnt, c); },
           [&](uint32_t f) {
             if (w.link < top_cap(a.max_sub)) a.top[w.link] = WideNode{w.bref, w.tri, w.level, f};
@@ -916,12 +958,12 @@ __global__ __launch_bounds__(BT) void k_walk_top(CollapseArgs a, const uint32_t*
   }
 }
 
-// The subtrees, a workgroup each: up to 256 waiting nodes are walked at a time,
+// The subtrees, a workgroup each: up to 128 waiting nodes are walked at a time,
 // last first, from a stack in LDS. Where the stack could fill up, fewer are
 // taken, down to one, which needs 7 entries a level.
 constexpr uint32_t REST_STACK = 3072, REST_SPARE = 7 * 128;
 
-__global__ __launch_bounds__(BT) void k_walk_rest(CollapseArgs a) {
+__global__ __launch_bounds__(WT) void k_walk_rest(CollapseArgs a) {
   __shared__ WideNode stack[REST_STACK];
   __shared__ uint32_t count, nodes, run;
   if (threadIdx.x == 0) run = a.cnt->error ? 0u : 1u;
@@ -943,22 +985,19 @@ __global__ __launch_bounds__(BT) void k_walk_rest(CollapseArgs a) {
       const uint32_t c = count;
       if (c == 0u) break;
       const uint32_t room = REST_STACK - REST_SPARE > c ? (REST_STACK - REST_SPARE - c) / 7u : 0u;
-      const uint32_t m = min(min(c, (uint32_t)BT), max(room, 1u));
+      const uint32_t m = min(min(c, WT / CG), max(room, 1u));
+      const uint32_t g = threadIdx.x / CG;
       WideNode w{};
-      if (threadIdx.x < m) w = stack[c - 1u - threadIdx.x];
+      if (g < m) w = stack[c - 1u - g];
       __syncthreads();
       if (threadIdx.x == 0) count = c - m;
       __syncthreads();
-      if (threadIdx.x < m) {
-        uint32_t at = 0;
+      if (g < m) {
         walk_node(
-            a, w,
-            [&](uint32_t ni) {
-              at = atomicAdd(&count, ni);
-              return atomicAdd(&nodes, ni);
-            },
+            a, w, threadIdx.x % CG, [&](uint32_t ni) { return atomicAdd(&nodes, ni); },
             [&](uint32_t, const WideNode& ch) {
-              if (at < REST_STACK) stack[at++] = ch;
+              const uint32_t at = atomicAdd(&count, 1u);
+              if (at < REST_STACK) stack[at] = ch;
               else atomicOr(&a.cnt->error, 2u);
             },
             [&](uint32_t i) {
@@ -1006,38 +1045,6 @@ __device__ inline void block_stats(CollapseStats& st) {
     for (int i = 1; i < BT / 64; i++) st.add(w[i]);
 }
 
-// Writing a node takes a group of CG lanes: every lane finds the children, lane
-// k then loads, quantises and writes child k, with shuffles for the node's box,
-// reductions and scans over the group.
-constexpr uint32_t CG = 8;
-
-template <class T>
-__device__ inline T group_sum(T v) {
-#pragma unroll
-  for (int d = 1; d < (int)CG; d <<= 1) v += __shfl_xor(v, d, CG);
-  return v;
-}
-__device__ inline float group_min(float v) {
-#pragma unroll
-  for (int d = 1; d < (int)CG; d <<= 1) v = fminf(v, __shfl_xor(v, d, CG));
-  return v;
-}
-__device__ inline float group_max(float v) {
-#pragma unroll
-  for (int d = 1; d < (int)CG; d <<= 1) v = fmaxf(v, __shfl_xor(v, d, CG));
-  return v;
-}
-// exclusive prefix over the group's lanes
-__device__ inline uint32_t group_prefix(uint32_t v, uint32_t k) {
-  uint32_t x = v;
-#pragma unroll
-  for (int d = 1; d < (int)CG; d <<= 1) {
-    const uint32_t y = __shfl_up(x, d, CG);
-    if (k >= (uint32_t)d) x += y;
-  }
-  return x - v;
-}
-
 // Writes node number `number` (w.link: the number of its first inner child).
 __device__ inline void emit_node(const CollapseArgs& a, const WideNode& w, uint32_t number, uint32_t k, CollapseStats& st) {
   const float eps = o2f(a.cnt->maxabs) * BOX_EPS_REL;
@@ -1070,13 +1077,13 @@ __device__ inline void emit_node(const CollapseArgs& a, const WideNode& w, uint3
     return;
   }
 
-  // children (the group's lanes take the same path); lane k keeps child k
+  // children; lane k keeps child k
   uint32_t mine = 0u;
   int n = 1;
   if (!is_inner(w.bref, a.isleaf)) {
     mine = w.bref;  // whole (small) scene as one leaf
   } else {
-    n = wide_children(a, w.bref, [&](int i, uint32_t c) { mine = (uint32_t)i == k ? c : mine; });
+    n = wide_children(a, w.bref, k, mine);
   }
 
   // this lane's child: box, primitive range and kind
@@ -1567,9 +1574,9 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   ca.leaf_src = S.leaf_src.as<uint32_t>();
   ca.info = out.info.as<NodeInfo>();
   ca.cap = cap;
-  hipLaunchKernelGGL(k_walk_top, dim3(1), dim3(BT), 0, s, ca, S.roots.as<uint32_t>(), S.roots.as<uint32_t>() + nscenes,
+  hipLaunchKernelGGL(k_walk_top, dim3(1), dim3(WT), 0, s, ca, S.roots.as<uint32_t>(), S.roots.as<uint32_t>() + nscenes,
                      S.roots.as<uint32_t>() + 2 * (size_t)nscenes);
-  hipLaunchKernelGGL(k_walk_rest, dim3(std::min(max_sub + 1u, 2048u)), dim3(BT), 0, s, ca);
+  hipLaunchKernelGGL(k_walk_rest, dim3(std::min(max_sub + 1u, 512u)), dim3(WT), 0, s, ca);
   S.scanner.exclusive(ca.count, S.walk_count.as<uint32_t>() + max_sub + 1, (size_t)max_sub + 1, s);
   const uint32_t egrid = std::min(div_up(cap, BT / CG), 4096u);
   S.walk_stats.reserve((size_t)egrid * sizeof(CollapseStats));

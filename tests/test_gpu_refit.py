@@ -46,9 +46,9 @@ def test_skewed_and_equal_primitives(rtc, oracle, device, quality):
 
 
 @pytest.mark.parametrize("width", [2, 3, 8])
-@pytest.mark.parametrize("n", [1, 9, 511, 513, 4097, 70001])
+@pytest.mark.parametrize("n", [1, 9, 511, 513, 2048, 2049, 4097, 70001])
 def test_widths_and_subtrees(rtc, oracle, n, width):
-    # the wide nodes are numbered by subtrees of at most 512 primitives or 1/256 of them
+    # the wide nodes are numbered by subtrees of at most 2048 primitives or 1/256 of them
     dev = rtc.Device(f"bvh_width={width}")
     check(rtc, oracle, dev, rtc.gen_soup(n, seed=n + 1, h=0.03), 1)
     dev.release()
