@@ -418,9 +418,9 @@ __global__ __launch_bounds__(BT) void k_radix_tree(const uint32_t* __restrict__ 
 __device__ inline float box_half_area(float4 l, float4 h) { return half_area(h.x - l.x, h.y - l.y, h.z - l.z); }
 
 
-// Bottom-up bounds and the SAH-optimal 8-wide collapse table. The second
-// child to arrive at a node (agent-scope acquire/release counter) finishes it
-// and moves up. For every binary node n and slot budget s = 1..8, cost8 holds
+// Bottom-up bounds and the SAH-optimal 8-wide collapse table, each node after
+// its two children.
+// For every binary node n and slot budget s = 1..8, cost8 holds
 // the least SAH cost of covering n's subtree with at most s subtrees:
 //   c(n,1) = min(leaf: cost_tri*count*A(n), node: cost_node*A(n) + d(n,8))
 //   d(n,s) = min_j c(left,j) + c(right,s-j)      (s >= 2)
@@ -451,48 +451,35 @@ struct RefitArgs {
   uint32_t* err;
 };
 
-__device__ inline bool refit_node(const RefitArgs& a, uint32_t node) {
+// `inner(c, slot, lo, hi, cost)` reads finished inner child number `slot` (0 or 1),
+// and `keep(lo, hi, cost)` gets the node's own box and costs.
+template <class Inner, class Keep>
+__device__ inline bool refit_node(const RefitArgs& a, uint32_t node, uint2 ch, uint32_t count, Inner inner_child,
+                                  Keep keep) {
   const uint32_t n = a.n;
-  const uint32_t* child = a.child;
-  const uint2* range = a.range;
-  const float4* slo = a.slo;
-  const float4* shi = a.shi;
-  float4* nlo = a.nlo;
-  float4* nhi = a.nhi;
-  float* cost8 = a.cost8;
-  uint8_t* split8 = a.split8;
-  uint8_t* isleaf = a.isleaf;
   const float cost_node = a.cost_node, cost_tri = a.cost_tri;
   const uint32_t max_leaf = a.max_leaf, width = a.width, min_leaf = a.min_leaf, block = a.block;
-  uint32_t* err = a.err;
   float4 bl[2], bh[2];
   float cc[2][8];
 #pragma unroll
   for (int k = 0; k < 2; k++) {
-    const uint32_t c = child[2 * node + k];
+    const uint32_t c = k ? ch.y : ch.x;
     if ((c & REF_LEAF) ? (c & ~REF_LEAF) >= n : c + 1 >= n) {
-      atomicOr(err, 1u);
+      atomicOr(a.err, 1u);
       return false;
     }
     if (c & REF_LEAF) {
-      bl[k] = slo[c & ~REF_LEAF];
-      bh[k] = shi[c & ~REF_LEAF];
+      bl[k] = a.slo[c & ~REF_LEAF];
+      bh[k] = a.shi[c & ~REF_LEAF];
       const float ct = cost_tri * box_half_area(bl[k], bh[k]);
 #pragma unroll
       for (int s = 0; s < 8; s++) cc[k][s] = ct;
     } else {
-      bl[k] = nlo[c];
-      bh[k] = nhi[c];
-      const float4* t = reinterpret_cast<const float4*>(cost8 + 8 * (size_t)c);
-      const float4 t0 = t[0], t1 = t[1];
-      cc[k][0] = t0.x; cc[k][1] = t0.y; cc[k][2] = t0.z; cc[k][3] = t0.w;
-      cc[k][4] = t1.x; cc[k][5] = t1.y; cc[k][6] = t1.z; cc[k][7] = t1.w;
+      inner_child(c, k, bl[k], bh[k], cc[k]);
     }
   }
   const float4 l = make_float4(fminf(bl[0].x, bl[1].x), fminf(bl[0].y, bl[1].y), fminf(bl[0].z, bl[1].z), 0.0f);
   const float4 h = make_float4(fmaxf(bh[0].x, bh[1].x), fmaxf(bh[0].y, bh[1].y), fmaxf(bh[0].z, bh[1].z), 0.0f);
-  const uint2 r = range[node];
-  const uint32_t count = r.y - r.x + 1;
   const float A = box_half_area(l, h);
   float d[9];
   uint32_t dj[9];
@@ -521,17 +508,54 @@ __device__ inline bool refit_node(const RefitArgs& a, uint32_t node) {
     if (d[s] < c[s - 2]) { c[s - 1] = d[s]; sp[s - 1] = dj[s]; }
     else { c[s - 1] = c[s - 2]; sp[s - 1] = 0x80u | dj[s]; }
   }
-  nlo[node] = l;
-  nhi[node] = h;
-  float4* t = reinterpret_cast<float4*>(cost8 + 8 * (size_t)node);
-  t[0] = make_float4(c[0], c[1], c[2], c[3]);
-  t[1] = make_float4(c[4], c[5], c[6], c[7]);
-  uint2* sp8 = reinterpret_cast<uint2*>(split8 + 8 * (size_t)node);
+  a.nlo[node] = l;
+  a.nhi[node] = h;
+  keep(l, h, c);
+  uint2* sp8 = reinterpret_cast<uint2*>(a.split8 + 8 * (size_t)node);
   *sp8 = make_uint2(sp[0] | (sp[1] << 8) | (sp[2] << 16) | (sp[3] << 24),
                     sp[4] | (sp[5] << 8) | (sp[6] << 16) | (sp[7] << 24));
-  isleaf[node] = leafc <= inner ? 1 : 0;
+  a.isleaf[node] = leafc <= inner ? 1 : 0;
   return true;
 }
+
+// A node's costs in HBM, for a parent that another workgroup finishes.
+__device__ inline void put_cost(const RefitArgs& a, uint32_t node, const float c[8]) {
+  float4* t = reinterpret_cast<float4*>(a.cost8 + 8 * (size_t)node);
+  t[0] = make_float4(c[0], c[1], c[2], c[3]);
+  t[1] = make_float4(c[4], c[5], c[6], c[7]);
+}
+__device__ inline void get_node(const RefitArgs& a, uint32_t node, float4& l, float4& h, float c[8]) {
+  l = a.nlo[node];
+  h = a.nhi[node];
+  const float4* t = reinterpret_cast<const float4*>(a.cost8 + 8 * (size_t)node);
+  const float4 t0 = t[0], t1 = t[1];
+  c[0] = t0.x; c[1] = t0.y; c[2] = t0.z; c[3] = t0.w;
+  c[4] = t1.x; c[5] = t1.y; c[6] = t1.z; c[7] = t1.w;
+}
+
+// What a workgroup keeps of its nodes in LDS, so that a parent's step waits
+// neither for its links nor for its children's results from HBM, and only the
+// costs that another workgroup reads are written there (56 B a node kept, 76 KB
+// a workgroup, two of them on a CU; Morton builds of 2^20 triangles 0.815 ->
+// 0.744 ms, of 20,000 0.226 -> 0.217).
+template <uint32_t N>
+struct RefitKept {
+  float v[14][N];  // box lo, hi, costs of 1..8 slots
+  uint2 child[N];
+  uint16_t parent[N];
+  __device__ inline void put(uint32_t i, float4 l, float4 h, const float c[8]) {
+    v[0][i] = l.x; v[1][i] = l.y; v[2][i] = l.z;
+    v[3][i] = h.x; v[4][i] = h.y; v[5][i] = h.z;
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[6 + k][i] = c[k];
+  }
+  __device__ inline void get(uint32_t i, float4& l, float4& h, float c[8]) const {
+    l = make_float4(v[0][i], v[1][i], v[2][i], 0.0f);
+    h = make_float4(v[3][i], v[4][i], v[5][i], 0.0f);
+#pragma unroll
+    for (int k = 0; k < 8; k++) c[k] = v[6 + k][i];
+  }
+};
 
 // Bottom-up order without a launch per depth: an inner node's id lies in its
 // range of positions, in the radix tree as in the binned-SAH tree, so the nodes
@@ -543,8 +567,9 @@ __device__ inline bool refit_node(const RefitArgs& a, uint32_t node) {
 // takes three launches, one of 20,000 two, where a launch per depth level took
 // 25, with the nodes sorted by depth and a read-back of the level sizes before
 // (Morton builds of 20,000 triangles: 0.56 -> 0.48 ms, of 4.2 M: 3.00 -> 2.82).
-// What bounds the pass on small trees is the chain of levels, about 1 us each.
+// What bounds the pass on small trees is the chain of levels, 0.7 us each.
 constexpr uint32_t REFIT_CHUNK = 1024, REFIT_FAN = 32;
+constexpr uint32_t SPAN_KEPT = 1024;   // and those of them that it keeps in LDS
 constexpr uint32_t REFIT_SPAN = 4608;  // listed nodes a workgroup takes (32 chunks of at most 2 x 70)
 
 // Nodes that became ready in round r are in list r % 2, their count in r % 3
@@ -560,6 +585,8 @@ __global__ __launch_bounds__(BT) void k_refit_chunk(RefitArgs a, const uint32_t*
   __shared__ uint16_t ready[2][REFIT_CHUNK];
   __shared__ RefitReady rd;
   __shared__ uint32_t nlist;
+  __shared__ RefitKept<REFIT_CHUNK> kept;
+  __shared__ uint16_t count[REFIT_CHUNK];
   const uint32_t base = blockIdx.x * REFIT_CHUNK, m = a.n - 1u;
   if (threadIdx.x < 3) rd.count[threadIdx.x] = 0u;
   if (threadIdx.x == 0) nlist = 0u;
@@ -567,11 +594,16 @@ __global__ __launch_bounds__(BT) void k_refit_chunk(RefitArgs a, const uint32_t*
   for (uint32_t k = threadIdx.x; k < REFIT_CHUNK; k += BT) {
     const uint32_t id = base + k;
     need[k] = 3u;  // never reaches 0: no node, or one of the list
-    if (id >= m || parent_int[id] == REF_EMPTY) continue;
+    const uint32_t parent = id < m ? parent_int[id] : REF_EMPTY;
+    if (parent == REF_EMPTY) continue;
     const uint2 r = a.range[id];
     if (r.x >= base && r.y - base < REFIT_CHUNK) {
-      const uint32_t inner = (a.child[2 * id] & REF_LEAF ? 0u : 1u) + (a.child[2 * id + 1] & REF_LEAF ? 0u : 1u);
+      const uint2 ch = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)id);
+      const uint32_t inner = (ch.x & REF_LEAF ? 0u : 1u) + (ch.y & REF_LEAF ? 0u : 1u);
       need[k] = inner;
+      kept.child[k] = ch;
+      kept.parent[k] = (uint16_t)min(parent - base, REFIT_CHUNK);  // (REFIT_CHUNK: not in the chunk)
+      count[k] = (uint16_t)(r.y - r.x + 1u);
       if (inner == 0u) ready[0][atomicAdd(&rd.count[0], 1u)] = (uint16_t)k;
     } else {
       list[base + atomicAdd(&nlist, 1u)] = id;
@@ -583,12 +615,21 @@ __global__ __launch_bounds__(BT) void k_refit_chunk(RefitArgs a, const uint32_t*
     if (cnt == 0u) break;
     if (threadIdx.x == 0) rd.count[(round + 2u) % 3u] = 0u;
     for (uint32_t t = threadIdx.x; t < cnt; t += BT) {
-      const uint32_t id = base + ready[round & 1u][t];
-      const uint32_t p = parent_int[id];
-      if (!refit_node(a, id)) continue;
+      const uint32_t k = ready[round & 1u][t], id = base + k;
+      const uint32_t p = kept.parent[k];
+      // (need is 3 where the parent is left to a later launch: only those children's costs are read from HBM)
+      const bool local = p < REFIT_CHUNK && need[p] != 3u;
+      const bool ok = refit_node(
+          a, id, kept.child[k], count[k],
+          [&](uint32_t c, int, float4& l, float4& h, float* cost) { kept.get(min(c - base, REFIT_CHUNK - 1u), l, h, cost); },
+          [&](float4 l, float4 h, const float* cost) {
+            if (local) kept.put(k, l, h, cost);
+            else put_cost(a, id, cost);
+          });
+      if (!ok) continue;
       visit[id] = 2u;  // what the tree check expects of a refitted node
-      if (p - base < REFIT_CHUNK && p < m && atomicSub(&need[p - base], 1u) == 1u)
-        ready[(round + 1u) & 1u][atomicAdd(&rd.count[(round + 1u) % 3u], 1u)] = (uint16_t)(p - base);
+      if (local && atomicSub(&need[p], 1u) == 1u)
+        ready[(round + 1u) & 1u][atomicAdd(&rd.count[(round + 1u) % 3u], 1u)] = (uint16_t)p;
     }
   }
   if (threadIdx.x == 0) list_count[blockIdx.x] = nlist;
@@ -606,6 +647,9 @@ __global__ __launch_bounds__(BT) void k_refit_span(RefitArgs a, const uint32_t* 
   __shared__ uint16_t ready[2][REFIT_SPAN];
   __shared__ RefitReady rd;
   __shared__ uint32_t nids, nout;
+  __shared__ RefitKept<SPAN_KEPT> kept;
+  __shared__ uint16_t cslot[2][SPAN_KEPT];  // slots of the children that are in this workgroup
+  __shared__ uint32_t count[SPAN_KEPT];
   const uint64_t base = (uint64_t)blockIdx.x * REFIT_FAN * cap, end = base + (uint64_t)REFIT_FAN * cap;
   const uint32_t m = a.n - 1u;
   if (threadIdx.x < 3) rd.count[threadIdx.x] = 0u;
@@ -632,12 +676,31 @@ __global__ __launch_bounds__(BT) void k_refit_span(RefitArgs a, const uint32_t* 
   }
   __syncthreads();
   const uint32_t n = min(nids, REFIT_SPAN);
+  // the slot of an inner node, REFIT_SPAN if it is not one of this workgroup's
+  auto slot_of = [&](uint32_t id) {
+    const uint32_t at = id < m ? visit[id] - 4u : REFIT_SPAN;
+    return at < n && ids[at] == id ? at : REFIT_SPAN;
+  };
   for (uint32_t k = threadIdx.x; k < n; k += BT) {
+    const uint32_t id = ids[k];
+    const uint2 ch = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)id);
     uint32_t wait = 0u;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const uint32_t c = a.child[2 * ids[k] + j];
-      if (!(c & REF_LEAF) && (c >= m || visit[c] != 2u)) wait++;
+      const uint32_t c = j ? ch.y : ch.x;
+      uint32_t at = SPAN_KEPT;
+      if (!(c & REF_LEAF)) {
+        const uint32_t v = c < m ? visit[c] : 0u;
+        if (v != 2u) wait++;
+        if (v >= 4u && v - 4u < n && ids[v - 4u] == c) at = min(v - 4u, SPAN_KEPT);
+      }
+      if (k < SPAN_KEPT) cslot[j][k] = (uint16_t)at;
+    }
+    if (k < SPAN_KEPT) {
+      const uint2 r = a.range[id];
+      kept.child[k] = ch;
+      kept.parent[k] = (uint16_t)slot_of(parent_int[id]);
+      count[k] = r.y - r.x + 1u;
     }
     need[k] = wait;
     if (wait == 0u) ready[0][atomicAdd(&rd.count[0], 1u)] = (uint16_t)k;
@@ -648,13 +711,35 @@ __global__ __launch_bounds__(BT) void k_refit_span(RefitArgs a, const uint32_t* 
     if (cnt == 0u) break;
     if (threadIdx.x == 0) rd.count[(round + 2u) % 3u] = 0u;
     for (uint32_t t = threadIdx.x; t < cnt; t += BT) {
-      const uint32_t id = ids[ready[round & 1u][t]];
-      const uint32_t p = parent_int[id];
-      const uint32_t at = p < m ? visit[p] - 4u : REFIT_SPAN;
-      if (!refit_node(a, id)) continue;
+      const uint32_t k = ready[round & 1u][t], id = ids[k];
+      uint2 ch;
+      uint32_t p, cnt, at[2] = {SPAN_KEPT, SPAN_KEPT};
+      if (k < SPAN_KEPT) {
+        ch = kept.child[k];
+        p = kept.parent[k];
+        cnt = count[k];
+        at[0] = cslot[0][k];
+        at[1] = cslot[1][k];
+      } else {
+        const uint2 r = a.range[id];
+        ch = *reinterpret_cast<const uint2*>(a.child + 2 * (size_t)id);
+        p = slot_of(parent_int[id]);
+        cnt = r.y - r.x + 1u;
+      }
+      const bool ok = refit_node(
+          a, id, ch, cnt,
+          [&](uint32_t c, int j, float4& l, float4& h, float* cost) {
+            if (at[j] < SPAN_KEPT) kept.get(at[j], l, h, cost);
+            else get_node(a, c, l, h, cost);
+          },
+          [&](float4 l, float4 h, const float* cost) {
+            if (k < SPAN_KEPT) kept.put(k, l, h, cost);
+            put_cost(a, id, cost);
+          });
+      if (!ok) continue;
       visit[id] = 2u;
-      if (at < n && ids[at] == p && atomicSub(&need[at], 1u) == 1u)
-        ready[(round + 1u) & 1u][atomicAdd(&rd.count[(round + 1u) % 3u], 1u)] = (uint16_t)at;
+      if (p < n && atomicSub(&need[p], 1u) == 1u)
+        ready[(round + 1u) & 1u][atomicAdd(&rd.count[(round + 1u) % 3u], 1u)] = (uint16_t)p;
     }
   }
   if (threadIdx.x == 0) out_count[blockIdx.x] = nout;
