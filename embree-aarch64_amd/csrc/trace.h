@@ -8,9 +8,8 @@ namespace rtg {
 
 // Launch-shape parameters of the traversal (chosen per device, tunable).
 struct TraceParams {
-  // LDS stack entries per lane (0: private stack, 8, 12 or 16; the kernel
-  // with a triangle cursor always has 8). On the 2^20-triangle soup with
-  // 2^24 incoherent rays, closest hit: 12 gave 2398 Mrays/s, 8 2345 and 16
+  // LDS stack entries per lane (0: private stack, 8, 12 or 16). On the
+  // 2^20-triangle soup with 2^24 incoherent rays, closest hit: 12 gave 2398 Mrays/s, 8 2345 and 16
   // 2089 (16 fits 5 blocks of 256 lanes per CU, 12 and 8 fit 6).
   int lds_slots = 12;
   int sort_rays = 0;        // trace in origin-Morton order (a permutation; records stay in place)
@@ -18,19 +17,17 @@ struct TraceParams {
   int persistent = 1;       // persistent waves pulling rays from a counter
   // Idle lanes of a wave that trigger a refill. A refill stalls the wave
   // for one ray-record load (and, once per RAY_RUN rays, a global counter's
-  // atomic); on the 2^20-triangle soup with 2^24 incoherent rays 10 gave
-  // 1936 Mrays/s closest hit (8-14 within 1 %, 24: 1854, 32: 1818) and 24
-  // gave 3795 Mrays/s occlusion (48: 3339).
+  // atomic). On the 2^20-triangle soup 2^24 incoherent rays take 6.71 ms at
+  // 8, 6.66 at 16, 6.80 at 32 and 7.12 at 40, the Pluecker test on a soup
+  // 1.04, 1.04, 1.11 and 1.11, camera rays on a terrain 403, 400, 420 and
+  // 425 us; occlusion rays in the soup 2.11 ms at 8, 2.09 at 16, 2.08 at 24,
+  // 2.10 at 32 and 2.19 at 40.
   int refill_min = 10;      // closest hit
   int refill_min_occ = 24;  // occlusion rays, which finish sooner
-  // Occlusion rays through a two-level scene: 10,000 instances, 12.6 M
-  // shadow rays gave 1169 Mrays/s at 8-12 against 1080 at 24 and 1129 at 16.
+  // Occlusion rays through a two-level scene: two million rays through 10,000
+  // instances and their shadow rays take 2.72 ms at 8, 2.76 at 16, 2.84 at 24
+  // and 2.98 at 32 (closest hit and occlusion alike).
   int refill_min_occ_inst = 12;
-  // Persistent kernel with a separate triangle cursor per lane: 0 never,
-  // 1 always, 2 for occlusion only. On the 2^20-triangle soup with 2^24
-  // incoherent rays it gave 3934 vs 3789 Mrays/s occlusion but 1724 vs 1939
-  // closest hit (speculative node visits before a pending leaf's hits).
-  int dual = 2;
   int groups = 1;           // small streams with eight lanes a ray (0: one lane, as large ones)
   int cus = 256;            // compute units (set from the device)
   int blocks_per_cu = 8;    // 256-thread blocks per compute unit for the persistent grid (at most those resident)

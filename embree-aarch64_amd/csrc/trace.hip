@@ -870,160 +870,6 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
   }
 }
 
-// Persistent traversal with a second cursor for triangles: a lane keeps
-// one leaf in progress (`tri`) next to its node cursor (`cur`), and each
-// loop iteration does one node step and one triangle step, so the wave's
-// triangle branch no longer runs while those lanes' node work waits (and the
-// other way round). A leaf met while a leaf is still in progress waits in
-// `cur`. Node entries are popped after the triangle step, so the cull test
-// sees the newest hit distance; nodes tested while a leaf is pending use the
-// older one (speculative; hits do not depend on it).
-template <bool OCCLUDED, bool ALIGNED, bool COUNT, bool PL>
-__global__ __launch_bounds__(TB, TRACE_MIN_BLOCKS) void k_trace_d(DevScene sc, char* __restrict__ rays, uint32_t M,
-                                                                    uint64_t stride, uint32_t inst_id,
-                                                                    uint32_t* __restrict__ cnt_nodes,
-                                                                    uint32_t* __restrict__ cnt_tris,
-                                                                    uint32_t* __restrict__ err,
-                                                                    const uint32_t* __restrict__ perm,
-                                                                    uint32_t* __restrict__ next, int refill_min,
-                                                                    RayRuns rr, uint32_t* node_visits) {
-  constexpr uint32_t NONE_REF = 0xffffffffu;  // no leaf in progress (as every lane without a ray)
-  const int lane = threadIdx.x & 63;
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  __shared__ uint64_t lds_stack[8 * TB];
-  uint64_t spill_mem[STACK_CAP];
-  RingStack<8> stack;
-  stack.init(lds_stack, spill_mem);
-  int smin = DIST_NONE;  // least entry distance on the stack (closest hit)
-
-  TRay r;
-  Hit best;
-  float lim = 0.0f;
-  uint32_t cur = REF_IDLE, tri = NONE_REF, ray = 0, nvis = 0, ntri = 0;
-  bool pool_empty = false;
-  WavePool pool;
-  pool.init(rr, M);
-  // (node and triangle counts are below 2^31 each, so the bound fits 32 bits)
-  const uint32_t max_iter = sc.num_nodes + sc.num_tris + 16u;
-  uint32_t iter = 0;
-
-  while (true) {
-    if (!pool_empty) {
-      const uint64_t idle = __ballot(cur == REF_IDLE);
-      const int nidle = __popcll(idle);
-      if (nidle >= refill_min) {
-        const uint32_t slot = pool.take(rr, next, M, nidle, (uint32_t)__popcll(idle & lt), lane);
-        pool_empty = pool.empty();
-        if (cur == REF_IDLE && slot != 0xffffffffu) {
-          ray = perm ? perm[slot] : slot;
-          float4 a, b;
-          float tfar;
-          load_ray<ALIGNED>(rays + (uint64_t)ray * stride, a, b, tfar);
-          if (a.w <= tfar) {
-            setup_ray(r, a, b, tfar);
-            best.t = INFINITY;
-            best.prim = best.geom = 0xffffffffu;
-            best.un = best.vn = best.dn = best.ngx = best.ngy = best.ngz = 0.0f;
-            lim = widen_up(tfar);
-            cur = sc.root;
-            stack.init(lds_stack, spill_mem);
-            smin = DIST_NONE;
-            nvis = ntri = 0;
-            iter = 0;
-          } else if (COUNT) {
-            cnt_nodes[ray] = 0;
-            cnt_tris[ray] = 0;
-          }
-        }
-      }
-    }
-    if (__ballot(cur != REF_IDLE) == 0) {
-      if (pool_empty) break;
-      continue;
-    }
-
-    if (++iter > max_iter && cur != REF_IDLE) {
-      raise_error(err, 2u);
-      cur = REF_DONE;
-    }
-    // a waiting leaf starts once the triangle cursor is free
-    if (tri == NONE_REF && (cur & REF_LEAF) && cur < REF_DONE) {
-      tri = cur & ~REF_LEAF;
-      cur = REF_EMPTY;
-    }
-    // node step
-    if (!(cur & REF_LEAF)) {
-      if (cur >= sc.num_nodes) {
-        raise_error(err, 4u);
-        cur = REF_DONE;
-      } else {
-        if (COUNT) {
-          nvis++;
-          if (node_visits) atomicAdd(&node_visits[cur], 1u);
-        }
-        NodeHit h;
-        intersect_node<OCCLUDED>(sc.nodes, cur, r, lim, h);
-        if (!(OCCLUDED ? push_any_order(h, stack, err, cur) : push_near_to_far(h, stack, smin, lim, err, cur)))
-          cur = REF_EMPTY;
-      }
-    }
-    // triangle step
-    if (tri != NONE_REF) {
-      if (tri >= sc.num_tris) {
-        raise_error(err, 4u);
-        cur = REF_DONE;
-      } else {
-        TriTest h;
-        const bool valid = tri_test<PL>(r, sc.tris + tri, h);
-        if (COUNT) ntri++;
-        tri = (h.flags & TRI_LAST) ? NONE_REF : tri + 1u;
-        if (valid) {
-          if (OCCLUDED) {
-            *reinterpret_cast<float*>(rays + (uint64_t)ray * stride + 32) = -INFINITY;
-            cur = REF_DONE;
-          } else {
-            // (a hit's geometry ID is below the initial one)
-            const bool better = h.t < best.t ||
-                                (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim)));
-            if (better) {
-              best.t = h.t;
-              best.un = h.un; best.vn = h.vn; best.dn = h.dn;
-              best.ngx = h.ngx; best.ngy = h.ngy; best.ngz = h.ngz;
-              best.prim = h.prim; best.geom = h.geom;
-              lim = widen_up(fminf(best.t, r.tfar));
-            }
-          }
-        }
-      }
-    }
-    // the node cursor takes the next entry that can still hold a closer hit
-    if (cur == REF_EMPTY) {
-      const int dlim = dist_limit(lim);
-      while (!stack.empty()) {
-        const uint2 e = stack.pop();
-        if (!OCCLUDED) smin = below_dist(e.y);
-        if (OCCLUDED || (int)e.y <= dlim) {
-          cur = e.x;
-          break;
-        }
-        if (smin > dlim) {
-          // every entry left is farther than the closest hit so far
-          stack.clear();
-          smin = DIST_NONE;
-          break;
-        }
-      }
-      if (cur == REF_EMPTY && tri == NONE_REF) cur = REF_DONE;
-    }
-    if (cur == REF_DONE) {
-      cur = REF_IDLE;
-      tri = NONE_REF;
-      if (COUNT) { cnt_nodes[ray] = nvis; cnt_tris[ray] = ntri; }
-      if (!OCCLUDED && best.geom != 0xffffffffu) write_hit(best, rays + (uint64_t)ray * stride, inst_id);
-    }
-  }
-}
-
 // ------------------------------------------------------- small streams --
 
 // A stream too small to fill the GPU with one ray per lane: eight lanes share
@@ -1548,7 +1394,6 @@ struct LaunchArgs {
   bool persistent;
   const TraceParams* tp;
   hipStream_t s;
-  bool dual;
 };
 
 template <bool OCC, bool AL, bool CNT, int SL, bool PL>
@@ -1558,18 +1403,11 @@ void launch_one(const LaunchArgs& a) {
                        a.stride, a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.node_visits);
     return;
   }
-  // (the dual-cursor kernel's ring has 8 slots whatever SL is)
-  const RayPlan p = ray_plan(
-      a.M, a.dual ? resident_blocks<k_trace_d<OCC, AL, CNT, PL>>() : resident_blocks<k_trace_p<OCC, AL, CNT, SL, PL>>(), *a.tp);
+  const RayPlan p = ray_plan(a.M, resident_blocks<k_trace_p<OCC, AL, CNT, SL, PL>>(), *a.tp);
   if (p.counter) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(COUNTERS), 0, a.s, a.counter);
-  if (a.dual)
-    hipLaunchKernelGGL((k_trace_d<OCC, AL, CNT, PL>), p.grid, dim3(TB), 0, a.s, a.sc, a.rays, a.M, a.stride,
-                       a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.counter, a.refill, p.runs,
-                       a.node_visits);
-  else
-    hipLaunchKernelGGL((k_trace_p<OCC, AL, CNT, SL, PL>), p.grid, dim3(TB), 0, a.s, a.sc, a.rays, a.M, a.stride,
-                       a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.counter, a.refill, p.runs,
-                       a.node_visits, nullptr, 0u);
+  hipLaunchKernelGGL((k_trace_p<OCC, AL, CNT, SL, PL>), p.grid, dim3(TB), 0, a.s, a.sc, a.rays, a.M, a.stride,
+                     a.inst_id, a.cnt_nodes, a.cnt_tris, a.err, a.perm, a.counter, a.refill, p.runs, a.node_visits,
+                     nullptr, 0u);
 }
 
 template <bool OCC, bool AL, bool CNT, bool PL>
@@ -1582,11 +1420,11 @@ void launch_slots(const LaunchArgs& a) {
 
 // The largest streams that eight lanes a ray serve better (us a call, with 14
 // of launching and of making the records; eight lanes against one):
-//                                     1024       16384      65536      131072
-//   camera, 131 k terrain          42 :  82   48 : 103   63 :  96   97 : 120
-//   random, 262 k soup            102 : 223  174 : 286  279 : 304  448 : 315
-//   random occlusion, 262 k soup   31 :  54   40 :  58   83 :  70  129 :  75
-//   camera, 16 k sphere            41 :  70   44 :  78   69 :  86   90 :  93
+//                                    8192      16384      32768      65536
+//   camera, 131 k terrain          49 :  75   47 :  88   58 :  86   61 :  80
+//   random, 262 k soup            143 : 247  171 : 248  194 : 253  270 : 258
+//   camera, 16 k sphere            44 :  63   43 :  66   55 :  71   68 :  72
+//   random occlusion, 262 k soup   33 :  54   41 :  53   51 :  60   83 :  64
 // From there on the GPU is full, and one lane a ray needs fewer instructions.
 constexpr uint32_t GROUP_MAX_RAYS = 65536, GROUP_MAX_RAYS_OCC = 32768;
 // A ray's stack is all in LDS: 256 entries are 16 KB a wave. (Trees of a few
@@ -1653,7 +1491,7 @@ void launch_trace(const DevScene& sc, void* rays, uint32_t M, uint64_t stride, b
     counter = sorter->counter.as<uint32_t>();
   }
   LaunchArgs la{sc, rp, M, stride, inst_id, cnt_nodes, cnt_tris, err, perm, persistent ? counter : nullptr, refill,
-                count ? node_visits : nullptr, persistent, &tp, s, tp.dual == 1 || (tp.dual == 2 && occluded)};
+                count ? node_visits : nullptr, persistent, &tp, s};
   if (sc.robust) launch_pl<true>(la, count, occluded, aligned);
   else launch_pl<false>(la, count, occluded, aligned);
   RTG_HIP(hipGetLastError());

@@ -23,7 +23,7 @@ typedef struct RTCDeviceTy* RTCDevice;
  * the reference's sahBlockSize; tree shape); spatial_budget (extra triangle
  * references spatial splits may add at RTC_BUILD_QUALITY_HIGH, as a fraction
  * of the triangles; default 0.3, 0 turns them off); trace_stack, refill_min, refill_min_occ,
- * refill_min_occ_inst, blocks_per_cu, persistent, dual, ray_sort
+ * refill_min_occ_inst, blocks_per_cu, persistent, ray_sort
  * (traversal launch settings, as rtcgAutotune writes them). The reference's
  * CPU keys (threads, isa, set_affinity, ...) and unknown keys are ignored as
  * the reference ignores unknown keys. The learned split cost is chosen per
