@@ -110,7 +110,7 @@ def profiled_traffic():
                 traffic = (rd + wr) * 1e9
             if line.strip().startswith("VALU instructions per ray"):
                 f = line.replace(",", " ").replace(";", " ").split()
-                limiter = {"kind": "VALU issue (SQ counters: VALU busy, divergent lanes)",
+                limiter = {"kind": "return path of the vector memory (TD busy) and VALU issue, divergent lanes",
                            "valu_instr_per_ray": float(f[4]), "salu_instr_per_ray": float(f[6]),
                            "lanes_active_per_valu_instr": float(f[f.index("instruction") + 1]),
                            "source": os.path.relpath(PROFILE, ROOT)}
@@ -126,10 +126,10 @@ def build_bytes_per_tri(n):
       Morton codes: box in, key + id out                                40
       radix sort: 4 passes of 8 B key + id in and out                   64
       boxes gathered in sorted order: id + box in, box out              68
-      copies into the level buffers: id + box in and out                72
-      each big level (segments above 4096): id + box read to bin and
-        again to flag, flags written and scanned, id + box + flag +
-        scan read and id + box + value + segment id written            176
+      ids copied into the level buffers                                  8
+      each big level (segments above 4096): segment id + box read to
+        bin, segment id + id + box read and id + box + value +
+        segment id written                                             120
       each mid or small level (segments of 17..4096): box read to bin
         and to flag, id + box read and id + box + value written        140
       tiny segments (2..16): id + box read, value + links written        56
@@ -140,7 +140,7 @@ def build_bytes_per_tri(n):
         reference, 3 indices and 3 vertices read, 48 B record written  140
     Big levels: ceil(log2(n / 4096)); mid and small levels: log2(4096 / 16) = 8."""
     big = max(0, int(np.ceil(np.log2(max(1.0, n / 4096.0)))))
-    return 84 + 40 + 64 + 68 + 72 + 176 * big + 140 * 8 + 56 + 68 + 64 + 22 + 140, big
+    return 84 + 40 + 64 + 68 + 8 + 120 * big + 140 * 8 + 56 + 68 + 64 + 22 + 140, big
 
 
 def time_trace(L, dev, sc, d_rays, d_src, n, steps):

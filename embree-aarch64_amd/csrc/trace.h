@@ -20,7 +20,7 @@ struct TraceParams {
   // atomic). On the 2^20-triangle soup 2^24 incoherent rays take 6.71 ms at
   // 8, 6.66 at 16, 6.80 at 32 and 7.12 at 40, the Pluecker test on a soup
   // 1.04, 1.04, 1.11 and 1.11, camera rays on a terrain 403, 400, 420 and
-  // 425 us; occlusion rays in the soup 2.11 ms at 8, 2.09 at 16, 2.08 at 24,
+  // 425 us; 2^23 occlusion rays in the soup 2.11 ms at 8, 2.09 at 16, 2.08 at 24,
   // 2.10 at 32 and 2.19 at 40.
   int refill_min = 10;      // closest hit
   int refill_min_occ = 24;  // occlusion rays, which finish sooner

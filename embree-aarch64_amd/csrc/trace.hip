@@ -394,9 +394,10 @@ __device__ inline bool push_any_order(const NodeHit& h, Stack& stack, uint32_t* 
 // conservative. The limit is compared with the sorted keys (which a push tests
 // anyway) instead of taking part in every child's slab test. (With integer
 // distances and this, 274 VALU instructions a ray instead of 290 on the
-// 2^20-triangle soup, 7.00 ms instead of 7.14 for 2^24 rays: the kernel is
-// bound as much by the return path of the vector memory, busy 95 % of the
-// time, where every lane's 16 bytes of a node are an access of their own.)
+// 2^20-triangle soup, 7.00 ms instead of 7.14 for 2^24 rays; with the lanes'
+// state in their references 229 and 6.72 ms. There the kernel is bound by the
+// return path of the vector memory, busy 96 % of the time, where every lane's
+// 16 bytes of a node are an access of their own.)
 template <class Stack>
 __device__ inline bool push_near_to_far(const NodeHit& h, Stack& stack, int& smin, float lim, uint32_t* err,
                                         uint32_t& next) {
