@@ -1210,21 +1210,22 @@ __device__ inline Split split_segment(const Seg& sg, const uint32_t* __restrict_
   return sp;
 }
 
-// One workgroup per mid segment of a level (between SMALL_MAX and MID_MAX
-// references).
+// Where a level's mid and small segments are read and written.
+struct LevelRefs {
+  const uint32_t* idx;
+  const float4 *blo, *bhi;
+  uint32_t* idx_o;
+  float4 *blo_o, *bhi_o;
+};
+
+// One mid segment (between SMALL_MAX and MID_MAX references) by a workgroup
+// of 256.
 template <bool LEARNED>
-__global__ __launch_bounds__(256, 4) void k_seg(const Seg* __restrict__ segs, const uint32_t* __restrict__ nseg,
-                                             const uint32_t* __restrict__ idx, const float4* __restrict__ blo,
-                                             const float4* __restrict__ bhi, uint32_t* __restrict__ idx_o,
-                                             float4* __restrict__ blo_o, float4* __restrict__ bhi_o, Lists nx,
-                                             Tree t, LearnedCost lc, LevelStart st) {
-  __shared__ SegLds<256> S;
-  start_level(st);
-  if (blockIdx.x >= *nseg) return;
-  const Seg sg = segs[blockIdx.x];
+__device__ inline void split_mid(const Seg& sg, const LevelRefs& R, const Lists& nx, const Tree& t,
+                                 const LearnedCost& lc, SegLds<256>& S) {
   float lcl[3], lch[3], rcl[3], rch[3];
-  const Split sp = split_segment<256, 16, false, LEARNED>(sg, idx, blo, bhi, idx_o, blo_o, bhi_o, t, lc, S, threadIdx.x, lcl,
-                                                 lch, rcl, rch);
+  const Split sp = split_segment<256, 16, false, LEARNED>(sg, R.idx, R.blo, R.bhi, R.idx_o, R.blo_o, R.bhi_o, t, lc, S,
+                                                          threadIdx.x, lcl, lch, rcl, rch);
   if (threadIdx.x == 0) {
     const uint32_t mid = sg.first + sp.nleft - 1, depth = sg.meta >> 1;
     emit_child(t, nx, mid, 0, depth, sg.first, sp.nleft, lcl, lch);
@@ -1232,31 +1233,28 @@ __global__ __launch_bounds__(256, 4) void k_seg(const Seg* __restrict__ segs, co
   }
 }
 
-// One wave per small segment of a level (up to SMALL_MAX references, or a
-// tree's root of any size up to that), SEGW_WAVES per workgroup; the grid
-// covers the list's capacity and the count is read on the device. The
-// workgroup reserves its children's list slots with one global atomic per
-// list: the level's segments number in the tens of thousands, and an atomic
-// per child on one address would serialise them. (A grid-stride loop over
-// the count doubles the kernel's registers.)
-constexpr int SEGW_TB = 512;
-constexpr int SEGW_WAVES = SEGW_TB / 64;
+// One wave per small segment (up to SMALL_MAX references, or a tree's root of
+// any size up to that), WAVES per workgroup. The workgroup reserves its
+// children's list slots with one global atomic per list: a level's segments
+// number in the tens of thousands, and an atomic per child on one address
+// would serialise them. (A grid-stride loop over the count doubles the
+// kernel's registers.)
 constexpr int SEGW_PER = (int)(SMALL_MAX / 64);
 
-template <bool LEARNED>
-__global__ __launch_bounds__(SEGW_TB) void k_seg_wave(const Seg* __restrict__ segs, const uint32_t* __restrict__ nseg,
-                                                      const uint32_t* __restrict__ idx, const float4* __restrict__ blo,
-                                                      const float4* __restrict__ bhi, uint32_t* __restrict__ idx_o,
-                                                      float4* __restrict__ blo_o, float4* __restrict__ bhi_o, Lists nx,
-                                                      Tree t, LearnedCost lc, LevelStart st) {
-  __shared__ SegLds<64> S[SEGW_WAVES];
-  __shared__ uint32_t lcount[4], lbase[4];
-  start_level(st);
+template <int WAVES>
+struct SmallLds {
+  SegLds<64> S[WAVES];
+  uint32_t lcount[4], lbase[4];
+};
+
+template <int WAVES, bool LEARNED>
+__device__ inline void split_smalls(const Seg* __restrict__ segs, uint32_t nseg, uint32_t block, const LevelRefs& R,
+                                    const Lists& nx, const Tree& t, const LearnedCost& lc, SmallLds<WAVES>& M) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t i = blockIdx.x * SEGW_WAVES + (uint32_t)wave;
-  if (threadIdx.x < 4) lcount[threadIdx.x] = 0u;
+  const uint32_t i = block * WAVES + (uint32_t)wave;
+  if (threadIdx.x < 4) M.lcount[threadIdx.x] = 0u;
   __syncthreads();
-  const bool active = i < *nseg && i < nx.cap[2];  // both parities' lists have this capacity
+  const bool active = i < nseg && i < nx.cap[2];  // both parities' lists have this capacity
   Seg sg;
   Split sp;
   float cb[2][6];  // children's centroid bounds: lo3, hi3
@@ -1264,29 +1262,70 @@ __global__ __launch_bounds__(SEGW_TB) void k_seg_wave(const Seg* __restrict__ se
   uint32_t slot[2] = {0u, 0u};
   if (active) {
     sg = segs[i];
-    sp = split_segment<64, SEGW_PER, true, LEARNED>(sg, idx, blo, bhi, idx_o, blo_o, bhi_o, t, lc, S[wave], lane,
-                                                    &cb[0][0], &cb[0][3], &cb[1][0], &cb[1][3]);
+    sp = split_segment<64, SEGW_PER, true, LEARNED>(sg, R.idx, R.blo, R.bhi, R.idx_o, R.blo_o, R.bhi_o, t, lc,
+                                                    M.S[wave], lane, &cb[0][0], &cb[0][3], &cb[1][0], &cb[1][3]);
     if (lane == 0) {
       const uint32_t mid = sg.first + sp.nleft - 1, depth = sg.meta >> 1;
       cls[0] = child_list(t, nx, mid, 0, depth, sg.first, sp.nleft);
       cls[1] = child_list(t, nx, mid, 1, depth, sg.first + sp.nleft, sg.count - sp.nleft);
 #pragma unroll
       for (int c = 0; c < 2; c++)
-        if (cls[c] >= 0) slot[c] = atomicAdd(&lcount[cls[c]], 1u);
+        if (cls[c] >= 0) slot[c] = atomicAdd(&M.lcount[cls[c]], 1u);
     }
   }
   __syncthreads();
-  if (threadIdx.x < 4 && lcount[threadIdx.x])
-    lbase[threadIdx.x] = atomicAdd(list_counter(t, nx, (int)threadIdx.x), lcount[threadIdx.x]);
+  if (threadIdx.x < 4 && M.lcount[threadIdx.x])
+    M.lbase[threadIdx.x] = atomicAdd(list_counter(t, nx, (int)threadIdx.x), M.lcount[threadIdx.x]);
   __syncthreads();
   if (active && lane == 0) {
     const uint32_t mid = sg.first + sp.nleft - 1, depth = sg.meta >> 1;
 #pragma unroll
     for (int c = 0; c < 2; c++)
       if (cls[c] >= 0)
-        put_child(t, nx, cls[c], lbase[cls[c]] + slot[c], mid, (uint32_t)c, depth, c ? sg.first + sp.nleft : sg.first,
+        put_child(t, nx, cls[c], M.lbase[cls[c]] + slot[c], mid, (uint32_t)c, depth, c ? sg.first + sp.nleft : sg.first,
                   c ? sg.count - sp.nleft : sp.nleft, &cb[c][0], &cb[c][3]);
   }
+}
+
+// The mid and small segments of a level that may have mid ones, in one launch:
+// the first `mids` workgroups a mid segment each, the others four small ones.
+// The grid covers what the lists may hold and the counts are read on the
+// device. (Two launches one after the other took a level's two latencies in
+// turn, 20 to 35 us each on small trees, 5 where a list is empty: builds of
+// 20,000 triangles 0.69 -> 0.62 ms, of 131,000 0.94 -> 0.88, of 2^20 2.33 ->
+// 2.29.)
+constexpr int SEG_TB = 256;
+
+template <bool LEARNED>
+__global__ __launch_bounds__(SEG_TB, LEARNED ? 3 : 4) void k_seg(const Seg* __restrict__ mid_segs, uint32_t mids,
+                                                   const Seg* __restrict__ small_segs,
+                                                   const uint32_t* __restrict__ nseg, LevelRefs R, Lists nx, Tree t,
+                                                   LearnedCost lc, LevelStart st) {
+  constexpr size_t A = sizeof(SegLds<SEG_TB>), B = sizeof(SmallLds<SEG_TB / 64>);
+  __shared__ __align__(16) char mem[A > B ? A : B];
+  start_level(st);
+  if (blockIdx.x < mids) {
+    if (blockIdx.x < nseg[1])
+      split_mid<LEARNED>(mid_segs[blockIdx.x], R, nx, t, lc, *reinterpret_cast<SegLds<SEG_TB>*>(mem));
+  } else {
+    const uint32_t block = blockIdx.x - mids, n = nseg[2];
+    if (block * (SEG_TB / 64) < n)
+      split_smalls<SEG_TB / 64, LEARNED>(small_segs, n, block, R, nx, t, lc,
+                                         *reinterpret_cast<SmallLds<SEG_TB / 64>*>(mem));
+  }
+}
+
+// The small segments of a level without mid ones: more of them to a workgroup,
+// so fewer reservations (2^20 triangles 2.35 ms, 2.40 with four a workgroup).
+constexpr int SEGW_TB = 512;
+constexpr int SEGW_WAVES = SEGW_TB / 64;
+
+template <bool LEARNED>
+__global__ __launch_bounds__(SEGW_TB) void k_seg_wave(const Seg* __restrict__ segs, const uint32_t* __restrict__ nseg,
+                                                      LevelRefs R, Lists nx, Tree t, LearnedCost lc, LevelStart st) {
+  __shared__ SmallLds<SEGW_WAVES> M;
+  start_level(st);
+  split_smalls<SEGW_WAVES, LEARNED>(segs, nseg[2], blockIdx.x, R, nx, t, lc, M);
 }
 
 // ------------------------------------------------------------ tiny segments --
@@ -1723,18 +1762,15 @@ void build_sah_tree(uint32_t n, uint32_t* vals, const float4* slo, const float4*
                          S.idx[in].as<uint32_t>(), lo_in, hi_in, n, bs, S.splits.as<Split>(),
                          S.before.as<uint32_t>(), S.sid[o].as<uint32_t>(), S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(), S.bhi[o].as<float4>(), vals, cnt);
     }
-    if (gb[1]) {
-      hipLaunchKernelGGL(lcost.P ? k_seg<true> : k_seg<false>, dim3(gb[1]), dim3(256), 0, s, S.segs[1][li].as<Seg>(),
-                         &cnt->nseg[li][1], S.idx[in].as<uint32_t>(), lo_in, hi_in, S.idx[o].as<uint32_t>(),
-                         S.blo[o].as<float4>(), S.bhi[o].as<float4>(), nx, t, lcost, st);
-      st = none;
-    }
-    // (a level without segments still posts that)
-    if (gb[2] || st.post)
-      hipLaunchKernelGGL(lcost.P ? k_seg_wave<true> : k_seg_wave<false>, dim3(std::max(div_up(gb[2], SEGW_WAVES), 1u)),
-                         dim3(SEGW_TB), 0, s, S.segs[2][li].as<Seg>(), &cnt->nseg[li][2], S.idx[in].as<uint32_t>(),
-                         lo_in, hi_in, S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(), S.bhi[o].as<float4>(), nx, t,
+    const LevelRefs R{S.idx[in].as<uint32_t>(), lo_in, hi_in, S.idx[o].as<uint32_t>(), S.blo[o].as<float4>(),
+                      S.bhi[o].as<float4>()};
+    if (gb[1])
+      hipLaunchKernelGGL(lcost.P ? k_seg<true> : k_seg<false>, dim3(gb[1] + div_up(gb[2], SEG_TB / 64)), dim3(SEG_TB),
+                         0, s, S.segs[1][li].as<Seg>(), gb[1], S.segs[2][li].as<Seg>(), &cnt->nseg[li][0], R, nx, t,
                          lcost, st);
+    else if (gb[2] || st.post)  // (a level without segments still posts that)
+      hipLaunchKernelGGL(lcost.P ? k_seg_wave<true> : k_seg_wave<false>, dim3(std::max(div_up(gb[2], SEGW_WAVES), 1u)),
+                         dim3(SEGW_TB), 0, s, S.segs[2][li].as<Seg>(), &cnt->nseg[li][0], R, nx, t, lcost, st);
     RTG_HIP(hipGetLastError());
   };
   uint32_t ntiny = 0;
