@@ -168,6 +168,56 @@ struct HostPool {
   }
 };
 
+// Asynchronous queries that may still run. A commit writes a tree's arrays in
+// place, so before that it waits for the device if a query of that tree was
+// queued since the last such wait; what it does before only uses scratch memory
+// and overlaps the query. (An event after each query, for the commit's stream to
+// wait on, costs every query: 1073 camera rays on a 131 k triangle terrain, call
+// after call, 38 us instead of 33. The wait costs a mesh of 20,000 triangles
+// that is committed and traced every frame 3 of 280 us, at the start of the
+// commit 21.)
+struct RunningQueries {
+  static constexpr size_t MAX = 64;
+  struct Entry {
+    const void* tree;
+    uint64_t last;  // number of its last query
+  };
+  std::mutex mtx;
+  std::vector<Entry> list;
+  uint64_t count = 0, any = 0;  // queries so far; the last one that may read any tree
+  bool captured = false;        // a graph with queries may be replayed at any time
+  // A query was queued on `stream`, of one tree (null: of several, a two-level one).
+  void note(hipStream_t stream, const void* tree) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    RTG_HIP(hipStreamIsCapturing(stream, &cs));
+    std::lock_guard<std::mutex> g(mtx);
+    if (cs != hipStreamCaptureStatusNone) captured = true;
+    count++;
+    for (Entry& e : list)
+      if (e.tree == tree) {
+        e.last = count;
+        return;
+      }
+    if (tree && list.size() < MAX) list.push_back({tree, count});
+    else any = count;
+  }
+  // What the caller does next may write `tree`.
+  void wait(const void* tree) {
+    uint64_t now;
+    {
+      std::lock_guard<std::mutex> g(mtx);
+      bool must = captured || any != 0;
+      for (const Entry& e : list) must = must || e.tree == tree;
+      if (!must) return;
+      now = count;
+    }
+    RTG_HIP(hipDeviceSynchronize());
+    std::lock_guard<std::mutex> g(mtx);
+    if (any <= now) any = 0;
+    list.erase(std::remove_if(list.begin(), list.end(), [&](const Entry& e) { return e.last <= now; }), list.end());
+  }
+};
+
 struct ThreadDev {
   hipStream_t stream = nullptr;
   rtg::PinnedBuf errword;  // traversal error bits: the host reads them after a synchronisation, without a copy
@@ -190,6 +240,7 @@ struct Device : RefObj {
   std::mutex build_mtx;
   rtg::BuildScratch scratch;
   rtg::DeviceBVH other;  // scratch of HIGH commits: the tree that was not kept (under build_mtx)
+  RunningQueries running;
   // tri_builder / builder setting: "default" lets the build quality choose
   // (reference bvh8_factory.cpp:865-870); an unknown name fails the commit.
   enum { TB_DEFAULT, TB_SAH, TB_MORTON, TB_UNKNOWN } tri_builder = TB_DEFAULT;
@@ -577,7 +628,7 @@ rtg::BuildParams scene_params(Scene* sc, rtg::LearnedCost& lc, const rtg::BuildP
 // of split at every node, kernels/builders/heuristic_spatial_array.h).
 void build_scene_tree(Scene* sc, Device* d, const std::vector<rtg::GeomDesc>& descs, const rtg::BuildParams& p,
                       hipStream_t st) {
-  rtg::build_bvh(descs, p, d->scratch, *sc->bvh, st);
+  rtg::build_bvh(descs, p, d->scratch, *sc->bvh, st, 1, nullptr, [&] { d->running.wait(sc->bvh.get()); });
   if (sc->bvh->stats.num_split == 0) return;
   rtg::BuildParams q = p;
   q.split_budget = 0.0f;
@@ -892,7 +943,7 @@ void build_top(Scene* sc, Device* d, ThreadDev& t) {
   d->monitor((ssize_t)n * (80 + 64));
   {
     std::lock_guard<std::mutex> bl(d->build_mtx);
-    rtg::build_bvh({gd}, p, d->scratch, sc->top, t.stream);
+    rtg::build_bvh({gd}, p, d->scratch, sc->top, t.stream, 1, nullptr, [&] { d->running.wait(&sc->top); });
   }
   sc->top_objects.reserve(objects.size() * sizeof(rtg::DevScene));
   RTG_HIP(hipMemcpyAsync(sc->top_objects.ptr, objects.data(), objects.size() * sizeof(rtg::DevScene),
@@ -947,6 +998,11 @@ void launch_scene(Scene* sc, uint32_t* err, rtg::RaySorter& sorter, void* rays, 
 void launch_scene(Scene* sc, ThreadDev& t, void* rays, unsigned M, size_t stride, bool occluded, uint32_t inst,
                   hipStream_t stream, const rtg::TraceParams& tp) {
   launch_scene(sc, t.errword.as<uint32_t>(), t.sorter, rays, M, stride, occluded, inst, stream, tp);
+}
+
+// An asynchronous query of the scene was queued on `stream`.
+void note_query(Scene* sc, hipStream_t stream) {
+  if (!scene_empty(sc)) sc->dev->running.note(stream, sc->two_level ? nullptr : (const void*)sc->bvh.get());
 }
 
 void single_level_only(Scene* sc, const char* what) {
@@ -1768,7 +1824,9 @@ static void async_trace(Scene* s, const RTCIntersectContext* ctx, void* rays, un
   d->activate();
   ThreadDev& t = d->td();
   const uint32_t inst = ctx ? ctx->instID[0] : RTC_INVALID_GEOMETRY_ID;
-  launch_scene(s, t, rays, M, stride, occluded, inst, stream ? (hipStream_t)stream : t.stream, d->trace_params());
+  const hipStream_t st = stream ? (hipStream_t)stream : t.stream;
+  launch_scene(s, t, rays, M, stride, occluded, inst, st, d->trace_params());
+  note_query(s, st);
 }
 
 RTC_API void rtcgIntersect1MAsync(RTCScene scene, const RTCIntersectContext* context, RTCRayHit* d_rayhit,
@@ -1822,7 +1880,10 @@ RTC_API void rtcgQuery1MNoAlloc(RTCScene scene, const RTCIntersectContext* conte
     rtg::launch_trace(s->bvh->view(s->slot), d_rays, M, byteStride, occluded != 0, inst, nullptr, nullptr, scr + 1,
                       st, tp, nullptr, nullptr, scr);
   }
-  if (hipStream) return;
+  if (hipStream) {
+    note_query(s, st);
+    return;
+  }
   RTG_HIP(hipStreamSynchronize(st));
   uint32_t err = 0;
   RTG_HIP(hipMemcpy(&err, scr + 1, 4, hipMemcpyDeviceToHost));

@@ -3,6 +3,7 @@
 // top-down collapse into quantised 8-wide nodes and Moeller-ready triangle
 // records.
 #pragma once
+#include <functional>
 #include <vector>
 
 #include "builder_sah.h"
@@ -131,7 +132,10 @@ struct UserTree {
 // Throws hip_error on a HIP failure.
 // With `user` set the build stops after the binary tree and hands it over
 // (one scene of GEOM_INSTANCES boxes; no nodes or records are written).
+// `before_write` (may be empty) is called once, before anything is queued that
+// writes or frees the arrays of `out`; the work before it only uses the scratch.
 void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& p, BuildScratch& scratch,
-               DeviceBVH& out, hipStream_t s, uint32_t nscenes = 1, UserTree* user = nullptr);
+               DeviceBVH& out, hipStream_t s, uint32_t nscenes = 1, UserTree* user = nullptr,
+               const std::function<void()>& before_write = nullptr);
 
 }  // namespace rtg

@@ -1378,7 +1378,7 @@ __global__ __launch_bounds__(BT) void k_sum_stats(const CollapseStats* __restric
 // ------------------------------------------------------------------ host --
 
 void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, BuildScratch& S, DeviceBVH& out,
-               hipStream_t s, uint32_t nscenes, UserTree* user) {
+               hipStream_t s, uint32_t nscenes, UserTree* user, const std::function<void()>& before_write) {
   auto t0 = std::chrono::steady_clock::now();
   out.generation++;
   out.stats = BuildStats();
@@ -1620,6 +1620,7 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
 
   // outputs: at most n + nscenes nodes, exactly n triangle records
   const uint32_t cap = n + nscenes;
+  if (before_write) before_write();
   out.nodes.reserve((size_t)cap * sizeof(QNode8));
   const bool inst_build = geoms[0].kind == GEOM_INSTANCES;
   for (const auto& g : geoms)
