@@ -1377,6 +1377,18 @@ __global__ __launch_bounds__(BT) void k_sum_stats(const CollapseStats* __restric
 
 // ------------------------------------------------------------------ host --
 
+namespace {
+// Leaves the stream idle however the build ends: the scratch and the staging
+// memory are the next build's, which may be another thread's on another stream.
+struct IdleAtEnd {
+  hipStream_t s;
+  bool idle = false;
+  ~IdleAtEnd() {
+    if (!idle) (void)hipStreamSynchronize(s);
+  }
+};
+}  // namespace
+
 void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, BuildScratch& S, DeviceBVH& out,
                hipStream_t s, uint32_t nscenes, UserTree* user, const std::function<void()>& before_write) {
   auto t0 = std::chrono::steady_clock::now();
@@ -1404,6 +1416,7 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
   const uint32_t min_leaf = prm.min_leaf < 1 ? 1 : (prm.min_leaf > max_leaf ? max_leaf : prm.min_leaf);
   const uint32_t block = prm.block < 1 ? 1 : prm.block;
 
+  IdleAtEnd at_end{s};
   if (nscenes == 0 || nscenes > 65535) throw hip_error(hipErrorInvalidValue, "scene count out of range");
   S.geoms.reserve(geoms.size() * sizeof(GeomDesc));
   const uint32_t geom_words = (uint32_t)(geoms.size() * sizeof(GeomDesc) / 4);
@@ -1612,6 +1625,7 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
     RTG_HIP(hipMemcpy2DAsync(user->pbox.data(), 32, S.slo.ptr, 16, 16, n, hipMemcpyDeviceToHost, s));
     RTG_HIP(hipMemcpy2DAsync(user->pbox.data() + 4, 32, S.shi.ptr, 16, 16, n, hipMemcpyDeviceToHost, s));
     RTG_HIP(hipStreamSynchronize(s));
+    at_end.idle = true;
     user->width = width;
     out.stats.num_prims = n;
     out.stats.ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1676,6 +1690,7 @@ void build_bvh(const std::vector<GeomDesc>& geoms, const BuildParams& prm, Build
                      prm.robust ? 1u : 0u, n);
   RTG_HIP(hipGetLastError());
   RTG_HIP(hipStreamSynchronize(s));
+  at_end.idle = true;
   S.post.wait(s);
   memcpy(&hc, S.post.words(), sizeof(hc));
   if (!trees.empty() && (hc.roots_seen != roots_expected || (hc.error & 5u)))
