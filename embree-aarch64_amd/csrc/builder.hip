@@ -1016,9 +1016,11 @@ __global__ __launch_bounds__(WT) void k_walk_top(CollapseArgs a, const uint32_t*
   for (uint32_t i = threadIdx.x; i < a.nscenes; i += WT) place(0, prims[i], WideNode{roots[i], first[i], 1u << 16, i});
   __syncthreads();
   while (true) {
+    // (each walked node may add 8 subtrees; every wave decides before any adds one)
     const uint32_t count = min(nlevel[in], TOP_SHARE);
-    // (each walked node may add 8 subtrees)
-    if (count == 0u || nsub + 8u * count > a.max_sub) break;
+    const bool last = count == 0u || nsub + 8u * count > a.max_sub;
+    __syncthreads();
+    if (last) break;
     for (uint32_t i = threadIdx.x / CG; i < count; i += WT / CG) {
       const WideNode w = level[in][i];
       walk_node(

@@ -1,4 +1,5 @@
-"""Builds that share a device's scratch memory with other threads' builds."""
+"""Builds that share a device's scratch memory with other threads' builds, and
+the walk of a tree whose top has nearly as many subtrees as there is room for."""
 import threading
 
 import numpy as np
@@ -47,3 +48,80 @@ def test_builds_beside_builds_without_a_valid_primitive(rtc, device, oracle, qua
         stop.set()
         other.join()
     assert not bad
+
+
+def clusters():
+    """The centres of 250 clusters on a grid, and a mesh of them: dense ones, each
+    with three small groups beside it that a split takes off first."""
+    rng = np.random.default_rng(9)
+    x = np.array([0, 1, 3, 4, 9, 10, 12, 13])  # (pairs, pairs of pairs, ...: every split lies between clusters)
+    at = np.stack(np.meshgrid(x, x, x[:4], indexing="ij"), -1).reshape(-1, 3)[:250]
+    beside = np.array([[0.25, 0.0, 0.0], [0.0, 0.25, 0.0], [-0.2, 0.0, 0.2]])
+    parts = []
+    for c in at:
+        parts.append(c + (rng.random((2380, 3)) - 0.5) * 0.01)
+        for b in beside:
+            parts.append(c + b + (rng.random((12, 3)) - 0.5) * 0.005)
+    p = np.concatenate(parts)
+    v = p[:, None, :] + (rng.random((len(p), 3, 3)) - 0.5) * 0.002
+    return at, v.reshape(-1, 3).astype(np.float32), np.arange(3 * len(p), dtype=np.uint32).reshape(-1, 3)
+
+
+def walk(nodes, tris):
+    """The level sizes of the tree's top and the subtrees there are before each,
+    as the collapse walks it (nodes of more than a 256th of the primitives, and
+    of more than 2048, are walked; the others are subtrees)."""
+    N = nodes.reshape(-1, 80)
+    base = N[:, 16:24].copy().view(np.uint32)
+    flags = tris.view(np.uint32).reshape(-1, 12)[:, 11]
+    ends = np.nonzero(flags & 1)[0]
+    n = len(flags)
+    size = np.zeros(len(N), np.int64)
+    kids = []
+    for i in range(len(N) - 1, -1, -1):  # (children follow their parents)
+        k = []
+        for m in N[i, 24:32]:
+            if m & 0x80:
+                k.append(int(base[i, 0]) + int(m & 0x7f))
+                size[i] += size[k[-1]]
+            elif m:
+                first = int(base[i, 1]) + int(m) - 1
+                size[i] += ends[np.searchsorted(ends, first)] - first + 1
+        kids.append(k)
+    kids.reverse()
+    assert size[0] == n
+    share = max(n // 256, 2048)
+    level, subs, out = [0], 0, []
+    while level:
+        out.append((len(level), subs))
+        children = [c for i in level for c in kids[i]]
+        level = [c for c in children if size[c] > share]
+        subs += len(children) - len(level)
+    return out + [(0, subs)]
+
+
+def test_top_walk_near_its_room_for_subtrees(rtc, oracle):
+    room = 2047  # subtrees of a build of one scene
+    dev = rtc.Device("bvh_width=2")
+    at, v, ix = clusters()
+    sc = rtc.Scene(dev, [(v, ix)]).commit()
+    nodes, tris = sc.read_bvh()
+    levels = walk(nodes, tris)
+    # a level that is walked, while its own subtrees leave too little room for as many again
+    assert any(subs + 8 * count <= room < then + 8 * count for (count, subs), (_, then) in zip(levels, levels[1:])), levels
+    # and one that is left as subtrees
+    assert any(count and subs + 8 * count > room for count, subs in levels), levels
+    prims = tris.view(np.uint32).reshape(-1, 12)[:, 3]
+    assert np.array_equal(np.sort(prims), np.arange(len(ix)))
+    rays = rtc.gen_random_rays(50000, seed=6, lo=0.0, hi=13.0)
+    rng = np.random.default_rng(10)
+    to = at[rng.integers(len(at), size=len(rays))] + (rng.random((len(rays), 3)) - 0.5) * 0.01
+    for k, axis in enumerate("xyz"):
+        rays[f"dir_{axis}"] = to[:, k] - rays[f"org_{axis}"]
+    want, out = rays.copy(), rays.copy()
+    oracle.BVH([(v, ix)]).intersect(want)
+    sc.intersect1M(out)
+    assert (want["geomID"] == 0).sum() > 10000
+    assert len(mismatches(out, want)) == 0
+    sc.release()
+    dev.release()
