@@ -727,18 +727,18 @@ void upload_geometry(Scene* sc, Device* d, ThreadDev& t, uint32_t scene, uint32_
   // buffers of the last commit are used again where they fit (an allocation of
   // this size, and the synchronisation of freeing the old one, cost more than
   // the copy on small scenes)
-  std::vector<rtg::DevBuf*> old;
-  old.swap(sc->gdata);
+  std::vector<std::unique_ptr<rtg::DevBuf>> old(sc->gdata.size());
+  for (size_t i = 0; i < old.size(); i++) old[i].reset(sc->gdata[i]);
+  sc->gdata.clear();
   sc->descs.clear();
   size_t used = 0;
   auto buffer = [&](size_t bytes) {
-    auto* b = used < old.size() ? old[used] : new rtg::DevBuf();
-    if (used < old.size()) old[used] = nullptr;
+    auto b = used < old.size() ? std::move(old[used]) : std::make_unique<rtg::DevBuf>();
     used++;
-    sc->gdata.push_back(b);
     if (b->bytes > 2 * bytes + (size_t(1) << 20)) b->release();
     b->reserve(bytes);
-    return b;
+    sc->gdata.push_back(b.get());
+    return b.release();
   };
   for (size_t id = 0; id < sc->geoms.size(); id++) {
     Geometry* g = sc->geoms[id];
@@ -767,7 +767,6 @@ void upload_geometry(Scene* sc, Device* d, ThreadDev& t, uint32_t scene, uint32_
     sc->descs.push_back(gd);
     out.push_back(gd);
   }
-  for (auto* b : old) delete b;
 }
 
 // ------------------------------------------------------------ instances --

@@ -1,5 +1,7 @@
-"""Builds that share a device's scratch memory with other threads' builds, and
-the walk of a tree whose top has nearly as many subtrees as there is room for."""
+"""Builds that share a device's scratch memory with other threads' builds,
+the walk of a tree whose top has nearly as many subtrees as there is room for,
+and commits that the memory monitor refuses."""
+import ctypes
 import threading
 
 import numpy as np
@@ -123,5 +125,37 @@ def test_top_walk_near_its_room_for_subtrees(rtc, oracle):
     sc.intersect1M(out)
     assert (want["geomID"] == 0).sum() > 10000
     assert len(mismatches(out, want)) == 0
+    sc.release()
+    dev.release()
+
+
+def test_refused_commits_keep_no_memory(rtc):
+    # the memory monitor refuses every other commit at its first, second, ... call
+    dev = rtc.Device("")
+    L = rtc.lib()
+    hip = ctypes.CDLL("libamdhip64.so")
+    left = [0]
+
+    @ctypes.CFUNCTYPE(ctypes.c_bool, ctypes.c_void_p, ctypes.c_ssize_t, ctypes.c_bool)
+    def monitor(_, size, post):
+        left[0] -= 1
+        return left[0] != 0
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    L.rtcSetDeviceMemoryMonitorFunction(dev.h, monitor, None)
+    sc = rtc.Scene(dev, [rtc.gen_soup(200000, seed=k) for k in range(3)]).commit()
+    start = None
+    for refused in (1, 2, 3, 1, 2, 3, 1, 2, 3):
+        left[0] = refused
+        L.rtcCommitScene(sc.h)
+        assert L.rtcGetDeviceError(dev.h) == rtc.RTC_ERROR_OUT_OF_MEMORY
+        left[0] = 0
+        sc.commit()
+        start = start or free()
+    assert start - free() < 8 << 20  # (a mesh's buffers are 10 MB)
     sc.release()
     dev.release()
