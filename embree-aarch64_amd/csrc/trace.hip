@@ -440,8 +440,9 @@ __device__ inline bool push_near_to_far(const NodeHit& h, Stack& stack, int& smi
   return true;
 }
 
-// A ray's best hit: none while geom is the invalid ID. u = un / dn and
-// v = vn / dn are divided when the hit is written: nearly every step of a wave
+// A ray's best hit: none while geom is the invalid ID. (The first one is taken
+// whatever its distance, which is NaN where T and |den| both overflow.) u = un / dn
+// and v = vn / dn are divided when the hit is written: nearly every step of a wave
 // improves some lane's hit, and would run the two divisions for it.
 struct Hit {
   float t, un, vn, dn, ngx, ngy, ngz;
@@ -624,7 +625,7 @@ __global__ __launch_bounds__(TB) void k_trace(DevScene sc, char* __restrict__ ra
             occluded = true;
             break;
           }
-          const bool better = h.t < best.t ||
+          const bool better = best.geom == 0xffffffffu || h.t < best.t ||
                               (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim)));
           if (better) {
             best.t = h.t;
@@ -835,8 +836,7 @@ __global__ __launch_bounds__(TB, LDS_SLOTS > 12 ? 5 : TRACE_MIN_BLOCKS) void k_t
             *reinterpret_cast<float*>((BATCH ? lrp : rays + (uint64_t)ray * stride) + 32) = -INFINITY;
             cur = REF_DONE;
           } else {
-            // (a hit's geometry ID is below the initial one)
-            const bool better = h.t < best.t ||
+            const bool better = best.geom == 0xffffffffu || h.t < best.t ||
                                 (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim)));
             if (better) {
               best.t = h.t;
@@ -1008,7 +1008,7 @@ __global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ 
           break;
         }
       } else {
-        if (valid && (h.t < best.t ||
+        if (valid && (best.geom == 0xffffffffu || h.t < best.t ||
                       (h.t == best.t && (h.geom < best.geom || (h.geom == best.geom && h.prim < best.prim))))) {
           best.t = h.t;
           best.un = h.un; best.vn = h.vn; best.dn = h.dn;
@@ -1044,19 +1044,22 @@ __global__ __launch_bounds__(64) void k_trace_g(DevScene sc, char* __restrict__ 
     return;
   }
   // the least (t, geomID, primID) of the group; a lane that holds it writes it
-  // (two may hold the same triangle, reached through two leaves)
-  float t = best.t;
+  // (two may hold the same triangle, reached through two leaves). Distances as
+  // ordered integers: NaN after every number, and a lane without a hit last.
+  int t = __float_as_int(best.t + 0.0f);
+  t = best.t != best.t || best.geom == 0xffffffffu ? 0x7fffffff : t ^ ((t >> 31) & 0x7fffffff);
+  const int mine = t;
   uint32_t geom = best.geom, prim = best.prim;
-  auto least = [&](float t2, uint32_t g2, uint32_t p2) {
+  auto least = [&](int t2, uint32_t g2, uint32_t p2) {
     const bool less = t2 < t || (t2 == t && (g2 < geom || (g2 == geom && p2 < prim)));
     t = less ? t2 : t;
     geom = less ? g2 : geom;
     prim = less ? p2 : prim;
   };
-  least(__uint_as_float(gx1(__float_as_uint(t))), gx1(geom), gx1(prim));
-  least(__uint_as_float(gx2(__float_as_uint(t))), gx2(geom), gx2(prim));
-  least(__uint_as_float(gx7(__float_as_uint(t))), gx7(geom), gx7(prim));
-  if (best.geom != 0xffffffffu && best.t == t && best.geom == geom && best.prim == prim) {
+  least((int)gx1((uint32_t)t), gx1(geom), gx1(prim));
+  least((int)gx2((uint32_t)t), gx2(geom), gx2(prim));
+  least((int)gx7((uint32_t)t), gx7(geom), gx7(prim));
+  if (best.geom != 0xffffffffu && mine == t && best.geom == geom && best.prim == prim) {
     float* f = reinterpret_cast<float*>(rp);
     uint32_t* u = reinterpret_cast<uint32_t*>(rp);
     f[8] = best.t;
@@ -1202,7 +1205,7 @@ __global__ __launch_bounds__(TB, 5) void k_trace_inst(DevTop top, char* __restri
             cur = REF_IDLE;
           } else {
             const bool better =
-                h.t < best.t ||
+                best.geom == 0xffffffffu || h.t < best.t ||
                 (h.t == best.t &&
                  (inst < best_inst ||
                   (inst == best_inst &&
