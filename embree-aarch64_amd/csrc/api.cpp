@@ -186,12 +186,10 @@ struct RunningQueries {
   std::vector<Entry> list;
   uint64_t count = 0, any = 0;  // queries so far; the last one that may read any tree
   bool captured = false;        // a graph with queries may be replayed at any time
-  // A query was queued on `stream`, of one tree (null: of several, a two-level one).
-  void note(hipStream_t stream, const void* tree) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    RTG_HIP(hipStreamIsCapturing(stream, &cs));
+  // A query was queued or captured, of one tree (null: of several, a two-level one).
+  void note(const void* tree, bool capturing) {
     std::lock_guard<std::mutex> g(mtx);
-    if (cs != hipStreamCaptureStatusNone) captured = true;
+    captured = captured || capturing;
     count++;
     for (Entry& e : list)
       if (e.tree == tree) {
@@ -224,7 +222,25 @@ struct ThreadDev {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   rtg::PinnedBuf small;    // records of small queries in host memory, which the kernel reads and writes in place
   std::unique_ptr<HostLane> lane;  // of large ones
-  rtg::RaySorter sorter;
+  rtg::RaySorter sorter;   // of the queries on `stream`
+  // Queries on other streams may overlap each other, so each stream has its own
+  // ray counters (2 KB); beyond MAX streams the one not used for longest gives
+  // its own back, which waits for the device. Captured queries share theirs.
+  static constexpr size_t MAX_STREAMS = 16;
+  std::vector<std::pair<hipStream_t, std::unique_ptr<rtg::RaySorter>>> foreign;  // last used first
+  rtg::RaySorter captured;
+  rtg::RaySorter& sorter_of(hipStream_t s, bool capturing) {
+    if (capturing) return captured;
+    if (s == stream) return sorter;
+    size_t i = 0;
+    while (i < foreign.size() && foreign[i].first != s) i++;
+    if (i == foreign.size()) {
+      if (i == MAX_STREAMS) foreign.pop_back(), i--;
+      foreign.emplace_back(s, std::make_unique<rtg::RaySorter>());
+    }
+    std::rotate(foreign.begin(), foreign.begin() + i, foreign.begin() + i + 1);
+    return *foreign[0].second;
+  }
   rtg::DevBuf batch, batch_counter;  // batched traversal: stream table, work counter
 };
 
@@ -271,6 +287,7 @@ struct Device : RefObj {
     RTG_HIP(hipEventCreate(&t->ev0));
     RTG_HIP(hipEventCreate(&t->ev1));
     t->errword.reserve(256);
+    t->captured.counter.reserve(rtg::COUNTER_BYTES);
     *t->errword.as<uint32_t>() = 0;
     threads[std::this_thread::get_id()] = t;
     return *t;
@@ -999,9 +1016,15 @@ void launch_scene(Scene* sc, ThreadDev& t, void* rays, unsigned M, size_t stride
   launch_scene(sc, t.errword.as<uint32_t>(), t.sorter, rays, M, stride, occluded, inst, stream, tp);
 }
 
-// An asynchronous query of the scene was queued on `stream`.
-void note_query(Scene* sc, hipStream_t stream) {
-  if (!scene_empty(sc)) sc->dev->running.note(stream, sc->two_level ? nullptr : (const void*)sc->bvh.get());
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  RTG_HIP(hipStreamIsCapturing(stream, &cs));
+  return cs != hipStreamCaptureStatusNone;
+}
+
+// An asynchronous query of the scene was queued (or captured).
+void note_query(Scene* sc, bool captured) {
+  if (!scene_empty(sc)) sc->dev->running.note(sc->two_level ? nullptr : (const void*)sc->bvh.get(), captured);
 }
 
 void single_level_only(Scene* sc, const char* what) {
@@ -1824,8 +1847,11 @@ static void async_trace(Scene* s, const RTCIntersectContext* ctx, void* rays, un
   ThreadDev& t = d->td();
   const uint32_t inst = ctx ? ctx->instID[0] : RTC_INVALID_GEOMETRY_ID;
   const hipStream_t st = stream ? (hipStream_t)stream : t.stream;
-  launch_scene(s, t, rays, M, stride, occluded, inst, st, d->trace_params());
-  note_query(s, st);
+  const bool cap = capturing(st);
+  rtg::TraceParams tp = d->trace_params();
+  if (cap) tp.sort_rays = 0;  // (no memory can be allocated for it)
+  launch_scene(s, t.errword.as<uint32_t>(), t.sorter_of(st, cap), rays, M, stride, occluded, inst, st, tp);
+  note_query(s, cap);
 }
 
 RTC_API void rtcgIntersect1MAsync(RTCScene scene, const RTCIntersectContext* context, RTCRayHit* d_rayhit,
@@ -1880,7 +1906,7 @@ RTC_API void rtcgQuery1MNoAlloc(RTCScene scene, const RTCIntersectContext* conte
                       st, tp, nullptr, nullptr, scr);
   }
   if (hipStream) {
-    note_query(s, st);
+    note_query(s, capturing(st));
     return;
   }
   RTG_HIP(hipStreamSynchronize(st));

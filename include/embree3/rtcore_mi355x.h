@@ -21,7 +21,9 @@ RTC_API void rtcgMemcpy(RTCDevice device, void* dst, const void* src, size_t byt
 /* Same contract as rtcIntersect1M / rtcOccluded1M, but the records live in
  * device memory and the call is asynchronous on `hipStream` (a hipStream_t;
  * NULL selects the calling thread's stream of this device). A commit of the
- * scene waits for the queries queued before it, which see the old geometry. */
+ * scene waits for the queries queued before it, which see the old geometry.
+ * Queries on several streams may overlap; those that one thread captured in
+ * graphs share their ray counters, so replays of its graphs must not. */
 RTC_API void rtcgIntersect1MAsync(RTCScene scene, const struct RTCIntersectContext* context, struct RTCRayHit* d_rayhit,
                                   unsigned int M, size_t byteStride, void* hipStream);
 RTC_API void rtcgOccluded1MAsync(RTCScene scene, const struct RTCIntersectContext* context, struct RTCRay* d_ray,

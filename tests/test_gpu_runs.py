@@ -192,3 +192,64 @@ def test_every_record_of_a_batch(rtc, device, scene, n):
     device.free(d)
     for s in scs:
         s.release()
+
+
+def test_queries_that_overlap_on_several_streams(rtc, device, scene):
+    # one thread, more streams than keep ray counters of their own, each with a
+    # closest-hit and an occlusion query too large for the waves' first runs
+    sc, rays, hits, shadow, dark = scene
+    hip = ctypes.CDLL("libamdhip64.so")
+    L, ctx, made = rtc.lib(), rtc.init_context(), []
+    for k in range(20):
+        s = ctypes.c_void_p()
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+        bufs = []
+        for src in (rays, shadow):
+            d = device.malloc(src.nbytes)
+            device.memcpy(d, src.ctypes.data, src.nbytes)
+            bufs.append(d)
+        made.append((s, bufs))
+    for s, (a, b) in made:
+        L.rtcgIntersect1MAsync(sc.h, ctypes.byref(ctx), a, len(rays), 80, s)
+        L.rtcgOccluded1MAsync(sc.h, ctypes.byref(ctx), b, len(shadow), 48, s)
+    device.check("queries")
+    for s, bufs in made:
+        assert hip.hipStreamSynchronize(s) == 0
+        for d, ref in zip(bufs, (hits, dark)):
+            out = np.empty_like(ref)
+            device.memcpy(out.ctypes.data, d, out.nbytes)
+            assert len(mismatches(out, ref)) == 0
+            device.free(d)
+        assert hip.hipStreamDestroy(s) == 0
+
+
+def test_captured_query(rtc, device, scene):
+    # captured on a stream of its own after a query on another one, replayed
+    # with eager queries between
+    sc, rays, hits, _, _ = scene
+    hip = ctypes.CDLL("libamdhip64.so")
+    L, ctx = rtc.lib(), rtc.init_context()
+    d, src = device.malloc(rays.nbytes), device.malloc(rays.nbytes)
+    device.memcpy(src, rays.ctypes.data, rays.nbytes)
+    s, graph, run = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+    assert hip.hipStreamBeginCapture(s, 2) == 0  # hipStreamCaptureModeRelaxed
+    L.rtcgIntersect1MAsync(sc.h, ctypes.byref(ctx), d, len(rays), 80, s)
+    assert hip.hipStreamEndCapture(s, ctypes.byref(graph)) == 0
+    device.check("capture")
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        device.memcpy(d, src, rays.nbytes)
+        assert hip.hipGraphLaunch(run, s) == 0
+        assert hip.hipStreamSynchronize(s) == 0
+        out = np.empty_like(rays)
+        device.memcpy(out.ctypes.data, d, out.nbytes)
+        assert len(mismatches(out, hits)) == 0
+        eager = rays[:100000].copy()
+        sc.intersect1M(eager)
+        assert len(mismatches(eager, hits[:100000])) == 0
+    assert hip.hipGraphExecDestroy(run) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamDestroy(s) == 0
+    device.free(d)
+    device.free(src)
