@@ -179,15 +179,15 @@ struct HostPool {
 struct RunningQueries {
   static constexpr size_t MAX = 64;
   struct Entry {
-    const void* tree;
+    uint64_t tree;  // DeviceBVH::id
     uint64_t last;  // number of its last query
   };
   std::mutex mtx;
   std::vector<Entry> list;
   uint64_t count = 0, any = 0;  // queries so far; the last one that may read any tree
   bool captured = false;        // a graph with queries may be replayed at any time
-  // A query was queued or captured, of one tree (null: of several, a two-level one).
-  void note(const void* tree, bool capturing) {
+  // A query was queued or captured, of one tree (0: of several, a two-level one).
+  void note(uint64_t tree, bool capturing) {
     std::lock_guard<std::mutex> g(mtx);
     captured = captured || capturing;
     count++;
@@ -200,7 +200,7 @@ struct RunningQueries {
     else any = count;
   }
   // What the caller does next may write `tree`.
-  void wait(const void* tree) {
+  void wait(uint64_t tree) {
     uint64_t now;
     {
       std::lock_guard<std::mutex> g(mtx);
@@ -645,7 +645,7 @@ rtg::BuildParams scene_params(Scene* sc, rtg::LearnedCost& lc, const rtg::BuildP
 // of split at every node, kernels/builders/heuristic_spatial_array.h).
 void build_scene_tree(Scene* sc, Device* d, const std::vector<rtg::GeomDesc>& descs, const rtg::BuildParams& p,
                       hipStream_t st) {
-  rtg::build_bvh(descs, p, d->scratch, *sc->bvh, st, 1, nullptr, [&] { d->running.wait(sc->bvh.get()); });
+  rtg::build_bvh(descs, p, d->scratch, *sc->bvh, st, 1, nullptr, [&] { d->running.wait(sc->bvh->id); });
   if (sc->bvh->stats.num_split == 0) return;
   rtg::BuildParams q = p;
   q.split_budget = 0.0f;
@@ -959,7 +959,7 @@ void build_top(Scene* sc, Device* d, ThreadDev& t) {
   d->monitor((ssize_t)n * (80 + 64));
   {
     std::lock_guard<std::mutex> bl(d->build_mtx);
-    rtg::build_bvh({gd}, p, d->scratch, sc->top, t.stream, 1, nullptr, [&] { d->running.wait(&sc->top); });
+    rtg::build_bvh({gd}, p, d->scratch, sc->top, t.stream, 1, nullptr, [&] { d->running.wait(sc->top.id); });
   }
   sc->top_objects.reserve(objects.size() * sizeof(rtg::DevScene));
   RTG_HIP(hipMemcpyAsync(sc->top_objects.ptr, objects.data(), objects.size() * sizeof(rtg::DevScene),
@@ -1024,7 +1024,7 @@ bool capturing(hipStream_t stream) {
 
 // An asynchronous query of the scene was queued (or captured).
 void note_query(Scene* sc, bool captured) {
-  if (!scene_empty(sc)) sc->dev->running.note(sc->two_level ? nullptr : (const void*)sc->bvh.get(), captured);
+  if (!scene_empty(sc)) sc->dev->running.note(sc->two_level ? 0 : sc->bvh->id, captured);
 }
 
 void single_level_only(Scene* sc, const char* what) {

@@ -3,6 +3,7 @@
 // top-down collapse into quantised 8-wide nodes and Moeller-ready triangle
 // records.
 #pragma once
+#include <atomic>
 #include <functional>
 #include <vector>
 
@@ -57,6 +58,11 @@ struct SceneSlot {
 // Owns the device arrays of one build: one scene, or every scene of a
 // batched build (they share the node and triangle arrays).
 struct DeviceBVH {
+  const uint64_t id = new_id();  // of no other tree of the process
+  static uint64_t new_id() {
+    static std::atomic<uint64_t> last{0};
+    return ++last;
+  }
   DevBuf nodes, tris, info;
   DevBuf insts;            // leaf records of an instance build (then tris is empty)
   bool instances = false;
