@@ -88,6 +88,10 @@ struct DeviceBVH {
   bool empty(uint32_t slot = 0) const { return stats.num_nodes == 0 || slot >= slots.size() || slots[slot].num_prims == 0; }
   BuildStats stats;  // of the whole build
   uint32_t robust = 0;
+  size_t bytes() const { return nodes.bytes + tris.bytes + info.bytes + insts.bytes; }
+  void release() {
+    for (DevBuf* b : {&nodes, &tris, &info, &insts}) b->release();
+  }
   // Exchanges the trees of two builds (a new generation for both).
   void swap_tree(DeviceBVH& o) {
     nodes.swap(o.nodes);

@@ -1,6 +1,6 @@
 """Builds that share a device's scratch memory with other threads' builds,
 the walk of a tree whose top has nearly as many subtrees as there is room for,
-and commits that the memory monitor refuses."""
+commits that the memory monitor refuses, and what HIGH commits keep."""
 import ctypes
 import threading
 
@@ -159,3 +159,28 @@ def test_refused_commits_keep_no_memory(rtc):
     assert start - free() < 8 << 20  # (a mesh's buffers are 10 MB)
     sc.release()
     dev.release()
+
+
+def test_high_commits_give_the_other_tree_back(rtc):
+    # what a device keeps after a HIGH commit of a large mesh is what a MEDIUM
+    # commit of as many references keeps, and the split's own scratch
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    def kept(n, quality):
+        dev = rtc.Device("")
+        sc = rtc.Scene(dev, [rtc.gen_soup(n, seed=1, h=0.02)], quality=quality).commit()
+        sc.release()
+        before = free()
+        dev.release()
+        return free() - before
+
+    n = 3000000
+    high = kept(n, rtc.RTC_BUILD_QUALITY_HIGH)
+    # (at most 1.3 n references are built over, and 48 bytes a triangle are the split's)
+    medium = kept(int(1.3 * n), rtc.RTC_BUILD_QUALITY_MEDIUM)
+    assert high < medium + 48 * n + (200 << 20)  # (a second tree has 208 bytes a triangle, 620 MB)
