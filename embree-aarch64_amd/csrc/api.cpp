@@ -19,10 +19,10 @@
 #include <condition_variable>
 #include <exception>
 #include <functional>
+#include <list>
 #include <memory>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -107,15 +107,36 @@ struct HostPool {
   std::mutex mtx;
   std::condition_variable wake, done;
   std::vector<Job*> jobs;  // with open places
-  std::vector<std::thread> threads;
+  struct Helper {
+    std::thread thread;
+    bool ended = false;  // without a stream or memory
+  };
+  std::list<Helper> helpers;
   bool stop = false;
-  void submit(Job& job, size_t helpers, int ordinal) {
+  void submit(Job& job, size_t wanted, int ordinal) {
     std::lock_guard<std::mutex> g(mtx);
-    job.open = std::min(helpers, MAX);
+    job.open = std::min(wanted, MAX);
     jobs.push_back(&job);
+    for (auto h = helpers.begin(); h != helpers.end();) {
+      if (h->ended) {
+        h->thread.join();  // (it takes no lock any more)
+        h = helpers.erase(h);
+      } else {
+        ++h;
+      }
+    }
     try {
-      while (threads.size() < job.open) threads.emplace_back([this, ordinal] { serve(ordinal); });
-    } catch (const std::system_error&) {  // no more threads: the caller does what they would have done
+      while (helpers.size() < job.open) {
+        helpers.emplace_back();
+        Helper& h = helpers.back();
+        try {
+          h.thread = std::thread([this, &h, ordinal] { serve(h, ordinal); });
+        } catch (...) {
+          helpers.pop_back();
+          throw;
+        }
+      }
+    } catch (...) {  // no more threads: the caller does what they would have done
     }
     wake.notify_all();
   }
@@ -124,7 +145,7 @@ struct HostPool {
     jobs.erase(std::remove(jobs.begin(), jobs.end(), &job), jobs.end());
     done.wait(g, [&] { return job.active == 0; });
   }
-  void serve(int ordinal) {
+  void serve(Helper& self, int ordinal) {
     std::unique_ptr<HostLane> lane;
     std::unique_lock<std::mutex> g(mtx);
     while (true) {
@@ -139,7 +160,11 @@ struct HostPool {
         }
         prepare(*lane);
       } catch (...) {
-        return;  // no stream or memory for a helper: the others do its part
+        // no stream or memory for a helper: the others do its part, and a later
+        // job starts another
+        std::lock_guard<std::mutex> l(mtx);
+        self.ended = true;
+        return;
       }
       g.lock();
       if (stop) return;
@@ -165,7 +190,7 @@ struct HostPool {
       stop = true;
     }
     wake.notify_all();
-    for (auto& t : threads) t.join();
+    for (auto& h : helpers) h.thread.join();
   }
 };
 
@@ -654,9 +679,8 @@ void build_scene_tree(Scene* sc, Device* d, const std::vector<rtg::GeomDesc>& de
   q.split_budget = 0.0f;
   // The arrays of the tree that is not kept stay for the next such commit if
   // they are no larger than OTHER_KEPT (2.5 M references), and are used again if
-  // they are not much larger than this one's: their allocation costs commits of
-  // 2^20 triangles 3 of 11 ms. Larger ones are given back (3 M triangles: 620 MB,
-  // 27 ms instead of 19).
+  // they are not much larger than this one's. Larger ones are given back (commits
+  // of 3 M triangles take 27 ms with that, 19 with the arrays kept).
   struct GiveBack {
     rtg::DeviceBVH& b;
     ~GiveBack() {
