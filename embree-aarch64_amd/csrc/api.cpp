@@ -195,29 +195,47 @@ struct HostPool {
 };
 
 // Asynchronous queries that may still run. A commit writes a tree's arrays in
-// place, so before that it waits for the device if a query of that tree was
-// queued since the last such wait; what it does before only uses scratch memory
-// and overlaps the query. (An event after each query, for the commit's stream to
-// wait on, costs every query: 1073 camera rays on a 131 k triangle terrain, call
-// after call, 38 us instead of 33. The wait costs a mesh of 20,000 triangles
-// that is committed and traced every frame 3 of 280 us, at the start of the
-// commit 21.)
+// place, so before that it waits for the queries of that tree; what it does
+// before only uses scratch memory and overlaps them. After a query of a scene
+// that was committed again before, an event is recorded, which the commit's
+// stream waits on. That costs every query (1073 camera rays on a 131 k triangle
+// terrain, call after call, 38 us instead of 33), so queries of other scenes are
+// only noted, and the first commit after them waits for the device once (every
+// time, that costs a frame of 280 us 3 to 70, more with each stream there is).
 struct RunningQueries {
-  static constexpr size_t MAX = 64;
-  struct Entry {
+  struct Noted {
     uint64_t tree;  // DeviceBVH::id
     uint64_t last;  // number of its last query
   };
+  struct Event {
+    hipStream_t stream = nullptr;
+    uint64_t tree = 0;  // 0: any (a two-level query reads several)
+    hipEvent_t ev = nullptr;
+    bool used = false;
+  };
+  static constexpr size_t MAX = 64, EVENTS = 16;
   std::mutex mtx;
-  std::vector<Entry> list;
-  uint64_t count = 0, any = 0;  // queries so far; the last one that may read any tree
+  std::vector<Noted> list;
+  Event events[EVENTS];         // made with the device, so that a query allocates nothing
+  uint64_t count = 0, any = 0;  // queries noted so far; the last one that may read any tree
   bool captured = false;        // a graph with queries may be replayed at any time
-  // A query was queued or captured, of one tree (0: of several, a two-level one).
-  void note(uint64_t tree, bool capturing) {
+  void make() {
+    // (no fence: the commit only must not write before the query has read)
+    for (Event& e : events)
+      RTG_HIP(hipEventCreateWithFlags(&e.ev, hipEventDisableTiming | hipEventDisableSystemFence));
+  }
+  ~RunningQueries() {
+    for (Event& e : events)
+      if (e.ev) (void)hipEventDestroy(e.ev);
+  }
+  // A query was queued on `stream` (or captured), of one tree (0: of several, a
+  // two-level one). again: its scene was committed more than once.
+  void note(hipStream_t stream, uint64_t tree, bool capturing, bool again) {
     std::lock_guard<std::mutex> g(mtx);
     captured = captured || capturing;
+    if (again && !capturing && record(stream, tree)) return;
     count++;
-    for (Entry& e : list)
+    for (Noted& e : list)
       if (e.tree == tree) {
         e.last = count;
         return;
@@ -225,20 +243,41 @@ struct RunningQueries {
     if (tree && list.size() < MAX) list.push_back({tree, count});
     else any = count;
   }
-  // What the caller does next may write `tree`.
-  void wait(uint64_t tree) {
+  bool record(hipStream_t stream, uint64_t tree) {
+    Event* to = nullptr;
+    // the event of the last query like this one (hipStreamPerThread is another
+    // stream in every thread; a stream's destruction waits for its work, so a
+    // handle that comes back as another stream's loses none)
+    for (Event& e : events)
+      if (e.used && e.stream == stream && e.tree == tree && stream != hipStreamPerThread) to = &e;
+    for (Event& e : events) {
+      if (to) break;
+      if (!e.used || hipEventQuery(e.ev) == hipSuccess) to = &e;
+    }
+    (void)hipGetLastError();  // (of a query that found its event still to come)
+    if (!to) return false;
+    RTG_HIP(hipEventRecord(to->ev, stream));
+    to->stream = stream;
+    to->tree = tree;
+    to->used = true;
+    return true;
+  }
+  // What the caller queues next on `stream` may write `tree`.
+  void wait(hipStream_t stream, uint64_t tree) {
     uint64_t now;
     {
       std::lock_guard<std::mutex> g(mtx);
+      for (const Event& e : events)
+        if (e.used && e.stream != stream && (!e.tree || e.tree == tree)) RTG_HIP(hipStreamWaitEvent(stream, e.ev, 0));
       bool must = captured || any != 0;
-      for (const Entry& e : list) must = must || e.tree == tree;
+      for (const Noted& e : list) must = must || e.tree == tree;
       if (!must) return;
       now = count;
     }
     RTG_HIP(hipDeviceSynchronize());
     std::lock_guard<std::mutex> g(mtx);
     if (any <= now) any = 0;
-    list.erase(std::remove_if(list.begin(), list.end(), [&](const Entry& e) { return e.last <= now; }), list.end());
+    list.erase(std::remove_if(list.begin(), list.end(), [&](const Noted& e) { return e.last <= now; }), list.end());
   }
 };
 
@@ -462,6 +501,7 @@ struct Scene : RefObj {
   RTCProgressMonitorFunction progress = nullptr;
   void* progress_ptr = nullptr;
   bool committed = false;
+  uint64_t commits = 0;
   std::mutex mtx;
   std::shared_ptr<rtg::DeviceBVH> bvh = std::make_shared<rtg::DeviceBVH>();  // shared by the scenes of a batch
   uint32_t slot = 0;                                                          // this scene's slot in bvh
@@ -673,7 +713,7 @@ constexpr size_t OTHER_KEPT = size_t(512) << 20;
 
 void build_scene_tree(Scene* sc, Device* d, const std::vector<rtg::GeomDesc>& descs, const rtg::BuildParams& p,
                       hipStream_t st) {
-  rtg::build_bvh(descs, p, d->scratch, *sc->bvh, st, 1, nullptr, [&] { d->running.wait(sc->bvh->id); });
+  rtg::build_bvh(descs, p, d->scratch, *sc->bvh, st, 1, nullptr, [&] { d->running.wait(st, sc->bvh->id); });
   if (sc->bvh->stats.num_split == 0) return;
   rtg::BuildParams q = p;
   q.split_budget = 0.0f;
@@ -999,7 +1039,7 @@ void build_top(Scene* sc, Device* d, ThreadDev& t) {
   d->monitor((ssize_t)n * (80 + 64));
   {
     std::lock_guard<std::mutex> bl(d->build_mtx);
-    rtg::build_bvh({gd}, p, d->scratch, sc->top, t.stream, 1, nullptr, [&] { d->running.wait(sc->top.id); });
+    rtg::build_bvh({gd}, p, d->scratch, sc->top, t.stream, 1, nullptr, [&] { d->running.wait(t.stream, sc->top.id); });
   }
   sc->top_objects.reserve(objects.size() * sizeof(rtg::DevScene));
   RTG_HIP(hipMemcpyAsync(sc->top_objects.ptr, objects.data(), objects.size() * sizeof(rtg::DevScene),
@@ -1062,9 +1102,9 @@ bool capturing(hipStream_t stream) {
   return cs != hipStreamCaptureStatusNone;
 }
 
-// An asynchronous query of the scene was queued (or captured).
-void note_query(Scene* sc, bool captured) {
-  if (!scene_empty(sc)) sc->dev->running.note(sc->two_level ? 0 : sc->bvh->id, captured);
+// An asynchronous query of the scene was queued on `stream` (or captured).
+void note_query(Scene* sc, hipStream_t stream, bool captured) {
+  if (!scene_empty(sc)) sc->dev->running.note(stream, sc->two_level ? 0 : sc->bvh->id, captured, sc->commits > 1);
 }
 
 void single_level_only(Scene* sc, const char* what) {
@@ -1095,6 +1135,7 @@ void commit_scene(Scene* sc) {
   RTG_HIP(hipStreamSynchronize(t.stream));
   build_top(sc, d, t);
   sc->committed = true;
+  sc->commits++;
   if (sc->progress && !sc->progress(sc->progress_ptr, 1.0)) RTC_THROW(RTC_ERROR_CANCELLED, "progress monitor forced termination");
 }
 
@@ -1120,7 +1161,9 @@ void check_trace_error(ThreadDev& t) {
 }
 
 // Rays up to which a query in host memory is traced in place in pinned memory
-// (one ray 17 us, 43 with copies; 4000 rays 100 us in place, 106 in chunks), and
+// (one ray 17 us, 43 with copies; 4000 rays 100 us in place, 106 in chunks; of
+// 1000 instances, whose kernel keeps the best hit in the record, 26 us against 30
+// and 8192 rays 236 us either way), and
 // records of a chunk of a larger one: each costs about 60 us of launches beside
 // its transfers, and there are a few for every thread.
 constexpr size_t SMALL_RAYS = 8192, HOST_CHUNK_MIN = 16384, HOST_CHUNK_MAX = 65536;
@@ -1239,6 +1282,7 @@ RTC_API RTCDevice rtcNewDevice(const char* config) {
   }
   d->activate();
   rtg::noalloc_setup(d->ordinal);
+  d->running.make();
   {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, d->ordinal) == hipSuccess && prop.multiProcessorCount > 0)
@@ -1901,7 +1945,7 @@ static void async_trace(Scene* s, const RTCIntersectContext* ctx, void* rays, un
   rtg::TraceParams tp = d->trace_params();
   if (cap) tp.sort_rays = 0;  // (no memory can be allocated for it)
   launch_scene(s, t.errword.as<uint32_t>(), t.sorter_of(st, cap), rays, M, stride, occluded, inst, st, tp);
-  note_query(s, cap);
+  note_query(s, st, cap);
 }
 
 RTC_API void rtcgIntersect1MAsync(RTCScene scene, const RTCIntersectContext* context, RTCRayHit* d_rayhit,
@@ -1956,7 +2000,7 @@ RTC_API void rtcgQuery1MNoAlloc(RTCScene scene, const RTCIntersectContext* conte
                       st, tp, nullptr, nullptr, scr);
   }
   if (hipStream) {
-    note_query(s, capturing(st));
+    note_query(s, st, capturing(st));
     return;
   }
   RTG_HIP(hipStreamSynchronize(st));
@@ -2621,6 +2665,7 @@ RTC_API void rtcgCommitScenes(RTCScene* scenes, unsigned int numScenes) {
     sc[i]->slot = i;
     build_top(sc[i], d, t);  // no instances: resets any earlier top tree
     sc[i]->committed = true;
+    sc[i]->commits++;
   }
   API_END(s0)
 }

@@ -86,14 +86,18 @@ def shared_scene(rtc, device, mesh, quality):
     return sc, change
 
 
+# a scene committed once is only noted, one committed again gets an event
+@pytest.mark.parametrize("commits", [1, 2])
 @pytest.mark.parametrize("call", ["async", "no_alloc"])
 @pytest.mark.parametrize("quality,size", [("LOW", 300), ("MEDIUM", 20000), ("HIGH", 20000)])
-def test_commit_after_a_queued_query(rtc, device, oracle, queue, quality, size, call):
+def test_commit_after_a_queued_query(rtc, device, oracle, queue, quality, size, call, commits):
     h, s, fill = queue
     v, ix = rtc.gen_soup(size, seed=7, h=0.05)
     sc, change = shared_scene(rtc, device, (v, ix), getattr(rtc, f"RTC_BUILD_QUALITY_{quality}"))
     first, second = (Records(rtc, device, 0.0, 1.0) for _ in range(2))
     want = first.expect(oracle, (v, ix))
+    for _ in range(commits - 1):
+        change(v)
     w = np.ascontiguousarray(v[::-1]) * np.float32(0.75)
     after = second.expect(oracle, (w, ix))
     L, ctx = rtc.lib(), rtc.init_context()
@@ -115,7 +119,8 @@ def test_commit_after_a_queued_query(rtc, device, oracle, queue, quality, size, 
     sc.release()
 
 
-def test_commit_of_a_two_level_scene_after_a_queued_query(rtc, device, oracle, queue):
+@pytest.mark.parametrize("commits", [1, 2])
+def test_commit_of_a_two_level_scene_after_a_queued_query(rtc, device, oracle, queue, commits):
     h, s, fill = queue
     v, ix = rtc.gen_sphere(24)
     obj = rtc.Scene(device, [(v, ix)]).commit()
@@ -137,6 +142,8 @@ def test_commit_of_a_two_level_scene_after_a_queued_query(rtc, device, oracle, q
     after = traced(other, second)
     other.release()
     top = place(0)
+    for _ in range(commits - 1):
+        top.commit()
     want = traced(top, first)
     assert len(mismatches(want, after)) > 100
     L, ctx = rtc.lib(), rtc.init_context()
@@ -160,12 +167,16 @@ def test_commit_of_a_two_level_scene_after_a_queued_query(rtc, device, oracle, q
     obj.release()
 
 
-def test_queries_of_many_scenes(rtc, device, oracle, queue):
-    """More scenes with queued queries than the library keeps apart."""
+@pytest.mark.parametrize("commits", [1, 2])
+def test_queries_of_many_scenes(rtc, device, oracle, queue, commits):
+    """More scenes with queued queries than the library has events for, or
+    keeps apart."""
     h, s, fill = queue
     v, ix = rtc.gen_soup(2000, seed=8, h=0.05)
     w = np.ascontiguousarray(v[::-1])
     scenes = [shared_scene(rtc, device, (v, ix), rtc.RTC_BUILD_QUALITY_LOW) for _ in range(70)]
+    for _, change in scenes * (commits - 1):
+        change(v)
     recs = [Records(rtc, device, 0.0, 1.0) for _ in scenes]
     want = recs[0].expect(oracle, (v, ix))
     L, ctx = rtc.lib(), rtc.init_context()
