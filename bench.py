@@ -110,7 +110,7 @@ def profiled_traffic():
                 traffic = (rd + wr) * 1e9
             if line.strip().startswith("VALU instructions per ray"):
                 f = line.replace(",", " ").replace(";", " ").split()
-                limiter = {"kind": "return path of the vector memory (TD busy) and VALU issue, divergent lanes",
+                limiter = {"kind": "VALU issue and vector memory returns inside the compute units, divergent lanes",
                            "valu_instr_per_ray": float(f[4]), "salu_instr_per_ray": float(f[6]),
                            "lanes_active_per_valu_instr": float(f[f.index("instruction") + 1]),
                            "source": os.path.relpath(PROFILE, ROOT)}

@@ -9,24 +9,27 @@ namespace rtg {
 // Launch-shape parameters of the traversal (chosen per device, tunable).
 struct TraceParams {
   // LDS stack entries per lane (0: private stack, 8, 12 or 16). On the
-  // 2^20-triangle soup with 2^24 incoherent rays, closest hit: 12 gave 2398 Mrays/s, 8 2345 and 16
-  // 2089 (16 fits 5 blocks of 256 lanes per CU, 12 and 8 fit 6).
+  // 2^20-triangle soup 2^24 incoherent rays, closest hit, take 6.26 ms at 12,
+  // 6.64 at 8 and 6.92 at 16 (16 fits 5 blocks of 256 lanes per CU, 12 and 8
+  // fit 6), 14.5 with a private stack; 2^23 occlusion rays there 1.96, 2.03,
+  // 2.18 and 3.65.
   int lds_slots = 12;
   int sort_rays = 0;        // trace in origin-Morton order (a permutation; records stay in place)
   uint32_t sort_min = 65536;  // smallest stream that is reordered
   int persistent = 1;       // persistent waves pulling rays from a counter
   // Idle lanes of a wave that trigger a refill. A refill stalls the wave
   // for one ray-record load (and, once per RAY_RUN rays, a global counter's
-  // atomic). On the 2^20-triangle soup 2^24 incoherent rays take 6.71 ms at
-  // 8, 6.66 at 16, 6.80 at 32 and 7.12 at 40, the Pluecker test on a soup
-  // 1.04, 1.04, 1.11 and 1.11, camera rays on a terrain 403, 400, 420 and
-  // 425 us; 2^23 occlusion rays in the soup 2.11 ms at 8, 2.09 at 16, 2.08 at 24,
-  // 2.10 at 32 and 2.19 at 40.
+  // atomic). The line is flat: 2^24 rays in the 2^20-triangle soup take 6.24 ms
+  // at 8, 6.25 at 10, 6.28 at 16, 6.33 at 24 and 6.52 at 32; the Pluecker test
+  // on a soup (985 to 1014 us) and camera rays on a terrain (322 to 332) show no
+  // order from 6 to 20. Occlusion rays, 2^23 in the soup: 1.98 ms at 8, 1.96 at
+  // 16, 1.97 at 24, 1.99 at 32 and 2.08 at 40; camera rays on a terrain 260, 260,
+  // 256, 264 and 264 us.
   int refill_min = 10;      // closest hit
   int refill_min_occ = 24;  // occlusion rays, which finish sooner
-  // Occlusion rays through a two-level scene: two million rays through 10,000
-  // instances and their shadow rays take 2.72 ms at 8, 2.76 at 16, 2.84 at 24
-  // and 2.98 at 32 (closest hit and occlusion alike).
+  // Occlusion rays through a two-level scene: two million camera rays through
+  // 10,000 instances and their shadow rays take 2.65 ms at 6, 2.69 at 8, 2.64 at
+  // 12, 2.65 at 16, 2.68 at 20 and 2.76 at 24 (closest hit and occlusion alike).
   int refill_min_occ_inst = 12;
   int groups = 1;           // small streams with eight lanes a ray (0: one lane, as large ones)
   int cus = 256;            // compute units (set from the device)

@@ -395,9 +395,7 @@ __device__ inline bool push_any_order(const NodeHit& h, Stack& stack, uint32_t* 
 // anyway) instead of taking part in every child's slab test. (With integer
 // distances and this, 274 VALU instructions a ray instead of 290 on the
 // 2^20-triangle soup, 7.00 ms instead of 7.14 for 2^24 rays; with the lanes'
-// state in their references 229 and 6.72 ms. There the kernel is bound by the
-// return path of the vector memory, busy 96 % of the time, where every lane's
-// 16 bytes of a node are an access of their own.)
+// state in their references 229 and 6.72 ms.)
 template <class Stack>
 __device__ inline bool push_near_to_far(const NodeHit& h, Stack& stack, int& smin, float lim, uint32_t* err,
                                         uint32_t& next) {
@@ -1422,14 +1420,21 @@ void launch_slots(const LaunchArgs& a) {
   else launch_one<OCC, AL, CNT, 16, PL>(a);
 }
 
-// The largest streams that eight lanes a ray serve better (us a call, with 14
-// of launching and of making the records; eight lanes against one):
-//                                    8192      16384      32768      65536
-//   camera, 131 k terrain          49 :  75   47 :  88   58 :  86   61 :  80
-//   random, 262 k soup            143 : 247  171 : 248  194 : 253  270 : 258
-//   camera, 16 k sphere            44 :  63   43 :  66   55 :  71   68 :  72
-//   random occlusion, 262 k soup   33 :  54   41 :  53   51 :  60   83 :  64
-// From there on the GPU is full, and one lane a ray needs fewer instructions.
+// The largest streams that eight lanes a ray serve better (kernel us, eight
+// lanes against one):
+//                                      8192       32768       49152       65536
+//   camera, 131 k terrain             49 :  85   53 :  87    66 :  96    69 :  80
+//   camera, 2.1 M terrain             64 : 107   81 : 111    90 : 131    85 : 119
+//   camera, 16 k sphere               49 :  73   59 :  79    67 :  84    73 :  80
+//   random, 250 k sphere              70 : 105   86 : 116   104 : 117   111 : 127
+//   random, 2^20 soup                262 : 394  280 : 408   313 : 397   351 : 401
+//   random, 262 k soup               147 : 247  197 : 243   223 : 240   265 : 236
+//   random, 262 k soup, robust       153 : 253  193 : 255   237 : 251   277 : 250
+//   random occlusion, 262 k soup      33 :  52   53 :  57    59 :  58    59 :  59
+//   random occlusion, 2^20 soup       46 :  68   75 :  85    82 :  85    83 :  84
+//   camera occlusion, 131 k terrain   39 :  63   41 :  71    72 :  72    62 :  65
+// The GPU fills up there, and one lane a ray needs fewer instructions. At 65536
+// closest-hit rays five of seven still gain, 9 to 29 %, and two lose 11 and 12 %.
 constexpr uint32_t GROUP_MAX_RAYS = 65536, GROUP_MAX_RAYS_OCC = 32768;
 // A ray's stack is all in LDS: 256 entries are 16 KB a wave. (Trees of a few
 // million triangles need fewer than 80.)
