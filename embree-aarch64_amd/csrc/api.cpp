@@ -205,7 +205,7 @@ struct HostPool {
 struct RunningQueries {
   struct Noted {
     uint64_t tree;  // DeviceBVH::id
-    uint64_t last;  // number of its last query
+    uint64_t last;  // number of its last query, or REPLAYED
   };
   struct Event {
     hipStream_t stream = nullptr;
@@ -218,7 +218,7 @@ struct RunningQueries {
   std::vector<Noted> list;
   Event events[EVENTS];         // made with the device, so that a query allocates nothing
   uint64_t count = 0, any = 0;  // queries noted so far; the last one that may read any tree
-  bool captured = false;        // a graph with queries may be replayed at any time
+  static constexpr uint64_t REPLAYED = UINT64_MAX;  // captured in a graph, which may run at any time
   void make() {
     // (no fence: the commit only must not write before the query has read)
     for (Event& e : events)
@@ -232,16 +232,15 @@ struct RunningQueries {
   // two-level one). again: its scene was committed more than once.
   void note(hipStream_t stream, uint64_t tree, bool capturing, bool again) {
     std::lock_guard<std::mutex> g(mtx);
-    captured = captured || capturing;
     if (again && !capturing && record(stream, tree)) return;
-    count++;
+    const uint64_t number = capturing ? REPLAYED : ++count;
     for (Noted& e : list)
       if (e.tree == tree) {
-        e.last = count;
+        e.last = std::max(e.last, number);
         return;
       }
-    if (tree && list.size() < MAX) list.push_back({tree, count});
-    else any = count;
+    if (tree && list.size() < MAX) list.push_back({tree, number});
+    else any = std::max(any, number);
   }
   bool record(hipStream_t stream, uint64_t tree) {
     Event* to = nullptr;
@@ -269,7 +268,7 @@ struct RunningQueries {
       std::lock_guard<std::mutex> g(mtx);
       for (const Event& e : events)
         if (e.used && e.stream != stream && (!e.tree || e.tree == tree)) RTG_HIP(hipStreamWaitEvent(stream, e.ev, 0));
-      bool must = captured || any != 0;
+      bool must = any != 0;
       for (const Noted& e : list) must = must || e.tree == tree;
       if (!must) return;
       now = count;

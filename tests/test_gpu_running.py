@@ -193,3 +193,29 @@ def test_queries_of_many_scenes(rtc, device, oracle, queue, commits):
         device.free(r.d)
     for sc, _ in scenes:
         sc.release()
+
+
+def test_commit_after_a_replayed_query(rtc, oracle, queue):
+    h, s, fill = queue
+    device = rtc.Device("")
+    v, ix = rtc.gen_soup(20000, seed=9, h=0.05)
+    sc, change = shared_scene(rtc, device, (v, ix), rtc.RTC_BUILD_QUALITY_LOW)
+    r = Records(rtc, device, 0.0, 1.0)
+    want = r.expect(oracle, (v, ix))
+    graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+    assert h.hipStreamBeginCapture(s, 2) == 0  # hipStreamCaptureModeRelaxed
+    rtc.lib().rtcgIntersect1MAsync(sc.h, ctypes.byref(rtc.init_context()), r.d, N, 80, s)
+    assert h.hipStreamEndCapture(s, ctypes.byref(graph)) == 0
+    device.check("capture")
+    assert h.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    fill()
+    assert h.hipGraphLaunch(run, s) == 0
+    assert h.hipStreamQuery(s) == NOT_READY
+    change(np.ascontiguousarray(v[::-1]))
+    assert h.hipStreamSynchronize(s) == 0
+    assert len(mismatches(r.get(), want)) == 0
+    assert h.hipGraphExecDestroy(run) == 0
+    assert h.hipGraphDestroy(graph) == 0
+    device.free(r.d)
+    sc.release()
+    device.release()
